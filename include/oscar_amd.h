@@ -249,6 +249,54 @@ int oscar_prefill_continuation(const float* q_rot, const float* k_new, const flo
                                const int64_t* stage_owner, int32_t stage_rows, float scale,
                                float* out, oscar_stream_t stream);
 
+/* The same read with its work spread over the whole GPU: the row blocks (128
+ * (token, head) rows) and their key blocks are cut into equal shares, and row
+ * blocks that a cut runs through are merged from fp32 partials.  workspace:
+ * device memory of at least oscar_prefill_workspace_bytes(num_new, Hq, Hk,
+ * cached_len) bytes (the new tokens' MFMA operands and the partials); its
+ * contents need no initialisation and mean nothing after the call.
+ */
+size_t oscar_prefill_workspace_bytes(int32_t num_new, int32_t num_heads, int32_t num_kv_heads, int64_t cached_len);
+int oscar_prefill_continuation_split(const float* q_rot, const float* k_new, const float* v_new,
+                                     int32_t num_new, int32_t num_heads, int32_t num_kv_heads,
+                                     int32_t head_size, const void* k_cache, const void* v_cache,
+                                     int32_t block_size, int64_t num_pages, int64_t k_stride_page,
+                                     int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page,
+                                     int64_t v_stride_token, int64_t v_stride_head,
+                                     const int32_t* block_table_row, int32_t block_table_cols,
+                                     int64_t cached_len, const float* stage_k, const float* stage_v,
+                                     const int64_t* stage_owner, int32_t stage_rows, float scale,
+                                     float* out, void* workspace, size_t workspace_size,
+                                     oscar_stream_t stream);
+
+/* The whole read of a step's long requests, bf16 in and out (the reference's
+ * per-request q / k / v rotations, dense read and output rotation,
+ * oscar_ascend/backend.py:361-415): every request in the same launches.
+ *   query_bf16 [tokens][query_token_stride], key_bf16 / value_bf16
+ *     [tokens][kv_token_stride]: the step's activations;
+ *   HOST arrays of num_requests: first_tokens (the request's first new token
+ *     in the step), new_tokens, cached_lens, table_rows (its block-table row);
+ *   rot_k_operand, rot_v_operand, rot_v_t_operand: oscar_rotation_operand of
+ *     R_k, R_v and R_v^T;
+ *   block_table [rows][block_table_stride];
+ *   out_bf16 [tokens][Hq][D]: rows of the requests' tokens are written;
+ *   workspace: at least oscar_prefill_rotated_workspace_bytes bytes.
+ */
+size_t oscar_prefill_rotated_workspace_bytes(int32_t num_requests, const int32_t* new_tokens,
+                                             const int64_t* cached_lens, int32_t num_heads, int32_t num_kv_heads);
+int oscar_prefill_rotated(const void* query_bf16, int64_t query_token_stride, const void* key_bf16,
+                          const void* value_bf16, int64_t kv_token_stride, int32_t num_requests,
+                          const int32_t* first_tokens, const int32_t* new_tokens, const int64_t* cached_lens,
+                          const int32_t* table_rows, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
+                          const void* rot_k_operand, const void* rot_v_operand, const void* rot_v_t_operand,
+                          const void* k_cache, const void* v_cache, int32_t block_size, int64_t num_pages,
+                          int64_t k_stride_page, int64_t k_stride_token, int64_t k_stride_head,
+                          int64_t v_stride_page, int64_t v_stride_token, int64_t v_stride_head,
+                          const int32_t* block_table, int64_t block_table_stride, int32_t block_table_cols,
+                          const float* stage_k, const float* stage_v, const int64_t* stage_owner,
+                          int32_t stage_rows, float scale, void* out_bf16, void* workspace,
+                          size_t workspace_size, oscar_stream_t stream);
+
 /* ---------------------------------------------------------------- step write
  * Everything a short step (num_tokens <= 1024 new tokens, e.g. MTP decode)
  * writes, in one launch: q_rot = query @ R_k, k_rot = key @ R_k, v_rot =

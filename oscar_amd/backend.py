@@ -426,24 +426,20 @@ class OscarAttentionBackendImpl:
                 attn_out[sl] = res
             else:
                 attn_out[idx] = res
-        # bf16 models rotate on MFMA (oscar_rotate_rows: about 2^-16 of each
-        # product, below the fp16 rounding the prefill kernel's operands take
-        # and the bf16 output's); other dtypes keep the fp32 matmuls.
-        mfma_rot = query.dtype == key.dtype == value.dtype == torch.bfloat16
-        _, _, op_k, op_v = layer._oscar_rot_ops
+        # bf16 models rotate on MFMA inside the read (about 2^-16 of each
+        # product, below the fp16 rounding the kernel's operands take and the
+        # bf16 output's); other dtypes keep the fp32 matmuls.
+        if large and query.dtype == key.dtype == value.dtype == torch.bfloat16:
+            _, _, op_k, op_v = layer._oscar_rot_ops
+            prefill.prefill_rotated(q3, k3, v3, [(a, b - a, max(seq - (b - a), 0), i) for i, a, b, seq in large],
+                                    op_k, op_v, layer._oscar_rvT_op, self.key_cache, self.value_cache, bt, self.scale,
+                                    attn_out, stage)
+            return attn_out
         for i, a, b, seq in large:
-            cached = seq - (b - a)
-            if mfma_rot:
-                qr, kr, vr = (quant.rotate_rows(q3[a:b], op_k), quant.rotate_rows(k3[a:b], op_k),
-                              quant.rotate_rows(v3[a:b], op_v))
-            else:
-                qr, kr, vr = q3[a:b].float() @ rk, k3[a:b].float() @ rk, v3[a:b].float() @ rv
-            out_rot = prefill.prefill_continuation(qr, kr, vr, self.key_cache, self.value_cache, bt[i],
-                                                   max(cached, 0), self.scale, stage)
-            if mfma_rot:
-                quant.rotate_rows(out_rot, layer._oscar_rvT_op, torch.bfloat16, out=attn_out[a:b])
-            else:
-                attn_out[a:b] = (out_rot @ rvT).to(query.dtype)
+            out_rot = prefill.prefill_continuation(q3[a:b].float() @ rk, k3[a:b].float() @ rk, v3[a:b].float() @ rv,
+                                                   self.key_cache, self.value_cache, bt[i], max(seq - (b - a), 0),
+                                                   self.scale, stage)
+            attn_out[a:b] = (out_rot @ rvT).to(query.dtype)
         return attn_out
 
 

@@ -1,5 +1,6 @@
-// Prefill continuation: causal attention of N new tokens over C cached INT2
-// tokens plus themselves (gfx950, 16-bit MFMA).
+// Prefill continuation: causal attention of the new tokens of one or more
+// requests over each request's C cached INT2 tokens plus themselves (gfx950,
+// f16 MFMA).
 //
 // Semantics (reference dense path): keys 0 .. C-1 are the dequantized history
 // (owner-matched FP32 staging values override INT2), keys C .. C+N-1 are the
@@ -10,39 +11,88 @@
 // tolerance even on x8 outlier channels.  Accumulation and softmax are fp32.
 // Rotated domain in, rotated-V domain out (fp32).
 //
-// One workgroup per 128 consecutive rows of one kv-head, a row being (new
-// token j, head-in-group); workgroups of later rows (more keys) are
-// dispatched first.  Keys are walked in 32-key blocks through two LDS tile
-// buffers, history blocks first, then new-token blocks.  Waves 4-7 produce:
-// the raw loads of block i + 2 (codes, meta, owner tags, or the new tokens'
-// fp32 values) are in flight while block i + 1's become fp16 K (token-major)
-// and V (feature-major) tiles.  Waves 0-3 consume, 32 rows each: S^T = K Q^T
-// (16 MFMA 32x32x16, two accumulator chains, Q^T from LDS) and O^T += V^T
-// P^T (16 MFMA) with base-2 online softmax and a lazily raised running max.
-// One barrier per block hands a buffer from producers to consumers; a
-// producer wave and a consumer wave share each SIMD, so dequantization
-// overlaps the MFMAs.
-#include "oscar_common.h"
+// Work: a row is (new token j, head in group) of one kv head; a workgroup of
+// eight wavefronts takes 256 consecutive rows (32 per wavefront) and walks
+// their keys in 32-key blocks, history blocks first, then new-token blocks
+// (from the request's first new token).
+//
+// Split (oscar_prefill_* with a workspace): the launch's row blocks, each as
+// long as its key blocks, form one line of units; every workgroup (one per CU)
+// takes an equal share of it, whatever row blocks that cuts.  A row block that
+// lies in one share is finished there; of a cut one each share writes fp32
+// partials (m, l, unnormalised O), which prefill_merge_kernel combines.
+//
+// A block is two phases of a wavefront:
+//   M (matrix): O^T += V^T P^T of block i - 1 and S^T = K Q^T of block i (16
+//     MFMA 32x32x16 each), and under them this wave's part of the tiles K of
+//     block i + 1 and V of block i, built from codes loaded a block ahead
+//     (new-token tiles are copied to LDS as they are, prefill_operands.h);
+//   S (softmax): base-2 online softmax of block i with a lazily raised running
+//     max, in registers.
+// One barrier per block, after S for wavefronts 0-3 and after M for 4-7: in
+// the interval between two barriers the former run M then S, the latter S
+// then M, so that on every SIMD one wave's MFMAs run under the other's
+// softmax.  K and V tiles are double-buffered in LDS (16 KB each); Q^T's first
+// kQReg k-steps stay in registers, the rest in LDS.
+//
+// What bounds it: the operand reads' LDS latency.  A phase M issues its 32
+// MFMAs in 2300 cycles where they need 1024 (timestamps), reads two pairs
+// ahead being what 256 registers hold; S takes 1100-1400.  Without a tile's
+// build, its loads, its exponentials or its PV it is 8-13 % faster each.  Two
+// barriers per block with the wavefronts 4-7 a phase behind (1.19x slower),
+// operand rows that two of sixteen lanes read from one bank slot (LDS active
+// 45 % against 29 % of the time), and workgroups of four wavefronts, two per
+// CU (1.25x slower) were left behind.  One request, 6 heads, D = 256: 9256
+// tokens over 15360 1988 -> 1220 us, 77 over 20011 1016 -> 46 us (+ merge 12),
+// 3001 alone 170 -> 62 us (+ merge 18).
+#include <type_traits>
+#include <utility>
+
+#include "prefill_operands.h"
 #include "../../include/oscar_amd.h"
 
 namespace oscar {
 namespace {
 
-constexpr int kBlk = 32;
+constexpr int kBlk = kKeyBlk;
 constexpr int kRowsPerWave = 32;
-constexpr int kWaves = 4;
-constexpr int kKs = kHeadDim + 8;     // halfs per K row in LDS
-constexpr int kVs = kBlk + 4;         // halfs per V feature row in LDS (72 B: 8-byte reads conflict-free)
-typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+constexpr int kWaves = 8;
+constexpr int kTileRows = kWaves * kRowsPerWave;
+constexpr int kQReg = 4;              // k-steps whose Q^T operand stays in registers
+constexpr int kAhead = 2;             // operand reads ahead of their MFMAs, in pairs
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.f;          // log2 headroom before a running max is raised
 constexpr float kVsMax = 240.f;       // p vs stays below 2^kLazy * 240 < 65504 (fp16) under the lazy max
+constexpr int kPartRows = kTileRows;
+constexpr size_t kPartFloats = (size_t)kPartRows * (kHeadDim + 2);   // O rows, then m, then l
+constexpr int kShares = 256;          // workgroups resident at once: one per CU
+// A piece of a row block costs as much as this many of its key blocks before
+// and after them (page lookup, Q^T, first tile; output or partial): 10-12 us
+// against 2.1 us a block.
+constexpr int kPieceCost = 7;
+constexpr int kMinShare = 10;         // units a share takes at least (see plan_share)
+constexpr int kMergeManyPieces = 6;   // partials a row from which its merge takes four waves
+
+struct PrefillItem {
+  int64_t unit0;       // first unit of the item: kPieceCost, then one per key block, for each row block of
+                       // each kv head
+  int64_t head_units;  // units per kv head
+  int32_t n_new;       // N
+  int32_t cached;      // C
+  int32_t req;         // block-table row
+  int32_t tok0;        // first token in q / k_new / v_new / out (fp32 inputs: of the whole call)
+  int32_t tile0;       // first new-token key tile
+  int32_t rb0;         // first row block of the item (kv heads x row blocks)
+};
 
 struct PrefillArgs {
+  const _Float16* q16;   // operands (prefill_operands.h), or null: the fp32 rows below
+  const float* qsum;
+  const _Float16* kimg;
+  const _Float16* vimg;
   const float* q;        // [N][Hq][D]
   const float* k_new;    // [N][Hk][D]
   const float* v_new;
-  int32_t n_new;
   int32_t num_heads, num_kv_heads, group;
   const uint8_t* k_cache;
   const uint8_t* v_cache;
@@ -51,26 +101,26 @@ struct PrefillArgs {
   FastDiv bs_div;        // block_size
   FastDiv rows_div;      // stage_rows (1 without an arena)
   int64_t num_pages;
-  const int32_t* bt;     // one request's block-table row
+  const int32_t* bt;
+  int64_t bt_stride;
   int32_t bt_cols;
-  int64_t cached;        // C
   const float* stage_k;
   const float* stage_v;
   const int64_t* owner;
   int32_t stage_rows;
   float scale_log2;
   float* out;
+  float* part;           // partial slots (two per share), or null: a workgroup takes a whole row block
+  int64_t share;         // units per workgroup
+  int64_t units;
+  int32_t nitems;
+  PrefillItem items[kMaxPrefillItems];
 };
 
-// Two key blocks of fp16 tiles: block k is computed from one while block
-// k + 1 is written into the other.
 struct PrefillLds {
-  _Float16 kh[2][kBlk * kKs];           // K operand, token-major (features permuted, see below)
-  _Float16 vt[2][kHeadDim * kVs];       // V operand, feature-major
-  float kpar[2][2][kBlk];               // per key: score = ta * (K'.q) + tb * sum(q)   [ta | tb]
-  float vpar[2][2][kBlk];               // per key: v = vs * V' + vz                    [vs | vz]
-  uint32_t big[2][4];                   // a key of the block has vs above kVsMax
-  _Float16 q[kWaves][16 * 2 * kRowsPerWave * 8];   // Q^T operands [wave][m][g][row][8]
+  _Float16 k[2][kKeyTileHalfs];         // K of block i in k[i & 1], V in v[i & 1]
+  _Float16 v[2][kKeyTileHalfs];
+  __attribute__((aligned(16))) _Float16 q[kWaves][16 - kQReg][64 * 8];   // Q^T operands of the k-steps past kQReg
 };
 constexpr size_t kPrefillLds = sizeof(PrefillLds);
 static_assert(kPrefillLds <= 160 * 1024, "LDS of one workgroup");
@@ -78,118 +128,170 @@ static_assert(kPrefillLds <= 160 * 1024, "LDS of one workgroup");
 __device__ __forceinline__ _Float16 to_h(float x) { return (_Float16)x; }
 
 // s_barrier without __syncthreads' memory fence (which would also wait for
-// the producers' outstanding global loads); LDS writes are complete at
-// lgkmcnt(0).
+// the outstanding global loads); LDS writes are complete at lgkmcnt(0).
 __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_s_waitcnt(0xC07F);       // lgkmcnt(0); vmcnt and expcnt left at their maxima
   asm volatile("s_barrier" ::: "memory");
 }
 
-__device__ __forceinline__ void wave_sync_lds() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// ... and with every copy to LDS of this wave complete (vmcnt(0)).
+__device__ __forceinline__ void copy_barrier() {
+  __builtin_amdgcn_s_waitcnt(0x0070);       // vmcnt(0), lgkmcnt(0), expcnt left at its maximum
+  asm volatile("s_barrier" ::: "memory");
 }
 
-// The key blocks a workgroup walks: first the history blocks (keys < C, in
-// 32-key blocks from 0), then the new-token blocks (from the block holding
-// key C).  A block that straddles C is walked twice, each time with the
-// other side's keys masked out.
-struct BlockPlan {
-  int64_t n_hist;     // history blocks
-  int64_t n_new;      // new-token blocks
-  int64_t new0;       // first key of the first new-token block
-};
-
-__device__ __forceinline__ BlockPlan block_plan(int64_t C, int64_t keys) {
-  BlockPlan b;
-  b.n_hist = (C + kBlk - 1) / kBlk;
-  b.new0 = (C / kBlk) * kBlk;
-  b.n_new = keys > C ? (keys - b.new0 + kBlk - 1) / kBlk : 0;
-  return b;
+__device__ __forceinline__ int row_blocks(const PrefillItem& it, int group) {
+  return (int)(((int64_t)it.n_new * group + kTileRows - 1) / kTileRows);
+}
+__device__ __forceinline__ int hist_blocks(const PrefillItem& it) { return (it.cached + kBlk - 1) / kBlk; }
+// Key blocks of row block rb: its last row's token sees new tokens 0 .. that token.
+__device__ __forceinline__ int key_blocks(const PrefillItem& it, int group, int rb) {
+  const int64_t last = min((int64_t)(rb + 1) * kTileRows, (int64_t)it.n_new * group) - 1;
+  return hist_blocks(it) + (int)(last / group) / kBlk + 1;
 }
 
-// Raw loads of one history block for one producer thread: K role (token ktt,
-// features 32 kfg .. +31) k = {codes lo, codes hi, meta, owner}; V role
-// (tokens 8 vtg + w, features 4 vfg .. +3) v[w] = {code byte, V meta, owner}.
-// Every thread issues all 27 loads whatever the block holds (tokens past C
-// and invalid pages read an in-bounds slot, masked later), so a wait counts
-// exactly one block's loads.
-struct HistLoad {
-  u32x4 k;
-  uint32_t vb[8], vm[8], vo[8];
+__device__ __forceinline__ int rb_units(const PrefillItem& it, int group, int rb) {
+  return kPieceCost + key_blocks(it, group, rb);
+}
+
+// Units of the item's row blocks before rb (every lane of the wave calls it
+// with the same rb).
+__device__ int64_t units_before(const PrefillItem& it, int group, int rb, int lane) {
+  int64_t n = 0;
+  for (int b = lane; b < rb; b += 64) n += rb_units(it, group, b);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) n += __shfl_xor(n, o, 64);
+  return n;
+}
+
+// Row block of unit u (relative to the kv head's first), and u within it: a
+// wave-wide scan over 64 row blocks a time.
+__device__ void locate_unit(const PrefillItem& it, int group, int64_t u, int lane, int& rb, int& at_unit) {
+  const int nrb = row_blocks(it, group);
+  for (int base = 0;; base += 64) {
+    const int b = base + lane;
+    const int n = b < nrb ? rb_units(it, group, b) : 0;
+    int64_t incl = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int64_t up = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += up;
+    }
+    const int64_t total = __shfl(incl, 63, 64);
+    if (u < total || base + 64 >= nrb) {
+      const int at = min(__popcll(__ballot(incl <= u)), 63);
+      rb = __builtin_amdgcn_readfirstlane(base + at);
+      at_unit = __builtin_amdgcn_readfirstlane((int)(u - (__shfl(incl, at, 64) - __shfl(n, at, 64))));
+      return;
+    }
+    u -= total;
+  }
+}
+
+// Raw bytes of one history block for one thread of wave w: K role (token 4w +
+// lane / 16, code word lane % 16: features 16 (lane % 16) .. +15) and owner
+// tag of token lane % 32; V role (token 4w + lane % 4, code word lane / 4);
+// meta of the key whose parameters this lane holds (par_key).  Every thread
+// issues its loads whatever the block holds (tokens past C and invalid pages
+// read an in-bounds slot, masked later).
+struct KLoad {
+  uint32_t kc;
+  int32_t own;
 };
 
-// Raw loads of one new-token block: K role k[i] = fp32 values 32 kfg + 4i ..,
-// V role v[w] = fp32 values 4 vfg .. +3 of token 8 vtg + w (16 loads, indices
-// clamped into range, masked later).
-struct NewLoad {
-  floatx4 k[8];
-  floatx4 v[8];
+// Score register q of lane half g is key 8 (q / 4) + 4g + q % 4 of the block:
+// lane q of each 16-lane row of half g holds that key's parameters.
+__device__ __forceinline__ int par_key(int lane) { return 8 * ((lane >> 2) & 3) + 4 * (lane >> 5) + (lane & 3); }
+
+// What the block loop reads every block, per segment (uniform).  The rest of
+// the arguments (the window arena's values) is read where it is needed,
+// through cold_args: kept in registers it spilled others of the loop.
+struct Hot {
+  const uint8_t* kbase;      // this kv head's slots of page 0
+  const uint8_t* vbase;
+  int64_t k_page, v_page;
+  uint32_t ktok, vtok;
+  const int64_t* owner;      // null: no arena
+  const int32_t* bt_row;
+  int32_t num_pages, bt_cols, cached, block_size;
+  FastDiv bs_div, rows_div;
+  float scale_log2;
 };
 
-// Page of the block at key k0 (uniform).  Read through the scalar cache, so
-// that waiting for it never waits for the vector loads in flight.
-__device__ __forceinline__ int32_t block_page(const PrefillArgs& a, int64_t k0) {
-  if (k0 >= a.cached) return -1;
-  const uint32_t pidx = fast_div((uint32_t)k0, a.bs_div);       // key positions stay below 2^31
-  if ((int64_t)pidx >= a.bt_cols) return -1;
+typedef __attribute__((address_space(4))) const PrefillArgs const_args;
+__device__ __forceinline__ const const_args* cold_args() {
+  const const_args* p = (const const_args*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
+// A thread's byte offsets: into a page's slots (ko, vo, mo), of its chunks in
+// the tiles it builds (ks, vs) and of the operands it reads (kr, vr).  The
+// tile offsets differ between chunks by bit flips only (see k_chunk, v_chunk),
+// so one register each serves all of them.
+struct Roles {
+  uint32_t ko, vo, mo;
+  uint32_t ks, vs, kr, vr;
+};
+
+// Keeps a loop-invariant value from being expanded into one register per use.
+__device__ __forceinline__ uint32_t opaque(uint32_t x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+__device__ __forceinline__ Roles make_roles(uint32_t k_tok, uint32_t v_tok, int w, int lane) {
+  Roles r;
+  const int t32 = lane & 31, ktt = 4 * w + (lane >> 4), par = (lane >> 2) & 3;
+  r.ko = (uint32_t)ktt * k_tok + kKCodeOff + 4 * (lane & 15);
+  r.vo = (uint32_t)(4 * w + (lane & 3)) * v_tok + 4 * (lane >> 2);
+  r.mo = (uint32_t)par_key(lane) * k_tok;
+  r.ks = ktt * 512 + 16 * k_chunk(2 * (lane & 15), ktt);
+  // tokens 4w .. 4w + 3 of feature 4 lane + par (see v_slot)
+  r.vs = (4 * lane + par) * 64 + 16 * v_chunk(2 * (w >> 2) + (w & 1), 4 * lane) + 8 * ((w >> 1) & 1);
+  r.kr = t32 * 512 + 16 * ((lane >> 5) ^ (lane & 15));
+  r.vr = t32 * 64 + 16 * v_chunk(lane >> 5, t32);
+  return r;
+}
+
+// Page of the history block at key k0 (uniform).  Read through the scalar
+// cache, so that waiting for it never waits for the vector loads in flight.
+__device__ __forceinline__ int32_t block_page(const Hot& h, int k0) {
+  if (k0 >= h.cached) return -1;
+  const uint32_t pidx = fast_div((uint32_t)k0, h.bs_div);
+  if ((int64_t)pidx >= h.bt_cols) return -1;
   typedef __attribute__((address_space(4))) const int32_t const_i32;
-  return ((const const_i32*)a.bt)[__builtin_amdgcn_readfirstlane(pidx)];
+  return ((const const_i32*)h.bt_row)[__builtin_amdgcn_readfirstlane(pidx)];
 }
+// ... checked where it is used, not where it is requested (which would wait).
+__device__ __forceinline__ int32_t valid_page(const Hot& h, int32_t page) { return page < h.num_pages ? page : -1; }
 
-__device__ __forceinline__ HistLoad load_hist(const PrefillArgs& a, int64_t k0, int32_t page, int kvh, int ktt,
-                                              int kfg, int vtg, int vfg) {
-  HistLoad L;
-  const bool page_ok = page >= 0 && page < a.num_pages;
-  const int64_t pg = page_ok ? page : 0;
-  const uint8_t* kpage = a.k_cache + pg * a.k_page + (int64_t)kvh * a.k_head;
-  const uint8_t* vpage = a.v_cache + pg * a.v_page + (int64_t)kvh * a.v_head;
+__device__ __forceinline__ KLoad load_k(const Hot& h, int k0, int32_t page, const Roles& r, int lane) {
+  KLoad L;
+  const int64_t pg = page >= 0 ? page : 0;
+  const uint32_t prow0 = fast_mod((uint32_t)k0, h.bs_div);
+  const uint8_t* kp = h.kbase + pg * h.k_page + (uint64_t)prow0 * h.ktok;
+  L.kc = *reinterpret_cast<const uint32_t*>(kp + r.ko);
   // Owner tags are pages (< 2^31) or -1: the low word of the little-endian
-  // int64 identifies them.  Without an arena the K slot's meta stands in.
-  const int32_t* opage = a.stage_rows > 0 ? reinterpret_cast<const int32_t*>(
-                                                a.owner + (int64_t)fast_mod((uint32_t)pg, a.rows_div) *
-                                                              a.block_size)
-                                          : reinterpret_cast<const int32_t*>(kpage);
-  const int ostride = a.stage_rows > 0 ? 2 : 0;
-  const int prow0 = (int)fast_mod((uint32_t)k0, a.bs_div);
-  const uint32_t ktok = (uint32_t)a.k_tok, vtok = (uint32_t)a.v_tok;
-  {
-    const int row = prow0 + ktt;
-    const uint8_t* ks = kpage + (uint32_t)row * ktok;
-    const u32x2 cw = *reinterpret_cast<const u32x2*>(ks + kKCodeOff + 8 * kfg);
-    L.k[0] = cw[0];
-    L.k[1] = cw[1];
-    L.k[2] = *reinterpret_cast<const uint32_t*>(ks);
-    L.k[3] = (uint32_t)opage[ostride * row];
-  }
-#pragma unroll
-  for (int w = 0; w < 8; ++w) {
-    const int row = prow0 + 8 * vtg + w;
-    L.vb[w] = vpage[(uint32_t)row * vtok + vfg];
-    L.vm[w] = *reinterpret_cast<const uint32_t*>(kpage + (uint32_t)row * ktok + 4);
-    L.vo[w] = (uint32_t)opage[ostride * row];
-  }
+  // int64 identifies them.  Without an arena the slots' own bytes stand in.
+  const uint8_t* op = h.owner != nullptr
+                          ? reinterpret_cast<const uint8_t*>(
+                                h.owner + (int64_t)fast_mod((uint32_t)pg, h.rows_div) * h.block_size + prow0)
+                          : kp;
+  L.own = *reinterpret_cast<const int32_t*>(op + 8 * (lane & 31));
   return L;
 }
 
-__device__ __forceinline__ NewLoad load_new(const PrefillArgs& a, int64_t k0, int kvh, int ktt, int kfg, int vtg,
-                                            int vfg) {
-  NewLoad L;
-  const int64_t C = a.cached, N = a.n_new;
-  const int64_t hs = (int64_t)a.num_kv_heads * kHeadDim;
-  {
-    const int64_t j = min(max(k0 + ktt - C, (int64_t)0), N - 1);
-    const floatx4* src = reinterpret_cast<const floatx4*>(a.k_new + j * hs + kvh * kHeadDim + 32 * kfg);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) L.k[i] = src[i];
-  }
-#pragma unroll
-  for (int w = 0; w < 8; ++w) {
-    const int64_t j = min(max(k0 + 8 * vtg + w - C, (int64_t)0), N - 1);
-    L.v[w] = *reinterpret_cast<const floatx4*>(a.v_new + j * hs + kvh * kHeadDim + 4 * vfg);
-  }
-  return L;
+__device__ __forceinline__ u32x2 load_meta(const Hot& h, int k0, int32_t page, const Roles& r) {
+  const int64_t pg = page >= 0 ? page : 0;
+  return *reinterpret_cast<const u32x2*>(h.kbase + pg * h.k_page +
+                                         (uint64_t)fast_mod((uint32_t)k0, h.bs_div) * h.ktok + r.mo);
+}
+
+__device__ __forceinline__ uint32_t load_v(const Hot& h, int k0, int32_t page, const Roles& r) {
+  const int64_t pg = page >= 0 ? page : 0;
+  const uint8_t* vp = h.vbase + pg * h.v_page + (uint64_t)fast_mod((uint32_t)k0, h.bs_div) * h.vtok;
+  return *reinterpret_cast<const uint32_t*>(vp + r.vo);
 }
 
 // fp16 pair (1 + c/4) of the codes at bits [sh, sh + 2) and [sh + 16, sh + 18)
@@ -199,43 +301,28 @@ __device__ __forceinline__ uint32_t magic_pair(uint32_t w, int sh) {
   return (x & 0x03000300u) | 0x3C003C00u;
 }
 
-// K tile rows hold each 16-feature group in the order 0, 8, 1, 9, .., 7, 15
-// (position p is feature (p >> 1) + 8 (p & 1)), so that one shift and mask of
-// a code dword yields a pair; the Q^T operand uses the same order.
-__device__ __forceinline__ int k_feature(int p) { return (p >> 1) + 8 * (p & 1); }
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 
-// 16-byte chunk q8 (0..3) of feature group kfg sits at position
-// (q8 + kfg / 2) mod 4 of the group's 64 bytes: the eight threads that write
-// one row store chunk q8 into eight different bank groups at once (unrotated,
-// the eight stores fell into two bank groups; measured C4 2.18 -> 2.08 ms).
-__device__ __forceinline__ int k_chunk_slot(int q8, int kfg) { return (q8 + (kfg >> 1)) & 3; }
-
-// A thread's 32 K values (features 32 kfg .. +31, natural order) into its
-// token's row in the permuted order.
-__device__ __forceinline__ void store_k_values(const float (&kv)[32], int ktt, int kfg, _Float16* kh) {
-  half8* dst = reinterpret_cast<half8*>(kh + ktt * kKs + 32 * kfg);
-#pragma unroll
-  for (int q8 = 0; q8 < 4; ++q8) {
-    half8 x;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = to_h(kv[16 * (q8 >> 1) + k_feature(8 * (q8 & 1) + e)]);
-    dst[k_chunk_slot(q8, kfg)] = x;
-  }
+// A thread's two K chunks and its four V features (feature 4 lane + f holds
+// tokens 4w .. +3) in the tiles.
+__device__ __forceinline__ half8* k_slot(_Float16* kt, uint32_t ks, int e) {
+  return reinterpret_cast<half8*>(reinterpret_cast<uint8_t*>(kt) + (ks ^ (16u * e)));
+}
+// f stands for feature f ^ par of the lane's four, par = (lane / 4) % 4, so
+// that sixteen lanes store into sixteen different 16-byte slots of the banks.
+__device__ __forceinline__ void* v_slot(_Float16* vt, uint32_t vs, int f) {
+  return reinterpret_cast<uint8_t*>(vt) + (vs ^ (64u * f));
 }
 
-// A thread's V values vv[u][w] (feature 4 vfg + u, token 8 vtg + w).
-__device__ __forceinline__ void store_v_values(const float (&vv)[4][8], int vtg, int vfg, _Float16* vt) {
+// A thread's 16 K values (features 16 k16 .. +15, fp32) into its token's row.
+__device__ __forceinline__ void store_k_values(const floatx4* __restrict__ src, uint32_t ks, _Float16* kt) {
+  const floatx4 x[4] = {src[0], src[1], src[2], src[3]};
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    half4 lo, hi;
+  for (int g = 0; g < 2; ++g) {
+    half8 h;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      lo[w] = to_h(vv[u][w]);
-      hi[w] = to_h(vv[u][4 + w]);
-    }
-    half4* d = reinterpret_cast<half4*>(vt + (4 * vfg + u) * kVs + 8 * vtg);
-    d[0] = lo;
-    d[1] = hi;
+    for (int e = 0; e < 8; ++e) h[e] = to_h(x[k_feature(8 * g + e) >> 2][k_feature(8 * g + e) & 3]);
+    *k_slot(kt, ks, g) = h;
   }
 }
 
@@ -247,415 +334,785 @@ __device__ __forceinline__ void store_v_values(const float (&vv)[4][8], int vtg,
 // FP32 values (rounded to fp16) with ta = scale, tb = 0, vs = 1, vz = 0.  Keys
 // past C or on an unmapped page get all-zero parameters (an unmapped page
 // reads as zeros; keys past C are masked by the consumer).
-__device__ __forceinline__ void store_hist(const PrefillArgs& a, const HistLoad& L, int64_t k0, int32_t page,
-                                           int kvh, int ktt, int kfg, int vtg, int vfg, _Float16* kh,
-                                           _Float16* vt, float (&kpar)[2][kBlk], float (&vpar)[2][kBlk],
-                                           uint32_t* big) {
-  const bool page_ok = page >= 0 && page < a.num_pages;
-  const bool arena = a.stage_rows > 0 && page_ok;
-  const int64_t seat0 = arena ? (int64_t)fast_mod((uint32_t)page, a.rows_div) * a.block_size : 0;
-  const int prow0 = (int)fast_mod((uint32_t)k0, a.bs_div);
-  const int64_t C = a.cached;
-  {
-    const bool live = page_ok && k0 + ktt < C;
-    const bool win = arena && live && (int32_t)L.k[3] == page;
-    if (!win) {
-      half8* dst = reinterpret_cast<half8*>(kh + ktt * kKs + 32 * kfg);
+
+// Bits of the block's window-owned tokens; live: live tokens of the block.
+__device__ __forceinline__ uint32_t window_mask(const Hot& h, int32_t own, int live, int32_t page, int lane) {
+  return (uint32_t)__ballot(h.owner != nullptr && (lane & 31) < live && own == page);
+}
+
+__device__ __forceinline__ int live_tokens(const Hot& h, int k0, int32_t page) {
+  return page >= 0 ? h.cached - k0 : 0;
+}
+
+__device__ __forceinline__ const float* stage_row(bool value, int32_t page, int k0, int t, int kvh) {
+  const const_args* a = cold_args();
+  const FastDiv rows{a->rows_div.d, a->rows_div.m, a->rows_div.l}, bs{a->bs_div.d, a->bs_div.m, a->bs_div.l};
+  const int64_t seat = (int64_t)fast_mod((uint32_t)page, rows) * a->block_size + fast_mod((uint32_t)k0, bs) + t;
+  return (value ? a->stage_v : a->stage_k) + (seat * a->num_kv_heads + kvh) * kHeadDim;
+}
+
+// This thread's part of the K tile from its code word: chunk e ...
+__device__ __forceinline__ void build_k(uint32_t w, uint32_t ks, _Float16* kt, int e) {
+  *k_slot(kt, ks, e) = __builtin_bit_cast(half8, u32x4{magic_pair(w, 8 * e), magic_pair(w, 8 * e + 2),
+                                                       magic_pair(w, 8 * e + 4), magic_pair(w, 8 * e + 6)});
+}
+
+// ... and of the V tile: the four tokens' code words of a lane quad, byte
+// transposed (lane j of the quad gets byte j of each), then the codes of its
+// byte's four features as fp16 of the four tokens.
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, 0xF, 0xF, true);
+}
+__device__ __forceinline__ uint32_t quad_transpose(uint32_t x, int lane) {
+  const uint32_t q0 = dpp_u32<0x00>(x), q1 = dpp_u32<0x55>(x), q2 = dpp_u32<0xAA>(x), q3 = dpp_u32<0xFF>(x);
+  const uint32_t sel = 0x0400u + 0x0101u * (uint32_t)(lane & 3);      // byte j of both words
+  const uint32_t lo = __builtin_amdgcn_perm(q1, q0, sel), hi = __builtin_amdgcn_perm(q3, q2, sel);
+  return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+__device__ __forceinline__ void build_v(uint32_t w, uint32_t vs, _Float16* vt, int f) {     // w: quad_transpose
+  const uint32_t y = ((w >> (((vs >> 5) & 6u) ^ (2u * f))) & 0x03030303u) | 0x3C3C3C3Cu;
+  // bytes {0, y.b0, 0, y.b1} and {0, y.b2, 0, y.b3}
+  *reinterpret_cast<u32x2*>(v_slot(vt, vs, f)) =
+      u32x2{__builtin_amdgcn_perm(0u, y, 0x010C000Cu), __builtin_amdgcn_perm(0u, y, 0x030C020Cu)};
+}
+
+// Window-owned tokens (rare), over what the builds above stored: their FP32
+// values rounded to fp16.  (opaque: nothing of this is worth a register in
+// the loop.)
+__device__ __forceinline__ void window_k(uint32_t wmask, int32_t page, int k0, int kvh, const Roles& r, int w,
+                                         int lane_, _Float16* kt) {
+  const int lane = (int)opaque((uint32_t)lane_), t = 4 * w + (lane >> 4);
+  if ((wmask >> t) & 1u)
+    store_k_values(reinterpret_cast<const floatx4*>(stage_row(false, page, k0, t, kvh) + 16 * (lane & 15)),
+                   opaque(r.ks), kt);
+}
+__device__ __forceinline__ void window_v(uint32_t wmask, uint32_t x, int32_t page, int k0, int kvh, const Roles& r,
+                                         int w, int lane_, _Float16* vt) {
+  const uint32_t nib = (wmask >> (4 * w)) & 15u;
+  if (nib == 0u) return;
+  const int lane = (int)opaque((uint32_t)lane_);
+  const uint32_t codes = quad_transpose(x, lane);
+  floatx4 y[4];
 #pragma unroll
-      for (int q8 = 0; q8 < 4; ++q8) {
-        const uint32_t w = L.k[q8 >> 1];
-        const int j0 = 4 * (q8 & 1);
-        dst[k_chunk_slot(q8, kfg)] = __builtin_bit_cast(
-            half8, u32x4{magic_pair(w, 2 * j0), magic_pair(w, 2 * j0 + 2), magic_pair(w, 2 * j0 + 4),
-                         magic_pair(w, 2 * j0 + 6)});
-      }
-    } else {
-      const floatx4* src = reinterpret_cast<const floatx4*>(
-          a.stage_k + ((seat0 + prow0 + ktt) * a.num_kv_heads + kvh) * kHeadDim + 32 * kfg);
-      float kv[32];
+  for (int k = 0; k < 4; ++k) {
+    if ((nib >> k) & 1u)
+      y[k] = *reinterpret_cast<const floatx4*>(stage_row(true, page, k0, 4 * w + k, kvh) + 4 * lane);
+    else
 #pragma unroll
-      for (int q4 = 0; q4 < 8; ++q4) {
-        const floatx4 x = src[q4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) kv[4 * q4 + e] = x[e];
-      }
-      store_k_values(kv, ktt, kfg, kh);
-    }
-    if (kfg == 0) {
-      const float sc = f16_bits_to_f32(L.k[2]), zr = f16_bits_to_f32(L.k[2] >> 16);
-      kpar[0][ktt] = win ? a.scale_log2 : (live ? 4.f * sc * a.scale_log2 : 0.f);
-      kpar[1][ktt] = (win || !live) ? 0.f : (zr - 4.f * sc) * a.scale_log2;
-    }
+      for (int e = 0; e < 4; ++e) y[k][e] = 1.f + 0.25f * (float)((codes >> (8 * k + 2 * e)) & 3u);
   }
-  {
-    uint32_t winmask = 0u, livemask = 0u;
+  const uint32_t vs = opaque(r.vs) ^ (64u * ((lane >> 2) & 3));      // (v_slot's f is then the feature)
 #pragma unroll
-    for (int w = 0; w < 8; ++w) {
-      const bool live = page_ok && k0 + 8 * vtg + w < C;
-      livemask |= live ? 1u << w : 0u;
-      winmask |= (arena && live && (int32_t)L.vo[w] == page) ? 1u << w : 0u;
-    }
-    if (winmask == 0u) {
-      // Code bytes of tokens 8 vtg + 0..3 and + 4..7; per feature u the codes
-      // at bits 2u of each byte become fp16 pairs (1 + c/4) of two tokens.
-      const uint32_t b0 = L.vb[0] | (L.vb[1] << 8) | (L.vb[2] << 16) | (L.vb[3] << 24);
-      const uint32_t b1 = L.vb[4] | (L.vb[5] << 8) | (L.vb[6] << 16) | (L.vb[7] << 24);
+  for (int e = 0; e < 4; ++e)
+    *reinterpret_cast<half4*>(v_slot(vt, vs, e)) = half4{to_h(y[0][e]), to_h(y[1][e]), to_h(y[2][e]), to_h(y[3][e])};
+}
+
+// A value held by lane r of each 16-lane row, in every lane of the row.
+template <int kLane>
+__device__ __forceinline__ float row_bcast(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + kLane, 0xF, 0xF, true));
+}
+// x[r] += y * (c of lane r of the row), r = 0 .. 15, and z += sum_r p[r] * (c of
+// lane r): fused multiply-adds that take the broadcast as they read it (the
+// compiler folds it into multiplies only and spends a move per broadcast
+// otherwise).  The two wait states are those a DPP read needs after a VALU
+// write of its source, which the compiler cannot see inside.
+#define OSCAR_FMAC(dst, c, y, r) "v_fmac_f32_dpp " dst ", " c ", " y " row_newbcast:" #r " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void fmac_bcast(float (&x)[16], float c, float y) {
+  asm("s_nop 1\n\t"
+      OSCAR_FMAC("%0", "%16", "%17", 0) OSCAR_FMAC("%1", "%16", "%17", 1) OSCAR_FMAC("%2", "%16", "%17", 2)
+      OSCAR_FMAC("%3", "%16", "%17", 3) OSCAR_FMAC("%4", "%16", "%17", 4) OSCAR_FMAC("%5", "%16", "%17", 5)
+      OSCAR_FMAC("%6", "%16", "%17", 6) OSCAR_FMAC("%7", "%16", "%17", 7) OSCAR_FMAC("%8", "%16", "%17", 8)
+      OSCAR_FMAC("%9", "%16", "%17", 9) OSCAR_FMAC("%10", "%16", "%17", 10) OSCAR_FMAC("%11", "%16", "%17", 11)
+      OSCAR_FMAC("%12", "%16", "%17", 12) OSCAR_FMAC("%13", "%16", "%17", 13) OSCAR_FMAC("%14", "%16", "%17", 14)
+      OSCAR_FMAC("%15", "%16", "%17", 15)
+      : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]),
+        "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]), "+v"(x[14]), "+v"(x[15])
+      : "v"(c), "v"(y));
+}
+__device__ __forceinline__ float dot_bcast(const float (&p)[16], float c, float z) {
+  asm("s_nop 1\n\t"
+      OSCAR_FMAC("%0", "%1", "%2", 0) OSCAR_FMAC("%0", "%1", "%3", 1) OSCAR_FMAC("%0", "%1", "%4", 2)
+      OSCAR_FMAC("%0", "%1", "%5", 3) OSCAR_FMAC("%0", "%1", "%6", 4) OSCAR_FMAC("%0", "%1", "%7", 5)
+      OSCAR_FMAC("%0", "%1", "%8", 6) OSCAR_FMAC("%0", "%1", "%9", 7) OSCAR_FMAC("%0", "%1", "%10", 8)
+      OSCAR_FMAC("%0", "%1", "%11", 9) OSCAR_FMAC("%0", "%1", "%12", 10) OSCAR_FMAC("%0", "%1", "%13", 11)
+      OSCAR_FMAC("%0", "%1", "%14", 12) OSCAR_FMAC("%0", "%1", "%15", 13) OSCAR_FMAC("%0", "%1", "%16", 14)
+      OSCAR_FMAC("%0", "%1", "%17", 15)
+      : "+v"(z)
+      : "v"(c), "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]), "v"(p[8]),
+        "v"(p[9]), "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
+  return z;
+}
+#undef OSCAR_FMAC
+template <typename F, int... kI>
+__device__ __forceinline__ void each16(F&& f, std::integer_sequence<int, kI...>) {
+  (f(std::integral_constant<int, kI>{}), ...);
+}
+
+// New-token tiles copied as they are: kCopyWaves waves take equal parts.
+typedef __attribute__((address_space(3))) void lds_void;
+template <int kCopyWaves>
+__device__ __forceinline__ void copy_tile(const _Float16* img, int64_t tile, _Float16* lds, int wave, int lane) {
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(img + tile * kKeyTileHalfs), (short)0, (int)(kKeyTileHalfs * sizeof(_Float16)), 0x00020000);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const uint32_t y0 = ((b0 >> (2 * u)) & 0x03030303u) | 0x3C3C3C3Cu;
-        const uint32_t y1 = ((b1 >> (2 * u)) & 0x03030303u) | 0x3C3C3C3Cu;
-        // bytes {0, y.b0, 0, y.b1} and {0, y.b2, 0, y.b3}
-        const u32x2 lo{__builtin_amdgcn_perm(0u, y0, 0x010C000Cu), __builtin_amdgcn_perm(0u, y0, 0x030C020Cu)};
-        const u32x2 hi{__builtin_amdgcn_perm(0u, y1, 0x010C000Cu), __builtin_amdgcn_perm(0u, y1, 0x030C020Cu)};
-        u32x2* d = reinterpret_cast<u32x2*>(vt + (4 * vfg + u) * kVs + 8 * vtg);
-        d[0] = lo;
-        d[1] = hi;
-      }
-    } else {
-      float vv[4][8];
-#pragma unroll
-      for (int w = 0; w < 8; ++w) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) vv[u][w] = 1.f + 0.25f * (float)((L.vb[w] >> (2 * u)) & 3u);
-        if ((winmask >> w) & 1u) {
-          const floatx4 y = *reinterpret_cast<const floatx4*>(
-              a.stage_v + ((seat0 + prow0 + 8 * vtg + w) * a.num_kv_heads + kvh) * kHeadDim + 4 * vfg);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) vv[u][w] = y[u];
-        }
-      }
-      store_v_values(vv, vtg, vfg, vt);
-    }
-    if (vfg == 0) {
-      bool bg = false;
-#pragma unroll
-      for (int w = 0; w < 8; ++w) {
-        const float sc = f16_bits_to_f32(L.vm[w]), zr = f16_bits_to_f32(L.vm[w] >> 16);
-        const bool live = (livemask >> w) & 1u, win = (winmask >> w) & 1u;
-        vpar[0][8 * vtg + w] = win ? 1.f : (live ? 4.f * sc : 0.f);
-        vpar[1][8 * vtg + w] = (win || !live) ? 0.f : zr - 4.f * sc;
-        bg = bg || (live && !win && 4.f * sc > kVsMax);
-      }
-      big[vtg] = bg ? 1u : 0u;
-    }
+  for (int i = 0; i < 16 / kCopyWaves; ++i) {
+    const int blk = 16 / kCopyWaves * wave + i;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void*)(lds + blk * 512), 16, (blk * 64 + lane) * 16, 0, 0, 0);
   }
 }
 
-// New-token tiles: the fp32 values rounded to fp16, ta = scale, tb = 0,
-// vs = 1, vz = 0.
-__device__ __forceinline__ void store_new(const PrefillArgs& a, const NewLoad& L, int ktt, int kfg, int vtg, int vfg,
-                                          _Float16* kh, _Float16* vt, float (&kpar)[2][kBlk],
-                                          float (&vpar)[2][kBlk], uint32_t* big) {
-  float kv[32];
-  float vv[4][8];
+// ... or, for callers without operands, rounded from the fp32 rows.
+__device__ __forceinline__ void store_new_k(const PrefillArgs& a, const PrefillItem& it, int j0, int kvh,
+                                            const Roles& r, int w, int lane, _Float16* kt) {
+  const int j = min(j0 + 4 * w + (lane >> 4), it.n_new - 1);
+  store_k_values(reinterpret_cast<const floatx4*>(a.k_new + ((int64_t)(it.tok0 + j) * a.num_kv_heads + kvh) * kHeadDim +
+                                                  16 * (lane & 15)),
+                 r.ks, kt);
+}
+__device__ __forceinline__ void store_new_v(const PrefillArgs& a, const PrefillItem& it, int j0, int kvh,
+                                            const Roles& r, int w, int lane, _Float16* vt) {
+  const uint32_t vs = r.vs ^ (64u * ((lane >> 2) & 3));
+  floatx4 x[4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) kv[4 * i + e] = L.k[i][e];
-#pragma unroll
-  for (int w = 0; w < 8; ++w)
-#pragma unroll
-    for (int u = 0; u < 4; ++u) vv[u][w] = L.v[w][u];
-  store_k_values(kv, ktt, kfg, kh);
-  store_v_values(vv, vtg, vfg, vt);
-  if (kfg == 0) {
-    kpar[0][ktt] = a.scale_log2;
-    kpar[1][ktt] = 0.f;
+  for (int k = 0; k < 4; ++k) {
+    const int j = min(j0 + 4 * w + k, it.n_new - 1);
+    x[k] = *reinterpret_cast<const floatx4*>(
+        a.v_new + ((int64_t)(it.tok0 + j) * a.num_kv_heads + kvh) * kHeadDim + 4 * lane);
   }
-  if (vfg == 0) {
 #pragma unroll
-    for (int w = 0; w < 8; ++w) {
-      vpar[0][8 * vtg + w] = 1.f;
-      vpar[1][8 * vtg + w] = 0.f;
-    }
-    big[vtg] = 0u;
-  }
+  for (int e = 0; e < 4; ++e)
+    *reinterpret_cast<half4*>(v_slot(vt, vs, e)) = half4{to_h(x[0][e]), to_h(x[1][e]), to_h(x[2][e]), to_h(x[3][e])};
 }
 
-// 8 wavefronts: waves 0-3 compute (32 rows each), waves 4-7 produce the
-// fp16 tiles of the next key block, two blocks of loads ahead.
-__global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs a) {
+template <bool kImages>
+__global__ __launch_bounds__(512, 2) void prefill_kernel(PrefillArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem_raw[];
   PrefillLds& S = *reinterpret_cast<PrefillLds*>(smem_raw);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool producer = wave >= kWaves;
   const int g = lane >> 5;
   const int col = lane & 31;
-  const int kvh = blockIdx.y;
-  const int64_t rows_total = (int64_t)a.n_new * a.group;
-  // Blocks of later rows see more keys: they are dispatched first.
-  const int64_t row0 = (int64_t)(gridDim.x - 1 - blockIdx.x) * (kWaves * kRowsPerWave);
-  const int64_t C = a.cached;
-  const int64_t last_row = min(row0 + kWaves * kRowsPerWave, rows_total) - 1;
-  const int64_t keys_blk = C + last_row / a.group + 1;
-  const BlockPlan plan = block_plan(C, keys_blk);
-  const int64_t nblk = plan.n_hist + plan.n_new;
-  auto block_k0 = [&](int64_t i) { return i < plan.n_hist ? i * kBlk : plan.new0 + (i - plan.n_hist) * kBlk; };
+  const bool second = wave >= kWaves / 2;     // its barrier comes between M and S
+  const Roles r = make_roles((uint32_t)a.k_tok, (uint32_t)a.v_tok, wave, lane);
 
-  if (producer) {
-    const int ptid = tid - kWaves * 64;
-    const int ktt = ptid >> 3, kfg = ptid & 7;       // K: token ktt, features 32*kfg .. +31
-    const int vtg = ptid >> 6, vfg = ptid & 63;      // V: tokens 8*vtg .. +7, features 4*vfg .. +3
-    // History pass: loads of block i + 2 out while block i + 1's are turned
-    // into tiles; then the same for the new-token pass.  The loop is unrolled
-    // twice so that the two load sets alternate in place: a load never lands
-    // in registers that still have to be copied, and each wait counts one
-    // block's loads.
-    const int64_t nh = plan.n_hist;
-    int64_t i = 0;
-    if (nh > 0) {
-      int32_t pg_a = block_page(a, 0), pg_b = block_page(a, kBlk);
-      HistLoad La = load_hist(a, 0, pg_a, kvh, ktt, kfg, vtg, vfg);
-      HistLoad Lb = load_hist(a, kBlk, pg_b, kvh, ktt, kfg, vtg, vfg);
-      int32_t pg_c = block_page(a, 2 * kBlk);
-      // top of the loop: La holds block i (page pg_a), Lb block i + 1 (pg_b),
-      // pg_c is block i + 2's page
-#pragma unroll 1
-      for (;;) {
-        store_hist(a, La, i * kBlk, pg_a, kvh, ktt, kfg, vtg, vfg, S.kh[i & 1], S.vt[i & 1], S.kpar[i & 1],
-                   S.vpar[i & 1], S.big[i & 1]);
-        const int32_t pg_d = block_page(a, (i + 3) * kBlk);
-        La = load_hist(a, (i + 2) * kBlk, pg_c, kvh, ktt, kfg, vtg, vfg);
-        pg_a = pg_c;
-        lds_barrier();        // tiles of block i ready / block i - 1 consumed
-        if (++i == nh) break;
-        store_hist(a, Lb, i * kBlk, pg_b, kvh, ktt, kfg, vtg, vfg, S.kh[i & 1], S.vt[i & 1], S.kpar[i & 1],
-                   S.vpar[i & 1], S.big[i & 1]);
-        pg_c = block_page(a, (i + 3) * kBlk);
-        Lb = load_hist(a, (i + 2) * kBlk, pg_d, kvh, ktt, kfg, vtg, vfg);
-        pg_b = pg_d;
-        lds_barrier();
-        if (++i == nh) break;
-      }
-    }
-    if (plan.n_new > 0) {
-      NewLoad La = load_new(a, plan.new0, kvh, ktt, kfg, vtg, vfg);
-      NewLoad Lb = load_new(a, plan.new0 + kBlk, kvh, ktt, kfg, vtg, vfg);
-#pragma unroll 1
-      for (;;) {
-        store_new(a, La, ktt, kfg, vtg, vfg, S.kh[i & 1], S.vt[i & 1], S.kpar[i & 1], S.vpar[i & 1],
-                  S.big[i & 1]);
-        La = load_new(a, block_k0(i) + 2 * kBlk, kvh, ktt, kfg, vtg, vfg);
-        lds_barrier();
-        if (++i == nblk) break;
-        store_new(a, Lb, ktt, kfg, vtg, vfg, S.kh[i & 1], S.vt[i & 1], S.kpar[i & 1], S.vpar[i & 1],
-                  S.big[i & 1]);
-        Lb = load_new(a, block_k0(i) + 2 * kBlk, kvh, ktt, kfg, vtg, vfg);
-        lds_barrier();
-        if (++i == nblk) break;
-      }
-    }
-    lds_barrier();            // the consumers' last block
-    return;
+  // ---- the workgroup's units [u, u1) ----
+  int64_t u, u1;
+  int item = 0, kvh, rb, ub;            // ub: u within row block rb
+  if (a.part == nullptr) {
+    // whole row blocks of one request, later ones (more keys) first
+    const int nrb = row_blocks(a.items[0], a.group);
+    kvh = (int)blockIdx.y;
+    rb = nrb - 1 - (int)blockIdx.x;
+    ub = 0;
+    u = 0;
+    u1 = rb_units(a.items[0], a.group, rb);
+  } else {
+    u = (int64_t)blockIdx.x * a.share;
+    u1 = min(u + a.share, a.units);
+    while (item + 1 < a.nitems && a.items[item + 1].unit0 <= u) ++item;
+    const int64_t rel = u - a.items[item].unit0;
+    kvh = (int)(rel / a.items[item].head_units);
+    locate_unit(a.items[item], a.group, rel - (int64_t)kvh * a.items[item].head_units, lane, rb, ub);
   }
 
-  // ---- consumers: 32 rows per wave ----
-  const int64_t wrow0 = row0 + wave * kRowsPerWave;
-  const int64_t row = wrow0 + col;
-  const bool row_ok = row < rows_total;
-  const int64_t wave_last = min(wrow0 + kRowsPerWave, rows_total) - 1;
-  const int64_t keys_wave = wrow0 < rows_total ? C + wave_last / a.group + 1 : 0;
-  const int64_t my_limit = row_ok ? C + row / a.group : -1;   // last visible key
-  // Keys every row of the wave sees (all rows in range): history keys
-  // 0 .. C - 1 in the history pass, C .. C + wrow0 / group in the new pass.
-  const bool wave_full = wrow0 + kRowsPerWave <= rows_total;
-  const int32_t full_hi_new = (int32_t)(C + wrow0 / a.group);
-  auto lo_wave = [&](bool hist) { return hist ? 0 : (int32_t)C; };
-  auto hi_wave = [&](bool hist) {
-    return wave_full ? (hist ? (int32_t)C - 1 : full_hi_new) : (int32_t)-1;
-  };
-  // Offsets (halves) of a K operand chunk for this lane's g: + 8g, or - 24g
-  // where the rotated slot wraps from 3 to 0.
-  const int kstep = 8 * g, kwrap = -24 * g;
-  float qsum;
-  {
-    // Q^T operands of the wave's rows in the K tiles' feature order: lane
-    // (row col, half g) holds positions 8g .. 8g + 7 of k-step m, i.e.
-    // features 16m + 4g + {0, 8, 1, 9, 2, 10, 3, 11}.  qsum: the row's sum of
-    // the fp16 values.
-    const int64_t j = row_ok ? row / a.group : 0;
-    const int h = kvh * a.group + (row_ok ? (int)(row % a.group) : 0);
-    const float* qp = a.q + (j * a.num_heads + h) * kHeadDim + 4 * g;
-    _Float16* qdst = S.q[wave] + (g * kRowsPerWave + col) * 8;
-    float qs = 0.f;
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      const floatx4 x0 = row_ok ? *reinterpret_cast<const floatx4*>(qp + 16 * m) : floatx4{};
-      const floatx4 x1 = row_ok ? *reinterpret_cast<const floatx4*>(qp + 16 * m + 8) : floatx4{};
-      const half8 v = half8{to_h(x0[0]), to_h(x1[0]), to_h(x0[1]), to_h(x1[1]),
-                            to_h(x0[2]), to_h(x1[2]), to_h(x0[3]), to_h(x1[3])};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) qs += (float)v[e];
-      *reinterpret_cast<half8*>(qdst + m * 2 * kRowsPerWave * 8) = v;
-    }
-    qsum = qs + shfl_xor_f32(qs, 32);
-  }
-  wave_sync_lds();
-
-  floatx16 acc[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) acc[t] = floatx16{};
-  float m_run = -__builtin_inff();
-  float l_run = 0.f, z_run = 0.f;     // this lane's keys' sums of p and p vz
-
 #pragma unroll 1
-  for (int64_t i = 0; i < nblk; ++i) {
-    lds_barrier();            // tiles of block i ready
-    const int64_t k0 = block_k0(i);
-    const bool hist = i < plan.n_hist;
-    if (k0 < keys_wave) {
-      const _Float16* kh = S.kh[i & 1];
-      const _Float16* vt = S.vt[i & 1];
-      const _Float16* krow = kh + col * kKs;
-      const half8* qsrc = reinterpret_cast<const half8*>(S.q[wave] + (g * kRowsPerWave + col) * 8);
-      // K operand of k-step m: chunk 2m + g of the row (feature group m / 2,
-      // chunk 2 (m % 2) + g), at its rotated slot; the lane's g enters as one
-      // of two per-lane offsets (with or without the wrap of the slot).
-      auto kchunk = [&](int m) {
-        const int c0 = (2 * (m & 1) + (m >> 2)) & 3;          // slot for g = 0
-        return *reinterpret_cast<const half8*>(krow + 8 * (4 * (m >> 1) + c0) + (c0 == 3 ? kwrap : kstep));
-      };
-      floatx16 s0 = floatx16{}, s1 = floatx16{};
-#pragma unroll
-      for (int m = 0; m < 16; m += 2) {
-        const half8 ka = kchunk(m);
-        const half8 kb2 = kchunk(m + 1);
-        s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qsrc[m * 2 * kRowsPerWave], s0, 0, 0, 0);
-        s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kb2, qsrc[(m + 1) * 2 * kRowsPerWave], s1, 0, 0, 0);
+  while (u < u1) {
+    const PrefillItem it = a.items[item];
+    // this piece: units ub .. ub + take - 1 of the row block, key blocks kb .. kend - 1
+    const int nblk = key_blocks(it, a.group, rb);
+    const int take = (int)min((int64_t)(kPieceCost + nblk - ub), u1 - u);
+    const int kb = max(ub - kPieceCost, 0), kend = ub + take - kPieceCost;
+    const int64_t start = u + max(kPieceCost - ub, 0);    // unit of key block kb
+    u += take;
+    const int rb_now = rb, kvh_now = kvh;
+    const bool rb_done = kend == nblk;
+    ub = 0;
+    if (rb_done && ++rb == row_blocks(it, a.group)) {
+      rb = 0;
+      if (++kvh == a.num_kv_heads) {
+        kvh = 0;
+        ++item;
       }
-      floatx16 s = s0 + s1;
-      // Visible keys of this pass: history keys < C in the history pass, new
-      // keys >= C in the new-token pass, causal for both.  A block every row
-      // of the wave sees whole skips the per-key test.
-      const int32_t lo = hist ? 0 : (int32_t)C;
-      const int32_t hi = hist ? (int32_t)min(C - 1, my_limit) : (int32_t)my_limit;
-      const bool whole = (int32_t)k0 >= lo_wave(hist) && (int32_t)k0 + kBlk - 1 <= hi_wave(hist);
-      // key 8 jj + 4g + i of the block is register 4 jj + i
-      const float* kpar0 = S.kpar[i & 1][0] + 4 * g;
-      const float* kpar1 = S.kpar[i & 1][1] + 4 * g;
+    }
+    if (kend <= kb) continue;             // the share ends before the row block's first key block
+    const int nh = hist_blocks(it);
+    const int rows_total = it.n_new * a.group;
+    const int row0 = rb_now * kTileRows;
+    const int wrow0 = row0 + wave * kRowsPerWave;
+    const bool wave_on = wrow0 < rows_total;
+    const int row = wrow0 + col;
+    const int rowc = min(row, rows_total - 1);
+    const int my_tok = rowc / a.group;                    // sees new tokens 0 .. my_tok
+    const int head = kvh_now * a.group + (rowc - my_tok * a.group);
+    const int first_tok = min(wrow0, rows_total - 1) / a.group;              // of the wave's rows
+    const int last_tok = (min(wrow0 + kRowsPerWave, rows_total) - 1) / a.group;
+
+    const Hot h{a.k_cache + (int64_t)kvh_now * a.k_head, a.v_cache + (int64_t)kvh_now * a.v_head, a.k_page, a.v_page,
+                (uint32_t)a.k_tok, (uint32_t)a.v_tok, a.stage_rows > 0 ? a.owner : nullptr,
+                a.bt + (int64_t)it.req * a.bt_stride, (int32_t)min(a.num_pages, (int64_t)INT32_MAX), a.bt_cols,
+                it.cached, a.block_size, a.bs_div, a.rows_div, a.scale_log2};
+
+    // ---- first blocks' loads, then the wave's Q^T operands.  In phase M of
+    // block i: lk holds block i + 1's words, lv block i's; pages p0 .. p2 are
+    // those of blocks i .. i + 2; meta (and cur) are block i's in phase S. ----
+    struct Block {
+      uint32_t win;       // window-owned tokens
+      int live;           // tokens in the history, from the first
+    };
+    KLoad lk{};
+    u32x2 meta{};
+    uint32_t lv = 0;
+    Block cur{0u, 0}, next{0u, 0};
+    int32_t p0 = -1, p1 = -1, p2 = -1;
+    if (kb < nh) {
+      p1 = valid_page(h, block_page(h, kb * kBlk));
+      lk = load_k(h, kb * kBlk, p1, r, lane);
+      lv = load_v(h, kb * kBlk, p1, r);
+      meta = load_meta(h, kb * kBlk, p1, r);
+      p2 = block_page(h, (kb + 1) * kBlk);
+    }
+    half8 qreg[kQReg];
+    float qsum;
+    if constexpr (kImages) {
+      const int64_t qrow = (int64_t)(it.tok0 + my_tok) * a.num_heads + head;
+      const half8* qp = reinterpret_cast<const half8*>(a.q16 + qrow * kHeadDim) + g;
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const floatx4 ta = *reinterpret_cast<const floatx4*>(kpar0 + 8 * jj);
-        const floatx4 tb = *reinterpret_cast<const floatx4*>(kpar1 + 8 * jj);
+      for (int m = 0; m < kQReg; ++m) qreg[m] = qp[2 * m];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[4 * jj + e] = fmaf(ta[e], s[4 * jj + e], tb[e] * qsum);
+      for (int m = kQReg; m < 16; ++m) *reinterpret_cast<half8*>(&S.q[wave][m - kQReg][lane * 8]) = qp[2 * m];
+      qsum = a.qsum[qrow];
+    } else {
+      const float* qp = a.q + ((int64_t)(it.tok0 + my_tok) * a.num_heads + head) * kHeadDim + 4 * g;
+      float qs = 0.f;
+#pragma unroll
+      for (int m = 0; m < 16; ++m) {
+        const floatx4 x0 = *reinterpret_cast<const floatx4*>(qp + 16 * m);
+        const floatx4 x1 = *reinterpret_cast<const floatx4*>(qp + 16 * m + 8);
+        const half8 v = half8{to_h(x0[0]), to_h(x1[0]), to_h(x0[1]), to_h(x1[1]),
+                              to_h(x0[2]), to_h(x1[2]), to_h(x0[3]), to_h(x1[3])};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qs += (float)v[e];
+        if (m < kQReg) qreg[m < kQReg ? m : 0] = v;
+        else *reinterpret_cast<half8*>(&S.q[wave][m < kQReg ? 0 : m - kQReg][lane * 8]) = v;
       }
-      float mb = -__builtin_inff();
-      if (whole) {
+      qsum = qs + shfl_xor_f32(qs, 32);
+    }
+
+    // the loop's waits must not count the loads above
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mb = fmaxf(mb, s[r]);
+    for (int m = 0; m < kQReg; ++m) asm volatile("" ::"v"(qreg[m]));
+    asm volatile("" ::"v"(qsum));
+
+    floatx16 acc[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[t] = floatx16{};
+    // Scores are taken relative to m_base, the row's lazily raised maximum (0
+    // until the row has seen a key); raise: what a block's maximum has to
+    // exceed to raise it.
+    float m_base = 0.f, raise = -__builtin_inff();
+    float l_run = 0.f, z_run = 0.f;     // this lane's keys' sums of p and p vz
+
+    // K tile of block i (its words in lk, page p1) and V tile of block i (its
+    // words in lv, page p0), with their window tokens.
+    auto tile_k = [&](int i) { return S.k[i & 1]; };
+    auto tile_v = [&](int i) { return S.v[i & 1]; };
+    auto block_of = [&](int i) {
+      const int live = live_tokens(h, i * kBlk, p1);
+      return Block{window_mask(h, lk.own, live, p1, lane), live};
+    };
+    auto hist_k = [&](int i) {
+      next = block_of(i);
+      const uint32_t ks = opaque(r.ks);
+      build_k(lk.kc, ks, tile_k(i), 0);
+      build_k(lk.kc, ks, tile_k(i), 1);
+      if (next.win != 0u) window_k(next.win, p1, i * kBlk, kvh_now, r, wave, lane, tile_k(i));
+    };
+    auto hist_v = [&](int i) {
+      const uint32_t vs = opaque(r.vs), w = quad_transpose(lv, lane);
+#pragma unroll
+      for (int f = 0; f < 4; ++f) build_v(w, vs, tile_v(i), f);
+      if (cur.win != 0u) window_v(cur.win, lv, p0, i * kBlk, kvh_now, r, wave, lane, tile_v(i));
+    };
+    auto new_k = [&](int i, auto copy_waves) {
+      constexpr int kCw = decltype(copy_waves)::value;
+      if constexpr (kImages) {
+        if (wave < kCw) copy_tile<kCw>(a.kimg, (int64_t)(it.tile0 + i - nh) * a.num_kv_heads + kvh_now, tile_k(i), wave, lane);
       } else {
+        store_new_k(a, it, (i - nh) * kBlk, kvh_now, r, wave, lane, tile_k(i));
+      }
+    };
+    auto new_v = [&](int i) {
+      if constexpr (kImages) {
+        if (!second) copy_tile<4>(a.vimg, (int64_t)(it.tile0 + i - nh) * a.num_kv_heads + kvh_now, tile_v(i), wave, lane);
+      } else {
+        store_new_v(a, it, (i - nh) * kBlk, kvh_now, r, wave, lane, tile_v(i));
+      }
+    };
+    // The words of block i + 1's V and block i + 2's K, while those exist.
+    auto load_next = [&](int i) {
+      p0 = p1;
+      p1 = valid_page(h, p2);
+      if (i + 1 < min(kend, nh)) lv = load_v(h, (i + 1) * kBlk, p0, r);
+      if (i + 2 < min(kend, nh)) {
+        lk = load_k(h, (i + 2) * kBlk, p1, r, lane);
+        p2 = block_page(h, (i + 3) * kBlk);
+      }
+    };
+    // Blocks before kseen are seen by a row of the wave.
+    const int kseen = !wave_on ? kb : min(kend, nh + last_tok / kBlk + 1);
+
+    floatx16 s;
+    half8 pb[2] = {half8{}, half8{}};
+
+    // ---- phase M: O^T += V^T P^T of block i - 1 (zero weights before the
+    // first block) and, with kQk, S^T = K Q^T of block i, MFMA by MFMA in
+    // turn, operand reads kAhead pairs ahead ----
+    auto matrix = [&](int i, auto qk_tag, auto&& piece) {
+      constexpr bool kQk = decltype(qk_tag)::value;
+      const uint32_t kr = opaque(r.kr), vr = opaque(r.vr);
+      const uint8_t* qb =
+          reinterpret_cast<const uint8_t*>(S.q) + opaque((uint32_t)(wave * (int)sizeof(S.q[0]) + 16 * lane));
+      const uint8_t* kt = reinterpret_cast<const uint8_t*>(tile_k(i));
+      const uint8_t* vt = reinterpret_cast<const uint8_t*>(tile_v(i - 1));
+      auto read_k = [&](int m) {
+        return *reinterpret_cast<const half8*>(kt + (kr ^ (16u * ((2 * m & 14) ^ (m >> 3)))) + 256 * (m >> 3));
+      };
+      // k-steps with Q^T in LDS first, then those in registers
+      auto read_q = [&](int m) { return *reinterpret_cast<const half8*>(qb + 1024 * (m - kQReg)); };
+      auto order = [](int n) { return n < 16 - kQReg ? n + kQReg : n - (16 - kQReg); };
+      // feature block n & 7 of PV k-step n >> 3
+      auto read_v = [&](int n) {
+        return *reinterpret_cast<const half8*>(vt + (vr ^ (32u * (n >> 3))) + 2048 * (n & 7));
+      };
+      half8 ka[kAhead], qa[kAhead], va[kAhead];
+      if constexpr (kQk) s = floatx16{};
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int32_t kp = (int32_t)k0 + 8 * (r >> 2) + 4 * g + (r & 3);
-          const float x = (kp >= lo && kp <= hi) ? s[r] : -__builtin_inff();
-          s[r] = x;
-          mb = fmaxf(mb, x);
+      for (int n = 0; n < kAhead; ++n) {
+        va[n] = read_v(n);
+        if constexpr (kQk) {
+          ka[n] = read_k(order(n));
+          qa[n] = read_q(order(n));
         }
       }
-      mb = fmaxf(mb, shfl_xor_f32(mb, 32));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < 16; ++n) {
+        // (the order below is the schedule: the compiler's own hoists the
+        // operand reads and spills)
+        const int nn = n + kAhead;
+        acc[n & 7] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[n % kAhead], pb[n >> 3], acc[n & 7], 0, 0, 0);
+        if (nn < 16) va[n % kAhead] = read_v(nn);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kQk) {
+          s = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+              ka[n % kAhead], order(n) < kQReg ? qreg[order(n) < kQReg ? order(n) : 0] : qa[n % kAhead], s, 0, 0, 0);
+          if (nn < 16) {
+            ka[n % kAhead] = read_k(order(nn));
+            if (order(nn) >= kQReg) qa[n % kAhead] = read_q(order(nn));
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        piece(n);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    auto nothing = [](int) {};
+
+    // ---- phase S: softmax of block i ----
+    auto softmax = [&](int i, bool hist) {
+      // This lane's key's parameters: score = par[0] (K'.q) + par[1] sum(q),
+      // v = par[2] V' + par[3]; eager: some key has vs above kVsMax.
+      floatx4 par{h.scale_log2, 0.f, 1.f, 0.f};
+      bool eager = false;
+      if (hist) {
+        const int key = par_key(lane);
+        const bool lv_ = key < cur.live, code = lv_ && ((cur.win >> key) & 1u) == 0u;
+        const float ks = 4.f * f16_bits_to_f32(meta[0]), kz = f16_bits_to_f32(meta[0] >> 16);
+        const float vs = 4.f * f16_bits_to_f32(meta[1]), vz = f16_bits_to_f32(meta[1] >> 16);
+        par[0] = code ? ks * h.scale_log2 : (lv_ ? h.scale_log2 : 0.f);
+        par[1] = code ? (kz - ks) * h.scale_log2 : 0.f;
+        par[2] = code ? vs : (lv_ ? 1.f : 0.f);
+        par[3] = code ? vz - vs : 0.f;
+        eager = __ballot(code && vs > kVsMax) != 0ull;
+        if (i + 1 < min(kend, nh)) meta = load_meta(h, (i + 1) * kBlk, p0, r);      // (p0: block i + 1's page by now)
+      }
+      constexpr auto regs = std::make_integer_sequence<int, 16>{};
+      // x = score - m_base; key 8 jj + 4g + e of the block is register 4 jj + e
+      float x[16];
+      each16([&](auto reg) {
+        constexpr int q = decltype(reg)::value;
+        x[q] = row_bcast<q>(par[0]) * s[q];
+      }, regs);
+      fmac_bcast(x, par[1], qsum);
+#pragma unroll
+      for (int q = 0; q < 16; ++q) x[q] -= m_base;
+      // Keys past C in the history's last block, causality in the new-token
+      // blocks; a block every row of the wave sees whole skips the test.
+      const int j0 = (i - nh) * kBlk;                     // first new token of a new-token block
+      const bool whole = hist ? (i + 1) * kBlk <= h.cached : j0 + kBlk - 1 <= first_tok;
+      if (!whole) {
+        const int lim = (hist ? h.cached - i * kBlk - 1 : my_tok - j0) - 4 * g;      // last visible key
+#pragma unroll
+        for (int q = 0; q < 16; ++q) x[q] = 8 * (q >> 2) + (q & 3) <= lim ? x[q] : -__builtin_inff();
+      }
+      float mb = x[0];
+#pragma unroll
+      for (int q = 1; q < 16; ++q) mb = fmaxf(mb, x[q]);
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(mb), __float_as_int(mb), false, false);
+      mb = fmaxf(__int_as_float(sw[0]), __int_as_float(sw[1]));
       // Lazy running max: raised only when a block exceeds it by more than
-      // 2^kLazy (p vs stays in fp16 range), or by any amount when a key of the
-      // block has vs above kVsMax; the first raise of a row needs no rescale.
-      const uint4 bg4 = *reinterpret_cast<const uint4*>(S.big[i & 1]);
-      const bool eager = (bg4[0] | bg4[1] | bg4[2] | bg4[3]) != 0u;
-      const bool need = mb > m_run + (eager ? 0.f : kLazy);
-      const bool resc = need && m_run != -__builtin_inff();
-      if (__ballot(resc)) {
-        const float alpha = resc ? __builtin_amdgcn_exp2f(m_run - mb) : 1.f;
+      // 2^kLazy (p vs stays in fp16 range), or by any amount when a key of
+      // the block has vs above kVsMax, or when the row has seen no key yet
+      // (which needs no rescale).
+      const bool need = mb > (eager ? fminf(raise, 0.f) : raise);
+      if (__ballot(need)) {
+        const float delta = need ? mb : 0.f;
+        const float alpha = raise == -__builtin_inff() ? 1.f : __builtin_amdgcn_exp2f(-delta);
 #pragma unroll
         for (int t = 0; t < 8; ++t) acc[t] *= alpha;
         l_run *= alpha;
         z_run *= alpha;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) x[q] -= delta;
+        m_base += delta;
+        raise = need ? kLazy : raise;
       }
-      if (need) m_run = mb;
-      // exp2(-inf - m) = 0 needs a finite m: rows that have seen no key yet use 0.
-      const float m_use = m_run == -__builtin_inff() ? 0.f : m_run;
-      float psum = 0.f, zsum = 0.f;
-      half8 pb[2];
-      const float* vpar0 = S.vpar[i & 1][0] + 4 * g;
-      const float* vpar1 = S.vpar[i & 1][1] + 4 * g;
+      float psum = 0.f;
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const floatx4 vs = *reinterpret_cast<const floatx4*>(vpar0 + 8 * jj);
-        const floatx4 vz = *reinterpret_cast<const floatx4*>(vpar1 + 8 * jj);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int r = 4 * jj + e;
-          const float p = __builtin_amdgcn_exp2f(s[r] - m_use);
-          psum += p;
-          zsum = fmaf(p, vz[e], zsum);
-          pb[r >> 3][r & 7] = to_h(p * vs[e]);
-        }
+      for (int q = 0; q < 16; ++q) {
+        x[q] = __builtin_amdgcn_exp2f(x[q]);
+        psum += x[q];
       }
       l_run += psum;
-      z_run += zsum;
-#pragma unroll
-      for (int mm = 0; mm < 2; ++mm) {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const _Float16* vrow = vt + (32 * t + col) * kVs + 16 * mm + 4 * g;
-          const u32x2 lo2 = *reinterpret_cast<const u32x2*>(vrow);
-          const u32x2 hi2 = *reinterpret_cast<const u32x2*>(vrow + 8);
-          const half8 va = __builtin_bit_cast(half8, u32x4{lo2[0], lo2[1], hi2[0], hi2[1]});
-          acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb[mm], acc[t], 0, 0, 0);
+      z_run = dot_bcast(x, par[3], z_run);
+      each16([&](auto reg) {
+        constexpr int q = decltype(reg)::value;
+        pb[q >> 3][q & 7] = to_h(row_bcast<q>(par[2]) * x[q]);
+      }, regs);
+    };
+
+    // ---- first K tile (and a zero V tile before it), then M and S per block ----
+    {
+      floatx4* z = reinterpret_cast<floatx4*>(tile_v(kb - 1));
+      z[tid] = floatx4{};
+      z[tid + 64 * kWaves] = floatx4{};
+      static_assert(2 * 64 * kWaves * sizeof(floatx4) == kKeyTileHalfs * sizeof(_Float16), "the tile");
+    }
+    if (kb < nh) {
+      hist_k(kb);
+      cur = next;
+      p0 = p1;
+      p1 = valid_page(h, p2);
+      if (kb + 1 < min(kend, nh)) {
+        lk = load_k(h, (kb + 1) * kBlk, p1, r, lane);
+        p2 = block_page(h, (kb + 2) * kBlk);
+      }
+      lds_barrier();
+    } else {
+      new_k(kb, std::integral_constant<int, kWaves>{});
+      copy_barrier();
+    }
+    int i = kb;
+    // blocks i and i + 1 in the history, i seen: builds under the MFMAs
+    const int hot = min(kseen, min(kend, nh) - 1);
+#pragma unroll 1
+    for (; i < hot; ++i) {
+      // (at the end of the phase, where the words have had longest to arrive)
+      uint32_t w = 0;
+      matrix(i, std::true_type{}, [&](int n) {
+        if (n == 9) w = quad_transpose(lv, lane);
+        if (n >= 10 && n < 14) build_v(w, opaque(r.vs), tile_v(i), n - 10);
+        if (n >= 14) build_k(lk.kc, opaque(r.ks), tile_k(i + 1), n - 14);
+      });
+      next = block_of(i + 1);
+      if ((next.win | cur.win) != 0u) {
+        if (next.win != 0u) window_k(next.win, p1, (i + 1) * kBlk, kvh_now, r, wave, lane, tile_k(i + 1));
+        if (cur.win != 0u) window_v(cur.win, lv, p0, i * kBlk, kvh_now, r, wave, lane, tile_v(i));
+      }
+      load_next(i);
+      if (second) lds_barrier();
+      softmax(i, true);
+      cur = next;
+      if (!second) lds_barrier();
+    }
+    // the history's last block and the new-token blocks
+    auto builds = [&](int i) {
+      if (i < nh) hist_v(i);
+      else new_v(i);
+      if (i + 1 < kend) {
+        if (i + 1 < nh) hist_k(i + 1);
+        else new_k(i + 1, std::integral_constant<int, 4>{});
+      }
+      if (i < nh) load_next(i);
+    };
+    // (a first-half wave's copies have had both phases)
+    auto first_end = [&](int i) {
+      if (kImages && i + 1 >= nh) copy_barrier();
+      else lds_barrier();
+    };
+#pragma unroll 1
+    for (; i < kseen; ++i) {
+      builds(i);
+      matrix(i, std::true_type{}, nothing);
+      if (second) lds_barrier();
+      softmax(i, i < nh);
+      cur = next;
+      if (!second) first_end(i);
+    }
+    // the last PV, then blocks that only other waves see
+    if (i < kend) builds(i);
+    matrix(i, std::false_type{}, nothing);
+#pragma unroll 1
+    while (i < kend) {
+      if (second) lds_barrier();
+      else first_end(i);
+      cur = next;
+      if (++i < kend) builds(i);
+    }
+    lds_barrier();              // the tiles are free
+
+    // ---- the row block's output, or this share's partial of it ----
+    const float l_tot = l_run + shfl_xor_f32(l_run, 32);
+    const float z_tot = z_run + shfl_xor_f32(z_run, 32);
+    // (this lane's row recomputed, so that nothing of it lives through the loop)
+    const int elane = (int)opaque((uint32_t)lane);
+    const int erow = wrow0 + (elane & 31), eg = elane >> 5;
+    if (erow < rows_total) {
+      const int etok = erow / a.group, ehead = kvh_now * a.group + (erow - etok * a.group);
+      const bool whole_rb = kb == 0 && kend == nblk;
+      float* op;
+      float inv = 1.f;
+      if (whole_rb) {
+        inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+        op = a.out + ((int64_t)(it.tok0 + etok) * a.num_heads + ehead) * kHeadDim;
+      } else {
+        const int64_t slot = 2 * (int64_t)blockIdx.x + (start != (int64_t)blockIdx.x * a.share ? 1 : 0);
+        float* part = a.part + slot * (int64_t)kPartFloats;
+        const int pr = wave * kRowsPerWave + (elane & 31);
+        op = part + pr * kHeadDim;
+        if (eg == 0) {
+          part[kPartRows * kHeadDim + pr] = raise == -__builtin_inff() ? raise : m_base;
+          part[kPartRows * (kHeadDim + 1) + pr] = l_tot;
         }
       }
+      op += 4 * eg;
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj)
+          *reinterpret_cast<floatx4*>(op + 32 * t + 8 * jj) =
+              floatx4{(acc[t][4 * jj] + z_tot) * inv, (acc[t][4 * jj + 1] + z_tot) * inv,
+                      (acc[t][4 * jj + 2] + z_tot) * inv, (acc[t][4 * jj + 3] + z_tot) * inv};
     }
-  }
-  lds_barrier();              // pairs with the producers' last barrier
-
-  const float l_tot = l_run + shfl_xor_f32(l_run, 32);
-  const float z_tot = z_run + shfl_xor_f32(z_run, 32);
-  if (!row_ok) return;
-  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  const int64_t j = row / a.group;
-  const int h = kvh * a.group + (int)(row % a.group);
-  float* op = a.out + (j * a.num_heads + h) * kHeadDim;
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) op[32 * t + 8 * (r >> 2) + 4 * g + (r & 3)] = (acc[t][r] + z_tot) * inv;
   }
 }
 
-std::atomic<uint64_t> g_lds_set{0};   // dynamic-LDS attribute set, one bit per device
+// Rows of the row blocks that the shares cut: their partials LSE-combined and
+// normalised.  kWavesPerRow waves share a row's partials (one where a row has
+// few of them, four where the work of few rows is spread over the GPU); lane
+// l holds features 4l .. 4l + 3, and the partials' (m, l) come in one
+// lane-parallel round per 64.  grid.x = row blocks x kTileRows x
+// kWavesPerRow / 4, 256 threads.
+template <int kWavesPerRow>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
+  constexpr int kRows = 4 / kWavesPerRow;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int grb = (int)blockIdx.x / (kTileRows / kRows);
+  int item = 0;
+  while (item + 1 < a.nitems && a.items[item + 1].rb0 <= grb) ++item;
+  const PrefillItem it = a.items[item];
+  const int nrb = row_blocks(it, a.group);
+  const int kvh = (grb - it.rb0) / nrb, rb = (grb - it.rb0) - kvh * nrb;
+  const int pr = ((int)blockIdx.x % (kTileRows / kRows)) * kRows + wave / kWavesPerRow;
+  const int row = rb * kTileRows + pr;
+  if (row >= it.n_new * a.group) return;
+  // units of the row block's first and last key block
+  const int64_t lo = it.unit0 + (int64_t)kvh * it.head_units + units_before(it, a.group, rb, lane) + kPieceCost;
+  const int64_t hi = lo + key_blocks(it, a.group, rb) - 1;
+  const int64_t w0 = lo / a.share, w1 = hi / a.share;
+  if (w0 == w1) return;                       // written whole by its share
+  const int n = (int)(w1 - w0) + 1;
+  auto slot = [&](int p) {
+    return a.part + (2 * (w0 + p) + (p == 0 && lo != w0 * a.share ? 1 : 0)) * (int64_t)kPartFloats;
+  };
+  float mx = -__builtin_inff();
+  for (int p = lane; p < n; p += 64) mx = fmaxf(mx, slot(p)[kPartRows * kHeadDim + pr]);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  // partials first, first + kWavesPerRow, ... of the row
+  const int first = wave % kWavesPerRow, mine = (n - first + kWavesPerRow - 1) / kWavesPerRow;
+  floatx4 acc = floatx4{};
+  float l = 0.f;
+  constexpr int kBatch = 8;
+  for (int p0 = 0; p0 < mine; p0 += 64) {
+    const int p = first + (p0 + lane) * kWavesPerRow;
+    float w = 0.f;
+    if (p < n) {
+      const float m = slot(p)[kPartRows * kHeadDim + pr];
+      w = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(m - mx);
+      l = fmaf(w, slot(p)[kPartRows * (kHeadDim + 1) + pr], l);
+    }
+    const int cnt = min(64, mine - p0);
+    for (int b = 0; b < cnt; b += kBatch) {
+      floatx4 x[kBatch];
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k)
+        x[k] = *reinterpret_cast<const floatx4*>(slot(first + (p0 + min(b + k, cnt - 1)) * kWavesPerRow) +
+                                                 pr * kHeadDim + 4 * lane);
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) {
+        const float wk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), (b + k) & 63));
+        if (b + k < cnt) acc += wk * x[k];
+      }
+    }
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) l += __shfl_xor(l, o, 64);
+  if constexpr (kWavesPerRow > 1) {
+    __shared__ floatx4 osum[kWavesPerRow][64];
+    __shared__ float lsum[kWavesPerRow];
+    osum[wave][lane] = acc;
+    if (lane == 0) lsum[wave] = l;
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int k = 1; k < kWavesPerRow; ++k) {
+      acc += osum[k][lane];
+      l += lsum[k];
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const int tok = row / a.group, head = kvh * a.group + (row - tok * a.group);
+  *reinterpret_cast<floatx4*>(a.out + ((int64_t)(it.tok0 + tok) * a.num_heads + head) * kHeadDim + 4 * lane) =
+      acc * inv;
+}
 
-}  // namespace
-}  // namespace oscar
+// Operands (prefill_operands.h) of rotated fp32 rows: one 16-byte chunk per
+// thread; query rows first (32 threads per row), then key tiles, then value
+// tiles.  Compact tokens are the inputs' tokens here.
+struct ConvertArgs {
+  const float* q;
+  const float* k;
+  const float* v;
+  int32_t num_heads, num_kv_heads;
+  PrefillOperands o;
+  int64_t q_chunks, kv_chunks;
+  OperandItems items;
+};
 
-using namespace oscar;
+__global__ __launch_bounds__(256) void convert_operands_kernel(ConvertArgs a) {
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (idx < a.q_chunks) {                      // a multiple of 256 or the tail's whole 32-thread rows
+    const int64_t row = idx >> 5;
+    const int c = (int)idx & 31;
+    const float* src = a.q + row * kHeadDim + 16 * (c >> 1) + 4 * (c & 1);
+    half8 o;
+    float qs = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      o[e] = to_h(src[(e >> 1) + 8 * (e & 1)]);
+      qs += (float)o[e];
+    }
+    reinterpret_cast<half8*>(a.o.q16)[idx] = o;
+#pragma unroll
+    for (int s = 16; s >= 1; s >>= 1) qs += __shfl_xor(qs, s, 64);
+    if (c == 0) a.o.qsum[row] = qs;
+    return;
+  }
+  int64_t r = idx - a.q_chunks;
+  const bool value = r >= a.kv_chunks;
+  if (value) r -= a.kv_chunks;
+  if (r >= a.kv_chunks) return;
+  const int64_t unit = r >> 10;                // (tile, kv head): 1024 chunks
+  const int tile = (int)(unit / a.num_kv_heads), head = (int)(unit - (int64_t)tile * a.num_kv_heads);
+  int i = 0;
+  while (i + 1 < a.items.n && a.items.it[i + 1].tile0 <= tile) ++i;
+  const OperandItem it = a.items.it[i];
+  const int j0 = (tile - it.tile0) * kBlk;
+  auto rowp = [&](const float* x, int t) {
+    return x + ((int64_t)(it.tok0 + min(j0 + t, it.n_new - 1)) * a.num_kv_heads + head) * kHeadDim;
+  };
+  half8 o;
+  if (!value) {
+    const int token = (int)(r >> 5) & 31, c = (int)r & 31;
+    const float* src = rowp(a.k, token) + 16 * (c >> 1) + 4 * (c & 1);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = to_h(src[(e >> 1) + 8 * (e & 1)]);
+    reinterpret_cast<half8*>(a.o.kimg)[unit * 1024 + token * 32 + k_chunk(c, token)] = o;
+  } else {
+    const int f = (int)r & 255, c = (int)(r >> 8) & 3;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = to_h(rowp(a.v, 16 * (c >> 1) + 8 * (e >> 2) + 4 * (c & 1) + (e & 3))[f]);
+    reinterpret_cast<half8*>(a.o.vimg)[unit * 1024 + f * 4 + v_chunk(c, f)] = o;
+  }
+}
 
-extern "C" int oscar_prefill_continuation(
-    const float* q_rot, const float* k_new, const float* v_new, int32_t num_new, int32_t num_heads,
-    int32_t num_kv_heads, int32_t head_size, const void* k_cache, const void* v_cache,
-    int32_t block_size, int64_t num_pages, int64_t k_stride_page, int64_t k_stride_token,
-    int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token, int64_t v_stride_head,
-    const int32_t* block_table_row, int32_t block_table_cols, int64_t cached_len,
-    const float* stage_k, const float* stage_v, const int64_t* stage_owner, int32_t stage_rows,
-    float scale, float* out, hipStream_t stream) {
+std::atomic<uint64_t> g_lds_set[2] = {{0}, {0}};   // dynamic-LDS attribute set, one bit per device
+
+// ---- host side ----
+int64_t host_head_units(int64_t n_new, int64_t cached, int64_t group) {
+  const int64_t rows = n_new * group, nrb = (rows + kTileRows - 1) / kTileRows, nh = (cached + kBlk - 1) / kBlk;
+  int64_t n = nrb * (nh + kPieceCost);
+  for (int64_t rb = 0; rb < nrb; ++rb) {
+    const int64_t last = ((rb + 1) * kTileRows < rows ? (rb + 1) * kTileRows : rows) - 1;
+    n += last / group / kBlk + 1;
+  }
+  return n;
+}
+
+// Units per workgroup: one round of kShares workgroups, of at least kMinShare
+// units each (a partial of 256 rows is 264 KB, written and read again).
+int64_t plan_share(int64_t units) {
+  const int64_t s = (units + kShares - 1) / kShares;
+  return s < kMinShare ? kMinShare : s;
+}
+
+struct Layout {          // byte offsets into the workspace
+  size_t q16, qsum, kimg, vimg, out, part, total;
+};
+
+size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+Layout workspace_layout(int64_t tokens, int64_t tiles, int64_t units, int32_t hq, int32_t hk, bool with_out) {
+  Layout w;
+  size_t o = 0;
+  w.q16 = o;
+  o = align256(o + (size_t)tokens * hq * kHeadDim * sizeof(_Float16));
+  w.qsum = o;
+  o = align256(o + (size_t)tokens * hq * sizeof(float));
+  w.kimg = o;
+  o = align256(o + (size_t)tiles * hk * kKeyTileHalfs * sizeof(_Float16));
+  w.vimg = o;
+  o = align256(o + (size_t)tiles * hk * kKeyTileHalfs * sizeof(_Float16));
+  w.out = o;
+  if (with_out) o = align256(o + (size_t)tokens * hq * kHeadDim * sizeof(float));
+  w.part = o;
+  const int64_t share = plan_share(units);
+  o += (size_t)(2 * ((units + share - 1) / share)) * kPartFloats * sizeof(float);
+  w.total = o;
+  return w;
+}
+
+// The cache, block table, arena and geometry half of the arguments, checked.
+int fill_common(PrefillArgs& a, int32_t num_heads, int32_t num_kv_heads, int32_t head_size, const void* k_cache,
+                const void* v_cache, int32_t block_size, int64_t num_pages, int64_t k_stride_page,
+                int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token,
+                int64_t v_stride_head, const int32_t* block_table, int64_t block_table_stride,
+                int32_t block_table_cols, const float* stage_k, const float* stage_v, const int64_t* stage_owner,
+                int32_t stage_rows, float scale) {
   if (head_size != kHeadDim) return kErrUnsupportedHeadDim;
-  if (num_new < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads ||
-      block_size <= 0 || num_pages <= 0 || cached_len < 0 || stage_rows < 0 || block_table_cols < 0)
-    return kErrInvalidArgument;
-  if (num_new == 0) return kOk;
-  // key positions and rows are handled in 32 bits inside the kernel
-  if (cached_len + num_new >= ((int64_t)1 << 31) || (int64_t)num_new * num_heads >= ((int64_t)1 << 31))
-    return kErrInvalidArgument;
-  if (!q_rot || !k_new || !v_new || !k_cache || !v_cache || !out) return kErrInvalidArgument;
-  if (cached_len > 0 && (!block_table_row || (cached_len + block_size - 1) / block_size > block_table_cols))
+  if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || block_size <= 0 || num_pages <= 0 ||
+      stage_rows < 0 || block_table_cols < 0 || !k_cache || !v_cache)
     return kErrInvalidArgument;
   if (stage_rows > 0 && (!stage_k || !stage_v || !stage_owner)) return kErrInvalidArgument;
   if (k_stride_head < kKCodeOff + kCodeBytes || v_stride_head < kCodeBytes || (k_stride_head & 7) ||
-      (k_stride_token & 7) || (k_stride_page & 7) || block_size % kBlk != 0)
+      (k_stride_token & 7) || (k_stride_page & 7) || (v_stride_head & 1) || (v_stride_token & 1) ||
+      (v_stride_page & 1) || block_size % kBlk != 0)
     return kErrUnsupportedGeometry;
-  PrefillArgs a{};
-  a.q = q_rot;
-  a.k_new = k_new;
-  a.v_new = v_new;
-  a.n_new = num_new;
   a.num_heads = num_heads;
   a.num_kv_heads = num_kv_heads;
   a.group = num_heads / num_kv_heads;
@@ -671,18 +1128,243 @@ extern "C" int oscar_prefill_continuation(
   a.bs_div = make_fast_div((uint32_t)block_size);
   a.rows_div = make_fast_div(stage_rows > 0 ? (uint32_t)stage_rows : 1u);
   a.num_pages = num_pages;
-  a.bt = block_table_row;
+  a.bt = block_table;
+  a.bt_stride = block_table_stride;
   a.bt_cols = block_table_cols;
-  a.cached = cached_len;
   a.stage_k = stage_k;
   a.stage_v = stage_v;
   a.owner = stage_owner;
   a.stage_rows = stage_rows;
   a.scale_log2 = scale * kLog2e;
+  return kOk;
+}
+
+// One request's sizes: positions and rows are handled in 32 bits in the kernel.
+int check_request(int64_t n_new, int64_t cached, int32_t num_heads, int32_t block_size, const int32_t* table,
+                  int32_t cols) {
+  if (n_new < 0 || cached < 0 || cached + n_new >= ((int64_t)1 << 31) || n_new * num_heads >= ((int64_t)1 << 31))
+    return kErrInvalidArgument;
+  if (cached > 0 && (!table || (cached + block_size - 1) / block_size > cols)) return kErrInvalidArgument;
+  return kOk;
+}
+
+void add_item(PrefillArgs& a, OperandItems& ops, int32_t n_new, int64_t cached, int32_t req, int32_t in_tok0) {
+  PrefillItem& it = a.items[a.nitems];
+  it.unit0 = a.units;
+  it.head_units = host_head_units(n_new, cached, a.group);
+  it.n_new = n_new;
+  it.cached = (int32_t)cached;
+  it.req = req;
+  it.tok0 = ops.tokens;
+  it.tile0 = ops.tiles;
+  it.rb0 = 0;
+  if (a.nitems > 0) {
+    const PrefillItem& p = a.items[a.nitems - 1];
+    it.rb0 = p.rb0 + (int32_t)(((int64_t)p.n_new * a.group + kTileRows - 1) / kTileRows) * a.num_kv_heads;
+  }
+  ops.it[ops.n++] = OperandItem{in_tok0, n_new, ops.tokens, ops.tiles};
+  ops.tokens += n_new;
+  ops.tiles += (n_new + kBlk - 1) / kBlk;
+  a.units += it.head_units * a.num_kv_heads;
+  ++a.nitems;
+}
+
+// The read over operands in the workspace: shares, then the merge of the row
+// blocks they cut.
+int launch_shares(PrefillArgs& a, hipStream_t stream) {
+  a.share = plan_share(a.units);
+  const int64_t wgs = (a.units + a.share - 1) / a.share;
+  if (set_dynamic_lds(reinterpret_cast<const void*>(prefill_kernel<true>), (int)kPrefillLds, g_lds_set[1]) != kOk)
+    return kErrLaunch;
+  hipLaunchKernelGGL((prefill_kernel<true>), dim3((unsigned)wgs), dim3(64 * kWaves), kPrefillLds, stream, a);
+  if (hipGetLastError() != hipSuccess) return kErrLaunch;
+  if (wgs > 1) {
+    const PrefillItem& p = a.items[a.nitems - 1];
+    const int64_t rbs = p.rb0 + (((int64_t)p.n_new * a.group + kTileRows - 1) / kTileRows) * a.num_kv_heads;
+    // few row blocks in many shares: a workgroup per row
+    if (rbs * kMergeManyPieces <= wgs)
+      hipLaunchKernelGGL((prefill_merge_kernel<4>), dim3((unsigned)(rbs * kTileRows)), dim3(256), 0, stream, a);
+    else
+      hipLaunchKernelGGL((prefill_merge_kernel<1>), dim3((unsigned)(rbs * kTileRows / 4)), dim3(256), 0, stream, a);
+    if (hipGetLastError() != hipSuccess) return kErrLaunch;
+  }
+  return kOk;
+}
+
+void bind_workspace(PrefillArgs& a, PrefillOperands& o, const Layout& w, uint8_t* ws) {
+  o.q16 = reinterpret_cast<_Float16*>(ws + w.q16);
+  o.qsum = reinterpret_cast<float*>(ws + w.qsum);
+  o.kimg = reinterpret_cast<_Float16*>(ws + w.kimg);
+  o.vimg = reinterpret_cast<_Float16*>(ws + w.vimg);
+  a.q16 = o.q16;
+  a.qsum = o.qsum;
+  a.kimg = o.kimg;
+  a.vimg = o.vimg;
+  a.part = reinterpret_cast<float*>(ws + w.part);
+}
+
+}  // namespace
+}  // namespace oscar
+
+using namespace oscar;
+
+extern "C" size_t oscar_prefill_workspace_bytes(int32_t num_new, int32_t num_heads, int32_t num_kv_heads,
+                                                int64_t cached_len) {
+  if (num_new <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || cached_len < 0) return 0;
+  const int64_t units = host_head_units(num_new, cached_len, num_heads / num_kv_heads) * num_kv_heads;
+  return workspace_layout(num_new, (num_new + kBlk - 1) / kBlk, units, num_heads, num_kv_heads, false).total;
+}
+
+extern "C" int oscar_prefill_continuation_split(
+    const float* q_rot, const float* k_new, const float* v_new, int32_t num_new, int32_t num_heads,
+    int32_t num_kv_heads, int32_t head_size, const void* k_cache, const void* v_cache,
+    int32_t block_size, int64_t num_pages, int64_t k_stride_page, int64_t k_stride_token,
+    int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token, int64_t v_stride_head,
+    const int32_t* block_table_row, int32_t block_table_cols, int64_t cached_len,
+    const float* stage_k, const float* stage_v, const int64_t* stage_owner, int32_t stage_rows,
+    float scale, float* out, void* workspace, size_t workspace_size, hipStream_t stream) {
+  PrefillArgs a{};
+  int st = fill_common(a, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages, k_stride_page,
+                       k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head, block_table_row,
+                       0, block_table_cols, stage_k, stage_v, stage_owner, stage_rows, scale);
+  if (st != kOk) return st;
+  if ((st = check_request(num_new, cached_len, num_heads, block_size, block_table_row, block_table_cols)) != kOk)
+    return st;
+  if (num_new == 0) return kOk;
+  if (!q_rot || !k_new || !v_new || !out || !workspace) return kErrInvalidArgument;
+  OperandItems ops{};
+  add_item(a, ops, num_new, cached_len, 0, 0);
+  const Layout w = workspace_layout(ops.tokens, ops.tiles, a.units, num_heads, num_kv_heads, false);
+  if (workspace_size < w.total) return kErrWorkspaceTooSmall;
+  ConvertArgs c{q_rot, k_new, v_new, num_heads, num_kv_heads, PrefillOperands{}, 0, 0, ops};
+  bind_workspace(a, c.o, w, static_cast<uint8_t*>(workspace));
   a.out = out;
+  c.q_chunks = (int64_t)ops.tokens * num_heads * (kHeadDim / 8);
+  c.kv_chunks = (int64_t)ops.tiles * num_kv_heads * (kKeyTileHalfs / 8);
+  const int64_t blocks = (c.q_chunks + 2 * c.kv_chunks + 255) / 256;
+  hipLaunchKernelGGL(convert_operands_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, c);
+  if (hipGetLastError() != hipSuccess) return kErrLaunch;
+  return launch_shares(a, stream);
+}
+
+extern "C" int oscar_prefill_continuation(
+    const float* q_rot, const float* k_new, const float* v_new, int32_t num_new, int32_t num_heads,
+    int32_t num_kv_heads, int32_t head_size, const void* k_cache, const void* v_cache,
+    int32_t block_size, int64_t num_pages, int64_t k_stride_page, int64_t k_stride_token,
+    int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token, int64_t v_stride_head,
+    const int32_t* block_table_row, int32_t block_table_cols, int64_t cached_len,
+    const float* stage_k, const float* stage_v, const int64_t* stage_owner, int32_t stage_rows,
+    float scale, float* out, hipStream_t stream) {
+  PrefillArgs a{};
+  int st = fill_common(a, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages, k_stride_page,
+                       k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head, block_table_row,
+                       0, block_table_cols, stage_k, stage_v, stage_owner, stage_rows, scale);
+  if (st != kOk) return st;
+  if ((st = check_request(num_new, cached_len, num_heads, block_size, block_table_row, block_table_cols)) != kOk)
+    return st;
+  if (num_new == 0) return kOk;
+  if (!q_rot || !k_new || !v_new || !out) return kErrInvalidArgument;
+  a.q = q_rot;
+  a.k_new = k_new;
+  a.v_new = v_new;
+  a.out = out;
+  OperandItems ops{};
+  add_item(a, ops, num_new, cached_len, 0, 0);
   const int64_t rows = (int64_t)num_new * a.group;
-  dim3 grid((unsigned)((rows + kWaves * kRowsPerWave - 1) / (kWaves * kRowsPerWave)), (unsigned)num_kv_heads);
-  if (set_dynamic_lds(reinterpret_cast<const void*>(prefill_kernel), (int)kPrefillLds, g_lds_set) != kOk) return kErrLaunch;
-  hipLaunchKernelGGL(prefill_kernel, grid, dim3(2 * kWaves * 64), kPrefillLds, stream, a);
+  const dim3 grid((unsigned)((rows + kTileRows - 1) / kTileRows), (unsigned)num_kv_heads);
+  if (set_dynamic_lds(reinterpret_cast<const void*>(prefill_kernel<false>), (int)kPrefillLds, g_lds_set[0]) != kOk)
+    return kErrLaunch;
+  hipLaunchKernelGGL((prefill_kernel<false>), grid, dim3(64 * kWaves), kPrefillLds, stream, a);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+extern "C" size_t oscar_prefill_rotated_workspace_bytes(int32_t num_requests, const int32_t* new_tokens,
+                                                        const int64_t* cached_lens, int32_t num_heads,
+                                                        int32_t num_kv_heads) {
+  if (num_requests <= 0 || !new_tokens || !cached_lens || num_heads <= 0 || num_kv_heads <= 0 ||
+      num_heads % num_kv_heads)
+    return 0;
+  size_t most = 0;
+  for (int32_t r0 = 0; r0 < num_requests; r0 += kMaxPrefillItems) {     // one launch's requests
+    int64_t tokens = 0, tiles = 0, units = 0;
+    for (int32_t i = r0; i < num_requests && i < r0 + kMaxPrefillItems; ++i) {
+      if (new_tokens[i] < 0 || cached_lens[i] < 0) return 0;
+      tokens += new_tokens[i];
+      tiles += (new_tokens[i] + kBlk - 1) / kBlk;
+      units += host_head_units(new_tokens[i], cached_lens[i], num_heads / num_kv_heads) * num_kv_heads;
+    }
+    const size_t n = workspace_layout(tokens, tiles, units, num_heads, num_kv_heads, true).total;
+    most = n > most ? n : most;
+  }
+  return most;
+}
+
+extern "C" int oscar_prefill_rotated(
+    const void* query_bf16, int64_t query_token_stride, const void* key_bf16, const void* value_bf16,
+    int64_t kv_token_stride, int32_t num_requests, const int32_t* first_tokens, const int32_t* new_tokens,
+    const int64_t* cached_lens, const int32_t* table_rows, int32_t num_heads, int32_t num_kv_heads,
+    int32_t head_size, const void* rot_k_operand, const void* rot_v_operand, const void* rot_v_t_operand,
+    const void* k_cache, const void* v_cache, int32_t block_size, int64_t num_pages, int64_t k_stride_page,
+    int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token,
+    int64_t v_stride_head, const int32_t* block_table, int64_t block_table_stride, int32_t block_table_cols,
+    const float* stage_k, const float* stage_v, const int64_t* stage_owner, int32_t stage_rows, float scale,
+    void* out_bf16, void* workspace, size_t workspace_size, hipStream_t stream) {
+  PrefillArgs base{};
+  int st = fill_common(base, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages,
+                       k_stride_page, k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
+                       block_table, block_table_stride, block_table_cols, stage_k, stage_v, stage_owner, stage_rows,
+                       scale);
+  if (st != kOk) return st;
+  if (num_requests < 0) return kErrInvalidArgument;
+  if (num_requests == 0) return kOk;
+  if (!query_bf16 || !key_bf16 || !value_bf16 || !first_tokens || !new_tokens || !cached_lens || !table_rows ||
+      !rot_k_operand || !rot_v_operand || !rot_v_t_operand || !out_bf16 || !workspace)
+    return kErrInvalidArgument;
+  // 16-byte vector accesses: every (token, head) row start 16-byte aligned
+  if (query_token_stride < (int64_t)num_heads * kHeadDim || kv_token_stride < (int64_t)num_kv_heads * kHeadDim ||
+      (query_token_stride & 7) || (kv_token_stride & 7) || (reinterpret_cast<uintptr_t>(query_bf16) & 15) ||
+      (reinterpret_cast<uintptr_t>(key_bf16) & 15) || (reinterpret_cast<uintptr_t>(value_bf16) & 15) ||
+      (reinterpret_cast<uintptr_t>(out_bf16) & 15) || (reinterpret_cast<uintptr_t>(rot_k_operand) & 15) ||
+      (reinterpret_cast<uintptr_t>(rot_v_operand) & 15) || (reinterpret_cast<uintptr_t>(rot_v_t_operand) & 15))
+    return kErrInvalidArgument;
+  for (int32_t i = 0; i < num_requests; ++i) {
+    if (first_tokens[i] < 0 || table_rows[i] < 0) return kErrInvalidArgument;
+    if ((st = check_request(new_tokens[i], cached_lens[i], num_heads, block_size, block_table, block_table_cols)) !=
+        kOk)
+      return st;
+  }
+  if (workspace_size < oscar_prefill_rotated_workspace_bytes(num_requests, new_tokens, cached_lens, num_heads,
+                                                             num_kv_heads))
+    return kErrWorkspaceTooSmall;
+  for (int32_t r0 = 0; r0 < num_requests; r0 += kMaxPrefillItems) {
+    PrefillArgs a = base;
+    OperandItems ops{};
+    for (int32_t i = r0; i < num_requests && i < r0 + kMaxPrefillItems; ++i)
+      if (new_tokens[i] > 0) add_item(a, ops, new_tokens[i], cached_lens[i], table_rows[i], first_tokens[i]);
+    if (a.nitems == 0) continue;
+    const Layout w = workspace_layout(ops.tokens, ops.tiles, a.units, num_heads, num_kv_heads, true);
+    uint8_t* ws = static_cast<uint8_t*>(workspace);
+    PrefillOperands o;
+    bind_workspace(a, o, w, ws);
+    a.out = reinterpret_cast<float*>(ws + w.out);
+    st = launch_rotate_operands(static_cast<const uint16_t*>(query_bf16), query_token_stride,
+                                static_cast<const uint16_t*>(key_bf16), static_cast<const uint16_t*>(value_bf16),
+                                kv_token_stride, num_heads, num_kv_heads, static_cast<const uint8_t*>(rot_k_operand),
+                                static_cast<const uint8_t*>(rot_v_operand), ops, o, stream);
+    if (st != kOk) return st;
+    if ((st = launch_shares(a, stream)) != kOk) return st;
+    // R_v^T and the bf16 cast: one launch per run of adjacent requests
+    for (int32_t i = 0; i < ops.n;) {
+      int32_t j = i + 1;
+      while (j < ops.n && ops.it[j].tok0 == ops.it[j - 1].tok0 + ops.it[j - 1].n_new) ++j;
+      const int64_t tokens = ops.it[j - 1].ctok0 + ops.it[j - 1].n_new - ops.it[i].ctok0;
+      st = oscar_rotate_rows(a.out + (int64_t)ops.it[i].ctok0 * num_heads * kHeadDim, 1, kHeadDim,
+                             tokens * num_heads, head_size, rot_v_t_operand,
+                             static_cast<uint16_t*>(out_bf16) + (int64_t)ops.it[i].tok0 * num_heads * kHeadDim, 1,
+                             kHeadDim, stream);
+      if (st != kOk) return st;
+      i = j;
+    }
+  }
+  return kOk;
 }

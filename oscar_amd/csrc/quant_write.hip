@@ -25,6 +25,7 @@
 // the window write of the step's bulk tokens from the same rotated values
 // (see window_epilogue), after a seat-winner pass over the step's slots.
 #include "int2_quant.h"
+#include "prefill_operands.h"
 #include "window_images.h"
 #include "../../include/oscar_amd.h"
 
@@ -534,21 +535,17 @@ __device__ constexpr int kRotWait(int m) {
                 : ((m >= 5 && m <= 7) ? 16 : m == 14 ? 4 : m == 15 ? 0 : 8);
 }
 
-template <bool kF32In, bool kBf16Out>
-__global__ __launch_bounds__(256, 2) void rotate_rows_kernel(const void* __restrict__ in, int64_t in_stride,
-                                                            int64_t rows, const uint8_t* __restrict__ rop,
-                                                            void* __restrict__ out, int64_t out_stride) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t ring[];
+// The rotation of one wave's 32 rows: lane l's row starts at xsrc (its input
+// features 128 (l >> 5) .. +127).  kSwap = false: register i of tile t is
+// output feature 128 (l >> 5) + 16 t + i of row l & 31.  kSwap = true (the
+// operands change sides): register i is row 8 (i >> 2) + 4 (l >> 5) + (i & 3)
+// and the lane is the operand's feature of tile t (rot_lane_feature).
+template <bool kF32In, bool kSwap>
+__device__ __forceinline__ void rotate_tile(const uint8_t* __restrict__ xsrc, const uint8_t* __restrict__ rop,
+                                            uint8_t* ring, int wave, int lane, floatx16 (&acc)[8]) {
   using Sched = RotSched<kF32In>;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int half = lane >> 5;
-  const int64_t row = (int64_t)blockIdx.x * (kFusedWaves * kTokPerWave) + wave * kTokPerWave + (lane & 31);
-  const bool live = row < rows;
-  const int64_t rr = live ? row : 0;        // a lane past the last row computes row 0 and stores nothing
   // input of K step m: features 128 half + 8m .. +7 (one 16-byte load, or two for fp32)
   u32x4 xr[Sched::kParts * Sched::kPartLoads];
-  const uint8_t* xsrc = static_cast<const uint8_t*>(in) + (rr * in_stride + kPerLane * half) * (kF32In ? 4 : 2);
   auto load_part = [&](int p) {
 #pragma unroll
     for (int i = 0; i < Sched::kPartLoads; ++i)
@@ -570,7 +567,6 @@ __global__ __launch_bounds__(256, 2) void rotate_rows_kernel(const void* __restr
   request(0);
   request(1);
   request(2);
-  floatx16 acc[8];
 #pragma unroll
   for (int t = 0; t < 8; ++t) acc[t] = floatx16{};
   constexpr int kPairs = kF32In ? 24 : 16;      // (fragment, operand) products per K step
@@ -619,7 +615,9 @@ __global__ __launch_bounds__(256, 2) void rotate_rows_kernel(const void* __restr
       const bf16x8 cur = a[i % kAhead];
       if (i + kAhead < kPairs)
         a[i % kAhead] = __builtin_bit_cast(bf16x8, a_src[((i + kAhead) & 15) * 64 + lane]);
-      acc[i & 7] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur, i < 16 ? xh : xl, acc[i & 7], 0, 0, 0);
+      const bf16x8 x = i < 16 ? xh : xl;
+      acc[i & 7] = kSwap ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, cur, acc[i & 7], 0, 0, 0)
+                         : __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur, x, acc[i & 7], 0, 0, 0);
     }
     __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
 #pragma unroll
@@ -628,6 +626,22 @@ __global__ __launch_bounds__(256, 2) void rotate_rows_kernel(const void* __restr
       if (i + kAhead < kPairs) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
   }
+}
+
+template <bool kF32In, bool kBf16Out>
+__global__ __launch_bounds__(256, 2) void rotate_rows_kernel(const void* __restrict__ in, int64_t in_stride,
+                                                            int64_t rows, const uint8_t* __restrict__ rop,
+                                                            void* __restrict__ out, int64_t out_stride) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t ring[];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int half = lane >> 5;
+  const int64_t row = (int64_t)blockIdx.x * (kFusedWaves * kTokPerWave) + wave * kTokPerWave + (lane & 31);
+  const bool live = row < rows;
+  const int64_t rr = live ? row : 0;        // a lane past the last row computes row 0 and stores nothing
+  floatx16 acc[8];
+  rotate_tile<kF32In, false>(static_cast<const uint8_t*>(in) + (rr * in_stride + kPerLane * half) * (kF32In ? 4 : 2),
+                             rop, ring, wave, lane, acc);
   if (!live) return;
   // register i of tile t: output feature 128 half + 16 t + i
   if constexpr (kBf16Out) {
@@ -649,6 +663,112 @@ __global__ __launch_bounds__(256, 2) void rotate_rows_kernel(const void* __restr
       for (int q = 0; q < 4; ++q)
         *reinterpret_cast<floatx4*>(dst + 16 * t + 4 * q) =
             floatx4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
+  }
+}
+
+// Operands of the prefill read (prefill_operands.h) from the step's bf16
+// query, key and value, in one launch: workgroups of 128 query rows, then of
+// four 32-token key tiles, then of four value tiles; each rotates as
+// rotate_rows_kernel does and rounds to fp16 what the read rounded when it
+// built its tiles from fp32 rows.  Queries and keys keep a row per lane; the
+// values' rotation runs with the operands exchanged, so that a lane holds one
+// feature of 16 tokens, which are its two 16-byte chunks of the V tile.
+struct RotateOperandArgs {
+  const uint16_t* q;
+  const uint16_t* k;
+  const uint16_t* v;
+  int64_t q_stride, kv_stride;
+  int32_t num_heads, num_kv_heads;
+  const uint8_t* rot_k;
+  const uint8_t* rot_v;
+  PrefillOperands o;
+  int32_t q_blocks, kv_blocks;
+  OperandItems items;
+};
+
+__global__ __launch_bounds__(256, 2) void rotate_operands_kernel(RotateOperandArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t ring[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = lane >> 5;
+  int blk = blockIdx.x;
+  floatx16 acc[8];
+  // the last item whose first unit (compact token or tile) is at or below u
+  auto item_of = [&](int u, bool tiles) {
+    int i = 0;
+    while (i + 1 < a.items.n && (tiles ? a.items.it[i + 1].tile0 : a.items.it[i + 1].ctok0) <= u) ++i;
+    return i;
+  };
+  if (blk < a.q_blocks) {
+    const int rows = a.items.tokens * a.num_heads;
+    const int row = blk * (kFusedWaves * kTokPerWave) + wave * kTokPerWave + (lane & 31);
+    const int rr = min(row, rows - 1);
+    const int ct = rr / a.num_heads, h = rr - ct * a.num_heads;
+    int i = 0;
+    while (i + 1 < a.items.n && a.items.it[i + 1].ctok0 <= ct) ++i;
+    const int64_t tok = a.items.it[i].tok0 + (ct - a.items.it[i].ctok0);
+    rotate_tile<false, false>(reinterpret_cast<const uint8_t*>(a.q + tok * a.q_stride + (int64_t)h * kHeadDim +
+                                                               kPerLane * half),
+                              a.rot_k, ring, wave, lane, acc);
+    half8* dst = reinterpret_cast<half8*>(a.o.q16 + (int64_t)rr * kHeadDim + kPerLane * half);
+    float qs = 0.f;
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        half8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          o[e] = (_Float16)acc[t][k_feature(8 * g + e)];
+          qs += (float)o[e];
+        }
+        if (row < rows) dst[2 * t + g] = o;
+      }
+    qs += shfl_xor_f32(qs, 32);
+    if (row < rows && half == 0) a.o.qsum[row] = qs;
+    return;
+  }
+  blk -= a.q_blocks;
+  const bool value = blk >= a.kv_blocks;
+  if (value) blk -= a.kv_blocks;
+  const int units = a.items.tiles * a.num_kv_heads;
+  const int u = blk * kFusedWaves + wave;                 // (tile, kv head) of this wave
+  const int uc = min(u, units - 1);
+  const int tile = uc / a.num_kv_heads, head = uc - tile * a.num_kv_heads;
+  const OperandItem it = a.items.it[item_of(tile, true)];
+  const int j = min((tile - it.tile0) * kKeyBlk + (lane & 31), it.n_new - 1);
+  const uint16_t* src = (value ? a.v : a.k) + (int64_t)(it.tok0 + j) * a.kv_stride + (int64_t)head * kHeadDim +
+                        kPerLane * half;
+  if (!value) {
+    rotate_tile<false, false>(reinterpret_cast<const uint8_t*>(src), a.rot_k, ring, wave, lane, acc);
+    if (u >= units) return;
+    const int token = lane & 31;
+    half8* dst = reinterpret_cast<half8*>(a.o.kimg + (int64_t)u * kKeyTileHalfs) + token * (kHeadDim / 8);
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        half8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (_Float16)acc[t][k_feature(8 * g + e)];
+        dst[k_chunk(2 * (8 * half + t) + g, token)] = o;
+      }
+    return;
+  }
+  rotate_tile<false, true>(reinterpret_cast<const uint8_t*>(src), a.rot_v, ring, wave, lane, acc);
+  if (u >= units) return;
+  half8* dst = reinterpret_cast<half8*>(a.o.vimg + (int64_t)u * kKeyTileHalfs);
+  const int r = lane & 31;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    const int f = 128 * ((r >> 2) & 1) + 16 * t + 4 * (r >> 3) + (r & 3);     // the operand's feature of this lane
+#pragma unroll
+    for (int mm = 0; mm < 2; ++mm) {
+      half8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = (_Float16)acc[t][8 * mm + e];
+      dst[f * (kKeyBlk / 8) + v_chunk(2 * mm + half, f)] = o;
+    }
   }
 }
 
@@ -690,8 +810,26 @@ int check_cache_args(CacheArgs& c) {
 
 std::atomic<uint64_t> g_lds_set{0};   // dynamic-LDS attribute set, one bit per device
 std::atomic<uint64_t> g_rot_lds_set[4] = {{0}, {0}, {0}, {0}};   // the same for the rotate_rows instances
+std::atomic<uint64_t> g_operand_lds_set{0};
 
 }  // namespace
+
+int launch_rotate_operands(const uint16_t* q, int64_t q_stride, const uint16_t* k, const uint16_t* v,
+                           int64_t kv_stride, int32_t num_heads, int32_t num_kv_heads, const uint8_t* rot_k,
+                           const uint8_t* rot_v, const OperandItems& items, const PrefillOperands& o,
+                           hipStream_t stream) {
+  RotateOperandArgs a{q, k, v, q_stride, kv_stride, num_heads, num_kv_heads, rot_k, rot_v, o, 0, 0, items};
+  const int64_t rows = (int64_t)items.tokens * num_heads, units = (int64_t)items.tiles * num_kv_heads;
+  a.q_blocks = (int32_t)((rows + kFusedWaves * kTokPerWave - 1) / (kFusedWaves * kTokPerWave));
+  a.kv_blocks = (int32_t)((units + kFusedWaves - 1) / kFusedWaves);
+  constexpr int kRingLds = kRing * kChunkBytes;
+  if (set_dynamic_lds(reinterpret_cast<const void*>(rotate_operands_kernel), kRingLds, g_operand_lds_set) != kOk)
+    return kErrLaunch;
+  hipLaunchKernelGGL(rotate_operands_kernel, dim3((unsigned)(a.q_blocks + 2 * a.kv_blocks)), dim3(256), kRingLds,
+                     stream, a);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
 }  // namespace oscar
 
 using namespace oscar;

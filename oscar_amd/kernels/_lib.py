@@ -59,6 +59,16 @@ SIGNATURES = {
                                             _c_p, _c_i32, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
                                             _c_i64, _c_i64, _c_p, _c_i32, _c_i64, _c_p, _c_p, _c_p,
                                             _c_i32, _c_f32, _c_p, _c_p]),
+    "oscar_prefill_workspace_bytes": (_c_sz, [_c_i32, _c_i32, _c_i32, _c_i64]),
+    "oscar_prefill_continuation_split": (_c_i32, [_c_p, _c_p, _c_p, _c_i32, _c_i32, _c_i32, _c_i32, _c_p,
+                                                  _c_p, _c_i32, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+                                                  _c_i64, _c_i64, _c_p, _c_i32, _c_i64, _c_p, _c_p, _c_p,
+                                                  _c_i32, _c_f32, _c_p, _c_p, _c_sz, _c_p]),
+    "oscar_prefill_rotated_workspace_bytes": (_c_sz, [_c_i32, _c_p, _c_p, _c_i32, _c_i32]),
+    "oscar_prefill_rotated": (_c_i32, [_c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i32, _c_p, _c_p, _c_p, _c_p, _c_i32,
+                                       _c_i32, _c_i32, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i32, _c_i64, _c_i64,
+                                       _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_i32, _c_p, _c_p,
+                                       _c_p, _c_i32, _c_f32, _c_p, _c_p, _c_sz, _c_p]),
     "oscar_staging_write": (_c_i32, [_c_p, _c_p, _c_i64, _c_p, _c_i32, _c_p, _c_p, _c_i32, _c_i32,
                                      _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_p, _c_p, _c_p, _c_p,
                                      _c_p, _c_p, _c_p, _c_p, _c_p]),
