@@ -1855,128 +1855,214 @@ __global__ __launch_bounds__(256) void paged_decode_merge_small_kernel(DecodeArg
   *reinterpret_cast<floatx4*>(a.out + ((int64_t)(it.qa + j) * a.num_heads + h) * kHeadDim + f0) = acc * inv;
 }
 
+// The item of (token, kv head): requests hold consecutive tokens, so it is the
+// last request that starts at or before the token (a request without tokens
+// starts where the next one does).  As in find_item, every lane reads two
+// requests' items and a ballot counts the starts.  Called by every lane of
+// the wavefront with wave-uniform arguments.
+__device__ __forceinline__ ItemInfo find_token_item(const DecodeArgs& a, int tok, int kvh) {
+  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  const int hk = a.num_kv_heads, n = a.nitems;     // items are [request][kv head]
+  if (n == hk) return a.items[kvh];
+  const int i0 = lane * hk + kvh, i1 = (lane + 64) * hk + kvh;
+  const int* f0 = reinterpret_cast<const int*>(&a.items[i0 < n ? i0 : kvh]);
+  const int* f1 = reinterpret_cast<const int*>(&a.items[i1 < n ? i1 : kvh]);
+  int w0[5], w1[5];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    w0[k] = f0[k];
+    w1[k] = f1[k];
+  }
+  static_assert(offsetof(ItemInfo, qa) == 0, "qa is the first word");
+  const int c = __popcll(__ballot(i0 < n && w0[0] <= tok)) + __popcll(__ballot(i1 < n && w1[0] <= tok));
+  const int req = __builtin_amdgcn_readfirstlane(c - 1);
+  int fld[5];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    const int v0 = __builtin_amdgcn_readlane(w0[k], req & 63), v1 = __builtin_amdgcn_readlane(w1[k], req & 63);
+    fld[k] = req < 64 ? v0 : v1;
+  }
+  ItemInfo it;
+  __builtin_memcpy(&it, fld, sizeof(it));
+  return it;
+}
+
 // Merge with the output rotation (the reference's `out @ R_v^T`,
 // backend.py:293-295) and the cast to the model dtype fused in: one
-// 1024-thread block per (output row, quarter of the output features) of an
-// item.  Every load goes out before any wait: the block's 64 columns of R_v^T
-// (wave w: rotated features 16w .. 16w + 15, lane: one output feature), every
-// partial's (m, l) (thread per partial) and the partial rows (wave w: partials
-// w, w + 16, ..., lane: four rotated features).  The block LSE-combines the
-// row over all 256 rotated features, normalises it, multiplies it by its
-// columns of R_v^T (the sixteen waves' sums added in wave order) and writes
-// fp32 or bf16 (RNE).
+// 1024-thread block per (kR consecutive output rows, 1 / kQ of the output
+// features).  Output rows are the launch's (token, head) pairs in memory
+// order, so a block's rows may belong to several requests and no block is
+// launched for a row that a request does not have.  The sixteen waves are
+// dealt to the rows, W = 16 / kR each.  Every load of the first round goes out
+// before any wait: the rows' partials' (m, l) (thread per partial), the
+// partial rows (wave wr of a row: partials wr, wr + W, ..., lane: four rotated
+// features) and, where a thread needs only 16 of them, the block's columns of
+// R_v^T (else they are fetched under the exchange of the row sums).  The block
+// LSE-combines each row over all 256 rotated features, normalises it,
+// multiplies it by its columns of R_v^T in fp32 (chunks of rotated features
+// per wave, added in chunk order) and writes fp32 or bf16 (RNE).
+// A block takes about 4 us whatever its rows (kernel arguments, partials,
+// exchange, R_v^T, exchange), one block fills a CU, and each of a group's kQ
+// blocks reads all of its partials; so what counts is one round of blocks and
+// few readers: 768 rows of 17 partials took 48.8 us as 3072 one-row quarters
+// (12 rounds of the 256 CUs), 14.6 as 8 rows x quarter, 10.5 as 8 rows x half
+// (192 blocks).  A ragged batch of 384 rows and up to 95 partials took 29 us
+// when every request had the blocks of the longest one, and takes 11 as 4
+// rows x half (4 x quarter 15, 8 x half 17).
 constexpr int kRotThreads = 1024;
 constexpr int kRotWaves = kRotThreads / 64;
 constexpr int kRotBatch = 16;                    // partial rows per thread per round
+constexpr int kRotMl = 2;                        // (m, l) pairs per thread, at most
 
+// Partials per row that kR rows per block can combine.
+constexpr int rot_max_partials(int kR) { return kRotMl * kRotThreads / kR; }
+static_assert(rot_max_partials(2) >= kMaxPartials, "one or two rows per block take any launch");
+
+template <int kR, int kQ>
 __global__ __launch_bounds__(kRotThreads) void paged_decode_merge_rotate_kernel(
-    DecodeArgs a, const float* __restrict__ rot_t, void* __restrict__ out, int64_t out_stride, int out_bf16) {
-  __shared__ float wpart[kMaxPartials];
+    DecodeArgs a, int tok0, int rows, FastDiv heads_div, FastDiv group_div, const float* __restrict__ rot_t, void* __restrict__ out, int64_t out_stride,
+    int out_bf16) {
+  constexpr int W = kRotWaves / kR;              // waves per row
+  constexpr int kMl = kR == 1 ? 1 : kRotMl;
+  constexpr int CW = 4 / kQ;                     // waves side by side over the block's output features
+  constexpr int KC = kRotWaves / CW;             // chunks of rotated features
+  constexpr int FK = kHeadDim / KC;              // rotated features per chunk
+  __shared__ float wpart[kR][kMl * 64 * W];
   __shared__ float red[2][kRotWaves];
-  __shared__ floatx4 osum[kRotWaves][64];
-  __shared__ __attribute__((aligned(16))) float orow[kHeadDim];
-  __shared__ float csum[kRotWaves][64];
-  static_assert(kMaxPartials <= kRotThreads, "one partial per thread");
-  // blockIdx.x = (r & 7) + 8 qd + 32 (r >> 3): workgroups are dealt to the 8
-  // XCDs by linear id mod 8, so the four quarter blocks of row r, which all
-  // read the row's every partial, share one XCD and its L2.
-  const int qd = (blockIdx.x >> 3) & 3;
-  const int r = (blockIdx.x & 7) + 8 * (blockIdx.x >> 5);
-  const int item = blockIdx.y;
-  const int rt = blockIdx.z;
-  const ItemInfo it = a.items[item];
-  const int rows = it.nq * a.group;
-  const int row = rt * kRows + r;
-  if (it.nq <= 0 || row >= rows) return;
+  // (the waves' row sums, then, once those are read, their output sums)
+  __shared__ floatx4 sums[kRotWaves * (kR < 4 ? 4 : kR) * 16];
+  floatx4 (&osum)[kRotWaves][64] = *reinterpret_cast<floatx4 (*)[kRotWaves][64]>(sums);
+  float (&csum)[KC][kR][CW * 64] = *reinterpret_cast<float (*)[KC][kR][CW * 64]>(sums);
+  __shared__ __attribute__((aligned(16))) float orow[kR][kHeadDim];
+  // blockIdx.x = (g & 7) + 8 (qd + kQ (g >> 3)) for row group g: workgroups
+  // are dealt to the 8 XCDs by linear id mod 8, so the kQ blocks of a group,
+  // which all read its rows' every partial, share one XCD and its L2.
+  const int qd = (blockIdx.x >> 3) % kQ;
+  const int row0 = kR * ((blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / kQ));
+  if (row0 >= rows) return;
   const int tid = threadIdx.x;
-  const int lane = tid & 63, w = tid >> 6;
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = w % W;
+
+  // ---- every load of the first round ----
+  float rv[FK];
+  const int col = CW == 1 ? lane : 64 * (w % CW) + lane;
+  const float* rcol = rot_t + (int64_t)(FK * (w / CW)) * kHeadDim + 64 * CW * qd + col;
+  auto load_rv = [&]() {
+#pragma unroll
+    for (int k = 0; k < FK; ++k) rv[k] = rcol[(int64_t)k * kHeadDim];
+  };
+  if constexpr (FK <= 16) load_rv();
+  // This wave's row: token and head, the item that holds it, its partials.
+  const int orow_id = row0 + w / W;
+  const bool live = orow_id < rows;
+  const int trow = live ? orow_id : rows - 1;
+  const int to = (int)fast_div((uint32_t)trow, heads_div);
+  const int tok = tok0 + to;
+  const int h = trow - to * a.num_heads;
+  const int kvh = (int)fast_div((uint32_t)h, group_div);
+  const ItemInfo it = find_token_item(a, tok, kvh);
+  const int row = (tok - it.qa) * a.group + (h - kvh * a.group);
+  const int rt = row / kRows, r = row % kRows;
   const int steps = (it.prefix + kStepTok - 1) / kStepTok;
   const int hs = min((int)it.nsplit, steps);
-  const int P = hs + a.fresh;
+  const int P = live ? hs + a.fresh : 0;
   const float* base = a.ws + partial_index(a, it, 0, rt) * kPartialFloats;
   const int64_t pstride = (int64_t)a.row_tiles * kPartialFloats;
   auto partial = [&](int p) { return base + (p < hs ? p : it.nsplit) * pstride; };
-
-  // ---- every load of the first round ----
-  float rv[kHeadDim / kRotWaves];
-  const float* rcol = rot_t + (int64_t)(16 * w) * kHeadDim + 64 * qd + lane;
+  float mp[kMl], lp[kMl];
 #pragma unroll
-  for (int k = 0; k < kHeadDim / kRotWaves; ++k) rv[k] = rcol[(int64_t)k * kHeadDim];
-  float mp = -__builtin_inff(), lp = 0.f;
-  if (tid < P) {
-    mp = partial(tid)[kPartO + r];
-    lp = partial(tid)[kPartO + kRows + r];
+  for (int i = 0; i < kMl; ++i) {
+    const int p = 64 * (wr + W * i) + lane;
+    mp[i] = -__builtin_inff();
+    lp[i] = 0.f;
+    if (p < P) {
+      mp[i] = partial(p)[kPartO + r];
+      lp[i] = partial(p)[kPartO + kRows + r];
+    }
   }
   floatx4 x[kRotBatch];
 #pragma unroll
   for (int k = 0; k < kRotBatch; ++k) {
-    const int p = w + kRotWaves * k;
+    const int p = wr + W * k;
     x[k] = p < P ? *reinterpret_cast<const floatx4*>(partial(p) + r * kHeadDim + 4 * lane) : floatx4{};
   }
 
   // ---- partial weights ----
-  float mloc = mp;
+  float mloc = mp[0];
+#pragma unroll
+  for (int i = 1; i < kMl; ++i) mloc = fmaxf(mloc, mp[i]);
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) mloc = fmaxf(mloc, __shfl_xor(mloc, o, 64));
   if (lane == 0) red[0][w] = mloc;
   __syncthreads();
-  float mx = red[0][0];
+  float mx = red[0][w - wr];
 #pragma unroll
-  for (int ww = 1; ww < kRotWaves; ++ww) mx = fmaxf(mx, red[0][ww]);
-  const float wgt = (mp == -__builtin_inff()) ? 0.f : exp2f(mp - mx);
-  if (tid < P) wpart[tid] = wgt;
-  float lsum = wgt * lp;
+  for (int ww = 1; ww < W; ++ww) mx = fmaxf(mx, red[0][w - wr + ww]);
+  float lsum = 0.f;
+#pragma unroll
+  for (int i = 0; i < kMl; ++i) {
+    const float wgt = (mp[i] == -__builtin_inff()) ? 0.f : exp2f(mp[i] - mx);
+    wpart[w / W][64 * (wr + W * i) + lane] = wgt;
+    lsum = i == 0 ? wgt * lp[i] : fmaf(wgt, lp[i], lsum);
+  }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) lsum += __shfl_xor(lsum, o, 64);
   if (lane == 0) red[1][w] = lsum;
   __syncthreads();
-  float L = 0.f;
-#pragma unroll
-  for (int ww = 0; ww < kRotWaves; ++ww) L += red[1][ww];
 
-  // ---- the row in the rotated domain ----
+  // ---- the rows in the rotated domain ----
   floatx4 acc = floatx4{};
 #pragma unroll
   for (int k = 0; k < kRotBatch; ++k) {
-    const int p = w + kRotWaves * k;
-    if (p < P) acc += wpart[p] * x[k];
+    const int p = wr + W * k;
+    if (p < P) acc += wpart[w / W][p] * x[k];
   }
-  for (int p0 = w + kRotWaves * kRotBatch; p0 < P; p0 += kRotWaves * kRotBatch) {
+  for (int p0 = wr + W * kRotBatch; p0 < P; p0 += W * kRotBatch) {
 #pragma unroll
     for (int k = 0; k < kRotBatch; ++k) {
-      const int p = p0 + kRotWaves * k;
+      const int p = p0 + W * k;
       x[k] = p < P ? *reinterpret_cast<const floatx4*>(partial(p) + r * kHeadDim + 4 * lane) : floatx4{};
     }
 #pragma unroll
     for (int k = 0; k < kRotBatch; ++k) {
-      const int p = p0 + kRotWaves * k;
-      if (p < P) acc += wpart[p] * x[k];
+      const int p = p0 + W * k;
+      if (p < P) acc += wpart[w / W][p] * x[k];
     }
   }
+  if constexpr (FK > 16) load_rv();
   osum[w][lane] = acc;
   __syncthreads();
-  if (w == 0) {
-    floatx4 o = osum[0][lane];
+  if (w < kR) {
+    floatx4 o = osum[w * W][lane];
+    float L = red[1][w * W];
 #pragma unroll
-    for (int ww = 1; ww < kRotWaves; ++ww) o += osum[ww][lane];
+    for (int ww = 1; ww < W; ++ww) {
+      o += osum[w * W + ww][lane];
+      L += red[1][w * W + ww];
+    }
     const float inv = L > 0.f ? 1.f / L : 0.f;
-    *reinterpret_cast<floatx4*>(&orow[4 * lane]) = o * inv;
+    *reinterpret_cast<floatx4*>(&orow[w][4 * lane]) = o * inv;
   }
   __syncthreads();
 
-  // ---- out[64 qd + lane] = sum_f orow[f] * R_v^T[f][64 qd + lane] ----
-  float y = 0.f;
+  // ---- out[c] = sum_f orow[f] * R_v^T[f][c] over the block's features c ----
 #pragma unroll
-  for (int k = 0; k < kHeadDim / kRotWaves; ++k) y = fmaf(orow[16 * w + k], rv[k], y);
-  csum[w][lane] = y;
+  for (int i = 0; i < kR; ++i) {
+    float y = 0.f;
+#pragma unroll
+    for (int k = 0; k < FK; ++k) y = fmaf(orow[i][FK * (w / CW) + k], rv[k], y);
+    csum[w / CW][i][col] = y;
+  }
   __syncthreads();
-  if (w == 0) {
-    float o = csum[0][lane];
+  const int i = w / CW;
+  if (i < kR && row0 + i < rows) {
+    float o = csum[0][i][col];
 #pragma unroll
-    for (int ww = 1; ww < kRotWaves; ++ww) o += csum[ww][lane];
-    const int j = row / a.group;
-    const int h = it.kvh * a.group + (row - j * a.group);
-    const int64_t idx = (int64_t)(it.qa + j) * out_stride + (int64_t)h * kHeadDim + 64 * qd + lane;
+    for (int ww = 1; ww < KC; ++ww) o += csum[ww][i][col];
+    const int to = (int)fast_div((uint32_t)(row0 + i), heads_div);
+    const int64_t idx = (int64_t)(tok0 + to) * out_stride + (int64_t)(row0 + i - to * a.num_heads) * kHeadDim +
+                        64 * CW * qd + col;
     if (out_bf16)
       reinterpret_cast<__bf16*>(out)[idx] = (__bf16)o;
     else
@@ -2279,9 +2365,29 @@ int launch_merge(const DecodeArgs& a, int64_t max_rows, unsigned nitems, const O
                  hipStream_t stream) {
   const int mr = merge_rows(max_rows);
   if (orot.rot_t != nullptr) {
-    dim3 grid((unsigned)(32 * ((mr + 7) / 8)), nitems, (unsigned)a.row_tiles);
-    hipLaunchKernelGGL(paged_decode_merge_rotate_kernel, grid, dim3(kRotThreads), 0, stream, a, orot.rot_t, orot.out,
-                       orot.out_stride, (int)orot.out_bf16);
+    const int tok0 = a.items[0].qa;
+    const ItemInfo& last = a.items[nitems - 1];
+    const int rows = (int)(last.qa + last.nq - tok0) * a.num_heads;
+    if (rows == 0) return kOk;
+    // Rows per block: the fewest that keep the launch's blocks within one
+    // round of the CUs, as far as the partials per row allow (one row of few
+    // is quickest by itself: 24 rows of 193 partials take 7.0 us, 6 of 9
+    // partials 4.9).
+    const int P = a.max_splits + a.fresh;
+    const FastDiv heads_div = make_fast_div((uint32_t)a.num_heads), group_div = make_fast_div((uint32_t)a.group);
+    auto blocks = [&](int kR, int kQ) { return 8u * kQ * (unsigned)((rows + 8 * kR - 1) / (8 * kR)); };
+    auto go = [&](auto kernel, int kR, int kQ) {
+      hipLaunchKernelGGL(kernel, dim3(blocks(kR, kQ)), dim3(kRotThreads), 0, stream, a, tok0, rows, heads_div, group_div, orot.rot_t,
+                         orot.out, orot.out_stride, (int)orot.out_bf16);
+    };
+    if (blocks(1, 4) <= 256)
+      go(paged_decode_merge_rotate_kernel<1, 4>, 1, 4);
+    else if (blocks(2, 4) <= 256 || P > rot_max_partials(4))
+      go(paged_decode_merge_rotate_kernel<2, 4>, 2, 4);
+    else if (blocks(4, 2) <= 256 || P > rot_max_partials(8))
+      go(paged_decode_merge_rotate_kernel<4, 2>, 4, 2);
+    else
+      go(paged_decode_merge_rotate_kernel<8, 2>, 8, 2);
   } else if (a.max_splits + a.fresh <= kSmallP) {
     dim3 grid((unsigned)((mr * 4 + 15) / 16), nitems, (unsigned)a.row_tiles);
     hipLaunchKernelGGL(paged_decode_merge_small_kernel, grid, dim3(256), 0, stream, a);
