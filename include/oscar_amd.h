@@ -397,6 +397,26 @@ int oscar_mtp_forward(const oscar_mtp_layer* layer, const oscar_mtp_step* step, 
                       int64_t kv_token_stride, void* out, int64_t out_token_stride, int32_t out_bf16,
                       oscar_stream_t stream);
 
+/* ---------------------------------------------------------------- DecodeOnly forward
+ * The forward of one layer in the DecodeOnly state (no fresh K/V, one query
+ * token per request): query @ R_k in fp32, oscar_decode_only, and @ R_v^T with
+ * the output cast in its merge, on one stream.  Replaces the reference's
+ * _forward_decode (oscar_ascend/backend.py:321-358).
+ * The layer is oscar_mtp_forward's (rot_v and the fp32 arena are not read);
+ * query_bf16 [num_requests][query_token_stride], out
+ * [num_requests][out_token_stride] bf16 (out_bf16 = 1) or fp32; seq_lens is a
+ * HOST array, the other arguments are oscar_decode_only's.  workspace: 16-byte
+ * aligned, >= oscar_decode_only_forward_workspace_bytes(...) bytes.  Every
+ * argument is checked before anything is enqueued.
+ */
+size_t oscar_decode_only_forward_workspace_bytes(int32_t num_requests, int32_t num_kv_heads, int32_t num_heads,
+                                                 int64_t max_history);
+int oscar_decode_only_forward(const oscar_mtp_layer* layer, const void* query_bf16, int64_t query_token_stride,
+                              const int32_t* block_table, int64_t block_table_stride, int32_t block_table_cols,
+                              const int32_t* seq_lens, int32_t num_requests, int64_t max_history, void* out,
+                              int64_t out_token_stride, int32_t out_bf16, void* workspace, size_t workspace_size,
+                              oscar_stream_t stream);
+
 /* ---------------------------------------------------------------- window write
  * Record the step's tokens in the FP32 sink/recent staging arena.
  * Replaces the torch body of _staging_write (oscar_ascend/backend.py:439-481)

@@ -297,6 +297,9 @@ class OscarAttentionBackendImpl:
             # has a read path (the reference's dense route needs the keys)
             if not _is_decode_only(getattr(attn_metadata, "attn_state", None)):
                 raise NotImplementedError("OSCAR reads without fresh K/V need the DecodeOnly attention state")
+            if self._decode_only_step(layer, query, kv_cache, attn_metadata, output):
+                self._oscar_stats["reads"] += 1
+                return output
             attn_out = self._decode_attention(layer, query, attn_metadata)
             self._oscar_stats["reads"] += 1
             output[:num_tokens] = attn_out.reshape(output[:num_tokens].shape).to(output.dtype)
@@ -369,6 +372,27 @@ class OscarAttentionBackendImpl:
                            arena if cfg.window_enabled else None, (cfg.sink_tokens // bs) * bs, cfg.recent_tokens)
         layer._oscar_mtp = ml
         return ml
+
+    def _decode_only_step(self, layer, query, kv_cache, attn_metadata, output) -> bool:
+        """The DecodeOnly forward of a bf16 model in one library call: fp32
+        query rotation, read, and R_v^T with the cast in its merge.  Returns
+        False (nothing done) for what takes the general route: other dtypes,
+        small pages, an arena that no step has written yet, a query count that
+        route refuses."""
+        cfg = self._oscar
+        N = query.shape[0]
+        if query.dtype != torch.bfloat16 or output.dtype != torch.bfloat16 or output.device != query.device \
+                or output.shape[0] < N or N == 0 or self.key_cache.shape[1] % 32 \
+                or query.numel() != N * self.num_heads * self.head_size:
+            return False
+        if cfg.window_enabled and not getattr(layer, "_oscar_stage_ready", False):
+            return False
+        qsl, seqs = metadata_batch_lists(attn_metadata)
+        if N != len(seqs) or any(b - a != 1 for a, b in itertools.pairwise(qsl[:N + 1])):
+            return False
+        dev = query.device
+        return step.decode_only_forward(self._mtp_layer(layer, kv_cache, dev), query, attn_metadata.block_tables,
+                                        seqs, output, _lib.stream_handle(dev))
 
     def _decode_attention(self, layer, query, attn_metadata) -> torch.Tensor:
         """backend.py:321-358, 500-586 — one query token per request over its

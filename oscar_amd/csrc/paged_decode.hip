@@ -74,6 +74,7 @@
 #include <type_traits>
 
 #include "oscar_common.h"
+#include "step_rotate.h"
 #include "window_images.h"
 #include "../../include/oscar_amd.h"
 
@@ -2581,6 +2582,84 @@ int scratch_address(void** out) {
   return kOk;
 }
 
+// oscar_decode_only; `before` enqueues what the read waits for once every
+// argument has been checked, and `orot` as in oscar_paged_decode_rotated.
+template <class Before>
+int decode_only(const float* q_rot, int32_t num_heads, int32_t num_kv_heads, int32_t head_size,
+                const void* k_cache, const void* v_cache, int32_t block_size, int64_t num_pages,
+                int64_t k_stride_page, int64_t k_stride_token, int64_t k_stride_head,
+                int64_t v_stride_page, int64_t v_stride_token, int64_t v_stride_head,
+                const int32_t* block_table, int64_t block_table_stride, int32_t block_table_cols,
+                const int32_t* seq_lens, int32_t num_requests, int64_t max_history,
+                const int64_t* stage_owner, const void* stage_k_image, const void* stage_v_image,
+                int32_t stage_rows, int32_t sink_tokens, int32_t recent_tokens, float scale,
+                int32_t tiles_per_split, float* out, const OutRotation& orot, void* workspace,
+                size_t workspace_size, hipStream_t stream, Before before) {
+  if (head_size != kHeadDim) return kErrUnsupportedHeadDim;
+  if (num_requests < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_kv_heads > kMaxInlineItems ||
+      num_heads % num_kv_heads != 0 || max_history < 0 ||
+      block_size <= 0 || num_pages <= 0 || block_table_cols < 0 || stage_rows < 0 || sink_tokens < 0 ||
+      recent_tokens < 0 || tiles_per_split < 0 || tiles_per_split > kMaxTilesPerSplit)
+    return kErrInvalidArgument;
+  if (num_requests == 0) return kOk;
+  DecodeArgs a{};
+  int rc = fill_common(a, q_rot, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages,
+                 k_stride_page, k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
+                 block_table, block_table_stride, block_table_cols, max_history, stage_owner, stage_k_image,
+                 stage_v_image, stage_rows, scale, out, workspace);
+  if (rc != kOk) return rc;
+  if (!seq_lens) return kErrInvalidArgument;
+  for (int32_t i = 0; i < num_requests; ++i)
+    if (seq_lens[i] < 0 || seq_lens[i] > max_history) return kErrInvalidArgument;
+  if (tiles_per_split > 0 && splits_for(max_history, tiles_per_split) > kMaxSplits) return kErrInvalidArgument;
+  if (tiles_per_split == 0 && (max_history + kStepTok - 1) / kStepTok > kMaxSplits * kMaxStepsPerSplit)
+    return kErrInvalidArgument;
+  const size_t partials = workspace_floats(num_requests, num_kv_heads, num_heads, 1, max_history,
+                                     tiles_per_split) * sizeof(float);
+  const int32_t per = requests_per_launch(num_kv_heads);
+  const size_t need = bounds_offset(partials) +
+                (size_t)(num_requests < per ? num_requests : per) * 2 * sizeof(int32_t);
+  if (workspace == nullptr || workspace_size < need) return kErrWorkspaceTooSmall;
+  const bool window = stage_rows > 0;
+  int32_t* bounds = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(workspace) + bounds_offset(partials));
+  const int32_t sink_eff = window ? (sink_tokens / block_size) * block_size : 0;
+  a.k_new = nullptr;
+  a.v_new = nullptr;
+  // One query per request: the small-row kernel reads when the group has at
+  // most 8 heads, and then finds the bounds itself when each of the sink and
+  // recent spans fits one position per thread; else the bounds kernel runs.
+  const bool fold = window && a.group <= kSmRows && sink_eff <= 256 && recent_tokens <= 256;
+  a.win = window && !fold ? bounds : nullptr;
+  a.win_fold = fold ? 1 : 0;
+  a.win_sink = sink_eff;
+  a.win_recent = recent_tokens;
+  a.fresh = 0;
+  a.row_tiles = (a.group + kRows - 1) / kRows;
+  if ((rc = set_split_lds()) != kOk) return rc;
+  if ((rc = before()) != kOk) return rc;
+  for (int32_t c0 = 0; c0 < num_requests; c0 += per) {
+    const int32_t nreq = num_requests - c0 < per ? num_requests - c0 : per;
+    for (int32_t i = 0; i < nreq; ++i)
+      for (int32_t h = 0; h < num_kv_heads; ++h)
+        a.items[i * num_kv_heads + h] = ItemInfo{c0 + i, seq_lens[c0 + i], 0, 1, (int16_t)i, (int16_t)h, 0};
+    a.block_table = block_table ? block_table + (int64_t)c0 * block_table_stride : nullptr;
+    const unsigned nitems = (unsigned)(nreq * num_kv_heads);
+    if (!plan_splits(a, nitems, max_history, tiles_per_split, 0)) return kErrInvalidArgument;
+    if (window && !fold) {
+      hipLaunchKernelGGL(decode_only_bounds_kernel, dim3((unsigned)nreq), dim3(kBoundsThreads), 0, stream, a, bounds,
+                   sink_eff, recent_tokens);
+      if (hipGetLastError() != hipSuccess) return kErrLaunch;
+    }
+    const unsigned gx = split_workgroups(a);
+    if (gx > 0) {
+      launch_split(a, nitems, dim3(gx, 1, (unsigned)a.row_tiles), stream);
+      if (hipGetLastError() != hipSuccess) return kErrLaunch;
+    }
+    if ((rc = launch_merge(a, a.group, nitems, orot, stream)) != kOk) return rc;
+  }
+  return kOk;
+}
+
 }  // namespace
 }  // namespace oscar
 
@@ -2680,68 +2759,51 @@ int oscar_decode_only(const float* q_rot, int32_t num_heads, int32_t num_kv_head
                       int32_t stage_rows, int32_t sink_tokens, int32_t recent_tokens, float scale,
                       int32_t tiles_per_split, float* out, void* workspace, size_t workspace_size,
                       hipStream_t stream) {
-  if (head_size != kHeadDim) return kErrUnsupportedHeadDim;
-  if (num_requests < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_kv_heads > kMaxInlineItems ||
-      num_heads % num_kv_heads != 0 || max_history < 0 ||
-      block_size <= 0 || num_pages <= 0 || block_table_cols < 0 || stage_rows < 0 || sink_tokens < 0 ||
-      recent_tokens < 0 || tiles_per_split < 0 || tiles_per_split > kMaxTilesPerSplit)
-    return kErrInvalidArgument;
+  return decode_only(q_rot, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages,
+                     k_stride_page, k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
+                     block_table, block_table_stride, block_table_cols, seq_lens, num_requests, max_history,
+                     stage_owner, stage_k_image, stage_v_image, stage_rows, sink_tokens, recent_tokens, scale,
+                     tiles_per_split, out, OutRotation{nullptr, nullptr, 0, 0}, workspace, workspace_size, stream,
+                     []() { return (int)kOk; });
+}
+
+size_t oscar_decode_only_forward_workspace_bytes(int32_t num_requests, int32_t num_kv_heads, int32_t num_heads,
+                                                 int64_t max_history) {
+  const size_t read = oscar_decode_only_workspace_bytes(num_requests, num_kv_heads, num_heads, max_history, 0);
+  return read == 0 ? 0 : (size_t)num_requests * num_heads * kHeadDim * sizeof(float) + read;
+}
+
+// The DecodeOnly forward of one layer: fp32 query rotation, read, and the
+// output rotation in its merge (three launches; the rotations were two
+// library matrix products between conversions and copies, 91 us of host and
+// launch time around a 25 us read of 8 x 32K tokens).
+int oscar_decode_only_forward(const oscar_mtp_layer* layer, const void* query_bf16, int64_t query_token_stride,
+                              const int32_t* block_table, int64_t block_table_stride, int32_t block_table_cols,
+                              const int32_t* seq_lens, int32_t num_requests, int64_t max_history, void* out,
+                              int64_t out_token_stride, int32_t out_bf16, void* workspace, size_t workspace_size,
+                              hipStream_t stream) {
+  if (!layer) return kErrInvalidArgument;
+  const oscar_mtp_layer& L = *layer;
+  const int32_t rows = L.stage_rows;
+  if (num_requests < 0 || L.num_heads <= 0 || out_bf16 < 0 || out_bf16 > 1) return kErrInvalidArgument;
   if (num_requests == 0) return kOk;
-  DecodeArgs a{};
-  int rc = fill_common(a, q_rot, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages,
-                       k_stride_page, k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
-                       block_table, block_table_stride, block_table_cols, max_history, stage_owner, stage_k_image,
-                       stage_v_image, stage_rows, scale, out, workspace);
-  if (rc != kOk) return rc;
-  if (!seq_lens) return kErrInvalidArgument;
-  for (int32_t i = 0; i < num_requests; ++i)
-    if (seq_lens[i] < 0 || seq_lens[i] > max_history) return kErrInvalidArgument;
-  if (tiles_per_split > 0 && splits_for(max_history, tiles_per_split) > kMaxSplits) return kErrInvalidArgument;
-  if (tiles_per_split == 0 && (max_history + kStepTok - 1) / kStepTok > kMaxSplits * kMaxStepsPerSplit)
+  const int64_t width = (int64_t)L.num_heads * kHeadDim;
+  if (!L.rot_k || !L.rot_v_t || !query_bf16 || !out || query_token_stride < width || out_token_stride < width ||
+      (reinterpret_cast<uintptr_t>(L.rot_k) & 15) || (reinterpret_cast<uintptr_t>(workspace) & 15))
     return kErrInvalidArgument;
-  const size_t partials = workspace_floats(num_requests, num_kv_heads, num_heads, 1, max_history,
-                                           tiles_per_split) * sizeof(float);
-  const int32_t per = requests_per_launch(num_kv_heads);
-  const size_t need = bounds_offset(partials) +
-                      (size_t)(num_requests < per ? num_requests : per) * 2 * sizeof(int32_t);
-  if (workspace == nullptr || workspace_size < need) return kErrWorkspaceTooSmall;
-  const bool window = stage_rows > 0;
-  int32_t* bounds = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(workspace) + bounds_offset(partials));
-  const int32_t sink_eff = window ? (sink_tokens / block_size) * block_size : 0;
-  a.k_new = nullptr;
-  a.v_new = nullptr;
-  // One query per request: the small-row kernel reads when the group has at
-  // most 8 heads, and then finds the bounds itself when each of the sink and
-  // recent spans fits one position per thread; else the bounds kernel runs.
-  const bool fold = window && a.group <= kSmRows && sink_eff <= 256 && recent_tokens <= 256;
-  a.win = window && !fold ? bounds : nullptr;
-  a.win_fold = fold ? 1 : 0;
-  a.win_sink = sink_eff;
-  a.win_recent = recent_tokens;
-  a.fresh = 0;
-  a.row_tiles = (a.group + kRows - 1) / kRows;
-  if ((rc = set_split_lds()) != kOk) return rc;
-  for (int32_t c0 = 0; c0 < num_requests; c0 += per) {
-    const int32_t nreq = num_requests - c0 < per ? num_requests - c0 : per;
-    for (int32_t i = 0; i < nreq; ++i)
-      for (int32_t h = 0; h < num_kv_heads; ++h)
-        a.items[i * num_kv_heads + h] = ItemInfo{c0 + i, seq_lens[c0 + i], 0, 1, (int16_t)i, (int16_t)h, 0};
-    a.block_table = block_table ? block_table + (int64_t)c0 * block_table_stride : nullptr;
-    const unsigned nitems = (unsigned)(nreq * num_kv_heads);
-    if (!plan_splits(a, nitems, max_history, tiles_per_split, 0)) return kErrInvalidArgument;
-    if (window && !fold) {
-      hipLaunchKernelGGL(decode_only_bounds_kernel, dim3((unsigned)nreq), dim3(kBoundsThreads), 0, stream, a, bounds,
-                         sink_eff, recent_tokens);
-      if (hipGetLastError() != hipSuccess) return kErrLaunch;
-    }
-    const unsigned gx = split_workgroups(a);
-    if (gx > 0) {
-      launch_split(a, nitems, dim3(gx, 1, (unsigned)a.row_tiles), stream);
-      if (hipGetLastError() != hipSuccess) return kErrLaunch;
-    }
-    if ((rc = launch_merge(a, a.group, nitems, OutRotation{nullptr, nullptr, 0, 0}, stream)) != kOk) return rc;
-  }
-  return kOk;
+  const size_t q_bytes = (size_t)num_requests * width * sizeof(float);
+  if (workspace == nullptr || workspace_size < q_bytes) return kErrWorkspaceTooSmall;
+  float* q_rot = static_cast<float*>(workspace);
+  return decode_only(q_rot, L.num_heads, L.num_kv_heads, L.head_size, L.k_cache, L.v_cache, L.block_size, L.num_pages,
+                     L.k_stride_page, L.k_stride_token, L.k_stride_head, L.v_stride_page, L.v_stride_token,
+                     L.v_stride_head, block_table, block_table_stride, block_table_cols, seq_lens, num_requests,
+                     max_history, rows > 0 ? L.stage_owner : nullptr, rows > 0 ? L.stage_k_image : nullptr,
+                     rows > 0 ? L.stage_v_image : nullptr, rows, L.sink_eff, L.recent, L.scale, 0,
+                     reinterpret_cast<float*>(out), OutRotation{L.rot_v_t, out, out_token_stride, out_bf16},
+                     static_cast<uint8_t*>(workspace) + q_bytes, workspace_size - q_bytes, stream, [&]() {
+                       return launch_rotate_queries(static_cast<const uint16_t*>(query_bf16), query_token_stride,
+                                                    num_requests, L.num_heads, L.rot_k, q_rot, stream);
+                     });
 }
 
 // The short-step forward of one layer: every argument of the decode is

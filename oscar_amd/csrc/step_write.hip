@@ -27,6 +27,7 @@
 // 256 |x| (ballots), quantizes with the exact thresholds of int2_quant.h,
 // writes the slot and, when it is its seat's winner, the window.
 #include "int2_quant.h"
+#include "step_rotate.h"
 #include "window_images.h"
 #include "../../include/oscar_amd.h"
 
@@ -363,7 +364,31 @@ __global__ __launch_bounds__(kThreads) void step_write_kernel(StepArgs a) {
   if (side < 2) write_vector(ctx, y, t, h, side, lane, my_slot, later, keep_word);
 }
 
+// Vectors per workgroup: one while the step has few vectors (every workgroup
+// streams R once; fewer vectors each finish sooner), up to four for larger
+// steps.
+int32_t vecs_per_group(int64_t vectors) { return vectors <= 512 ? 1 : (vectors <= 2048 ? 2 : 4); }
+
 }  // namespace
+}  // namespace oscar
+
+namespace oscar {
+
+int launch_rotate_queries(const uint16_t* q, int64_t q_stride, int32_t n_tokens, int32_t num_heads, const float* rot_k,
+                          float* q_rot, hipStream_t stream) {
+  StepArgs a{};
+  a.q = q;
+  a.q_stride = q_stride;
+  a.n_tokens = n_tokens;
+  a.num_heads = num_heads;
+  a.rot_k = rot_k;
+  a.q_rot = q_rot;
+  a.vecs_per_group = vecs_per_group((int64_t)n_tokens * num_heads);
+  const int64_t groups = ((int64_t)n_tokens * num_heads + a.vecs_per_group - 1) / a.vecs_per_group;
+  hipLaunchKernelGGL(step_write_kernel, dim3((unsigned)groups), dim3(kThreads), 0, stream, a);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
 }  // namespace oscar
 
 using namespace oscar;
@@ -447,11 +472,7 @@ extern "C" int oscar_step_write(const void* query_bf16, int64_t query_token_stri
       if (pos >= (int64_t)seq_lens[i] - recent || pos < sink_eff) a.keep[t >> 5] |= 1u << (t & 31);
     }
   }
-  // Vectors per workgroup: one while the step has few vectors (every
-  // workgroup streams R once; fewer vectors each finish sooner), up to four
-  // for larger steps.
-  const int64_t vectors = (int64_t)num_tokens * (num_heads + 2 * num_kv_heads);
-  a.vecs_per_group = vectors <= 512 ? 1 : (vectors <= 2048 ? 2 : 4);
+  a.vecs_per_group = vecs_per_group((int64_t)num_tokens * (num_heads + 2 * num_kv_heads));
   a.kv_groups = (int32_t)(((int64_t)num_tokens * num_kv_heads + a.vecs_per_group - 1) / a.vecs_per_group);
   const int64_t q_groups = ((int64_t)num_tokens * num_heads + a.vecs_per_group - 1) / a.vecs_per_group;
   hipLaunchKernelGGL(step_write_kernel, dim3((unsigned)(2 * a.kv_groups + q_groups)), dim3(kThreads), 0, stream, a);

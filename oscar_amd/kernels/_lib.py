@@ -55,6 +55,9 @@ SIGNATURES = {
                                    _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_i32,
                                    _c_p, _c_i32, _c_i64, _c_p, _c_p, _c_p, _c_i32, _c_i32, _c_i32,
                                    _c_f32, _c_i32, _c_p, _c_p, _c_sz, _c_p]),
+    "oscar_decode_only_forward_workspace_bytes": (_c_sz, [_c_i32, _c_i32, _c_i32, _c_i64]),
+    "oscar_decode_only_forward": (_c_i32, [_c_p, _c_p, _c_i64, _c_p, _c_i64, _c_i32, _c_p, _c_i32, _c_i64, _c_p,
+                                           _c_i64, _c_i32, _c_p, _c_sz, _c_p]),
     "oscar_prefill_continuation": (_c_i32, [_c_p, _c_p, _c_p, _c_i32, _c_i32, _c_i32, _c_i32, _c_p,
                                             _c_p, _c_i32, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
                                             _c_i64, _c_i64, _c_p, _c_i32, _c_i64, _c_p, _c_p, _c_p,

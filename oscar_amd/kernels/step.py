@@ -277,3 +277,34 @@ def mtp_forward(layer: MtpLayer, st: MtpStep, query, key, value, out, stream: in
     if status != 0:
         raise _lib.OscarKernelError(f"oscar_mtp_forward failed: {_lib.STATUS.get(status, status)}")
     return out
+
+
+def decode_only_forward(layer: MtpLayer, query, block_table, seqs, out, stream: int) -> bool:
+    """One layer's DecodeOnly forward (backend.py:321-358) through
+    oscar_decode_only_forward: query [B, Hq*D] (or [B, Hq, D]) bf16, one row
+    per request of the host lengths ``seqs``, out rows [>= B] bf16 or fp32 in
+    the model domain.  Returns False, with nothing enqueued, when the output's
+    rows do not hold Hq * D contiguous features."""
+    B = len(seqs)
+    hq, hk, D = layer.num_heads, layer.num_kv_heads, layer.head_size
+    os_ = _row_stride(out, B, hq * D)
+    if os_ < 0:
+        return False
+    if any(s < 0 for s in seqs) or block_table.ndim != 2 or block_table.shape[0] < B:
+        raise ValueError("DecodeOnly needs a non-negative length and a block-table row per request")
+    qs = _row_stride(query, B, hq * D)
+    if qs < 0:
+        query, qs = _rows(query, B, hq * D)
+    if block_table.dtype != torch.int32 or block_table.device != query.device or block_table.stride(1) != 1:
+        block_table = block_table.to(device=query.device, dtype=torch.int32).contiguous()
+    seq_t = (_i32 * B)(*seqs)
+    longest = max(seqs)
+    lib = _lib.load()
+    ws = decode.workspace(query.device, lib.oscar_decode_only_forward_workspace_bytes(B, hk, hq, longest))
+    status = lib.oscar_decode_only_forward(layer.ref, query.data_ptr(), qs, block_table.data_ptr(),
+                                           block_table.stride(0), block_table.shape[1], ctypes.addressof(seq_t), B,
+                                           longest, out.data_ptr(), os_, int(out.dtype == torch.bfloat16),
+                                           ws.data_ptr(), ws.numel(), stream)
+    if status != 0:
+        raise _lib.OscarKernelError(f"oscar_decode_only_forward failed: {_lib.STATUS.get(status, status)}")
+    return True
