@@ -74,7 +74,7 @@
 #include <type_traits>
 
 #include "oscar_common.h"
-#include "step_rotate.h"
+#include "step_launch.h"
 #include "window_images.h"
 #include "../../include/oscar_amd.h"
 

@@ -26,6 +26,7 @@
 // (see window_epilogue), after a seat-winner pass over the step's slots.
 #include "int2_quant.h"
 #include "prefill_operands.h"
+#include "step_launch.h"
 #include "window_images.h"
 #include "../../include/oscar_amd.h"
 
@@ -953,13 +954,13 @@ int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_t
     const uint8_t* ok = static_cast<const uint8_t*>(rot_k_operand) + kMfmaOperandBytes;
     const uint8_t* ov = static_cast<const uint8_t*>(rot_v_operand) + kMfmaOperandBytes;
     const bool win = w.rows > 0;
-    return oscar_step_write(nullptr, 0, key_bf16, value_bf16, token_stride, (int32_t)num_tokens, 0, num_kv_heads,
-                            head_size, reinterpret_cast<const float*>(ok), reinterpret_cast<const float*>(ov),
-                            slot_mapping, win ? w.query_start : nullptr, win ? w.seq_lens : nullptr,
-                            win ? w.num_requests : 0, k_cache, v_cache, block_size, num_pages, k_stride_page,
-                            k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
-                            clip_index_k, clip_index_v, w.stage_k, w.stage_v, w.owner, w.kimg, w.vimg, w.rows,
-                            w.sink_eff, w.recent, nullptr, nullptr, nullptr, stream);
+    return step_write(true, nullptr, 0, key_bf16, value_bf16, token_stride, (int32_t)num_tokens, 0, num_kv_heads,
+                      head_size, reinterpret_cast<const float*>(ok), reinterpret_cast<const float*>(ov),
+                      slot_mapping, win ? w.query_start : nullptr, win ? w.seq_lens : nullptr,
+                      win ? w.num_requests : 0, k_cache, v_cache, block_size, num_pages, k_stride_page,
+                      k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
+                      clip_index_k, clip_index_v, w.stage_k, w.stage_v, w.owner, w.kimg, w.vimg, w.rows,
+                      w.sink_eff, w.recent, nullptr, nullptr, nullptr, stream);
   }
   if (set_dynamic_lds(reinterpret_cast<const void*>(quant_write_fused_kernel), (int)kFusedLds, g_lds_set) != kOk) return kErrLaunch;
   const int64_t per_block = kFusedWaves * kTokPerWave;

@@ -27,7 +27,7 @@
 // 256 |x| (ballots), quantizes with the exact thresholds of int2_quant.h,
 // writes the slot and, when it is its seat's winner, the window.
 #include "int2_quant.h"
-#include "step_rotate.h"
+#include "step_launch.h"
 #include "window_images.h"
 #include "../../include/oscar_amd.h"
 
@@ -68,7 +68,10 @@ struct StepArgs {
   float* v_rot;
   int32_t vecs_per_group;       // 1, 2 or 4
   int32_t kv_groups;            // workgroups per side (K, V)
-  uint32_t keep[kMaxStepTokens / 32];   // bit t: the window keeps token t
+  uint32_t keep[kMaxStepTokens / 32];   // bit t: the window keeps token t (host request layout)
+  const int32_t* query_start;   // the request layout on the device, or null: keep holds the rule
+  const int32_t* seq_lens;
+  int32_t num_requests, sink_eff, recent;
 };
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t x) { return __uint_as_float((uint32_t)x << 16); }
@@ -285,6 +288,23 @@ __device__ void write_vector(const WriteCtx& a, const floatx4& y, int t, int h, 
   }
 }
 
+// The window's keep rule of token t from the request layout on the device: t
+// lies in the last request that starts at or before it, at position
+// seq - (end - t).  Called by every lane of the wavefront with the same t; a
+// token outside the layout is not kept.
+__device__ bool layout_keeps(const StepArgs& a, int t, int lane) {
+  int starts = 0;                       // entries of query_start (the end included) at or before t
+#pragma unroll 1
+  for (int base = 0; base <= a.num_requests; base += 64) {
+    const int i = base + lane;
+    starts += __popcll(__ballot(i <= a.num_requests && a.query_start[min(i, a.num_requests)] <= t));
+  }
+  if (starts < 1 || starts > a.num_requests) return false;
+  const int64_t seq = a.seq_lens[starts - 1];
+  const int64_t pos = seq - a.query_start[starts] + t;
+  return pos >= seq - a.recent || pos < a.sink_eff;
+}
+
 __global__ __launch_bounds__(kThreads) void step_write_kernel(StepArgs a) {
   __shared__ __attribute__((aligned(16))) float xs[kGroupVecs][kHeadDim];
   __shared__ __attribute__((aligned(16))) float part[kWaves][kGroupVecs][kHeadDim];
@@ -324,7 +344,7 @@ __global__ __launch_bounds__(kThreads) void step_write_kernel(StepArgs a) {
   ctx.clip = side == 0 ? c.clip_k : c.clip_v;
   if (side < 2 && w < nv) {
     const int t = (e0 + w) / heads;
-    keep_word = a.keep[t >> 5];
+    keep_word = a.query_start != nullptr ? (layout_keeps(a, t, lane) ? ~0u : 0u) : a.keep[t >> 5];
     my_slot = ctx.slots[t];
     later = t + 1 + lane < ctx.n_tokens ? ctx.slots[t + 1 + lane] : -1;
   }
@@ -391,19 +411,19 @@ int launch_rotate_queries(const uint16_t* q, int64_t q_stride, int32_t n_tokens,
 
 }  // namespace oscar
 
-using namespace oscar;
+namespace oscar {
 
-extern "C" int oscar_step_write(const void* query_bf16, int64_t query_token_stride, const void* key_bf16,
-                                const void* value_bf16, int64_t kv_token_stride, int32_t num_tokens,
-                                int32_t num_heads, int32_t num_kv_heads, int32_t head_size, const float* rot_k,
-                                const float* rot_v, const int64_t* slot_mapping, const int32_t* query_start_loc,
-                                const int32_t* seq_lens, int32_t num_requests, void* k_cache, void* v_cache,
-                                int32_t block_size, int64_t num_pages, int64_t k_stride_page,
-                                int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page,
-                                int64_t v_stride_token, int64_t v_stride_head, int32_t clip_index_k,
-                                int32_t clip_index_v, float* stage_k, float* stage_v, int64_t* stage_owner,
-                                void* stage_k_image, void* stage_v_image, int32_t stage_rows, int32_t sink_eff,
-                                int32_t recent, float* q_rot, float* k_rot, float* v_rot, hipStream_t stream) {
+int step_write(bool layout_on_device, const void* query_bf16, int64_t query_token_stride,
+               const void* key_bf16, const void* value_bf16, int64_t kv_token_stride, int32_t num_tokens,
+               int32_t num_heads, int32_t num_kv_heads, int32_t head_size, const float* rot_k,
+               const float* rot_v, const int64_t* slot_mapping, const int32_t* query_start_loc,
+               const int32_t* seq_lens, int32_t num_requests, void* k_cache, void* v_cache,
+               int32_t block_size, int64_t num_pages, int64_t k_stride_page,
+               int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page,
+               int64_t v_stride_token, int64_t v_stride_head, int32_t clip_index_k,
+               int32_t clip_index_v, float* stage_k, float* stage_v, int64_t* stage_owner,
+               void* stage_k_image, void* stage_v_image, int32_t stage_rows, int32_t sink_eff,
+               int32_t recent, float* q_rot, float* k_rot, float* v_rot, hipStream_t stream) {
   if (head_size != kHeadDim) return kErrUnsupportedHeadDim;
   if (num_tokens < 0 || num_tokens > kMaxStepTokens || num_requests < 0 || num_heads < 0 ||
       num_kv_heads <= 0 || num_heads % num_kv_heads != 0 || block_size <= 0 || num_pages <= 0 ||
@@ -462,9 +482,16 @@ extern "C" int oscar_step_write(const void* query_bf16, int64_t query_token_stri
   a.q_rot = q_rot;
   a.k_rot = k_rot;
   a.v_rot = v_rot;
-  // Window keep rule per token (host lists, as the reference's): token t of
-  // request i sits at seq[i] - qsl[i + 1] + t.
-  for (int32_t i = 0; i < num_requests; ++i) {
+  // Window keep rule per token: token t of request i sits at seq[i] - qsl[i +
+  // 1] + t (from host lists here, as the reference's; else in the kernel).
+  if (layout_on_device && num_requests > 0) {
+    a.query_start = query_start_loc;
+    a.seq_lens = seq_lens;
+    a.num_requests = num_requests;
+    a.sink_eff = sink_eff;
+    a.recent = recent;
+  }
+  for (int32_t i = 0; i < num_requests && !layout_on_device; ++i) {
     const int32_t lo = query_start_loc[i] < 0 ? 0 : query_start_loc[i];
     const int32_t hi = query_start_loc[i + 1] < num_tokens ? query_start_loc[i + 1] : num_tokens;
     for (int32_t t = lo; t < hi; ++t) {
@@ -477,4 +504,27 @@ extern "C" int oscar_step_write(const void* query_bf16, int64_t query_token_stri
   const int64_t q_groups = ((int64_t)num_tokens * num_heads + a.vecs_per_group - 1) / a.vecs_per_group;
   hipLaunchKernelGGL(step_write_kernel, dim3((unsigned)(2 * a.kv_groups + q_groups)), dim3(kThreads), 0, stream, a);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+}  // namespace oscar
+
+using namespace oscar;
+
+extern "C" int oscar_step_write(const void* query_bf16, int64_t query_token_stride, const void* key_bf16,
+                                const void* value_bf16, int64_t kv_token_stride, int32_t num_tokens,
+                                int32_t num_heads, int32_t num_kv_heads, int32_t head_size, const float* rot_k,
+                                const float* rot_v, const int64_t* slot_mapping, const int32_t* query_start_loc,
+                                const int32_t* seq_lens, int32_t num_requests, void* k_cache, void* v_cache,
+                                int32_t block_size, int64_t num_pages, int64_t k_stride_page,
+                                int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page,
+                                int64_t v_stride_token, int64_t v_stride_head, int32_t clip_index_k,
+                                int32_t clip_index_v, float* stage_k, float* stage_v, int64_t* stage_owner,
+                                void* stage_k_image, void* stage_v_image, int32_t stage_rows, int32_t sink_eff,
+                                int32_t recent, float* q_rot, float* k_rot, float* v_rot, hipStream_t stream) {
+  return step_write(false, query_bf16, query_token_stride, key_bf16, value_bf16, kv_token_stride, num_tokens, num_heads,
+                    num_kv_heads, head_size, rot_k, rot_v, slot_mapping, query_start_loc, seq_lens,
+                    num_requests, k_cache, v_cache, block_size, num_pages, k_stride_page,
+                    k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
+                    clip_index_k, clip_index_v, stage_k, stage_v, stage_owner, stage_k_image,
+                    stage_v_image, stage_rows, sink_eff, recent, q_rot, k_rot, v_rot, stream);
 }
