@@ -470,6 +470,36 @@ int oscar_quant_write_window(const void* key_bf16, const void* value_bf16, int64
                              float* stage_k, float* stage_v, int64_t* stage_owner, int64_t* seat_winner,
                              void* stage_k_image, void* stage_v_image, oscar_stream_t stream);
 
+/* ---------------------------------------------------------------- step forward
+ * The whole forward of one layer for a step with long requests: the INT2 and
+ * window write of every token, the paged read of the requests of 1 ..
+ * max_short query tokens (max_short <= 16) and the prefill read of the longer
+ * ones, on one stream.  Replaces the reference's forward with mixed or long
+ * requests (oscar_ascend/backend.py:239-319, 361-415).  The pieces are
+ * oscar_quant_write_window (oscar_quant_write without an arena),
+ * oscar_paged_decode_rotated over fp32 rotations, and oscar_prefill_rotated.
+ *   layer: oscar_mtp_forward's, block_size a multiple of 32, with the rotations' operands
+ *     (oscar_rotation_operand of R_k, R_v and R_v^T) and, with an arena, its
+ *     seat_winner buffer (oscar_staging_write's);
+ *   query_bf16 [tokens][query_token_stride], key_bf16 / value_bf16
+ *     [tokens][kv_token_stride]: 16-byte aligned, strides multiples of 8;
+ *   query_start_loc [num_requests + 1] (from 0, its last entry the tokens) and
+ *     seq_lens [num_requests]: HOST arrays, read during the call; slot_mapping
+ *     [tokens], block_table [num_requests][block_table_stride];
+ *   out_bf16 [tokens][num_heads][D], 16-byte aligned;
+ *   workspace: 16-byte aligned, >= oscar_step_forward_workspace_bytes(...).
+ */
+size_t oscar_step_forward_workspace_bytes(int32_t num_requests, const int32_t* query_start_loc,
+                                          const int32_t* seq_lens, int32_t num_heads, int32_t num_kv_heads,
+                                          int32_t max_short);
+int oscar_step_forward(const oscar_mtp_layer* layer, const void* rot_k_operand, const void* rot_v_operand,
+                       const void* rot_v_t_operand, int64_t* seat_winner, const void* query_bf16,
+                       int64_t query_token_stride, const void* key_bf16, const void* value_bf16,
+                       int64_t kv_token_stride, const int64_t* slot_mapping, const int32_t* block_table,
+                       int64_t block_table_stride, int32_t block_table_cols, const int32_t* query_start_loc,
+                       const int32_t* seq_lens, int32_t num_requests, int32_t max_short, void* out_bf16,
+                       void* workspace, size_t workspace_size, oscar_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

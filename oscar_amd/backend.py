@@ -308,6 +308,9 @@ class OscarAttentionBackendImpl:
         if self._short_step(layer, query, key, value, kv_cache, attn_metadata, output, capturing):
             self._oscar_stats["reads"] += 1
             return output
+        if self._long_step(layer, query, key, value, kv_cache, attn_metadata, output):
+            self._oscar_stats["reads"] += 1
+            return output
         self._write_step(layer, key, value, kv_cache, attn_metadata)
 
         attn_out = self._read(layer, query, key, value, attn_metadata)
@@ -346,6 +349,43 @@ class OscarAttentionBackendImpl:
         self._oscar_stats["kv_bytes_written"] += N * self.num_kv_heads * 160
         if output.shape[0] > N:
             output[N:].zero_()
+        return True
+
+    def _long_step(self, layer, query, key, value, kv_cache, attn_metadata, output) -> bool:
+        """The whole forward of a bf16 step with long requests in one library
+        call (write, window, paged read of the short requests, prefill read
+        of the long ones).  Returns False (nothing done) when the step's
+        types, shapes or layout need the general route."""
+        cfg = self._oscar
+        N = attn_metadata.num_actual_tokens
+        num_tokens = query.shape[0]
+        bf16 = torch.bfloat16
+        if N <= 0 or query.ndim != 3 or not query.dtype == key.dtype == value.dtype == output.dtype == bf16 \
+                or min(num_tokens, key.shape[0], value.shape[0]) < N or output.shape[0] < num_tokens \
+                or self.key_cache.shape[1] % 32:
+            return False
+        dev = query.device
+        if not key.device == value.device == output.device == self.key_cache.device == dev:
+            return False
+        limit = cfg.paged_max_q_len if cfg.use_paged else 0
+        slots, bt = attn_metadata.slot_mapping, attn_metadata.block_tables
+        qsl, seqs = metadata_batch_lists(attn_metadata)
+        B = len(qsl) - 1
+        if B < 1 or len(seqs) < B or qsl[0] != 0 or qsl[-1] != N or not 0 <= limit <= decode.MAX_QUERY_LEN \
+                or any(not 0 <= b - a <= s for (a, b), s in zip(itertools.pairwise(qsl), seqs)) \
+                or slots.ndim != 1 or slots.shape[0] < N or bt.ndim != 2 or bt.shape[0] < B or bt.shape[1] == 0:
+            return False
+        self._layer_rots(layer, dev)
+        ml = self._mtp_layer(layer, kv_cache, dev)
+        _, _, op_k, op_v = layer._oscar_rot_ops
+        winner = layer._oscar_seat_winner if cfg.window_enabled else None
+        if not step.step_forward(ml, (op_k, op_v, layer._oscar_rvT_op), winner, decode.request_layout(qsl, seqs[:B]),
+                                 limit, slots, bt, query, key, value, output, _lib.stream_handle(dev)):
+            return False
+        self._oscar_stats["writes"] += 1
+        self._oscar_stats["kv_bytes_written"] += N * self.num_kv_heads * 160
+        if num_tokens > N:
+            output[N:num_tokens].zero_()
         return True
 
     def _mtp_layer(self, layer, kv_cache, dev) -> step.MtpLayer:

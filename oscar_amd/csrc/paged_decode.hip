@@ -99,17 +99,19 @@ typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 
 // Work items of one launch travel inside the kernel arguments (no device
 // round trip for the metadata); larger batches are launched in chunks.
-constexpr int kMaxInlineItems = 128;
+constexpr int kMaxInlineItems = 128;    // (and kv heads, so that kvh fits its byte)
 
 struct ItemInfo {
   int32_t qa;        // first query row (token) of the request
   int32_t prefix;    // history length
   int32_t pbase;     // first partial slot of the item: history splits 0 .. nsplit - 1, then the fresh one
-  int16_t nq;        // query tokens of the request
-  int16_t req;       // block-table row (request index within the launch chunk)
-  int16_t kvh;       // kv head
+  int32_t out0;      // first output token of the request (rotated merge)
+  int32_t req;       // block-table row, from the launch chunk's first
+  int8_t nq;         // query tokens of the request
+  int8_t kvh;        // kv head
   int16_t nsplit;    // history splits of the item: split s takes steps s, s + nsplit, s + 2 nsplit, ...
 };
+constexpr int kItemWords = sizeof(ItemInfo) / sizeof(int);
 
 struct DecodeArgs {
   const float* q;          // [n, Hq, D]
@@ -195,13 +197,13 @@ __device__ __forceinline__ ItemInfo find_item(const DecodeArgs& a, int b, int& i
   const int skip = a.fresh - a.fresh_block;     // fresh slots without a workgroup of their own
   const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
   // (unconditional loads, lanes past the last item reading item 0, so that
-  // all ten go out before one wait)
+  // all of them go out before one wait)
   const int n = a.nitems;
   const int* f0 = reinterpret_cast<const int*>(&a.items[lane < n ? lane : 0]);
   const int* f1 = reinterpret_cast<const int*>(&a.items[lane + 64 < n ? lane + 64 : 0]);
-  int w0[5], w1[5];
+  int w0[kItemWords], w1[kItemWords];
 #pragma unroll
-  for (int k = 0; k < 5; ++k) {
+  for (int k = 0; k < kItemWords; ++k) {
     w0[k] = f0[k];
     w1[k] = f1[k];
   }
@@ -210,13 +212,12 @@ __device__ __forceinline__ ItemInfo find_item(const DecodeArgs& a, int b, int& i
   const int s1 = lane + 64 < n ? w1[2] - (lane + 64) * skip : 0x7fffffff;
   item = __popcll(__ballot(s0 <= b)) + __popcll(__ballot(s1 <= b)) - 1;
   item = __builtin_amdgcn_readfirstlane(item);
-  int fld[5];
+  int fld[kItemWords];
 #pragma unroll
-  for (int k = 0; k < 5; ++k) {
+  for (int k = 0; k < kItemWords; ++k) {
     const int v0 = __builtin_amdgcn_readlane(w0[k], item & 63), v1 = __builtin_amdgcn_readlane(w1[k], item & 63);
     fld[k] = item < 64 ? v0 : v1;
   }
-  static_assert(sizeof(ItemInfo) == 5 * sizeof(int), "ItemInfo is five words");
   ItemInfo it;
   __builtin_memcpy(&it, fld, sizeof(it));
   local = b - (it.pbase - item * skip);
@@ -1868,18 +1869,18 @@ __device__ __forceinline__ ItemInfo find_token_item(const DecodeArgs& a, int tok
   const int i0 = lane * hk + kvh, i1 = (lane + 64) * hk + kvh;
   const int* f0 = reinterpret_cast<const int*>(&a.items[i0 < n ? i0 : kvh]);
   const int* f1 = reinterpret_cast<const int*>(&a.items[i1 < n ? i1 : kvh]);
-  int w0[5], w1[5];
+  int w0[kItemWords], w1[kItemWords];
 #pragma unroll
-  for (int k = 0; k < 5; ++k) {
+  for (int k = 0; k < kItemWords; ++k) {
     w0[k] = f0[k];
     w1[k] = f1[k];
   }
   static_assert(offsetof(ItemInfo, qa) == 0, "qa is the first word");
   const int c = __popcll(__ballot(i0 < n && w0[0] <= tok)) + __popcll(__ballot(i1 < n && w1[0] <= tok));
   const int req = __builtin_amdgcn_readfirstlane(c - 1);
-  int fld[5];
+  int fld[kItemWords];
 #pragma unroll
-  for (int k = 0; k < 5; ++k) {
+  for (int k = 0; k < kItemWords; ++k) {
     const int v0 = __builtin_amdgcn_readlane(w0[k], req & 63), v1 = __builtin_amdgcn_readlane(w1[k], req & 63);
     fld[k] = req < 64 ? v0 : v1;
   }
@@ -1935,6 +1936,7 @@ __global__ __launch_bounds__(kRotThreads) void paged_decode_merge_rotate_kernel(
   floatx4 (&osum)[kRotWaves][64] = *reinterpret_cast<floatx4 (*)[kRotWaves][64]>(sums);
   float (&csum)[KC][kR][CW * 64] = *reinterpret_cast<float (*)[KC][kR][CW * 64]>(sums);
   __shared__ __attribute__((aligned(16))) float orow[kR][kHeadDim];
+  __shared__ int otok[kR];                       // the rows' output tokens
   // blockIdx.x = (g & 7) + 8 (qd + kQ (g >> 3)) for row group g: workgroups
   // are dealt to the 8 XCDs by linear id mod 8, so the kQ blocks of a group,
   // which all read its rows' every partial, share one XCD and its L2.
@@ -1996,6 +1998,7 @@ __global__ __launch_bounds__(kRotThreads) void paged_decode_merge_rotate_kernel(
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) mloc = fmaxf(mloc, __shfl_xor(mloc, o, 64));
   if (lane == 0) red[0][w] = mloc;
+  if (lane == 0 && wr == 0) otok[w / W] = it.out0 + (tok - it.qa);
   __syncthreads();
   float mx = red[0][w - wr];
 #pragma unroll
@@ -2062,7 +2065,7 @@ __global__ __launch_bounds__(kRotThreads) void paged_decode_merge_rotate_kernel(
 #pragma unroll
     for (int ww = 1; ww < KC; ++ww) o += csum[ww][i][col];
     const int to = (int)fast_div((uint32_t)(row0 + i), heads_div);
-    const int64_t idx = (int64_t)(tok0 + to) * out_stride + (int64_t)(row0 + i - to * a.num_heads) * kHeadDim +
+    const int64_t idx = (int64_t)otok[i] * out_stride + (int64_t)(row0 + i - to * a.num_heads) * kHeadDim +
                         64 * CW * qd + col;
     if (out_bf16)
       reinterpret_cast<__bf16*>(out)[idx] = (__bf16)o;
@@ -2435,6 +2438,7 @@ struct DecodeLaunch {
   const int32_t* block_table;
   int64_t bt_stride;
   int32_t num_requests;
+  int32_t spans;                // > 0: only the requests of 1 .. spans tokens, queries packed
   int32_t max_query_len;
   int32_t num_kv_heads;
   int64_t max_history;
@@ -2451,7 +2455,7 @@ int prepare_decode(DecodeLaunch& L, const float* q_rot, const float* k_new, cons
                    int32_t num_requests, int32_t max_query_len, int64_t max_history, const int64_t* stage_owner,
                    const void* stage_k_image, const void* stage_v_image, int32_t stage_rows, float scale,
                    int32_t tiles_per_split, float* out, const OutRotation& orot, void* workspace,
-                   size_t workspace_size) {
+                   size_t workspace_size, int32_t spans = 0) {
   L.empty = true;
   if (head_size != kHeadDim) return kErrUnsupportedHeadDim;
   if (num_tokens < 0 || num_requests < 0 || num_heads <= 0 || num_kv_heads <= 0 ||
@@ -2472,13 +2476,23 @@ int prepare_decode(DecodeLaunch& L, const float* q_rot, const float* k_new, cons
   if (query_start_loc[0] < 0 || query_start_loc[num_requests] > num_tokens) return kErrInvalidArgument;
   for (int32_t i = 0; i < num_requests; ++i) {
     const int32_t nq = query_start_loc[i + 1] - query_start_loc[i];
+    if (spans > 0 && nq > spans) continue;
     if (nq < 0 || nq > max_query_len || seq_lens[i] < nq || (int64_t)(seq_lens[i] - nq) > max_history)
       return kErrInvalidArgument;
   }
   if (tiles_per_split > 0 && splits_for(max_history, tiles_per_split) > kMaxSplits) return kErrInvalidArgument;
   if (tiles_per_split == 0 && (max_history + kStepTok - 1) / kStepTok > kMaxSplits * kMaxStepsPerSplit)
     return kErrInvalidArgument;
-  const size_t need = workspace_floats(num_requests, num_kv_heads, num_heads, max_query_len, max_history,
+  int32_t reading = num_requests;
+  if (spans > 0) {
+    reading = 0;
+    for (int32_t i = 0; i < num_requests; ++i) {
+      const int32_t nq = query_start_loc[i + 1] - query_start_loc[i];
+      reading += nq > 0 && nq <= spans;
+    }
+    if (reading == 0) return kOk;
+  }
+  const size_t need = workspace_floats(reading, num_kv_heads, num_heads, max_query_len, max_history,
                                        tiles_per_split) * sizeof(float);
   if (workspace == nullptr || workspace_size < need) return kErrWorkspaceTooSmall;
   a.k_new = k_new;
@@ -2495,6 +2509,7 @@ int prepare_decode(DecodeLaunch& L, const float* q_rot, const float* k_new, cons
   L.block_table = block_table;
   L.bt_stride = block_table_stride;
   L.num_requests = num_requests;
+  L.spans = spans;
   L.max_query_len = max_query_len;
   L.num_kv_heads = num_kv_heads;
   L.empty = false;
@@ -2508,15 +2523,23 @@ int launch_decode(DecodeLaunch& L, hipStream_t stream) {
   // partials reuse the same workspace (the merge of one chunk precedes the
   // next split in stream order).
   const int32_t per = requests_per_launch(L.num_kv_heads);
-  for (int32_t c0 = 0; c0 < L.num_requests; c0 += per) {
-    const int32_t nreq = L.num_requests - c0 < per ? L.num_requests - c0 : per;
-    for (int32_t i = 0; i < nreq; ++i) {
-      const int32_t qa = L.qsl[c0 + i];
-      const int32_t nq = L.qsl[c0 + i + 1] - qa;
+  int32_t packed = 0;                   // query tokens of the requests so far
+  for (int32_t c0 = 0; c0 < L.num_requests;) {
+    int32_t nreq = 0, first = c0;
+    for (; c0 < L.num_requests && nreq < per; ++c0) {
+      const int32_t tok = L.qsl[c0];
+      const int32_t nq = L.qsl[c0 + 1] - tok;
+      if (L.spans > 0 && (nq <= 0 || nq > L.spans)) continue;
+      if (nreq == 0) first = c0;
+      const int32_t qa = L.spans > 0 ? packed : tok;
       for (int32_t h = 0; h < L.num_kv_heads; ++h)
-        a.items[i * L.num_kv_heads + h] = ItemInfo{qa, L.seqs[c0 + i] - nq, 0, (int16_t)nq, (int16_t)i, (int16_t)h, 0};
+        a.items[nreq * L.num_kv_heads + h] =
+            ItemInfo{qa, L.seqs[c0] - nq, 0, tok, c0 - first, (int8_t)nq, (int8_t)h, 0};
+      packed += nq;
+      ++nreq;
     }
-    a.block_table = L.block_table ? L.block_table + (int64_t)c0 * L.bt_stride : nullptr;
+    if (nreq == 0) break;
+    a.block_table = L.block_table ? L.block_table + (int64_t)first * L.bt_stride : nullptr;
     const unsigned nitems = (unsigned)(nreq * L.num_kv_heads);
     // Per-item splits; the fresh partial gets a workgroup of its own when one
     // more per item still fits the resident budget, else it rides on a
@@ -2641,7 +2664,7 @@ int decode_only(const float* q_rot, int32_t num_heads, int32_t num_kv_heads, int
     const int32_t nreq = num_requests - c0 < per ? num_requests - c0 : per;
     for (int32_t i = 0; i < nreq; ++i)
       for (int32_t h = 0; h < num_kv_heads; ++h)
-        a.items[i * num_kv_heads + h] = ItemInfo{c0 + i, seq_lens[c0 + i], 0, 1, (int16_t)i, (int16_t)h, 0};
+        a.items[i * num_kv_heads + h] = ItemInfo{c0 + i, seq_lens[c0 + i], 0, c0 + i, i, 1, (int8_t)h, 0};
     a.block_table = block_table ? block_table + (int64_t)c0 * block_table_stride : nullptr;
     const unsigned nitems = (unsigned)(nreq * num_kv_heads);
     if (!plan_splits(a, nitems, max_history, tiles_per_split, 0)) return kErrInvalidArgument;
@@ -2843,3 +2866,24 @@ int oscar_mtp_forward(const oscar_mtp_layer* layer, const oscar_mtp_step* step, 
 }
 
 }  // extern "C"
+
+namespace oscar {
+
+int launch_decode_spans(const oscar_mtp_layer& L, const DecodeSpans& d, void* out_bf16, int64_t out_token_stride,
+                        void* workspace, size_t workspace_size, hipStream_t stream) {
+  const int32_t rows = L.stage_rows;
+  DecodeLaunch D;
+  const int rc = prepare_decode(D, d.q_rot, d.k_rot, d.v_rot, d.query_start_loc[d.num_requests], L.num_heads,
+                                L.num_kv_heads, L.head_size, L.k_cache, L.v_cache, L.block_size, L.num_pages,
+                                L.k_stride_page, L.k_stride_token, L.k_stride_head, L.v_stride_page, L.v_stride_token,
+                                L.v_stride_head, d.block_table, d.block_table_stride, d.block_table_cols,
+                                d.query_start_loc, d.seq_lens, d.num_requests, d.max_query_len, d.max_history,
+                                rows > 0 ? L.stage_owner : nullptr, rows > 0 ? L.stage_k_image : nullptr,
+                                rows > 0 ? L.stage_v_image : nullptr, rows, L.scale, 0,
+                                reinterpret_cast<float*>(out_bf16),
+                                OutRotation{L.rot_v_t, out_bf16, out_token_stride, 1}, workspace, workspace_size,
+                                d.spans);
+  return rc != kOk ? rc : launch_decode(D, stream);
+}
+
+}  // namespace oscar

@@ -310,9 +310,26 @@ __device__ void window_epilogue(const float (&v)[kPerLane], int64_t tok, int64_t
   }
 }
 
+// A step's request layout on its way from the host to the device: the first
+// n of the ints go to dst.
+constexpr int kLayoutInts = 896;
+struct HostLayout {
+  int32_t* dst;
+  int32_t n;
+  int32_t v[kLayoutInts];
+};
+
+__global__ __launch_bounds__(256) void store_layout_kernel(HostLayout h) {
+  for (int i = threadIdx.x; i < h.n; i += 256) h.dst[i] = h.v[i];
+}
+
+// (its first workgroup also stores a request layout that came with the launch)
 __global__ __launch_bounds__(256) void quant_window_winner_kernel(const int64_t* __restrict__ slots, int32_t n_tokens,
-                                                                   int64_t* winner, int32_t block_size, int32_t rows) {
+                                                                   int64_t* winner, int32_t block_size, int32_t rows,
+                                                                   HostLayout h) {
   __shared__ int64_t epoch;
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < h.n; i += 256) h.dst[i] = h.v[i];
   seat_winner_pass(slots, n_tokens, winner, (int64_t)rows * block_size, block_size, rows, &epoch);
 }
 
@@ -921,13 +938,20 @@ int oscar_quant_write_prerotated(const float* k_rot, const float* v_rot, int64_t
 
 namespace {
 
-// oscar_quant_write with an optional window arena (w.rows > 0).
+// A request layout in host arrays; its device copy is the window arguments'.
+struct StepLayout {
+  const int32_t* query_start;
+  const int32_t* seq_lens;
+};
+
+// oscar_quant_write with an optional window arena (w.rows > 0), whose request
+// layout is in w's device arrays, or to be stored there from host's.
 int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_tokens, int32_t num_kv_heads,
                      int32_t head_size, int64_t token_stride, const void* rot_k_operand, const void* rot_v_operand,
                      const int64_t* slot_mapping, void* k_cache, void* v_cache, int32_t block_size,
                      int64_t num_pages, int64_t k_stride_page, int64_t k_stride_token, int64_t k_stride_head,
                      int64_t v_stride_page, int64_t v_stride_token, int64_t v_stride_head, int32_t clip_index_k,
-                     int32_t clip_index_v, const WindowArgs& w, hipStream_t stream) {
+                     int32_t clip_index_v, const WindowArgs& w, const StepLayout* host, hipStream_t stream) {
   if (head_size != kHeadDim) return kErrUnsupportedHeadDim;
   if (num_tokens < 0 || num_kv_heads <= 0 || clip_index_k >= kHeadDim || clip_index_v >= kHeadDim)
     return kErrInvalidArgument;
@@ -954,9 +978,10 @@ int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_t
     const uint8_t* ok = static_cast<const uint8_t*>(rot_k_operand) + kMfmaOperandBytes;
     const uint8_t* ov = static_cast<const uint8_t*>(rot_v_operand) + kMfmaOperandBytes;
     const bool win = w.rows > 0;
-    return step_write(true, nullptr, 0, key_bf16, value_bf16, token_stride, (int32_t)num_tokens, 0, num_kv_heads,
+    return step_write(host == nullptr, nullptr, 0, key_bf16, value_bf16, token_stride, (int32_t)num_tokens, 0, num_kv_heads,
                       head_size, reinterpret_cast<const float*>(ok), reinterpret_cast<const float*>(ov),
-                      slot_mapping, win ? w.query_start : nullptr, win ? w.seq_lens : nullptr,
+                      slot_mapping, win ? (host ? host->query_start : w.query_start) : nullptr,
+                      win ? (host ? host->seq_lens : w.seq_lens) : nullptr,
                       win ? w.num_requests : 0, k_cache, v_cache, block_size, num_pages, k_stride_page,
                       k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
                       clip_index_k, clip_index_v, w.stage_k, w.stage_v, w.owner, w.kimg, w.vimg, w.rows,
@@ -966,8 +991,24 @@ int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_t
   const int64_t per_block = kFusedWaves * kTokPerWave;
   dim3 grid((unsigned)((num_tokens + per_block - 1) / per_block), (unsigned)(num_kv_heads * 2));
   if (w.rows > 0) {
+    HostLayout h{};
+    if (host != nullptr) {
+      // query_start, then seq_lens, in one array; the last part goes with the
+      // winner pass, the others in launches of their own
+      const int64_t starts = (int64_t)w.num_requests + 1, ints = starts + w.num_requests;
+      for (int64_t i0 = 0; i0 < ints; i0 += kLayoutInts) {
+        h.dst = const_cast<int32_t*>(w.query_start) + i0;
+        h.n = (int32_t)(ints - i0 < kLayoutInts ? ints - i0 : kLayoutInts);
+        for (int32_t i = 0; i < h.n; ++i)
+          h.v[i] = i0 + i < starts ? host->query_start[i0 + i] : host->seq_lens[i0 + i - starts];
+        if (i0 + h.n < ints) {
+          hipLaunchKernelGGL(store_layout_kernel, dim3(1), dim3(256), 0, stream, h);
+          if (hipGetLastError() != hipSuccess) return kErrLaunch;
+        }
+      }
+    }
     hipLaunchKernelGGL(quant_window_winner_kernel, dim3((unsigned)((num_tokens + 255) / 256)), dim3(256), 0, stream,
-                       slot_mapping, (int32_t)num_tokens, w.winner, block_size, w.rows);
+                       slot_mapping, (int32_t)num_tokens, w.winner, block_size, w.rows, h);
     if (hipGetLastError() != hipSuccess) return kErrLaunch;
   }
   hipLaunchKernelGGL(quant_write_fused_kernel, grid, dim3(kFusedWaves * 64), kFusedLds, stream,
@@ -993,7 +1034,7 @@ int oscar_quant_write(const void* key_bf16, const void* value_bf16, int64_t num_
   return quant_write_impl(key_bf16, value_bf16, num_tokens, num_kv_heads, head_size, token_stride, rot_k_operand,
                           rot_v_operand, slot_mapping, k_cache, v_cache, block_size, num_pages, k_stride_page,
                           k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
-                          clip_index_k, clip_index_v, WindowArgs{}, stream);
+                          clip_index_k, clip_index_v, WindowArgs{}, nullptr, stream);
 }
 
 int oscar_quant_write_window(const void* key_bf16, const void* value_bf16, int64_t num_tokens,
@@ -1023,7 +1064,27 @@ int oscar_quant_write_window(const void* key_bf16, const void* value_bf16, int64
   return quant_write_impl(key_bf16, value_bf16, num_tokens, num_kv_heads, head_size, token_stride, rot_k_operand,
                           rot_v_operand, slot_mapping, k_cache, v_cache, block_size, num_pages, k_stride_page,
                           k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
-                          clip_index_k, clip_index_v, w, stream);
+                          clip_index_k, clip_index_v, w, nullptr, stream);
 }
 
 }  // extern "C"
+
+namespace oscar {
+
+int quant_write_step(const oscar_mtp_layer& L, const void* rot_k_operand, const void* rot_v_operand,
+                     int64_t* seat_winner, const void* key_bf16, const void* value_bf16, int64_t kv_token_stride,
+                     int32_t num_tokens, const int64_t* slot_mapping, const int32_t* query_start_loc,
+                     const int32_t* seq_lens, int32_t num_requests, int32_t* layout, hipStream_t stream) {
+  WindowArgs w{};
+  const StepLayout host{query_start_loc, seq_lens};
+  if (L.stage_rows > 0)
+    w = WindowArgs{layout, layout + num_requests + 1, num_requests, L.stage_rows, L.sink_eff, L.recent,
+                   L.num_kv_heads, L.stage_k, L.stage_v, L.stage_owner, seat_winner,
+                   static_cast<_Float16*>(L.stage_k_image), static_cast<_Float16*>(L.stage_v_image)};
+  return quant_write_impl(key_bf16, value_bf16, num_tokens, L.num_kv_heads, L.head_size, kv_token_stride,
+                          rot_k_operand, rot_v_operand, slot_mapping, L.k_cache, L.v_cache, L.block_size, L.num_pages,
+                          L.k_stride_page, L.k_stride_token, L.k_stride_head, L.v_stride_page, L.v_stride_token,
+                          L.v_stride_head, L.clip_index_k, L.clip_index_v, w, &host, stream);
+}
+
+}  // namespace oscar

@@ -1,7 +1,8 @@
-// The short-step write (step_write.hip) as the other sources launch it.
+// What the sources launch of one another in a step's forward.
 #pragma once
 
 #include "oscar_common.h"
+#include "../../include/oscar_amd.h"
 
 namespace oscar {
 
@@ -9,6 +10,50 @@ namespace oscar {
 // [n_tokens][q_stride]; q_rot and rot_k 16-byte aligned, n_tokens >= 1.
 int launch_rotate_queries(const uint16_t* q, int64_t q_stride, int32_t n_tokens, int32_t num_heads, const float* rot_k,
                           float* q_rot, hipStream_t stream);
+
+// Runs of consecutive tokens, packed: token p of the packed order, pos[r] <= p
+// < pos[r + 1], is token tok[r] + p - pos[r] of the step.
+constexpr int kMaxTokenRuns = 64;
+struct TokenRuns {
+  int32_t n;                          // runs
+  int32_t tokens;                     // of all runs
+  int32_t pos[kMaxTokenRuns];
+  int32_t tok[kMaxTokenRuns];
+};
+
+// q_rot [tokens][num_heads][D], k_rot / v_rot [tokens][num_kv_heads][D] fp32 of
+// the runs' tokens (step_write.hip).
+int launch_rotate_runs(const uint16_t* q, int64_t q_stride, const uint16_t* k, const uint16_t* v, int64_t kv_stride,
+                       const TokenRuns& runs, int32_t num_heads, int32_t num_kv_heads, const float* rot_k,
+                       const float* rot_v, float* q_rot, float* k_rot, float* v_rot, hipStream_t stream);
+
+// The paged read of the requests of 1 .. spans query tokens of a step, from
+// their packed rotated q / k / v to their rows of the step's bf16 output
+// (paged_decode.hip).
+struct DecodeSpans {
+  const float* q_rot;                 // [packed tokens][Hq][D]
+  const float* k_rot;
+  const float* v_rot;
+  const int32_t* query_start_loc;     // host, the step's
+  const int32_t* seq_lens;            // host
+  int32_t num_requests;               // of the step
+  int32_t spans;                      // most query tokens of a request that is read
+  int32_t max_query_len;              // of those requests
+  int64_t max_history;
+  const int32_t* block_table;
+  int64_t block_table_stride;
+  int32_t block_table_cols;
+};
+int launch_decode_spans(const oscar_mtp_layer& layer, const DecodeSpans& d, void* out_bf16, int64_t out_token_stride,
+                        void* workspace, size_t workspace_size, hipStream_t stream);
+
+// oscar_quant_write_window (stage_rows > 0) or oscar_quant_write of a step
+// whose request layout is in host arrays; layout: 2 num_requests + 1 ints of
+// device scratch (quant_write.hip).
+int quant_write_step(const oscar_mtp_layer& layer, const void* rot_k_operand, const void* rot_v_operand,
+                     int64_t* seat_winner, const void* key_bf16, const void* value_bf16, int64_t kv_token_stride,
+                     int32_t num_tokens, const int64_t* slot_mapping, const int32_t* query_start_loc,
+                     const int32_t* seq_lens, int32_t num_requests, int32_t* layout, hipStream_t stream);
 
 // oscar_step_write, with the request layout in host arrays, or
 // (layout_on_device) in device arrays that are read on the stream.

@@ -72,6 +72,7 @@ struct StepArgs {
   const int32_t* query_start;   // the request layout on the device, or null: keep holds the rule
   const int32_t* seq_lens;
   int32_t num_requests, sink_eff, recent;
+  TokenRuns runs;               // n > 0: the inputs' tokens of the packed order
 };
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t x) { return __uint_as_float((uint32_t)x << 16); }
@@ -292,7 +293,7 @@ __device__ void write_vector(const WriteCtx& a, const floatx4& y, int t, int h, 
 // lies in the last request that starts at or before it, at position
 // seq - (end - t).  Called by every lane of the wavefront with the same t; a
 // token outside the layout is not kept.
-__device__ bool layout_keeps(const StepArgs& a, int t, int lane) {
+__device__ __forceinline__ bool layout_keeps(const StepArgs& a, int t, int lane) {
   int starts = 0;                       // entries of query_start (the end included) at or before t
 #pragma unroll 1
   for (int base = 0; base <= a.num_requests; base += 64) {
@@ -303,6 +304,14 @@ __device__ bool layout_keeps(const StepArgs& a, int t, int lane) {
   const int64_t seq = a.seq_lens[starts - 1];
   const int64_t pos = seq - a.query_start[starts] + t;
   return pos >= seq - a.recent || pos < a.sink_eff;
+}
+
+// Token of the step at packed position p (wave-uniform; every lane calls).
+__device__ __forceinline__ int run_token(const TokenRuns& r, int p, int lane) {
+  static_assert(kMaxTokenRuns == 64, "a run per lane");
+  const int pos = lane < r.n ? r.pos[lane] : 0x7fffffff, tok = r.tok[lane];
+  const int i = __builtin_amdgcn_readfirstlane(__popcll(__ballot(pos <= p)) - 1);
+  return __builtin_amdgcn_readlane(tok, i) + p - __builtin_amdgcn_readlane(pos, i);
 }
 
 __global__ __launch_bounds__(kThreads) void step_write_kernel(StepArgs a) {
@@ -342,15 +351,16 @@ __global__ __launch_bounds__(kThreads) void step_write_kernel(StepArgs a) {
   ctx.stage = side == 0 ? c.stage_k : c.stage_v;
   ctx.img = side == 0 ? c.kimg : c.vimg;
   ctx.clip = side == 0 ? c.clip_k : c.clip_v;
-  if (side < 2 && w < nv) {
+  if (side < 2 && w < nv && ctx.slots != nullptr) {
     const int t = (e0 + w) / heads;
     keep_word = a.query_start != nullptr ? (layout_keeps(a, t, lane) ? ~0u : 0u) : a.keep[t >> 5];
     my_slot = ctx.slots[t];
     later = t + 1 + lane < ctx.n_tokens ? ctx.slots[t + 1 + lane] : -1;
   }
   for (int idx = tid; idx < nv * kHeadDim; idx += kThreads) {
-    const int vv = idx >> 8, f = idx & 255;
-    const int e = e0 + vv, t = e / heads, h = e - t * heads;
+    const int vv = __builtin_amdgcn_readfirstlane(idx >> 8), f = idx & 255;
+    const int e = e0 + vv, h = e % heads;
+    const int t = a.runs.n > 0 ? run_token(a.runs, e / heads, lane) : e / heads;
     xs[vv][f] = bf16_to_f32(src[(int64_t)t * stride + (int64_t)h * kHeadDim + f]);
   }
   __syncthreads();
@@ -381,13 +391,22 @@ __global__ __launch_bounds__(kThreads) void step_write_kernel(StepArgs a) {
   const int e = e0 + w, t = e / heads, h = e - t * heads;
   float* out = side == 0 ? c.k_rot : (side == 1 ? c.v_rot : c.q_rot);
   if (out != nullptr) *reinterpret_cast<floatx4*>(out + ((int64_t)t * heads + h) * kHeadDim + 4 * lane) = y;
-  if (side < 2) write_vector(ctx, y, t, h, side, lane, my_slot, later, keep_word);
+  if (side < 2 && ctx.slots != nullptr) write_vector(ctx, y, t, h, side, lane, my_slot, later, keep_word);
 }
 
 // Vectors per workgroup: one while the step has few vectors (every workgroup
 // streams R once; fewer vectors each finish sooner), up to four for larger
 // steps.
-int32_t vecs_per_group(int64_t vectors) { return vectors <= 512 ? 1 : (vectors <= 2048 ? 2 : 4); }
+int launch(StepArgs& a, hipStream_t stream) {
+  const int64_t n = a.n_tokens;
+  const int64_t vectors = n * (a.num_heads + 2 * a.num_kv_heads);
+  const int64_t per = vectors <= 512 ? 1 : (vectors <= 2048 ? 2 : 4);
+  a.vecs_per_group = (int32_t)per;
+  a.kv_groups = (int32_t)((n * a.num_kv_heads + per - 1) / per);
+  const int64_t q_groups = (n * a.num_heads + per - 1) / per;
+  hipLaunchKernelGGL(step_write_kernel, dim3((unsigned)(2 * a.kv_groups + q_groups)), dim3(kThreads), 0, stream, a);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
 
 }  // namespace
 }  // namespace oscar
@@ -403,15 +422,33 @@ int launch_rotate_queries(const uint16_t* q, int64_t q_stride, int32_t n_tokens,
   a.num_heads = num_heads;
   a.rot_k = rot_k;
   a.q_rot = q_rot;
-  a.vecs_per_group = vecs_per_group((int64_t)n_tokens * num_heads);
-  const int64_t groups = ((int64_t)n_tokens * num_heads + a.vecs_per_group - 1) / a.vecs_per_group;
-  hipLaunchKernelGGL(step_write_kernel, dim3((unsigned)groups), dim3(kThreads), 0, stream, a);
-  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+  return launch(a, stream);
 }
 
 }  // namespace oscar
 
 namespace oscar {
+
+int launch_rotate_runs(const uint16_t* q, int64_t q_stride, const uint16_t* k, const uint16_t* v, int64_t kv_stride,
+                       const TokenRuns& runs, int32_t num_heads, int32_t num_kv_heads, const float* rot_k,
+                       const float* rot_v, float* q_rot, float* k_rot, float* v_rot, hipStream_t stream) {
+  StepArgs a{};
+  a.q = q;
+  a.k = k;
+  a.v = v;
+  a.q_stride = q_stride;
+  a.kv_stride = kv_stride;
+  a.n_tokens = runs.tokens;
+  a.num_heads = num_heads;
+  a.num_kv_heads = num_kv_heads;
+  a.rot_k = rot_k;
+  a.rot_v = rot_v;
+  a.q_rot = q_rot;
+  a.k_rot = k_rot;
+  a.v_rot = v_rot;
+  a.runs = runs;
+  return launch(a, stream);
+}
 
 int step_write(bool layout_on_device, const void* query_bf16, int64_t query_token_stride,
                const void* key_bf16, const void* value_bf16, int64_t kv_token_stride, int32_t num_tokens,
@@ -499,11 +536,7 @@ int step_write(bool layout_on_device, const void* query_bf16, int64_t query_toke
       if (pos >= (int64_t)seq_lens[i] - recent || pos < sink_eff) a.keep[t >> 5] |= 1u << (t & 31);
     }
   }
-  a.vecs_per_group = vecs_per_group((int64_t)num_tokens * (num_heads + 2 * num_kv_heads));
-  a.kv_groups = (int32_t)(((int64_t)num_tokens * num_kv_heads + a.vecs_per_group - 1) / a.vecs_per_group);
-  const int64_t q_groups = ((int64_t)num_tokens * num_heads + a.vecs_per_group - 1) / a.vecs_per_group;
-  hipLaunchKernelGGL(step_write_kernel, dim3((unsigned)(2 * a.kv_groups + q_groups)), dim3(kThreads), 0, stream, a);
-  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+  return launch(a, stream);
 }
 
 }  // namespace oscar

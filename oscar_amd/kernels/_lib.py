@@ -72,6 +72,9 @@ SIGNATURES = {
                                        _c_i32, _c_i32, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i32, _c_i64, _c_i64,
                                        _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_i32, _c_p, _c_p,
                                        _c_p, _c_i32, _c_f32, _c_p, _c_p, _c_sz, _c_p]),
+    "oscar_step_forward_workspace_bytes": (_c_sz, [_c_i32, _c_p, _c_p, _c_i32, _c_i32, _c_i32]),
+    "oscar_step_forward": (_c_i32, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_p,
+                                    _c_i64, _c_i32, _c_p, _c_p, _c_i32, _c_i32, _c_p, _c_p, _c_sz, _c_p]),
     "oscar_staging_write": (_c_i32, [_c_p, _c_p, _c_i64, _c_p, _c_i32, _c_p, _c_p, _c_i32, _c_i32,
                                      _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_p, _c_p, _c_p, _c_p,
                                      _c_p, _c_p, _c_p, _c_p, _c_p]),

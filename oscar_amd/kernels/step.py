@@ -308,3 +308,38 @@ def decode_only_forward(layer: MtpLayer, query, block_table, seqs, out, stream: 
     if status != 0:
         raise _lib.OscarKernelError(f"oscar_decode_only_forward failed: {_lib.STATUS.get(status, status)}")
     return True
+
+
+def step_forward(layer: MtpLayer, operands, winner, layout: decode.RequestLayout, max_short: int, slot_mapping,
+                 block_table, query, key, value, out, stream: int) -> bool:
+    """One layer's forward of a step with long requests through
+    oscar_step_forward: query [N, Hq*D] (or [N, Hq, D]) and key / value bf16,
+    out [>= N, Hq*D] bf16 rows.  ``operands``: those of R_k, R_v and R_v^T;
+    ``winner``: the arena's seat-winner buffer.  Returns False, with nothing
+    enqueued, when a tensor is not laid out as the library reads it in place."""
+    B = len(layout.lengths)
+    N = layout.qsl[-1]
+    hq, hk, D = layer.num_heads, layer.num_kv_heads, layer.head_size
+    qs = _row_stride(query, N, hq * D)
+    ks = _row_stride(key, N, hk * D)
+    if qs < hq * D or ks < hk * D or qs % 8 or ks % 8 or _row_stride(value, N, hk * D) != ks \
+            or _row_stride(out, N, hq * D) != hq * D:
+        return False
+    ptrs = query.data_ptr(), key.data_ptr(), value.data_ptr(), out.data_ptr()
+    if any(p % 16 for p in ptrs):
+        return False
+    dev = query.device
+    if slot_mapping.dtype != torch.int64 or slot_mapping.device != dev or not slot_mapping.is_contiguous():
+        slot_mapping = slot_mapping.to(device=dev, dtype=torch.int64).contiguous()
+    if block_table.dtype != torch.int32 or block_table.device != dev or block_table.stride(1) != 1:
+        block_table = block_table.to(device=dev, dtype=torch.int32).contiguous()
+    lib = _lib.load()
+    qsl, seqs = ctypes.addressof(layout.qstart), ctypes.addressof(layout.seq_t)
+    ws = decode.workspace(dev, lib.oscar_step_forward_workspace_bytes(B, qsl, seqs, hq, hk, max_short))
+    status = lib.oscar_step_forward(layer.ref, *(o.data_ptr() for o in operands), _lib.ptr(winner), ptrs[0], qs,
+                                    ptrs[1], ptrs[2], ks, slot_mapping.data_ptr(), block_table.data_ptr(),
+                                    block_table.stride(0), block_table.shape[1], qsl, seqs, B, max_short, ptrs[3],
+                                    ws.data_ptr(), ws.numel(), stream)
+    if status != 0:
+        raise _lib.OscarKernelError(f"oscar_step_forward failed: {_lib.STATUS.get(status, status)}")
+    return True
