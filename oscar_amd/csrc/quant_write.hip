@@ -254,38 +254,141 @@ struct WindowArgs {
   _Float16* vimg;
 };
 
-// The window half of the bulk write (the reference's _staging_write,
-// backend.py:439-481) for this lane's token (slot >= 0): if the token won
-// its seat, it sets the seat's owner (the K side of head 0 does) to its page
-// when it lies in the sink or recent window and to -1 otherwise; a kept token
-// then stores this lane's 128 unclipped rotated values (features 128 half ..
-// +127 of this side and head) and their fp16 image parts.  The lane's token
-// half is exactly one lane of the K image (token row prow % 32, half g), so
-// the K parts go out as 16-byte blocks; the V image holds tokens in slots, so
-// each V value is two 2-byte stores.
-__device__ void window_epilogue(const float (&v)[kPerLane], int64_t tok, int64_t slot, int head, int side, int half,
-                                int block_size, const WindowArgs& w) {
-  int64_t seat, page;
-  if (!won_seat(w.winner, (int64_t)w.rows * block_size, slot, tok, block_size, w.rows, seat, page)) return;
-  int lo = 0, hi = w.num_requests - 1;       // request of the token: last i with query_start[i] <= tok
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (w.query_start[mid] <= tok) lo = mid; else hi = mid - 1;
-  }
-  const int64_t seq = w.seq_lens[lo];
-  const int64_t pos = seq - w.query_start[lo + 1] + tok;
-  const bool keep = pos >= seq - w.recent || pos < w.sink_eff;
-  if (side == 0 && head == 0 && half == 0) w.owner[seat] = keep ? page : -1;
-  if (!keep) return;
-  float* dst = (side == 0 ? w.stage_k : w.stage_v) + (seat * w.num_kv_heads + head) * kHeadDim + kPerLane * half;
+__device__ __forceinline__ int64_t read_lane64(int64_t x, int lane) {
+  return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), lane) << 32) |
+                   (uint32_t)__builtin_amdgcn_readlane((int)x, lane));
+}
+
+// LDS of a wave's V image transpose: 32 features of each lane half by the 32
+// token slots of a tile, rows of 36 words (16-byte reads), the halves 32 words
+// apart modulo the 64 banks.
+constexpr int kTrRow = 36;
+constexpr int kTrHalf = 32 * kTrRow + 32;
+static_assert(2 * kTrHalf * sizeof(float) <= sizeof(SelLds), "the transpose reuses the selection's LDS");
+
+// The V image of the wave's tokens in one 32-token tile: `mine` on the lanes
+// whose token (token slot tt of the tile) is stored, full: the tile's 8-token
+// chunks (bytes of the mask) that those tokens fill, which alone are written.
+// A lane holds one token's features, an image chunk one feature's eight
+// tokens, so the values go through LDS, 32 features of each half at a time,
+// and out as 16-byte stores.  (Two-byte stores, token by token, touch 64
+// lines per wave and instruction; 256 of them took 23 us of a 45 us write
+// that is one workgroup deep; image and arena take 7 this way, 14 where 28
+// tokens of short requests go one by one.)
+__device__ __forceinline__ void store_v_tile(const float (&v)[kPerLane], bool mine, int tt, uint32_t full,
+                                             _Float16* img, float* T, int lane) {
+  const int half = lane >> 5;
+  const int r = tt & 7;                                    // place of the token in its chunk
+  const int place = (tt & 24) | (r == 1 ? 2 : (r == 2 ? 1 : (r == 5 ? 6 : (r == 6 ? 5 : r))));
 #pragma unroll
-  for (int k = 0; k < kPerLane / 4; ++k)
-    reinterpret_cast<floatx4*>(dst)[k] = floatx4{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
+  for (int p = 0; p < 4; ++p) {
+    wave_sync_lds();
+    if (mine) {
+#pragma unroll
+      for (int j = 0; j < 32; ++j) T[half * kTrHalf + j * kTrRow + place] = v[32 * p + j];
+    }
+    wave_sync_lds();
+    // chunk lane & 15 (m), then b, token group and half: 512-byte runs
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int u = 64 * i + lane;
+      const int ml = u & 15, grp = (u >> 4) & 3, b = (u >> 6) & 1, h = u >> 7;
+      const int j = 4 * (ml >> 1) + 2 * b + (ml & 1);      // feature 128 h + 32 p + j
+      if (((full >> (8 * grp)) & 1u) == 0u) continue;
+      const float* src = T + h * kTrHalf + j * kTrRow + 8 * grp;
+      const floatx4 x0 = reinterpret_cast<const floatx4*>(src)[0], x1 = reinterpret_cast<const floatx4*>(src)[1];
+      half8 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        _Float16 a, c;
+        fp16_parts(e < 4 ? x0[e] : x1[e - 4], a, c);
+        hi[e] = a;
+        lo[e] = c;
+      }
+      _Float16* d = img + vimg_offset(128 * h + 32 * p + j, 8 * grp);
+      *reinterpret_cast<half8*>(d) = hi;
+      *reinterpret_cast<half8*>(d + kVPartHalfs) = lo;
+    }
+  }
+}
+
+// The V image of single tokens (bits of `single`, both lanes of each): 64
+// features of a token at a time, 2-byte stores.  (A store per feature of the
+// lanes' own tokens would be 256 instructions however few the tokens; 8 a
+// token this way.)
+__device__ __forceinline__ void store_v_tokens(const float (&v)[kPerLane], uint64_t single, int64_t tile, int tt,
+                                               _Float16* vimg, float* T, int lane) {
+  const int half = lane >> 5, j = lane & 31;
+  const bool mine = ((single >> lane) & 1ull) != 0ull;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    wave_sync_lds();
+    if (mine) {
+#pragma unroll
+      for (int i = 0; i < 32; ++i) T[half * kTrHalf + i * kTrRow + j] = v[32 * p + i];
+    }
+    wave_sync_lds();
+    // (four tokens in flight; the last one again when fewer are left)
+#pragma unroll 1
+    for (uint32_t left = (uint32_t)single; left != 0u;) {
+      float x[4];
+      _Float16* d[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = (int)__builtin_ctz(left);
+        if (e == 3 || (left & (left - 1)) != 0u) left &= left - 1;
+        x[e] = T[half * kTrHalf + j * kTrRow + t];
+        d[e] = vimg + read_lane64(tile, t) * kVImgHalfs +
+               vimg_offset(kPerLane * half + 32 * p + j, __builtin_amdgcn_readlane(tt, t));
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) fp16_parts(x[e], d[e][0], d[e][kVPartHalfs]);
+    }
+  }
+}
+
+// The window half of the bulk write (the reference's _staging_write,
+// backend.py:439-481) for this lane's token (slot; negative: none): if the
+// token won its seat, it sets the seat's owner (the K side of head 0 does) to
+// its page when it lies in the sink or recent window and to -1 otherwise; a
+// kept token then stores this lane's 128 unclipped rotated values (features
+// 128 half .. +127 of this side and head) and their fp16 image parts.  The
+// lane's token half is exactly one lane of the K image (token row prow % 32,
+// half g), so the K parts go out as 16-byte blocks; the V image holds tokens
+// in slots, which neighbouring tokens fill together (store_v_tile).  Called
+// by every lane of the wavefront; sel: its selection LDS, free by now.
+__device__ __forceinline__ void window_epilogue(const float (&v)[kPerLane], int64_t tok, int64_t slot, int head,
+                                                int side, int lane, int block_size, const WindowArgs& w,
+                                                SelLds& sel) {
+  const int half = lane >> 5;
+  int64_t seat = 0, page = 0;
+  bool keep = false;
+  if (slot >= 0 &&
+      won_seat(w.winner, (int64_t)w.rows * block_size, slot, tok, block_size, w.rows, seat, page)) {
+    int lo = 0, hi = w.num_requests - 1;     // request of the token: last i with query_start[i] <= tok
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (w.query_start[mid] <= tok) lo = mid; else hi = mid - 1;
+    }
+    const int64_t seq = w.seq_lens[lo];
+    const int64_t pos = seq - w.query_start[lo + 1] + tok;
+    keep = pos >= seq - w.recent || pos < w.sink_eff;
+    if (side == 0 && head == 0 && half == 0) w.owner[seat] = keep ? page : -1;
+  }
+  uint64_t pending = __ballot(keep);         // (both halves of a token agree)
+  if (pending == 0ull) return;
+  if (keep) {
+    float* dst = (side == 0 ? w.stage_k : w.stage_v) + (seat * w.num_kv_heads + head) * kHeadDim + kPerLane * half;
+#pragma unroll
+    for (int k = 0; k < kPerLane / 4; ++k)
+      reinterpret_cast<floatx4*>(dst)[k] = floatx4{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
+  }
   if (w.kimg == nullptr) return;
   const int prow = (int)(slot - page * block_size);
   const int64_t tile = image_of(seat / block_size, prow, block_size, head, w.num_kv_heads);
   const int tt = prow & 31;
   if (side == 0) {
+    if (!keep) return;
     // block m = 2j + a, slot u = 2i + b: local feature 16j + 4a + i + 8b
     _Float16* img = w.kimg + tile * kKImgHalfs + (tt + 32 * half) * 8;
 #pragma unroll
@@ -300,14 +403,32 @@ __device__ void window_epilogue(const float (&v)[kPerLane], int64_t tok, int64_t
       *reinterpret_cast<half8*>(img + m * 64 * 8) = h;
       *reinterpret_cast<half8*>(img + kImgHalfs + m * 64 * 8) = l;
     }
-  } else {
-    _Float16* img = w.vimg + tile * kVImgHalfs;
-#pragma unroll
-    for (int k = 0; k < kPerLane; ++k) {
-      _Float16* d = img + vimg_offset(kPerLane * half + k, tt);
-      fp16_parts(v[k], d[0], d[kVPartHalfs]);
-    }
+    return;
   }
+  // The wave's tiles in turn (32 consecutive tokens lie in one or two); tokens
+  // whose chunk the wave does not fill are stored one by one.
+  uint64_t single = 0ull;
+  while (pending != 0ull) {
+    const int leader = (int)__builtin_ctzll(pending);
+    const int64_t first = read_lane64(tile, leader);
+    const bool mine = ((pending >> lane) & 1ull) != 0ull && tile == first;
+    const uint64_t group = __ballot(mine);
+    pending &= ~group;
+    if (__popcll(group) < 16) {              // no 8 tokens (of two lanes each)
+      single |= group;
+      continue;
+    }
+    uint32_t have = mine ? 1u << tt : 0u;    // token slots of the tile, then its whole chunks' low bits
+#pragma unroll
+    for (int o = 16; o >= 1; o >>= 1) have |= (uint32_t)__shfl_xor((int)have, o, 64);
+    uint32_t full = 0u;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) full |= ((have >> (8 * g)) & 0xFFu) == 0xFFu ? 1u << (8 * g) : 0u;
+    if (full != 0u)
+      store_v_tile(v, mine, tt, full, w.vimg + first * kVImgHalfs, reinterpret_cast<float*>(&sel), lane);
+    single |= __ballot(mine && ((full >> (tt & 24)) & 1u) == 0u);
+  }
+  if (single != 0ull) store_v_tokens(v, single, tile, tt, w.vimg, reinterpret_cast<float*>(&sel), lane);
 }
 
 // A step's request layout on its way from the host to the device: the first
@@ -521,7 +642,7 @@ __global__ __launch_bounds__(256, 2) void quant_write_fused_kernel(
   const QParams p = vector_params(v, side == 0 ? clip_k : clip_v, sel, lane);
   const int64_t slot = live ? slots[tok] : -1;
   quantize_store(v, p, slot, head, side, half, c);
-  if (w.rows > 0 && slot >= 0) window_epilogue(v, tok, slot, head, side, half, c.block_size, w);
+  if (w.rows > 0) window_epilogue(v, tok, slot, head, side, lane, c.block_size, w, sel);
 }
 
 // ---------------------------------------------------------------------------
