@@ -83,6 +83,7 @@ struct PrefillItem {
   int32_t tok0;        // first token in q / k_new / v_new / out (fp32 inputs: of the whole call)
   int32_t tile0;       // first new-token key tile
   int32_t rb0;         // first row block of the item (kv heads x row blocks)
+  int32_t out0;        // first token in the step's output (rotated output)
 };
 
 struct PrefillArgs {
@@ -910,41 +911,18 @@ __global__ __launch_bounds__(512, 2) void prefill_kernel(PrefillArgs a) {
   }
 }
 
-// Rows of the row blocks that the shares cut: their partials LSE-combined and
-// normalised.  kWavesPerRow waves share a row's partials (one where a row has
-// few of them, four where the work of few rows is spread over the GPU); lane
-// l holds features 4l .. 4l + 3, and the partials' (m, l) come in one
-// lane-parallel round per 64.  grid.x = row blocks x kTileRows x
-// kWavesPerRow / 4, 256 threads.
-template <int kWavesPerRow>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
-  constexpr int kRows = 4 / kWavesPerRow;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int grb = (int)blockIdx.x / (kTileRows / kRows);
-  int item = 0;
-  while (item + 1 < a.nitems && a.items[item + 1].rb0 <= grb) ++item;
-  const PrefillItem it = a.items[item];
-  const int nrb = row_blocks(it, a.group);
-  const int kvh = (grb - it.rb0) / nrb, rb = (grb - it.rb0) - kvh * nrb;
-  const int pr = ((int)blockIdx.x % (kTileRows / kRows)) * kRows + wave / kWavesPerRow;
-  const int row = rb * kTileRows + pr;
-  if (row >= it.n_new * a.group) return;
-  // units of the row block's first and last key block
-  const int64_t lo = it.unit0 + (int64_t)kvh * it.head_units + units_before(it, a.group, rb, lane) + kPieceCost;
-  const int64_t hi = lo + key_blocks(it, a.group, rb) - 1;
-  const int64_t w0 = lo / a.share, w1 = hi / a.share;
-  if (w0 == w1) return;                       // written whole by its share
-  const int n = (int)(w1 - w0) + 1;
-  auto slot = [&](int p) {
-    return a.part + (2 * (w0 + p) + (p == 0 && lo != w0 * a.share ? 1 : 0)) * (int64_t)kPartFloats;
-  };
+// Row pr of a row block from its n partials (slot(p)), LSE-combined and
+// normalised: lane l's features 4l .. 4l + 3.  With kWavesPerRow waves (the
+// workgroup's all), wave `first` takes partials first, first + kWavesPerRow,
+// ...; the (m, l) come in one lane-parallel round per 64 partials.
+template <int kWavesPerRow, class Slot>
+__device__ __forceinline__ floatx4 merge_row(const Slot& slot, int n, int pr, int first, int lane) {
   float mx = -__builtin_inff();
   for (int p = lane; p < n; p += 64) mx = fmaxf(mx, slot(p)[kPartRows * kHeadDim + pr]);
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
   // partials first, first + kWavesPerRow, ... of the row
-  const int first = wave % kWavesPerRow, mine = (n - first + kWavesPerRow - 1) / kWavesPerRow;
+  const int mine = (n - first + kWavesPerRow - 1) / kWavesPerRow;
   floatx4 acc = floatx4{};
   float l = 0.f;
   constexpr int kBatch = 8;
@@ -975,20 +953,223 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   if constexpr (kWavesPerRow > 1) {
     __shared__ floatx4 osum[kWavesPerRow][64];
     __shared__ float lsum[kWavesPerRow];
-    osum[wave][lane] = acc;
-    if (lane == 0) lsum[wave] = l;
+    osum[first][lane] = acc;
+    if (lane == 0) lsum[first] = l;
     __syncthreads();
-    if (wave != 0) return;
+    acc = osum[0][lane];
+    l = lsum[0];
 #pragma unroll
     for (int k = 1; k < kWavesPerRow; ++k) {
       acc += osum[k][lane];
       l += lsum[k];
     }
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  return acc * (l > 0.f ? 1.f / l : 0.f);
+}
+
+// Rows of the row blocks that the shares cut: their partials LSE-combined and
+// normalised.  kWavesPerRow waves share a row's partials (one where a row has
+// few of them, four where the work of few rows is spread over the GPU).
+// grid.x = row blocks x kTileRows x
+// kWavesPerRow / 4, 256 threads.
+template <int kWavesPerRow>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
+  constexpr int kRows = 4 / kWavesPerRow;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int grb = (int)blockIdx.x / (kTileRows / kRows);
+  int item = 0;
+  while (item + 1 < a.nitems && a.items[item + 1].rb0 <= grb) ++item;
+  const PrefillItem it = a.items[item];
+  const int nrb = row_blocks(it, a.group);
+  const int kvh = (grb - it.rb0) / nrb, rb = (grb - it.rb0) - kvh * nrb;
+  const int pr = ((int)blockIdx.x % (kTileRows / kRows)) * kRows + wave / kWavesPerRow;
+  const int row = rb * kTileRows + pr;
+  if (row >= it.n_new * a.group) return;
+  // units of the row block's first and last key block
+  const int64_t lo = it.unit0 + (int64_t)kvh * it.head_units + units_before(it, a.group, rb, lane) + kPieceCost;
+  const int64_t hi = lo + key_blocks(it, a.group, rb) - 1;
+  const int64_t w0 = lo / a.share, w1 = hi / a.share;
+  if (w0 == w1) return;                       // written whole by its share
+  const int n = (int)(w1 - w0) + 1;
+  auto slot = [&](int p) {
+    return a.part + (2 * (w0 + p) + (p == 0 && lo != w0 * a.share ? 1 : 0)) * (int64_t)kPartFloats;
+  };
+  const floatx4 o = merge_row<kWavesPerRow>(slot, n, pr, wave % kWavesPerRow, lane);
+  if (wave % kWavesPerRow != 0) return;
   const int tok = row / a.group, head = kvh * a.group + (row - tok * a.group);
-  *reinterpret_cast<floatx4*>(a.out + ((int64_t)(it.tok0 + tok) * a.num_heads + head) * kHeadDim + 4 * lane) =
-      acc * inv;
+  *reinterpret_cast<floatx4*>(a.out + ((int64_t)(it.tok0 + tok) * a.num_heads + head) * kHeadDim + 4 * lane) = o;
+}
+
+// The read's bf16 output: rows merged where the shares cut their row block
+// (merged: that is done, the rows are in a.out), multiplied by R_v^T and
+// rounded.  A workgroup takes 32 rows of a row block.  Its eight waves first
+// combine four rows each (lane l: features 4l .. 4l + 3), all rows' (m, l) in
+// one load where a row has at most 16 pieces, and leave them in LDS as the
+// bf16 high and low parts of MFMA operands; then wave t computes output
+// features {128 h + 16 t + i} of every row, its operand fragments of R_v^T
+// (rotation_operand's, high and low parts) straight from L2, kOutAhead steps
+// ahead of their use.  Products and their order are rotate_rows_kernel's:
+// R high x high, R low x high, R high x low.
+// Reading the partials (83 MB at 3001 tokens) bounds it from below; two
+// workgroups a CU overlap one's reads with the other's products.  The merge
+// and the rotation of the merged rows took 18 + 18 us (3001 tokens), 23 + 16
+// (1024 over 4K), 9 + 15 (77 over 20K) and 48 + 35 (9256 over 15K) as kernels
+// of their own; this takes 27, 22, 9 + 8.5 and 51.  64 rows a workgroup, whose
+// registers leave one to a CU, took 28, -, 9 + 11 and 55.
+constexpr int kOutAhead = 4;
+constexpr int kOutRows = 32;          // rows of a workgroup
+constexpr int kOutMine = kOutRows / 8;
+
+__global__ __launch_bounds__(512, 4) void prefill_output_kernel(PrefillArgs a, int merged,
+                                                                const uint8_t* __restrict__ rop,
+                                                                uint16_t* __restrict__ out) {
+  // [part][k-step][row ^ k-step, half][8]: chunk rows swizzled so that a
+  // wave's 16 k-steps of one row fall on different banks
+  __shared__ __attribute__((aligned(16))) __bf16 xs[2][16][64][8];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int grb = (int)blockIdx.x / (kTileRows / kOutRows);
+  const int pr0 = ((int)blockIdx.x % (kTileRows / kOutRows)) * kOutRows;
+  int item = 0;
+  while (item + 1 < a.nitems && a.items[item + 1].rb0 <= grb) ++item;
+  const PrefillItem it = a.items[item];
+  const int nrb = row_blocks(it, a.group);
+  const int kvh = (grb - it.rb0) / nrb, rb = (grb - it.rb0) - kvh * nrb;
+  const int rows = it.n_new * a.group;
+  if (rb * kTileRows + pr0 >= rows) return;
+
+  const u32x4* frag = reinterpret_cast<const u32x4*>(rop) + wave * 64 + lane;
+  auto load_r = [&](int m, int p) { return __builtin_bit_cast(bf16x8, frag[(m * 16 + p * 8) * 64]); };
+  bf16x8 f[kOutAhead][2];
+#pragma unroll
+  for (int m = 0; m < kOutAhead; ++m) {
+    f[m][0] = load_r(m, 0);
+    f[m][1] = load_r(m, 1);
+  }
+
+  // ---- rows pr0 + mine0 .. + kOutMine - 1 of the row block ----
+  const int mine0 = kOutMine * wave;
+  int n = 1;
+  int64_t w0 = 0;
+  bool second = false;                        // the first piece is its share's second partial
+  if (!merged) {
+    const int64_t lo = it.unit0 + (int64_t)kvh * it.head_units + units_before(it, a.group, rb, lane) + kPieceCost;
+    const int64_t hi = lo + key_blocks(it, a.group, rb) - 1;
+    w0 = lo / a.share;
+    n = (int)(hi / a.share - w0) + 1;
+    second = lo != w0 * a.share;
+  }
+  auto slot = [&](int p) { return a.part + (2 * (w0 + p) + (p == 0 && second ? 1 : 0)) * (int64_t)kPartFloats; };
+  auto put = [&](int i, const floatx4& x) {
+    const int rr = mine0 + i, m = (lane & 31) >> 1;
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    bf16x4 h, l;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      h[e] = (__bf16)x[e];
+      l[e] = (__bf16)(x[e] - (float)h[e]);
+    }
+    const int at = (rr ^ m) + (lane & 32), sub = 4 * (lane & 1);
+    *reinterpret_cast<bf16x4*>(&xs[0][m][at][sub]) = h;
+    *reinterpret_cast<bf16x4*>(&xs[1][m][at][sub]) = l;
+  };
+  const int row0 = rb * kTileRows + pr0 + mine0;
+  const int left = min(kOutMine, rows - row0);   // (<= 0: none of the wave's rows)
+  constexpr int kFew = 64 / kOutMine, kBatch = 8;
+  if (n == 1) {
+    floatx4 x[kOutMine];
+#pragma unroll
+    for (int i = 0; i < kOutMine; ++i) {
+      const int row = row0 + (i < left ? i : 0), tok = row / a.group, head = kvh * a.group + (row - tok * a.group);
+      x[i] = floatx4{};
+      if (i < left)
+        x[i] = *reinterpret_cast<const floatx4*>(a.out + ((int64_t)(it.tok0 + tok) * a.num_heads + head) * kHeadDim +
+                                                 4 * lane);
+    }
+#pragma unroll
+    for (int i = 0; i < kOutMine; ++i) put(i, x[i]);
+  } else if (n <= kFew) {
+    // lane kFew i + p: piece p of row i
+    const int wi = lane / kFew, wp = lane % kFew;
+    float mp = -__builtin_inff(), lp = 0.f;
+    if (wp < n && wi < left) {
+      const float* part = slot(wp) + kPartRows * kHeadDim + pr0 + mine0 + wi;
+      mp = part[0];
+      lp = part[kPartRows];
+    }
+    // the rows' pieces in batches, the next batch requested before one is used
+    constexpr int kSteps = kOutMine * (kFew / kBatch);
+    floatx4 x[2][kBatch];
+    auto load_batch = [&](int s) {
+      const int i = s / (kFew / kBatch), p0 = kBatch * (s % (kFew / kBatch));
+      if (p0 >= n) return;
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) {
+        x[s & 1][k] = floatx4{};
+        if (p0 + k < n && i < left)
+          x[s & 1][k] =
+              *reinterpret_cast<const floatx4*>(slot(p0 + k) + (int64_t)(pr0 + mine0 + i) * kHeadDim + 4 * lane);
+      }
+    };
+    load_batch(0);
+    float mx = mp;
+#pragma unroll
+    for (int o = kFew / 2; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    const float w = mp == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(mp - mx);
+    float l = w * lp;
+#pragma unroll
+    for (int o = kFew / 2; o >= 1; o >>= 1) l += __shfl_xor(l, o, 64);
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    floatx4 acc = floatx4{};
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      const int i = s / (kFew / kBatch), p0 = kBatch * (s % (kFew / kBatch));
+      if (s + 1 < kSteps) load_batch(s + 1);
+      if (p0 < n) {
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k)
+          if (p0 + k < n)
+            acc += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), kFew * i + p0 + k)) * x[s & 1][k];
+      }
+      if (p0 + kBatch == kFew) {
+        put(i, acc * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), kFew * i)));
+        acc = floatx4{};
+      }
+    }
+  } else {
+#pragma unroll 1
+    for (int i = 0; i < kOutMine; ++i) put(i, i < left ? merge_row<1>(slot, n, pr0 + mine0 + i, 0, lane) : floatx4{});
+  }
+  __syncthreads();
+
+  floatx16 acc = floatx16{};
+#pragma unroll
+  for (int m = 0; m < 16; ++m) {
+    const bf16x8 rh = f[m % kOutAhead][0], rl = f[m % kOutAhead][1];
+    if (m + kOutAhead < 16) {
+      f[m % kOutAhead][0] = load_r(m + kOutAhead, 0);
+      f[m % kOutAhead][1] = load_r(m + kOutAhead, 1);
+    }
+    const int at = ((lane & 31) ^ m) + (lane & 32);
+    const bf16x8 h = *reinterpret_cast<const bf16x8*>(&xs[0][m][at][0]);
+    const bf16x8 l = *reinterpret_cast<const bf16x8*>(&xs[1][m][at][0]);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rh, h, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rl, h, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rh, l, acc, 0, 0, 0);
+  }
+  const int row = rb * kTileRows + pr0 + (lane & 31);
+  if (row >= rows) return;
+  const int tok = row / a.group, head = kvh * a.group + (row - tok * a.group);
+  __bf16* d = reinterpret_cast<__bf16*>(out) + ((int64_t)(it.out0 + tok) * a.num_heads + head) * kHeadDim +
+              128 * (lane >> 5) + 16 * wave;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    bf16x8 o;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) o[u] = (__bf16)acc[8 * q + u];
+    reinterpret_cast<bf16x8*>(d)[q] = o;
+  }
 }
 
 // Operands (prefill_operands.h) of rotated fp32 rows: one 16-byte chunk per
@@ -1156,6 +1337,7 @@ void add_item(PrefillArgs& a, OperandItems& ops, int32_t n_new, int64_t cached, 
   it.cached = (int32_t)cached;
   it.req = req;
   it.tok0 = ops.tokens;
+  it.out0 = in_tok0;
   it.tile0 = ops.tiles;
   it.rb0 = 0;
   if (a.nitems > 0) {
@@ -1169,26 +1351,52 @@ void add_item(PrefillArgs& a, OperandItems& ops, int32_t n_new, int64_t cached, 
   ++a.nitems;
 }
 
-// The read over operands in the workspace: shares, then the merge of the row
-// blocks they cut.
-int launch_shares(PrefillArgs& a, hipStream_t stream) {
+// Row blocks of a launch.
+int64_t launch_row_blocks(const PrefillArgs& a) {
+  const PrefillItem& p = a.items[a.nitems - 1];
+  return p.rb0 + (((int64_t)p.n_new * a.group + kTileRows - 1) / kTileRows) * a.num_kv_heads;
+}
+
+// The read over operands in the workspace by shares; returns their number in
+// wgs.
+int launch_shares(PrefillArgs& a, int64_t& wgs, hipStream_t stream) {
   a.share = plan_share(a.units);
-  const int64_t wgs = (a.units + a.share - 1) / a.share;
+  wgs = (a.units + a.share - 1) / a.share;
   if (set_dynamic_lds(reinterpret_cast<const void*>(prefill_kernel<true>), (int)kPrefillLds, g_lds_set[1]) != kOk)
     return kErrLaunch;
   hipLaunchKernelGGL((prefill_kernel<true>), dim3((unsigned)wgs), dim3(64 * kWaves), kPrefillLds, stream, a);
-  if (hipGetLastError() != hipSuccess) return kErrLaunch;
-  if (wgs > 1) {
-    const PrefillItem& p = a.items[a.nitems - 1];
-    const int64_t rbs = p.rb0 + (((int64_t)p.n_new * a.group + kTileRows - 1) / kTileRows) * a.num_kv_heads;
-    // few row blocks in many shares: a workgroup per row
-    if (rbs * kMergeManyPieces <= wgs)
-      hipLaunchKernelGGL((prefill_merge_kernel<4>), dim3((unsigned)(rbs * kTileRows)), dim3(256), 0, stream, a);
-    else
-      hipLaunchKernelGGL((prefill_merge_kernel<1>), dim3((unsigned)(rbs * kTileRows / 4)), dim3(256), 0, stream, a);
-    if (hipGetLastError() != hipSuccess) return kErrLaunch;
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+// Few row blocks in many shares: a workgroup per row merges them.
+bool many_pieces(const PrefillArgs& a, int64_t wgs) { return launch_row_blocks(a) * kMergeManyPieces <= wgs; }
+
+int launch_merge(const PrefillArgs& a, int64_t wgs, hipStream_t stream) {
+  if (wgs <= 1) return kOk;
+  const int64_t rbs = launch_row_blocks(a);
+  if (many_pieces(a, wgs))
+    hipLaunchKernelGGL((prefill_merge_kernel<4>), dim3((unsigned)(rbs * kTileRows)), dim3(256), 0, stream, a);
+  else
+    hipLaunchKernelGGL((prefill_merge_kernel<1>), dim3((unsigned)(rbs * kTileRows / 4)), dim3(256), 0, stream, a);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+// The bf16 output of the shares: merge and rotation in one pass, unless rows
+// average more pieces than a wave's one round of (m, l) takes: a workgroup per
+// row then merges them first (77 tokens over 20K: two row blocks of 128
+// pieces, which the 16 workgroups of the output pass could not read quickly).
+int launch_output(const PrefillArgs& a, int64_t wgs, const void* rop, void* out_bf16, hipStream_t stream) {
+  const int64_t rbs = launch_row_blocks(a);
+  const bool many = wgs > 1 && rbs * (64 / kOutMine) <= wgs;
+  if (many) {
+    const int st = launch_merge(a, wgs, stream);
+    if (st != kOk) return st;
   }
-  return kOk;
+  const uint8_t* r = static_cast<const uint8_t*>(rop);
+  uint16_t* o = static_cast<uint16_t*>(out_bf16);
+  hipLaunchKernelGGL(prefill_output_kernel, dim3((unsigned)(rbs * (kTileRows / kOutRows))), dim3(512), 0, stream, a,
+                     (int)many, r, o);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
 void bind_workspace(PrefillArgs& a, PrefillOperands& o, const Layout& w, uint8_t* ws) {
@@ -1244,7 +1452,9 @@ extern "C" int oscar_prefill_continuation_split(
   const int64_t blocks = (c.q_chunks + 2 * c.kv_chunks + 255) / 256;
   hipLaunchKernelGGL(convert_operands_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, c);
   if (hipGetLastError() != hipSuccess) return kErrLaunch;
-  return launch_shares(a, stream);
+  int64_t wgs = 0;
+  if ((st = launch_shares(a, wgs, stream)) != kOk) return st;
+  return launch_merge(a, wgs, stream);
 }
 
 extern "C" int oscar_prefill_continuation(
@@ -1352,19 +1562,9 @@ extern "C" int oscar_prefill_rotated(
                                 kv_token_stride, num_heads, num_kv_heads, static_cast<const uint8_t*>(rot_k_operand),
                                 static_cast<const uint8_t*>(rot_v_operand), ops, o, stream);
     if (st != kOk) return st;
-    if ((st = launch_shares(a, stream)) != kOk) return st;
-    // R_v^T and the bf16 cast: one launch per run of adjacent requests
-    for (int32_t i = 0; i < ops.n;) {
-      int32_t j = i + 1;
-      while (j < ops.n && ops.it[j].tok0 == ops.it[j - 1].tok0 + ops.it[j - 1].n_new) ++j;
-      const int64_t tokens = ops.it[j - 1].ctok0 + ops.it[j - 1].n_new - ops.it[i].ctok0;
-      st = oscar_rotate_rows(a.out + (int64_t)ops.it[i].ctok0 * num_heads * kHeadDim, 1, kHeadDim,
-                             tokens * num_heads, head_size, rot_v_t_operand,
-                             static_cast<uint16_t*>(out_bf16) + (int64_t)ops.it[i].tok0 * num_heads * kHeadDim, 1,
-                             kHeadDim, stream);
-      if (st != kOk) return st;
-      i = j;
-    }
+    int64_t wgs = 0;
+    if ((st = launch_shares(a, wgs, stream)) != kOk) return st;
+    if ((st = launch_output(a, wgs, rot_v_t_operand, out_bf16, stream)) != kOk) return st;
   }
   return kOk;
 }
