@@ -24,6 +24,8 @@
 // With a window arena (oscar_quant_write_window) the fused kernel also does
 // the window write of the step's bulk tokens from the same rotated values
 // (see window_epilogue), after a seat-winner pass over the step's slots.
+#include <type_traits>
+
 #include "int2_quant.h"
 #include "prefill_operands.h"
 #include "step_launch.h"
@@ -675,11 +677,9 @@ __device__ constexpr int kRotWait(int m) {
 }
 
 // The rotation of one wave's 32 rows: lane l's row starts at xsrc (its input
-// features 128 (l >> 5) .. +127).  kSwap = false: register i of tile t is
-// output feature 128 (l >> 5) + 16 t + i of row l & 31.  kSwap = true (the
-// operands change sides): register i is row 8 (i >> 2) + 4 (l >> 5) + (i & 3)
-// and the lane is the operand's feature of tile t (rot_lane_feature).
-template <bool kF32In, bool kSwap>
+// features 128 (l >> 5) .. +127); register i of tile t is output feature 128 (l
+// >> 5) + 16 t + i of row l & 31.
+template <bool kF32In>
 __device__ __forceinline__ void rotate_tile(const uint8_t* __restrict__ xsrc, const uint8_t* __restrict__ rop,
                                             uint8_t* ring, int wave, int lane, floatx16 (&acc)[8]) {
   using Sched = RotSched<kF32In>;
@@ -755,8 +755,7 @@ __device__ __forceinline__ void rotate_tile(const uint8_t* __restrict__ xsrc, co
       if (i + kAhead < kPairs)
         a[i % kAhead] = __builtin_bit_cast(bf16x8, a_src[((i + kAhead) & 15) * 64 + lane]);
       const bf16x8 x = i < 16 ? xh : xl;
-      acc[i & 7] = kSwap ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, cur, acc[i & 7], 0, 0, 0)
-                         : __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur, x, acc[i & 7], 0, 0, 0);
+      acc[i & 7] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur, x, acc[i & 7], 0, 0, 0);
     }
     __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
 #pragma unroll
@@ -779,8 +778,8 @@ __global__ __launch_bounds__(256, 2) void rotate_rows_kernel(const void* __restr
   const bool live = row < rows;
   const int64_t rr = live ? row : 0;        // a lane past the last row computes row 0 and stores nothing
   floatx16 acc[8];
-  rotate_tile<kF32In, false>(static_cast<const uint8_t*>(in) + (rr * in_stride + kPerLane * half) * (kF32In ? 4 : 2),
-                             rop, ring, wave, lane, acc);
+  rotate_tile<kF32In>(static_cast<const uint8_t*>(in) + (rr * in_stride + kPerLane * half) * (kF32In ? 4 : 2),
+                     rop, ring, wave, lane, acc);
   if (!live) return;
   // register i of tile t: output feature 128 half + 16 t + i
   if constexpr (kBf16Out) {
@@ -806,12 +805,20 @@ __global__ __launch_bounds__(256, 2) void rotate_rows_kernel(const void* __restr
 }
 
 // Operands of the prefill read (prefill_operands.h) from the step's bf16
-// query, key and value, in one launch: workgroups of 128 query rows, then of
-// four 32-token key tiles, then of four value tiles; each rotates as
-// rotate_rows_kernel does and rounds to fp16 what the read rounded when it
-// built its tiles from fp32 rows.  Queries and keys keep a row per lane; the
-// values' rotation runs with the operands exchanged, so that a lane holds one
-// feature of 16 tokens, which are its two 16-byte chunks of the V tile.
+// query, key and value, in one launch: workgroups of 32 query rows, then of
+// one 32-token key tile, then of one value tile.  The eight waves bring the
+// rows to LDS as MFMA operands; then wave t computes rotated features {128 h +
+// 16 t + i} of every row, its operand fragments of R (bf16 high, then low
+// part) straight from L2, kOpAhead steps ahead of their use, and rounds to
+// fp16 what the read rounded when it built its tiles from fp32 rows.  Queries
+// and keys keep a row per lane; the values' product runs with the operands
+// exchanged, so that a lane holds one feature of 16 tokens, which are its two
+// 16-byte chunks of the V tile.
+// Small calls are bound by one workgroup's latency, large ones by reading R
+// (256 KB a workgroup) from L2.  128 rows to a workgroup with R through an LDS
+// ring took 18.4 us for 3001 tokens, 12.6 for 1024, 11.0 for 77 and 41 for
+// 9256 (six query heads); this takes 14.9, 7.6, 5.8 and 38.  64 rows, which
+// read R half as often, took 15.2, 9.5, 7.9 and 34: only the last is better.
 struct RotateOperandArgs {
   const uint16_t* q;
   const uint16_t* k;
@@ -824,90 +831,115 @@ struct RotateOperandArgs {
   int32_t q_blocks, kv_blocks;
   OperandItems items;
 };
+constexpr int kOpAhead = 4;
 
-__global__ __launch_bounds__(256, 2) void rotate_operands_kernel(RotateOperandArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t ring[];
+__global__ __launch_bounds__(512, 4) void rotate_operands_kernel(RotateOperandArgs a) {
+  // [k-step][row ^ k-step, half][8]: swizzled so that the 16 k-steps of one
+  // row fall on different banks
+  __shared__ __attribute__((aligned(16))) uint16_t xs[kSteps][64][8];
+  __shared__ float qs[8][32];
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int half = lane >> 5;
   int blk = blockIdx.x;
-  floatx16 acc[8];
-  // the last item whose first unit (compact token or tile) is at or below u
-  auto item_of = [&](int u, bool tiles) {
-    int i = 0;
-    while (i + 1 < a.items.n && (tiles ? a.items.it[i + 1].tile0 : a.items.it[i + 1].ctok0) <= u) ++i;
-    return i;
+  const int kind = blk < a.q_blocks ? 0 : (blk < a.q_blocks + a.kv_blocks ? 1 : 2);    // query, key, value
+  blk -= kind == 0 ? 0 : (kind == 1 ? a.q_blocks : a.q_blocks + a.kv_blocks);
+  const u32x4* frag = reinterpret_cast<const u32x4*>(kind == 2 ? a.rot_v : a.rot_k) + wave * 64 + lane;
+  auto load_r = [&](int m, int p) { return __builtin_bit_cast(bf16x8, frag[(m * 16 + p * 8) * 64]); };
+  bf16x8 f[kOpAhead][2];
+#pragma unroll
+  for (int m = 0; m < kOpAhead; ++m) {
+    f[m][0] = load_r(m, 0);
+    f[m][1] = load_r(m, 1);
+  }
+
+  // ---- rows to LDS: piece u & 31 (eight features) of row u >> 5 ----
+  const int rows = a.items.tokens * a.num_heads;
+  u32x4 piece[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int u = (int)threadIdx.x + 512 * i, r = u >> 5;
+    const uint16_t* src;
+    if (kind == 0) {
+      const int rr = min(blk * 32 + r, rows - 1), ct = rr / a.num_heads, h = rr - ct * a.num_heads;
+      int it = 0;
+      while (it + 1 < a.items.n && a.items.it[it + 1].ctok0 <= ct) ++it;
+      src = a.q + (int64_t)(a.items.it[it].tok0 + (ct - a.items.it[it].ctok0)) * a.q_stride + (int64_t)h * kHeadDim;
+    } else {
+      const int tile = blk / a.num_kv_heads, head = blk - tile * a.num_kv_heads;
+      int n = 0;
+      while (n + 1 < a.items.n && a.items.it[n + 1].tile0 <= tile) ++n;
+      const OperandItem it = a.items.it[n];
+      const int j = min((tile - it.tile0) * kKeyBlk + r, it.n_new - 1);
+      src = (kind == 2 ? a.v : a.k) + (int64_t)(it.tok0 + j) * a.kv_stride + (int64_t)head * kHeadDim;
+    }
+    piece[i] = reinterpret_cast<const u32x4*>(src)[u & 31];
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int u = (int)threadIdx.x + 512 * i, r = u >> 5, m = u & 15;
+    *reinterpret_cast<u32x4*>(&xs[m][(r ^ m) + 32 * ((u >> 4) & 1)][0]) = piece[i];
+  }
+  __syncthreads();
+
+  floatx16 acc = floatx16{};
+  auto product = [&](auto swap_tag) {
+    constexpr bool kSwap = decltype(swap_tag)::value;
+#pragma unroll
+    for (int m = 0; m < kSteps; ++m) {
+      const bf16x8 rh = f[m % kOpAhead][0], rl = f[m % kOpAhead][1];
+      if (m + kOpAhead < kSteps) {
+        f[m % kOpAhead][0] = load_r(m + kOpAhead, 0);
+        f[m % kOpAhead][1] = load_r(m + kOpAhead, 1);
+      }
+      const bf16x8 x = *reinterpret_cast<const bf16x8*>(&xs[m][((lane & 31) ^ m) + (lane & 32)][0]);
+      acc = kSwap ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, rh, acc, 0, 0, 0)
+                  : __builtin_amdgcn_mfma_f32_32x32x16_bf16(rh, x, acc, 0, 0, 0);
+      acc = kSwap ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, rl, acc, 0, 0, 0)
+                  : __builtin_amdgcn_mfma_f32_32x32x16_bf16(rl, x, acc, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);      // (keeps the scheduler from hoisting every step's reads)
+    }
   };
-  if (blk < a.q_blocks) {
-    const int rows = a.items.tokens * a.num_heads;
-    const int row = blk * (kFusedWaves * kTokPerWave) + wave * kTokPerWave + (lane & 31);
-    const int rr = min(row, rows - 1);
-    const int ct = rr / a.num_heads, h = rr - ct * a.num_heads;
-    int i = 0;
-    while (i + 1 < a.items.n && a.items.it[i + 1].ctok0 <= ct) ++i;
-    const int64_t tok = a.items.it[i].tok0 + (ct - a.items.it[i].ctok0);
-    rotate_tile<false, false>(reinterpret_cast<const uint8_t*>(a.q + tok * a.q_stride + (int64_t)h * kHeadDim +
-                                                               kPerLane * half),
-                              a.rot_k, ring, wave, lane, acc);
-    half8* dst = reinterpret_cast<half8*>(a.o.q16 + (int64_t)rr * kHeadDim + kPerLane * half);
-    float qs = 0.f;
-#pragma unroll
-    for (int t = 0; t < 8; ++t)
-#pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        half8 o;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          o[e] = (_Float16)acc[t][k_feature(8 * g + e)];
-          qs += (float)o[e];
-        }
-        if (row < rows) dst[2 * t + g] = o;
-      }
-    qs += shfl_xor_f32(qs, 32);
-    if (row < rows && half == 0) a.o.qsum[row] = qs;
-    return;
-  }
-  blk -= a.q_blocks;
-  const bool value = blk >= a.kv_blocks;
-  if (value) blk -= a.kv_blocks;
-  const int units = a.items.tiles * a.num_kv_heads;
-  const int u = blk * kFusedWaves + wave;                 // (tile, kv head) of this wave
-  const int uc = min(u, units - 1);
-  const int tile = uc / a.num_kv_heads, head = uc - tile * a.num_kv_heads;
-  const OperandItem it = a.items.it[item_of(tile, true)];
-  const int j = min((tile - it.tile0) * kKeyBlk + (lane & 31), it.n_new - 1);
-  const uint16_t* src = (value ? a.v : a.k) + (int64_t)(it.tok0 + j) * a.kv_stride + (int64_t)head * kHeadDim +
-                        kPerLane * half;
-  if (!value) {
-    rotate_tile<false, false>(reinterpret_cast<const uint8_t*>(src), a.rot_k, ring, wave, lane, acc);
-    if (u >= units) return;
-    const int token = lane & 31;
-    half8* dst = reinterpret_cast<half8*>(a.o.kimg + (int64_t)u * kKeyTileHalfs) + token * (kHeadDim / 8);
-#pragma unroll
-    for (int t = 0; t < 8; ++t)
-#pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        half8 o;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = (_Float16)acc[t][k_feature(8 * g + e)];
-        dst[k_chunk(2 * (8 * half + t) + g, token)] = o;
-      }
-    return;
-  }
-  rotate_tile<false, true>(reinterpret_cast<const uint8_t*>(src), a.rot_v, ring, wave, lane, acc);
-  if (u >= units) return;
-  half8* dst = reinterpret_cast<half8*>(a.o.vimg + (int64_t)u * kKeyTileHalfs);
-  const int r = lane & 31;
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const int f = 128 * ((r >> 2) & 1) + 16 * t + 4 * (r >> 3) + (r & 3);     // the operand's feature of this lane
+  if (kind == 2) {
+    product(std::true_type{});
+    const int r = lane & 31;
+    const int ft = 128 * ((r >> 2) & 1) + 16 * wave + 4 * (r >> 3) + (r & 3);   // the operand's feature of this lane
+    half8* dst = reinterpret_cast<half8*>(a.o.vimg + (int64_t)blk * kKeyTileHalfs);
 #pragma unroll
     for (int mm = 0; mm < 2; ++mm) {
       half8 o;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = (_Float16)acc[t][8 * mm + e];
-      dst[f * (kKeyBlk / 8) + v_chunk(2 * mm + half, f)] = o;
+      for (int e = 0; e < 8; ++e) o[e] = (_Float16)acc[8 * mm + e];
+      dst[ft * (kKeyBlk / 8) + v_chunk(2 * mm + half, ft)] = o;
     }
+    return;
+  }
+  product(std::false_type{});
+  const int row = blk * 32 + (lane & 31);
+  half8* dst = kind == 0 ? reinterpret_cast<half8*>(a.o.q16 + (int64_t)row * kHeadDim)
+                         : reinterpret_cast<half8*>(a.o.kimg + (int64_t)blk * kKeyTileHalfs) +
+                               (lane & 31) * (kHeadDim / 8);
+  float sum = 0.f;
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    half8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      o[e] = (_Float16)acc[k_feature(8 * g + e)];
+      sum += (float)o[e];
+    }
+    const int c = 2 * (8 * half + wave) + g;
+    if (kind == 1 || row < rows) dst[kind == 0 ? c : k_chunk(c, lane & 31)] = o;
+  }
+  if (kind == 1) return;
+  sum += shfl_xor_f32(sum, 32);
+  if (half == 0) qs[wave][lane] = sum;
+  __syncthreads();
+  if ((int)threadIdx.x < 32) {
+    float total = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) total += qs[w][threadIdx.x];
+    if (row < rows) a.o.qsum[row] = total;
   }
 }
 
@@ -949,7 +981,6 @@ int check_cache_args(CacheArgs& c) {
 
 std::atomic<uint64_t> g_lds_set{0};   // dynamic-LDS attribute set, one bit per device
 std::atomic<uint64_t> g_rot_lds_set[4] = {{0}, {0}, {0}, {0}};   // the same for the rotate_rows instances
-std::atomic<uint64_t> g_operand_lds_set{0};
 
 }  // namespace
 
@@ -959,13 +990,9 @@ int launch_rotate_operands(const uint16_t* q, int64_t q_stride, const uint16_t* 
                            hipStream_t stream) {
   RotateOperandArgs a{q, k, v, q_stride, kv_stride, num_heads, num_kv_heads, rot_k, rot_v, o, 0, 0, items};
   const int64_t rows = (int64_t)items.tokens * num_heads, units = (int64_t)items.tiles * num_kv_heads;
-  a.q_blocks = (int32_t)((rows + kFusedWaves * kTokPerWave - 1) / (kFusedWaves * kTokPerWave));
-  a.kv_blocks = (int32_t)((units + kFusedWaves - 1) / kFusedWaves);
-  constexpr int kRingLds = kRing * kChunkBytes;
-  if (set_dynamic_lds(reinterpret_cast<const void*>(rotate_operands_kernel), kRingLds, g_operand_lds_set) != kOk)
-    return kErrLaunch;
-  hipLaunchKernelGGL(rotate_operands_kernel, dim3((unsigned)(a.q_blocks + 2 * a.kv_blocks)), dim3(256), kRingLds,
-                     stream, a);
+  a.q_blocks = (int32_t)((rows + 31) / 32);
+  a.kv_blocks = (int32_t)units;
+  hipLaunchKernelGGL(rotate_operands_kernel, dim3((unsigned)(a.q_blocks + 2 * a.kv_blocks)), dim3(512), 0, stream, a);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
