@@ -1,29 +1,29 @@
 // Fused rotate + sort-clip + INT2 quantize + 4-codes-per-byte pack + paged
 // slot write (gfx950).
 //
-// Work layout: one wavefront owns 32 tokens of one (kv-head, K-or-V) side.
-// Lane l holds token (l & 31), features 128*(l >> 5) .. +127 of that token in
-// 128 fp32 registers, so every per-vector reduction is lane-local plus one
-// exchange with lane l ^ 32.  That is exactly the fp32 accumulator layout of
-// a 32x32 MFMA tile whose columns are tokens, which the fused entry point
-// uses for the 256x256 rotation (bf16 hi + lo split of R, two passes; the
-// operand streams through a 4-deep LDS ring filled by direct-to-LDS loads).
+// Work layout of the fused entry: a workgroup of eight wavefronts takes 32
+// tokens of one (kv-head, K-or-V) side.  Each wavefront computes an eighth of
+// the 256x256 rotation's output features for all of them on MFMA (bf16 hi + lo
+// split of R, two passes); the values change hands through LDS, after which a
+// row of 16 lanes holds a vector and everything that concerns it stays in the
+// row.  The pre-rotated entry has one wavefront to 32 tokens, lane l holding
+// features 128 (l >> 5) .. +127 of token l & 31.
 //
 // Clip threshold (the idx-th smallest |x| of a vector, i.e. its kk-th largest
 // with kk = 256 - idx) without sorting: a 64-bucket histogram of |x| keyed on
 // the float bits (bucket = key(max|x|) - key(|x|), key = bits >> S, S = 18:
 // 1/32 octave per bucket over two octaves) built with LDS atomics gives the
-// bucket holding the answer and its rank j inside that bucket; the bucket's
-// few values are gathered into small per-lane LDS lists and the j-th largest
-// of them is taken exactly (ties counted).  Vectors whose answer lies outside
-// the histogram's range or whose bucket overflows the lists use a bitwise
-// radix select instead (exact, slow, rare).
+// bucket holding the answer and its rank inside that bucket; the bucket's few
+// values are gathered into small LDS lists and the answer is taken exactly
+// (ties counted).  Vectors whose answer lies outside the histogram's range or
+// whose bucket overflows the lists use a bitwise radix select instead (exact,
+// slow, rare).
 //
 // Quantization: the exact divide-free thresholds of int2_quant.h.
 //
 // With a window arena (oscar_quant_write_window) the fused kernel also does
-// the window write of the step's bulk tokens from the same rotated values
-// (see window_epilogue), after a seat-winner pass over the step's slots.
+// the window write of the step's bulk tokens from the same rotated values,
+// after a seat-winner pass over the step's slots.
 #include <type_traits>
 
 #include "int2_quant.h"
@@ -261,178 +261,6 @@ __device__ __forceinline__ int64_t read_lane64(int64_t x, int lane) {
                    (uint32_t)__builtin_amdgcn_readlane((int)x, lane));
 }
 
-// LDS of a wave's V image transpose: 32 features of each lane half by the 32
-// token slots of a tile, rows of 36 words (16-byte reads), the halves 32 words
-// apart modulo the 64 banks.
-constexpr int kTrRow = 36;
-constexpr int kTrHalf = 32 * kTrRow + 32;
-static_assert(2 * kTrHalf * sizeof(float) <= sizeof(SelLds), "the transpose reuses the selection's LDS");
-
-// The V image of the wave's tokens in one 32-token tile: `mine` on the lanes
-// whose token (token slot tt of the tile) is stored, full: the tile's 8-token
-// chunks (bytes of the mask) that those tokens fill, which alone are written.
-// A lane holds one token's features, an image chunk one feature's eight
-// tokens, so the values go through LDS, 32 features of each half at a time,
-// and out as 16-byte stores.  (Two-byte stores, token by token, touch 64
-// lines per wave and instruction; 256 of them took 23 us of a 45 us write
-// that is one workgroup deep; image and arena take 7 this way, 14 where 28
-// tokens of short requests go one by one.)
-__device__ __forceinline__ void store_v_tile(const float (&v)[kPerLane], bool mine, int tt, uint32_t full,
-                                             _Float16* img, float* T, int lane) {
-  const int half = lane >> 5;
-  const int r = tt & 7;                                    // place of the token in its chunk
-  const int place = (tt & 24) | (r == 1 ? 2 : (r == 2 ? 1 : (r == 5 ? 6 : (r == 6 ? 5 : r))));
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    wave_sync_lds();
-    if (mine) {
-#pragma unroll
-      for (int j = 0; j < 32; ++j) T[half * kTrHalf + j * kTrRow + place] = v[32 * p + j];
-    }
-    wave_sync_lds();
-    // chunk lane & 15 (m), then b, token group and half: 512-byte runs
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int u = 64 * i + lane;
-      const int ml = u & 15, grp = (u >> 4) & 3, b = (u >> 6) & 1, h = u >> 7;
-      const int j = 4 * (ml >> 1) + 2 * b + (ml & 1);      // feature 128 h + 32 p + j
-      if (((full >> (8 * grp)) & 1u) == 0u) continue;
-      const float* src = T + h * kTrHalf + j * kTrRow + 8 * grp;
-      const floatx4 x0 = reinterpret_cast<const floatx4*>(src)[0], x1 = reinterpret_cast<const floatx4*>(src)[1];
-      half8 hi, lo;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        _Float16 a, c;
-        fp16_parts(e < 4 ? x0[e] : x1[e - 4], a, c);
-        hi[e] = a;
-        lo[e] = c;
-      }
-      _Float16* d = img + vimg_offset(128 * h + 32 * p + j, 8 * grp);
-      *reinterpret_cast<half8*>(d) = hi;
-      *reinterpret_cast<half8*>(d + kVPartHalfs) = lo;
-    }
-  }
-}
-
-// The V image of single tokens (bits of `single`, both lanes of each): 64
-// features of a token at a time, 2-byte stores.  (A store per feature of the
-// lanes' own tokens would be 256 instructions however few the tokens; 8 a
-// token this way.)
-__device__ __forceinline__ void store_v_tokens(const float (&v)[kPerLane], uint64_t single, int64_t tile, int tt,
-                                               _Float16* vimg, float* T, int lane) {
-  const int half = lane >> 5, j = lane & 31;
-  const bool mine = ((single >> lane) & 1ull) != 0ull;
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    wave_sync_lds();
-    if (mine) {
-#pragma unroll
-      for (int i = 0; i < 32; ++i) T[half * kTrHalf + i * kTrRow + j] = v[32 * p + i];
-    }
-    wave_sync_lds();
-    // (four tokens in flight; the last one again when fewer are left)
-#pragma unroll 1
-    for (uint32_t left = (uint32_t)single; left != 0u;) {
-      float x[4];
-      _Float16* d[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = (int)__builtin_ctz(left);
-        if (e == 3 || (left & (left - 1)) != 0u) left &= left - 1;
-        x[e] = T[half * kTrHalf + j * kTrRow + t];
-        d[e] = vimg + read_lane64(tile, t) * kVImgHalfs +
-               vimg_offset(kPerLane * half + 32 * p + j, __builtin_amdgcn_readlane(tt, t));
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) fp16_parts(x[e], d[e][0], d[e][kVPartHalfs]);
-    }
-  }
-}
-
-// The window half of the bulk write (the reference's _staging_write,
-// backend.py:439-481) for this lane's token (slot; negative: none): if the
-// token won its seat, it sets the seat's owner (the K side of head 0 does) to
-// its page when it lies in the sink or recent window and to -1 otherwise; a
-// kept token then stores this lane's 128 unclipped rotated values (features
-// 128 half .. +127 of this side and head) and their fp16 image parts.  The
-// lane's token half is exactly one lane of the K image (token row prow % 32,
-// half g), so the K parts go out as 16-byte blocks; the V image holds tokens
-// in slots, which neighbouring tokens fill together (store_v_tile).  Called
-// by every lane of the wavefront; sel: its selection LDS, free by now.
-__device__ __forceinline__ void window_epilogue(const float (&v)[kPerLane], int64_t tok, int64_t slot, int head,
-                                                int side, int lane, int block_size, const WindowArgs& w,
-                                                SelLds& sel) {
-  const int half = lane >> 5;
-  int64_t seat = 0, page = 0;
-  bool keep = false;
-  if (slot >= 0 &&
-      won_seat(w.winner, (int64_t)w.rows * block_size, slot, tok, block_size, w.rows, seat, page)) {
-    int lo = 0, hi = w.num_requests - 1;     // request of the token: last i with query_start[i] <= tok
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (w.query_start[mid] <= tok) lo = mid; else hi = mid - 1;
-    }
-    const int64_t seq = w.seq_lens[lo];
-    const int64_t pos = seq - w.query_start[lo + 1] + tok;
-    keep = pos >= seq - w.recent || pos < w.sink_eff;
-    if (side == 0 && head == 0 && half == 0) w.owner[seat] = keep ? page : -1;
-  }
-  uint64_t pending = __ballot(keep);         // (both halves of a token agree)
-  if (pending == 0ull) return;
-  if (keep) {
-    float* dst = (side == 0 ? w.stage_k : w.stage_v) + (seat * w.num_kv_heads + head) * kHeadDim + kPerLane * half;
-#pragma unroll
-    for (int k = 0; k < kPerLane / 4; ++k)
-      reinterpret_cast<floatx4*>(dst)[k] = floatx4{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
-  }
-  if (w.kimg == nullptr) return;
-  const int prow = (int)(slot - page * block_size);
-  const int64_t tile = image_of(seat / block_size, prow, block_size, head, w.num_kv_heads);
-  const int tt = prow & 31;
-  if (side == 0) {
-    if (!keep) return;
-    // block m = 2j + a, slot u = 2i + b: local feature 16j + 4a + i + 8b
-    _Float16* img = w.kimg + tile * kKImgHalfs + (tt + 32 * half) * 8;
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      half8 h, l;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const float x = v[16 * (m >> 1) + 4 * (m & 1) + (u >> 1) + 8 * (u & 1)];
-        h[u] = (_Float16)x;
-        l[u] = (_Float16)(x - (float)h[u]);
-      }
-      *reinterpret_cast<half8*>(img + m * 64 * 8) = h;
-      *reinterpret_cast<half8*>(img + kImgHalfs + m * 64 * 8) = l;
-    }
-    return;
-  }
-  // The wave's tiles in turn (32 consecutive tokens lie in one or two); tokens
-  // whose chunk the wave does not fill are stored one by one.
-  uint64_t single = 0ull;
-  while (pending != 0ull) {
-    const int leader = (int)__builtin_ctzll(pending);
-    const int64_t first = read_lane64(tile, leader);
-    const bool mine = ((pending >> lane) & 1ull) != 0ull && tile == first;
-    const uint64_t group = __ballot(mine);
-    pending &= ~group;
-    if (__popcll(group) < 16) {              // no 8 tokens (of two lanes each)
-      single |= group;
-      continue;
-    }
-    uint32_t have = mine ? 1u << tt : 0u;    // token slots of the tile, then its whole chunks' low bits
-#pragma unroll
-    for (int o = 16; o >= 1; o >>= 1) have |= (uint32_t)__shfl_xor((int)have, o, 64);
-    uint32_t full = 0u;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) full |= ((have >> (8 * g)) & 0xFFu) == 0xFFu ? 1u << (8 * g) : 0u;
-    if (full != 0u)
-      store_v_tile(v, mine, tt, full, w.vimg + first * kVImgHalfs, reinterpret_cast<float*>(&sel), lane);
-    single |= __ballot(mine && ((full >> (tt & 24)) & 1u) == 0u);
-  }
-  if (single != 0ull) store_v_tokens(v, single, tile, tt, w.vimg, reinterpret_cast<float*>(&sel), lane);
-}
-
 // A step's request layout on its way from the host to the device: the first
 // n of the ints go to dst.
 constexpr int kLayoutInts = 896;
@@ -515,8 +343,6 @@ constexpr size_t kMfmaOperandBytes = (size_t)kSteps * kChunkBytes;
 constexpr size_t kOperandBytes = kMfmaOperandBytes + sizeof(float) * kHeadDim * kHeadDim;
 constexpr int64_t kShortWriteVectors = 2048;   // at most 1024 tokens (the step write's limit)
 constexpr int kDmaPerChunk = kChunkBytes / (kFusedWaves * 64 * 16);   // 2 per thread
-constexpr size_t kFusedLds = kFusedWaves * sizeof(SelLds) > kRing * kChunkBytes
-                                 ? kFusedWaves * sizeof(SelLds) : (size_t)kRing * kChunkBytes;
 
 // Workgroup barrier without a memory fence: __syncthreads() would also wait
 // for every outstanding global access (vmcnt(0)) and so drain the ring's
@@ -535,116 +361,403 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
 
-__global__ __launch_bounds__(256, 2) void quant_write_fused_kernel(
+// DPP moves within a row of 16 lanes.
+template <int kCtrl>
+__device__ __forceinline__ uint32_t row_dpp(uint32_t x) {      // lanes without a source read 0
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, 0xF, 0xF, true);
+}
+constexpr int kRowRor = 0x120, kRowShr = 0x110;                // + distance
+
+template <class Op>
+__device__ __forceinline__ uint32_t row_reduce(uint32_t x, Op op) {   // result in every lane of the row
+  x = op(x, row_dpp<kRowRor + 8>(x));
+  x = op(x, row_dpp<kRowRor + 4>(x));
+  x = op(x, row_dpp<kRowRor + 2>(x));
+  return op(x, row_dpp<kRowRor + 1>(x));
+}
+
+__device__ __forceinline__ uint32_t row_scan(uint32_t x) {            // inclusive sum
+  x += row_dpp<kRowShr + 1>(x);
+  x += row_dpp<kRowShr + 2>(x);
+  x += row_dpp<kRowShr + 4>(x);
+  return x + row_dpp<kRowShr + 8>(x);
+}
+
+// The bulk write's workgroup: eight waves and 32 tokens of one (kv-head, K or
+// V) side.  Lane 16 i + j of a wave ends up with features 16 j .. 16 j + 15 of
+// the wave's token i, so that whatever concerns a vector stays in one row of
+// 16 lanes.
+constexpr int kFwTokens = 32;
+constexpr int kFwThreads = 512;
+constexpr int kFwTokPerWave = 4;
+constexpr int kFwPerLane = 16;
+constexpr int kFwAhead = 3;
+
+// LDS of the threshold search, per wave: a histogram and a candidate list per
+// token, and a word per lane that absorbs what belongs in neither (one word
+// per token would serialise its 16 lanes: 91 instead of 72 us for 65536
+// tokens).
+struct RowSelLds {
+  uint32_t hist[kFwTokPerWave][kHistStride];
+  uint32_t list[kFwTokPerWave][16];
+  uint32_t other[64];
+};
+
+// The idx-th smallest |x| (float bits) of the 256 values a row of lanes
+// holds, without sorting: select_clip_bits' histogram and candidates, a
+// vector to a row.  amax_bits = bits of max |x|.
+__device__ __forceinline__ uint32_t row_select(const float (&v)[kFwPerLane], int idx, uint32_t amax_bits,
+                                               RowSelLds& L, int lane) {
+  const uint32_t kk = (uint32_t)(kHeadDim - idx);
+  const int i4 = lane >> 4, j = lane & 15;
+  const int S = kk <= 40 ? 18 : 20;
+  uint32_t* flat = &L.hist[0][0];
+  constexpr int kWords = kFwTokPerWave * kHistStride;
+#pragma unroll
+  for (int i = 0; i < (kWords + 63) / 64; ++i)
+    if (i * 64 + lane < kWords) flat[i * 64 + lane] = 0u;
+  wave_sync_lds();
+  typedef __attribute__((address_space(3))) uint32_t lds_u32;
+  uint32_t* H = L.hist[i4];
+  const uint32_t kh = amax_bits >> S;
+  const uint32_t first = (uint32_t)(uintptr_t)(lds_u32*)H + 4u;      // bucket 63's word
+  const uint32_t other = (uint32_t)(uintptr_t)(lds_u32*)&L.other[lane];
+  const uint32_t low = kh - (uint32_t)(kHistBuckets - 1);
+#pragma unroll
+  for (int i = 0; i < kFwPerLane; ++i) {
+    const uint32_t b = __builtin_amdgcn_ubfe(__float_as_uint(v[i]), S, 31 - S) - low;
+    const uint32_t addr = b < (uint32_t)kHistBuckets ? first + 4u * b : other;
+    __atomic_fetch_add((lds_u32*)(uintptr_t)addr, 1u, __ATOMIC_RELAXED);
+  }
+  wave_sync_lds();
+  // Bucket b* where the count from the top reaches kk: lane j scans buckets
+  // 4j .. 4j + 3 from the top (words 64 - b).
+  uint32_t cnt[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) cnt[i] = H[kHistBuckets - 4 * j - i];
+  const uint32_t tot = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+  const uint32_t upto = row_scan(tot);
+  uint32_t run = upto - tot, hit = 0u;                  // hit: (bucket + 1) << 16 | count above it
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (run < kk && run + cnt[i] >= kk) hit = ((uint32_t)(4 * j + i + 1) << 16) | run;
+    run += cnt[i];
+  }
+  auto umax = [](uint32_t a, uint32_t b) { return max(a, b); };
+  hit = row_reduce(hit, umax);
+  const uint32_t keystar = kh + 1u - (hit >> 16), rem = kk - (hit & 0xFFFFu);
+  bool fb = hit == 0u || keystar == 0u;
+  // The values of bucket b*, packed over the row.
+  const uint32_t lo2 = keystar << (S + 1), w2 = 2u << S;
+  uint32_t n = 0u;
+#pragma unroll
+  for (int i = 0; i < kFwPerLane; ++i) n += ((__float_as_uint(v[i]) << 1) - lo2 < w2) ? 1u : 0u;
+  const uint32_t end = row_scan(n);
+  const uint32_t total = row_reduce(end, umax);
+  fb = fb || total > 16u;
+  uint32_t* list = L.list[i4];
+  uint32_t at = end - n;
+#pragma unroll
+  for (int i = 0; i < kFwPerLane; ++i) {
+    const uint32_t u = __float_as_uint(v[i]);
+    const bool match = (u << 1) - lo2 < w2;
+    *(match && at < 16u ? list + at : &L.other[lane]) = u & 0x7FFFFFFFu;
+    at += match ? 1u : 0u;
+  }
+  wave_sync_lds();
+  // The rem-th largest of the candidates, ties counted.
+  const uint32_t c = (uint32_t)j < total ? list[j] : 0u;
+  uint32_t gt = 0u, ge = 1u;
+  auto rank = [&](uint32_t o) {
+    gt += o > c ? 1u : 0u;
+    ge += o >= c ? 1u : 0u;
+  };
+  rank(row_dpp<kRowRor + 1>(c));
+  rank(row_dpp<kRowRor + 2>(c));
+  rank(row_dpp<kRowRor + 3>(c));
+  rank(row_dpp<kRowRor + 4>(c));
+  rank(row_dpp<kRowRor + 5>(c));
+  rank(row_dpp<kRowRor + 6>(c));
+  rank(row_dpp<kRowRor + 7>(c));
+  rank(row_dpp<kRowRor + 8>(c));
+  rank(row_dpp<kRowRor + 9>(c));
+  rank(row_dpp<kRowRor + 10>(c));
+  rank(row_dpp<kRowRor + 11>(c));
+  rank(row_dpp<kRowRor + 12>(c));
+  rank(row_dpp<kRowRor + 13>(c));
+  rank(row_dpp<kRowRor + 14>(c));
+  rank(row_dpp<kRowRor + 15>(c));
+  uint32_t res = row_reduce(gt < rem && rem <= ge ? c : 0u, umax);
+  if (__ballot(fb) != 0ull) {
+    // outside the histogram, or a crowded bucket: bitwise radix select (exact)
+    uint32_t prefix = 0u;
+#pragma unroll 1
+    for (int b = 30; b >= 0; --b) {
+      const uint32_t probe = prefix | (1u << b);
+      const float pf = __uint_as_float(probe);
+      uint32_t below = 0u;
+#pragma unroll
+      for (int i = 0; i < kFwPerLane; ++i) below += fabsf(v[i]) < pf ? 1u : 0u;
+      below = row_reduce(below, [](uint32_t a, uint32_t b2) { return a + b2; });
+      if ((uint32_t)idx >= below) prefix = probe;
+    }
+    if (fb) res = prefix;
+  }
+  return res;
+}
+
+// The V image of the workgroup's kept tokens, from their rotated values in
+// LDS (value(r, f): feature f of token r): seat_tile / seat_slot are token
+// lane & 31's image tile and its slot there (-1: not kept).  Wave w stores
+// features 32 w .. 32 w + 31.  An image chunk holds eight tokens of one
+// feature: chunks the workgroup's tokens fill leave as 16-byte stores, the
+// tokens of others go one by one.  (Two-byte stores for all of them, 256 a
+// token, took 23 us.)
+template <class Value>
+__device__ __forceinline__ void store_v_images(const Value& value, int64_t seat_tile, int seat_slot, uint8_t* inv,
+                                               _Float16* vimg, int wave, int lane) {
+  const int me = lane & 31;
+  uint32_t pending = (uint32_t)__ballot(seat_slot >= 0);
+  uint32_t single = 0u;
+  while (pending != 0u) {
+    const int leader = (int)__builtin_ctz(pending);
+    const int64_t tile = read_lane64(seat_tile, leader);
+    const bool mine = ((pending >> me) & 1u) != 0u && seat_tile == tile;
+    const uint32_t group = (uint32_t)__ballot(mine);
+    pending &= ~group;
+    uint32_t have = mine ? 1u << seat_slot : 0u, full = 0u;
+    if (__popc(group) >= 8) {
+#pragma unroll
+      for (int o = 16; o >= 1; o >>= 1) have |= (uint32_t)__shfl_xor((int)have, o, 64);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) full |= ((have >> (8 * g)) & 0xFFu) == 0xFFu ? 1u << (8 * g) : 0u;
+    }
+    single |= (uint32_t)__ballot(mine && ((full >> (seat_slot & 24)) & 1u) == 0u);
+    if (full == 0u) continue;
+    if (mine && lane < 32) inv[seat_slot] = (uint8_t)me;      // token of each slot
+    wave_sync_lds();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int u = 64 * i + lane;
+      const int ml = u & 15, b = (u >> 4) & 1, grp = u >> 5;
+      if (((full >> (8 * grp)) & 1u) == 0u) continue;
+      const int f = 32 * wave + 4 * (ml >> 1) + 2 * b + (ml & 1);
+      half8 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int t = e == 1 ? 2 : (e == 2 ? 1 : (e == 5 ? 6 : (e == 6 ? 5 : e)));
+        _Float16 x, y;
+        fp16_parts(value(inv[8 * grp + t], f), x, y);
+        hi[e] = x;
+        lo[e] = y;
+      }
+      _Float16* d = vimg + tile * kVImgHalfs + vimg_offset(f, 8 * grp);
+      *reinterpret_cast<half8*>(d) = hi;
+      *reinterpret_cast<half8*>(d + kVPartHalfs) = lo;
+    }
+    wave_sync_lds();
+  }
+  // two tokens at a time, a feature per lane (the last token twice if odd)
+  while (single != 0u) {
+    const int t0 = (int)__builtin_ctz(single);
+    single &= single - 1u;
+    const int t1 = single != 0u ? (int)__builtin_ctz(single) : t0;
+    single &= single - 1u;
+    const int64_t tile0 = read_lane64(seat_tile, t0), tile1 = read_lane64(seat_tile, t1);
+    const int slot0 = __builtin_amdgcn_readlane(seat_slot, t0), slot1 = __builtin_amdgcn_readlane(seat_slot, t1);
+    const int f = 32 * wave + me;
+    const bool first = lane < 32;
+    _Float16* d = vimg + (first ? tile0 : tile1) * kVImgHalfs + vimg_offset(f, first ? slot0 : slot1);
+    fp16_parts(value(first ? t0 : t1, f), d[0], d[kVPartHalfs]);
+  }
+}
+
+// Rotation, clip, quantization and slot write of 32 tokens, and their window
+// write.  The waves bring the tokens' rows to LDS as MFMA operands; wave t
+// computes rotated features {128 h + 16 t + i} of every token, its operand
+// fragments of R (bf16 high, then low part) straight from L2, kFwAhead steps
+// ahead; the values then change hands through LDS (64-byte chunks, swizzled)
+// so that each vector lies in one row of 16 lanes.
+// Writes up to 8K tokens are bound by one workgroup's latency, larger ones by
+// the products (two bf16 passes, 28 us for 65536 tokens at the rate of a
+// large library product) beside the selection's vector instructions, which a
+// CU's three workgroups overlap.  With 128 tokens to a workgroup of four
+// wavefronts, each with 32 tokens of its own and R through an LDS ring, 3001
+// tokens took 29 us with the window (their selection 10, its image 7), 1052
+// of a mixed step 36, 9256 29 and 65536 without one 71; this takes 11, 15, 20
+// and 67.  64 tokens to a workgroup (half the reading of R): 17, -, 25, 68.
+__global__ __launch_bounds__(kFwThreads, 4) void quant_write_fused_kernel(
     const uint16_t* __restrict__ key, const uint16_t* __restrict__ value, int64_t n_tokens,
     int64_t token_stride, const uint8_t* __restrict__ rot_k, const uint8_t* __restrict__ rot_v,
     const int64_t* __restrict__ slots, CacheArgs c, int clip_k, int clip_v, WindowArgs w) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t ring[];     // ring, then the selection buffers
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
+  // [k-step][row ^ k-step, half]; the selection's LDS once the products are done
+  __shared__ __attribute__((aligned(16))) uint16_t xs[kSteps][64][8];
+  static_assert(sizeof(RowSelLds) * (kFwThreads / 64) <= sizeof(xs), "the selection reuses the operands' LDS");
+  RowSelLds* sel = reinterpret_cast<RowSelLds*>(xs);
+  __shared__ floatx4 ys[kFwTokens * kHeadDim / 4];
+  __shared__ int64_t seat_tile[kFwTokens];
+  __shared__ int32_t seat_slot[kFwTokens];
+  __shared__ uint8_t inv[kFwThreads / 64][32];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int head = blockIdx.y >> 1;
   const int side = blockIdx.y & 1;
   const int half = lane >> 5;
-  const int64_t tok = (int64_t)blockIdx.x * (kFusedWaves * kTokPerWave) + wave * kTokPerWave + (lane & 31);
-  const bool live = tok < n_tokens;
-  const uint8_t* rop = side == 0 ? rot_k : rot_v;
+  const int64_t tok0 = (int64_t)blockIdx.x * kFwTokens;
+  const u32x4* frag = reinterpret_cast<const u32x4*>(side == 0 ? rot_k : rot_v) + wave * 64 + lane;
+  auto load_r = [&](int m, int p) { return __builtin_bit_cast(bf16x8, frag[(m * 16 + p * 8) * 64]); };
 
-  // B operand of K step m: this lane's token, input features 128*half + 8m .. +7.
-  // Loaded in two halves, each one 128-byte line of the lane's half-row:
-  // steps 0..7 up front, steps 8..15 during step 4, so the first step waits
-  // for half the loads and each line is still fetched in one burst.
-  const uint16_t* xsrc = (side == 0 ? key : value) + (live ? tok : 0) * token_stride +
-                         (int64_t)head * kHeadDim + half * kPerLane;
-  // A lane past the last token reads token 0: its MFMA column (and the
-  // vector the selection then computes) is never stored.
-  auto load_x = [&](int m) -> bf16x8 {
-    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(xsrc + 8 * m));
-  };
-  bf16x8 xlo[8], xhi[8];
+  // ---- rows to LDS: piece u & 31 (eight features) of token u >> 5; tokens
+  // past the last read it again and store nothing ----
+  u32x4 piece[2];
 #pragma unroll
-  for (int m = 0; m < 8; ++m) xlo[m] = load_x(m);
-  // Thread's share of a chunk: wave w copies 1 KB blocks 4w .. 4w + 3.  The
-  // copies are buffer loads: unlike the flat-encoded global form, they count
-  // only in vmcnt, so the operand reads from LDS below keep a partial
-  // lgkmcnt wait each instead of draining every outstanding LDS read.
-  typedef __attribute__((address_space(3))) void lds_void;
-  const __amdgpu_buffer_rsrc_t rop_rsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void*)rop, (short)0, (int)(kSteps * kChunkBytes), 0x00020000);
-  auto request = [&](int chunk) {
+  for (int i = 0; i < 2; ++i) {
+    const int u = (int)threadIdx.x + kFwThreads * i;
+    const int64_t tok = min(tok0 + (u >> 5), n_tokens - 1);
+    piece[i] = reinterpret_cast<const u32x4*>((side == 0 ? key : value) + tok * token_stride +
+                                              (int64_t)head * kHeadDim)[u & 31];
+  }
+  // this lane's token from the exchange on
+  const int r = kFwTokPerWave * wave + (lane >> 4), j = lane & 15;
+  const int64_t tok = tok0 + r;
+  const int64_t slot = tok < n_tokens ? slots[tok] : -1;
+  bf16x8 f[kFwAhead][2];
 #pragma unroll
-    for (int i = 0; i < kDmaPerChunk; ++i) {
-      const int blk = kDmaPerChunk * wave + i;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rop_rsrc, (lds_void*)(uintptr_t)(uint32_t)(uintptr_t)(ring + (chunk % kRing) * kChunkBytes + blk * 1024),
-          16, chunk * kChunkBytes + (blk * 64 + lane) * 16, 0, 0, 0);
-    }
-  };
-  request(0);
-  request(1);
-  request(2);
-
-  floatx16 acc[8];
+  for (int m = 0; m < kFwAhead; ++m) {
+    f[m][0] = load_r(m, 0);
+    f[m][1] = load_r(m, 1);
+  }
 #pragma unroll
-  for (int t = 0; t < 8; ++t) acc[t] = floatx16{};
-
+  for (int i = 0; i < 2; ++i) {
+    const int u = (int)threadIdx.x + kFwThreads * i, m = u & 15;
+    *reinterpret_cast<u32x4*>(&xs[m][((u >> 5) ^ m) + 32 * ((u >> 4) & 1)][0]) = piece[i];
+  }
+  __syncthreads();
+  floatx16 acc = floatx16{};
 #pragma unroll
   for (int m = 0; m < kSteps; ++m) {
-    // This thread's copies of chunk m (and x_m) have landed (later ones may
-    // still be in flight); after the barrier every thread's have, and chunk
-    // m - 1's slot is free for chunk m + 3.  Issue order: x_0..7, chunks
-    // 0..2, then per step chunk m + 3, and x_8..15 after chunk 7 (step 4);
-    // what was issued after chunk m is left outstanding.
-    if (m >= 5 && m <= 7) wait_vmcnt<2 * kDmaPerChunk + 8>();
-    else if (m + 2 < kSteps) wait_vmcnt<2 * kDmaPerChunk>();
-    else if (m + 1 < kSteps) wait_vmcnt<kDmaPerChunk>();
-    else wait_vmcnt<0>();
-    lds_barrier();
-    if (m + 3 < kSteps) request(m + 3);
-    // The waits of steps 5-7 count x_8..15 after chunk 7's copies: keep the
-    // scheduler from hoisting any of those loads above the request (one
-    // hoisted load would leave chunk 7's last copy unwaited at step 7).
-    __builtin_amdgcn_sched_barrier(0);
-    if (m == 4) {
-#pragma unroll
-      for (int k = 0; k < 8; ++k) xhi[k] = load_x(8 + k);
+    const bf16x8 rh = f[m % kFwAhead][0], rl = f[m % kFwAhead][1];
+    if (m + kFwAhead < kSteps) {
+      f[m % kFwAhead][0] = load_r(m + kFwAhead, 0);
+      f[m % kFwAhead][1] = load_r(m + kFwAhead, 1);
     }
-    const bf16x8 xm = m < 8 ? xlo[m] : xhi[m - 8];
-    const u32x4* a_src = reinterpret_cast<const u32x4*>(ring + (m % kRing) * kChunkBytes);
-    // Operand reads run kAhead MFMAs ahead of their use (register rotation);
-    // the 8 tiles' hi passes come first, then their lo passes.
-    constexpr int kAhead = 6;
-    bf16x8 a[kAhead];
-#pragma unroll
-    for (int i = 0; i < kAhead; ++i) a[i] = __builtin_bit_cast(bf16x8, a_src[i * 64 + lane]);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const bf16x8 cur = a[i % kAhead];
-      if (i + kAhead < 16) a[i % kAhead] = __builtin_bit_cast(bf16x8, a_src[(i + kAhead) * 64 + lane]);
-      acc[i & 7] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur, xm, acc[i & 7], 0, 0, 0);
-    }
-    // Keep that pipeline in the schedule: kAhead LDS reads, then each MFMA
-    // followed by the read kAhead positions ahead.
-    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (i + kAhead < 16) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
+    const bf16x8 x = *reinterpret_cast<const bf16x8*>(&xs[m][((lane & 31) ^ m) + (lane & 32)][0]);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rh, x, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rl, x, acc, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);      // (keeps the scheduler from hoisting every step's reads)
   }
-  __syncthreads();      // the ring becomes the waves' selection buffers
 
-  float v[kPerLane];
+  // ---- exchange: 16-byte quarter q of token r's chunk jj (features 16 jj ..)
+  // lies where 16 tokens of one chunk, and the 16 chunks of one token, fall on
+  // different banks ----
+  auto place = [](int rr, int jj, int q) {
+    return rr * 64 + ((jj ^ (rr & 15)) * 4) + (q ^ ((rr >> 2) & 3) ^ ((jj >> 2) & 3));
+  };
 #pragma unroll
-  for (int t = 0; t < 8; ++t) {
+  for (int q = 0; q < 4; ++q)
+    ys[place(lane & 31, 8 * half + wave, q)] = floatx4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+  __syncthreads();
+  float v[kFwPerLane];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v[16 * t + i] = acc[t][i];
+  for (int q = 0; q < 4; ++q) {
+    const floatx4 y = ys[place(r, j, q)];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[4 * q + e] = y[e];
   }
-  SelLds& sel = reinterpret_cast<SelLds*>(ring)[wave];
-  const QParams p = vector_params(v, side == 0 ? clip_k : clip_v, sel, lane);
-  const int64_t slot = live ? slots[tok] : -1;
-  quantize_store(v, p, slot, head, side, half, c);
-  if (w.rows > 0) window_epilogue(v, tok, slot, head, side, lane, c.block_size, w, sel);
+
+  // ---- quantize and store ----
+  float mx = v[0], mn = v[0];
+#pragma unroll
+  for (int i = 1; i < kFwPerLane; ++i) {
+    mx = fmaxf(mx, v[i]);
+    mn = fminf(mn, v[i]);
+  }
+  mx = __uint_as_float(row_reduce(__float_as_uint(mx), [](uint32_t a, uint32_t b) {
+    return __float_as_uint(fmaxf(__uint_as_float(a), __uint_as_float(b)));
+  }));
+  mn = __uint_as_float(row_reduce(__float_as_uint(mn), [](uint32_t a, uint32_t b) {
+    return __float_as_uint(fminf(__uint_as_float(a), __uint_as_float(b)));
+  }));
+  const int clip = side == 0 ? clip_k : clip_v;
+  float thr = __builtin_inff();
+  if (clip >= 0) {
+    const uint32_t amax_bits = max(__float_as_uint(mx) & 0x7FFFFFFFu, __float_as_uint(mn) & 0x7FFFFFFFu);
+    thr = __uint_as_float(row_select(v, clip, amax_bits, sel[wave], lane));
+  }
+  const QParams p = make_qparams(mn, mx, thr, clip >= 0);
+  uint32_t word = 0;
+#pragma unroll
+  for (int i = kFwPerLane - 1; i >= 0; --i) word = (word << 2) | int2_code(v[i], p);
+  if (slot >= 0 && slot < c.num_slots) {
+    const int64_t page = fast_div((uint32_t)slot, c.bs_div);
+    const int64_t row = slot - page * c.block_size;
+    uint8_t* kslot = c.k_cache + page * c.k_page + row * c.k_tok + (int64_t)head * c.k_head;
+    uint8_t* codes = side == 0 ? kslot + kKCodeOff
+                               : c.v_cache + page * c.v_page + row * c.v_tok + (int64_t)head * c.v_head;
+    reinterpret_cast<uint32_t*>(codes)[j] = word;
+    if (j == 0) *reinterpret_cast<uint32_t*>(kslot + 4 * side) = p.meta;
+  }
+  if (w.rows <= 0) return;
+
+  // ---- window (the reference's _staging_write, backend.py:439-481): the
+  // token that won its seat sets the seat's owner (the K side of head 0 does)
+  // to its page when it lies in the sink or recent window and to -1
+  // otherwise; a kept token's unclipped rotated values go to the arena and, as
+  // fp16 parts, to the operand images ----
+  int64_t seat = 0, page = 0;
+  bool keep = false;
+  if (slot >= 0 &&
+      won_seat(w.winner, (int64_t)w.rows * c.block_size, slot, tok, c.block_size, w.rows, seat, page)) {
+    int lo = 0, hi = w.num_requests - 1;     // request of the token: last i with query_start[i] <= tok
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (w.query_start[mid] <= tok) lo = mid; else hi = mid - 1;
+    }
+    const int64_t seq = w.seq_lens[lo];
+    const int64_t pos = seq - w.query_start[lo + 1] + tok;
+    keep = pos >= seq - w.recent || pos < w.sink_eff;
+    if (side == 0 && head == 0 && j == 0) w.owner[seat] = keep ? page : -1;
+  }
+  const bool v_images = side == 1 && w.kimg != nullptr;
+  int64_t tile = 0;
+  int tt = -1;
+  if (keep) {
+    floatx4* dst = reinterpret_cast<floatx4*>((side == 0 ? w.stage_k : w.stage_v) +
+                                              (seat * w.num_kv_heads + head) * kHeadDim + kFwPerLane * j);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) dst[q] = floatx4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+    if (w.kimg != nullptr) {
+      const int prow = (int)(slot - page * c.block_size);
+      tile = image_of(seat / c.block_size, prow, c.block_size, head, w.num_kv_heads);
+      tt = prow & 31;
+      if (side == 0) {
+        // block m = 2 (j & 7) + b, lane tt + 32 (j >> 3), slot u: local feature 4b + (u >> 1) + 8 (u & 1)
+        _Float16* img = w.kimg + tile * kKImgHalfs + (2 * (j & 7) * 64 + tt + 32 * (j >> 3)) * 8;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          half8 h, l;
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            _Float16 x, y;
+            fp16_parts(v[4 * b + (u >> 1) + 8 * (u & 1)], x, y);
+            h[u] = x;
+            l[u] = y;
+          }
+          *reinterpret_cast<half8*>(img + b * 64 * 8) = h;
+          *reinterpret_cast<half8*>(img + kImgHalfs + b * 64 * 8) = l;
+        }
+      }
+    }
+  }
+  if (!v_images) return;
+  if (j == 0) {
+    seat_tile[r] = tile;
+    seat_slot[r] = tt;
+  }
+  __syncthreads();
+  const float* yf = reinterpret_cast<const float*>(ys);
+  store_v_images([&](int rr, int ff) { return yf[4 * place(rr, ff >> 4, (ff >> 2) & 3) + (ff & 3)]; },
+                 seat_tile[lane & 31], seat_slot[lane & 31], inv[wave], w.vimg, wave, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -979,7 +1092,6 @@ int check_cache_args(CacheArgs& c) {
   return kOk;
 }
 
-std::atomic<uint64_t> g_lds_set{0};   // dynamic-LDS attribute set, one bit per device
 std::atomic<uint64_t> g_rot_lds_set[4] = {{0}, {0}, {0}, {0}};   // the same for the rotate_rows instances
 
 }  // namespace
@@ -1119,9 +1231,10 @@ int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_t
   if (st != kOk) return st;
   // Short writes (at most kShortWriteVectors key + value vectors): the fp32
   // rotation of the short-step write (1024-thread workgroups of one to four
-  // vectors, R read from the operand's fp32 copy), instead of a 128-token
-  // MFMA tile that streams the whole operand through one CU's LDS for a few
-  // tokens (4 tokens: 19.4 -> 6.2 us).
+  // vectors, R read from the operand's fp32 copy).  (They took it when the
+  // tile kernel was slower for few tokens, 19.4 against 6.2 us for four; it
+  // stays because its rotation is the fp32 one, which the tiles' two bf16
+  // parts only approach.)
   if (2 * num_tokens * num_kv_heads <= kShortWriteVectors) {
     const uint8_t* ok = static_cast<const uint8_t*>(rot_k_operand) + kMfmaOperandBytes;
     const uint8_t* ov = static_cast<const uint8_t*>(rot_v_operand) + kMfmaOperandBytes;
@@ -1135,9 +1248,7 @@ int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_t
                       clip_index_k, clip_index_v, w.stage_k, w.stage_v, w.owner, w.kimg, w.vimg, w.rows,
                       w.sink_eff, w.recent, nullptr, nullptr, nullptr, stream);
   }
-  if (set_dynamic_lds(reinterpret_cast<const void*>(quant_write_fused_kernel), (int)kFusedLds, g_lds_set) != kOk) return kErrLaunch;
-  const int64_t per_block = kFusedWaves * kTokPerWave;
-  dim3 grid((unsigned)((num_tokens + per_block - 1) / per_block), (unsigned)(num_kv_heads * 2));
+  dim3 grid((unsigned)((num_tokens + kFwTokens - 1) / kFwTokens), (unsigned)(num_kv_heads * 2));
   if (w.rows > 0) {
     HostLayout h{};
     if (host != nullptr) {
@@ -1159,7 +1270,7 @@ int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_t
                        slot_mapping, (int32_t)num_tokens, w.winner, block_size, w.rows, h);
     if (hipGetLastError() != hipSuccess) return kErrLaunch;
   }
-  hipLaunchKernelGGL(quant_write_fused_kernel, grid, dim3(kFusedWaves * 64), kFusedLds, stream,
+  hipLaunchKernelGGL(quant_write_fused_kernel, grid, dim3(kFwThreads), 0, stream,
                      static_cast<const uint16_t*>(key_bf16), static_cast<const uint16_t*>(value_bf16),
                      num_tokens, token_stride, static_cast<const uint8_t*>(rot_k_operand),
                      static_cast<const uint8_t*>(rot_v_operand), slot_mapping, c,
