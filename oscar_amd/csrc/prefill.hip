@@ -42,9 +42,10 @@
 // barriers per block with the wavefronts 4-7 a phase behind (1.19x slower),
 // operand rows that two of sixteen lanes read from one bank slot (LDS active
 // 45 % against 29 % of the time), and workgroups of four wavefronts, two per
-// CU (1.25x slower) were left behind.  One request, 6 heads, D = 256: 9256
-// tokens over 15360 1988 -> 1220 us, 77 over 20011 1016 -> 46 us (+ merge 12),
-// 3001 alone 170 -> 62 us (+ merge 18).
+// CU (1.25x slower) were left behind.  Before and after its blocks a piece
+// takes about 5 and 2.5 us: unit, pages and Q^T, first words, first tile; and
+// the partial.  One request, 6 heads, D = 256, this kernel: 9256 tokens over
+// 15360 1988 -> 1200 us, 77 over 20011 1016 -> 34 us, 3001 alone 170 -> 50 us.
 #include <type_traits>
 #include <utility>
 
@@ -67,10 +68,11 @@ constexpr int kPartRows = kTileRows;
 constexpr size_t kPartFloats = (size_t)kPartRows * (kHeadDim + 2);   // O rows, then m, then l
 constexpr int kShares = 256;          // workgroups resident at once: one per CU
 // A piece of a row block costs as much as this many of its key blocks before
-// and after them (page lookup, Q^T, first tile; output or partial): 10-12 us
-// against 2.1 us a block.
-constexpr int kPieceCost = 7;
-constexpr int kMinShare = 10;         // units a share takes at least (see plan_share)
+// and after them (page lookup, Q^T, first tile; output or partial, which the
+// output pass reads again): 7.5 us and that pass against 2.1 us a block.  (4
+// to 7 are within 2 us of each other on the cases timed.)
+constexpr int kPieceCost = 5;
+constexpr int kMinShare = 5;          // units a share takes at least (see plan_share)
 constexpr int kMergeManyPieces = 6;   // partials a row from which its merge takes four waves
 
 struct PrefillItem {
@@ -128,6 +130,12 @@ static_assert(kPrefillLds <= 160 * 1024, "LDS of one workgroup");
 
 __device__ __forceinline__ _Float16 to_h(float x) { return (_Float16)x; }
 
+__device__ __forceinline__ void wave_sync_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // s_barrier without __syncthreads' memory fence (which would also wait for
 // the outstanding global loads); LDS writes are complete at lgkmcnt(0).
 __device__ __forceinline__ void lds_barrier() {
@@ -155,34 +163,55 @@ __device__ __forceinline__ int rb_units(const PrefillItem& it, int group, int rb
   return kPieceCost + key_blocks(it, group, rb);
 }
 
+// Sum over the lanes up to and including this one (wave-wide, DPP).
+__device__ __forceinline__ uint32_t wave_scan(uint32_t x) {
+  auto up = [](uint32_t v, auto ctrl, auto rows) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+  };
+  using std::integral_constant;
+  x += up(x, integral_constant<int, 0x111>{}, integral_constant<int, 0xF>{});     // row_shr:1, 2, 4, 8
+  x += up(x, integral_constant<int, 0x112>{}, integral_constant<int, 0xF>{});
+  x += up(x, integral_constant<int, 0x114>{}, integral_constant<int, 0xF>{});
+  x += up(x, integral_constant<int, 0x118>{}, integral_constant<int, 0xF>{});
+  x += up(x, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});     // row_bcast:15 into rows 1 and 3
+  x += up(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});     // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
+// The sum of 64 row blocks' units as a wave scan, in two 32-bit halves: a row
+// block has less than 2^28 units, so 16 low bits of each sum below 2^22 and
+// the rest below 2^18.
+__device__ __forceinline__ int64_t units_scan(int n) {
+  return ((int64_t)wave_scan((uint32_t)n >> 16) << 16) + wave_scan((uint32_t)n & 0xFFFFu);
+}
+__device__ __forceinline__ int64_t lane64(int64_t x, int lane) {
+  return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), lane) << 32) |
+                   (uint32_t)__builtin_amdgcn_readlane((int)x, lane));
+}
+
 // Units of the item's row blocks before rb (every lane of the wave calls it
 // with the same rb).
-__device__ int64_t units_before(const PrefillItem& it, int group, int rb, int lane) {
+__device__ __forceinline__ int64_t units_before(const PrefillItem& it, int group, int rb, int lane) {
   int64_t n = 0;
-  for (int b = lane; b < rb; b += 64) n += rb_units(it, group, b);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) n += __shfl_xor(n, o, 64);
+  for (int base = 0; base < rb; base += 64)
+    n += lane64(units_scan(base + lane < rb ? rb_units(it, group, base + lane) : 0), 63);
   return n;
 }
 
 // Row block of unit u (relative to the kv head's first), and u within it: a
 // wave-wide scan over 64 row blocks a time.
-__device__ void locate_unit(const PrefillItem& it, int group, int64_t u, int lane, int& rb, int& at_unit) {
+__device__ __forceinline__ void locate_unit(const PrefillItem& it, int group, int64_t u, int lane, int& rb,
+                                            int& at_unit) {
   const int nrb = row_blocks(it, group);
   for (int base = 0;; base += 64) {
     const int b = base + lane;
     const int n = b < nrb ? rb_units(it, group, b) : 0;
-    int64_t incl = n;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int64_t up = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += up;
-    }
-    const int64_t total = __shfl(incl, 63, 64);
+    const int64_t incl = units_scan(n);
+    const int64_t total = lane64(incl, 63);
     if (u < total || base + 64 >= nrb) {
       const int at = min(__popcll(__ballot(incl <= u)), 63);
-      rb = __builtin_amdgcn_readfirstlane(base + at);
-      at_unit = __builtin_amdgcn_readfirstlane((int)(u - (__shfl(incl, at, 64) - __shfl(n, at, 64))));
+      rb = base + at;
+      at_unit = (int)(u - (lane64(incl, at) - __builtin_amdgcn_readlane(n, at)));
       return;
     }
     u -= total;
@@ -255,16 +284,14 @@ __device__ __forceinline__ Roles make_roles(uint32_t k_tok, uint32_t v_tok, int 
   return r;
 }
 
-// Page of the history block at key k0 (uniform).  Read through the scalar
-// cache, so that waiting for it never waits for the vector loads in flight.
-__device__ __forceinline__ int32_t block_page(const Hot& h, int k0) {
-  if (k0 >= h.cached) return -1;
-  const uint32_t pidx = fast_div((uint32_t)k0, h.bs_div);
-  if ((int64_t)pidx >= h.bt_cols) return -1;
-  typedef __attribute__((address_space(4))) const int32_t const_i32;
-  return ((const const_i32*)h.bt_row)[__builtin_amdgcn_readfirstlane(pidx)];
+// Pages of the 64 history blocks from block b on, one a lane (negative: none);
+// checked against the pool where they are taken out.
+__device__ __forceinline__ int32_t load_pages(const Hot& h, int b, int lane) {
+  const uint32_t k0 = (uint32_t)(b + lane) * kBlk, pidx = fast_div(k0, h.bs_div);
+  const bool ok = k0 < (uint32_t)h.cached && pidx < (uint32_t)h.bt_cols;
+  const int32_t p = h.bt_row[ok ? pidx : 0];
+  return ok ? p : -1;
 }
-// ... checked where it is used, not where it is requested (which would wait).
 __device__ __forceinline__ int32_t valid_page(const Hot& h, int32_t page) { return page < h.num_pages ? page : -1; }
 
 __device__ __forceinline__ KLoad load_k(const Hot& h, int k0, int32_t page, const Roles& r, int lane) {
@@ -316,8 +343,7 @@ __device__ __forceinline__ void* v_slot(_Float16* vt, uint32_t vs, int f) {
 }
 
 // A thread's 16 K values (features 16 k16 .. +15, fp32) into its token's row.
-__device__ __forceinline__ void store_k_values(const floatx4* __restrict__ src, uint32_t ks, _Float16* kt) {
-  const floatx4 x[4] = {src[0], src[1], src[2], src[3]};
+__device__ __forceinline__ void store_k_values(const floatx4 (&x)[4], uint32_t ks, _Float16* kt) {
 #pragma unroll
   for (int g = 0; g < 2; ++g) {
     half8 h;
@@ -379,34 +405,41 @@ __device__ __forceinline__ void build_v(uint32_t w, uint32_t vs, _Float16* vt, i
 }
 
 // Window-owned tokens (rare), over what the builds above stored: their FP32
-// values rounded to fp16.  (opaque: nothing of this is worth a register in
-// the loop.)
-__device__ __forceinline__ void window_k(uint32_t wmask, int32_t page, int k0, int kvh, const Roles& r, int w,
-                                         int lane_, _Float16* kt) {
+// values rounded to fp16, those of a K tile (kmask, page kpage, keys from k0)
+// and of a V tile (vmask, its code words in x, page vpage, keys from v0).  The
+// loads of both go out before either is waited for: a wait of its own for
+// each cost a block 1 us.  (opaque: nothing of this is worth a register in the
+// loop.)
+__device__ __forceinline__ void window_tiles(uint32_t kmask, int32_t kpage, int k0, _Float16* kt, uint32_t vmask,
+                                             uint32_t x, int32_t vpage, int v0, _Float16* vt, int kvh, const Roles& r,
+                                             int w, int lane_) {
   const int lane = (int)opaque((uint32_t)lane_), t = 4 * w + (lane >> 4);
-  if ((wmask >> t) & 1u)
-    store_k_values(reinterpret_cast<const floatx4*>(stage_row(false, page, k0, t, kvh) + 16 * (lane & 15)),
-                   opaque(r.ks), kt);
-}
-__device__ __forceinline__ void window_v(uint32_t wmask, uint32_t x, int32_t page, int k0, int kvh, const Roles& r,
-                                         int w, int lane_, _Float16* vt) {
-  const uint32_t nib = (wmask >> (4 * w)) & 15u;
-  if (nib == 0u) return;
-  const int lane = (int)opaque((uint32_t)lane_);
-  const uint32_t codes = quad_transpose(x, lane);
-  floatx4 y[4];
+  const bool mine = ((kmask >> t) & 1u) != 0u;
+  const uint32_t nib = (vmask >> (4 * w)) & 15u;
+  floatx4 xk[4] = {}, y[4];
+  if (mine) {
+    const floatx4* src = reinterpret_cast<const floatx4*>(stage_row(false, kpage, k0, t, kvh) + 16 * (lane & 15));
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if ((nib >> k) & 1u)
-      y[k] = *reinterpret_cast<const floatx4*>(stage_row(true, page, k0, 4 * w + k, kvh) + 4 * lane);
-    else
-#pragma unroll
-      for (int e = 0; e < 4; ++e) y[k][e] = 1.f + 0.25f * (float)((codes >> (8 * k + 2 * e)) & 3u);
+    for (int e = 0; e < 4; ++e) xk[e] = src[e];
   }
-  const uint32_t vs = opaque(r.vs) ^ (64u * ((lane >> 2) & 3));      // (v_slot's f is then the feature)
+  if (nib != 0u) {
+    const uint32_t codes = quad_transpose(x, lane);
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
-    *reinterpret_cast<half4*>(v_slot(vt, vs, e)) = half4{to_h(y[0][e]), to_h(y[1][e]), to_h(y[2][e]), to_h(y[3][e])};
+    for (int k = 0; k < 4; ++k) {
+      if ((nib >> k) & 1u)
+        y[k] = *reinterpret_cast<const floatx4*>(stage_row(true, vpage, v0, 4 * w + k, kvh) + 4 * lane);
+      else
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[k][e] = 1.f + 0.25f * (float)((codes >> (8 * k + 2 * e)) & 3u);
+    }
+  }
+  if (mine) store_k_values(xk, opaque(r.ks), kt);
+  if (nib != 0u) {
+    const uint32_t vs = opaque(r.vs) ^ (64u * ((lane >> 2) & 3));      // (v_slot's f is then the feature)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      *reinterpret_cast<half4*>(v_slot(vt, vs, e)) = half4{to_h(y[0][e]), to_h(y[1][e]), to_h(y[2][e]), to_h(y[3][e])};
+  }
 }
 
 // A value held by lane r of each 16-lane row, in every lane of the row.
@@ -468,9 +501,10 @@ __device__ __forceinline__ void copy_tile(const _Float16* img, int64_t tile, _Fl
 __device__ __forceinline__ void store_new_k(const PrefillArgs& a, const PrefillItem& it, int j0, int kvh,
                                             const Roles& r, int w, int lane, _Float16* kt) {
   const int j = min(j0 + 4 * w + (lane >> 4), it.n_new - 1);
-  store_k_values(reinterpret_cast<const floatx4*>(a.k_new + ((int64_t)(it.tok0 + j) * a.num_kv_heads + kvh) * kHeadDim +
-                                                  16 * (lane & 15)),
-                 r.ks, kt);
+  const floatx4* src = reinterpret_cast<const floatx4*>(
+      a.k_new + ((int64_t)(it.tok0 + j) * a.num_kv_heads + kvh) * kHeadDim + 16 * (lane & 15));
+  const floatx4 x[4] = {src[0], src[1], src[2], src[3]};
+  store_k_values(x, r.ks, kt);
 }
 __device__ __forceinline__ void store_new_v(const PrefillArgs& a, const PrefillItem& it, int j0, int kvh,
                                             const Roles& r, int w, int lane, _Float16* vt) {
@@ -515,7 +549,7 @@ __global__ __launch_bounds__(512, 2) void prefill_kernel(PrefillArgs a) {
     u1 = min(u + a.share, a.units);
     while (item + 1 < a.nitems && a.items[item + 1].unit0 <= u) ++item;
     const int64_t rel = u - a.items[item].unit0;
-    kvh = (int)(rel / a.items[item].head_units);
+    kvh = rel < a.items[item].head_units ? 0 : (int)(rel / a.items[item].head_units);
     locate_unit(a.items[item], a.group, rel - (int64_t)kvh * a.items[item].head_units, lane, rb, ub);
   }
 
@@ -557,8 +591,8 @@ __global__ __launch_bounds__(512, 2) void prefill_kernel(PrefillArgs a) {
                 it.cached, a.block_size, a.bs_div, a.rows_div, a.scale_log2};
 
     // ---- first blocks' loads, then the wave's Q^T operands.  In phase M of
-    // block i: lk holds block i + 1's words, lv block i's; pages p0 .. p2 are
-    // those of blocks i .. i + 2; meta (and cur) are block i's in phase S. ----
+    // block i: lk holds block i + 1's words, lv block i's; pages p0 and p1
+    // are those of blocks i and i + 1; meta (and cur) are block i's in phase S. ----
     struct Block {
       uint32_t win;       // window-owned tokens
       int live;           // tokens in the history, from the first
@@ -567,24 +601,35 @@ __global__ __launch_bounds__(512, 2) void prefill_kernel(PrefillArgs a) {
     u32x2 meta{};
     uint32_t lv = 0;
     Block cur{0u, 0}, next{0u, 0};
-    int32_t p0 = -1, p1 = -1, p2 = -1;
-    if (kb < nh) {
-      p1 = valid_page(h, block_page(h, kb * kBlk));
-      lk = load_k(h, kb * kBlk, p1, r, lane);
-      lv = load_v(h, kb * kBlk, p1, r);
-      meta = load_meta(h, kb * kBlk, p1, r);
-      p2 = block_page(h, (kb + 1) * kBlk);
-    }
-    half8 qreg[kQReg];
-    float qsum;
+    int32_t p0 = -1, p1 = -1;
+    // (pages come from registers: a table read in the loop would be waited
+    // for with the LDS reads at the next barrier)
+    int pbase = kb;
+    int32_t pgv = -1;
+    auto page_at = [&](int i) { return valid_page(h, __builtin_amdgcn_readlane(pgv, i - pbase)); };
+    if (kb < nh) pgv = load_pages(h, kb, lane);
+    half8 qreg[kQReg], qlds[16 - kQReg];
+    float qsum = 0.f;
     if constexpr (kImages) {
       const int64_t qrow = (int64_t)(it.tok0 + my_tok) * a.num_heads + head;
       const half8* qp = reinterpret_cast<const half8*>(a.q16 + qrow * kHeadDim) + g;
 #pragma unroll
       for (int m = 0; m < kQReg; ++m) qreg[m] = qp[2 * m];
 #pragma unroll
-      for (int m = kQReg; m < 16; ++m) *reinterpret_cast<half8*>(&S.q[wave][m - kQReg][lane * 8]) = qp[2 * m];
+      for (int m = kQReg; m < 16; ++m) qlds[m - kQReg] = qp[2 * m];
       qsum = a.qsum[qrow];
+    }
+    __builtin_amdgcn_sched_barrier(0);      // (pages and queries in one round)
+    if (kb < nh) {
+      p1 = page_at(kb);
+      lk = load_k(h, kb * kBlk, p1, r, lane);
+      lv = load_v(h, kb * kBlk, p1, r);
+      meta = load_meta(h, kb * kBlk, p1, r);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kImages) {
+#pragma unroll
+      for (int m = kQReg; m < 16; ++m) *reinterpret_cast<half8*>(&S.q[wave][m - kQReg][lane * 8]) = qlds[m - kQReg];
     } else {
       const float* qp = a.q + ((int64_t)(it.tok0 + my_tok) * a.num_heads + head) * kHeadDim + 4 * g;
       float qs = 0.f;
@@ -629,13 +674,15 @@ __global__ __launch_bounds__(512, 2) void prefill_kernel(PrefillArgs a) {
       const uint32_t ks = opaque(r.ks);
       build_k(lk.kc, ks, tile_k(i), 0);
       build_k(lk.kc, ks, tile_k(i), 1);
-      if (next.win != 0u) window_k(next.win, p1, i * kBlk, kvh_now, r, wave, lane, tile_k(i));
+      if (next.win != 0u)
+        window_tiles(next.win, p1, i * kBlk, tile_k(i), 0u, 0u, -1, 0, tile_v(i), kvh_now, r, wave, lane);
     };
     auto hist_v = [&](int i) {
       const uint32_t vs = opaque(r.vs), w = quad_transpose(lv, lane);
 #pragma unroll
       for (int f = 0; f < 4; ++f) build_v(w, vs, tile_v(i), f);
-      if (cur.win != 0u) window_v(cur.win, lv, p0, i * kBlk, kvh_now, r, wave, lane, tile_v(i));
+      if (cur.win != 0u)
+        window_tiles(0u, -1, 0, tile_k(i), cur.win, lv, p0, i * kBlk, tile_v(i), kvh_now, r, wave, lane);
     };
     auto new_k = [&](int i, auto copy_waves) {
       constexpr int kCw = decltype(copy_waves)::value;
@@ -655,12 +702,13 @@ __global__ __launch_bounds__(512, 2) void prefill_kernel(PrefillArgs a) {
     // The words of block i + 1's V and block i + 2's K, while those exist.
     auto load_next = [&](int i) {
       p0 = p1;
-      p1 = valid_page(h, p2);
-      if (i + 1 < min(kend, nh)) lv = load_v(h, (i + 1) * kBlk, p0, r);
-      if (i + 2 < min(kend, nh)) {
-        lk = load_k(h, (i + 2) * kBlk, p1, r, lane);
-        p2 = block_page(h, (i + 3) * kBlk);
+      if (i + 2 - pbase >= 64) {
+        pbase = i + 2;
+        pgv = load_pages(h, pbase, lane);
       }
+      p1 = page_at(i + 2);
+      if (i + 1 < min(kend, nh)) lv = load_v(h, (i + 1) * kBlk, p0, r);
+      if (i + 2 < min(kend, nh)) lk = load_k(h, (i + 2) * kBlk, p1, r, lane);
     };
     // Blocks before kseen are seen by a row of the wave.
     const int kseen = !wave_on ? kb : min(kend, nh + last_tok / kBlk + 1);
@@ -806,11 +854,8 @@ __global__ __launch_bounds__(512, 2) void prefill_kernel(PrefillArgs a) {
       hist_k(kb);
       cur = next;
       p0 = p1;
-      p1 = valid_page(h, p2);
-      if (kb + 1 < min(kend, nh)) {
-        lk = load_k(h, (kb + 1) * kBlk, p1, r, lane);
-        p2 = block_page(h, (kb + 2) * kBlk);
-      }
+      p1 = page_at(kb + 1);
+      if (kb + 1 < min(kend, nh)) lk = load_k(h, (kb + 1) * kBlk, p1, r, lane);
       lds_barrier();
     } else {
       new_k(kb, std::integral_constant<int, kWaves>{});
@@ -830,8 +875,8 @@ __global__ __launch_bounds__(512, 2) void prefill_kernel(PrefillArgs a) {
       });
       next = block_of(i + 1);
       if ((next.win | cur.win) != 0u) {
-        if (next.win != 0u) window_k(next.win, p1, (i + 1) * kBlk, kvh_now, r, wave, lane, tile_k(i + 1));
-        if (cur.win != 0u) window_v(cur.win, lv, p0, i * kBlk, kvh_now, r, wave, lane, tile_v(i));
+        window_tiles(next.win, p1, (i + 1) * kBlk, tile_k(i + 1), cur.win, lv, p0, i * kBlk, tile_v(i), kvh_now, r,
+                     wave, lane);
       }
       load_next(i);
       if (second) lds_barrier();
@@ -878,35 +923,56 @@ __global__ __launch_bounds__(512, 2) void prefill_kernel(PrefillArgs a) {
     // ---- the row block's output, or this share's partial of it ----
     const float l_tot = l_run + shfl_xor_f32(l_run, 32);
     const float z_tot = z_run + shfl_xor_f32(z_run, 32);
-    // (this lane's row recomputed, so that nothing of it lives through the loop)
+    // A lane holds quarters of 16-byte pieces of one row; through the wave's
+    // own Q^T area (its last scores are done), 64 features of its 32 rows at a
+    // time, they leave as whole 256-byte runs.  (Straight from the registers,
+    // 32 bytes of 32 rows an instruction, a partial took 3.8 us.)  The lane's
+    // row recomputed, so that nothing of it lives through the loop.
     const int elane = (int)opaque((uint32_t)lane);
-    const int erow = wrow0 + (elane & 31), eg = elane >> 5;
-    if (erow < rows_total) {
-      const int etok = erow / a.group, ehead = kvh_now * a.group + (erow - etok * a.group);
-      const bool whole_rb = kb == 0 && kend == nblk;
-      float* op;
-      float inv = 1.f;
-      if (whole_rb) {
-        inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-        op = a.out + ((int64_t)(it.tok0 + etok) * a.num_heads + ehead) * kHeadDim;
-      } else {
-        const int64_t slot = 2 * (int64_t)blockIdx.x + (start != (int64_t)blockIdx.x * a.share ? 1 : 0);
-        float* part = a.part + slot * (int64_t)kPartFloats;
-        const int pr = wave * kRowsPerWave + (elane & 31);
-        op = part + pr * kHeadDim;
-        if (eg == 0) {
-          part[kPartRows * kHeadDim + pr] = raise == -__builtin_inff() ? raise : m_base;
-          part[kPartRows * (kHeadDim + 1) + pr] = l_tot;
-        }
+    const int er = elane & 31, eg = elane >> 5;
+    const bool whole_rb = kb == 0 && kend == nblk;
+    const float inv = whole_rb ? (l_tot > 0.f ? 1.f / l_tot : 0.f) : 1.f;
+    float* base = a.out;
+    if (!whole_rb) {
+      const int64_t slot = 2 * (int64_t)blockIdx.x + (start != (int64_t)blockIdx.x * a.share ? 1 : 0);
+      base = a.part + slot * (int64_t)kPartFloats;
+      if (eg == 0 && wrow0 + er < rows_total) {
+        const int pr = wave * kRowsPerWave + er;
+        base[kPartRows * kHeadDim + pr] = raise == -__builtin_inff() ? raise : m_base;
+        base[kPartRows * (kHeadDim + 1) + pr] = l_tot;
       }
-      op += 4 * eg;
+    }
+    // rows 4 i + lane / 16 of the wave, piece lane % 16 of a run
+    uint32_t off[8];
 #pragma unroll
-      for (int t = 0; t < 8; ++t)
+    for (int i = 0; i < 8; ++i) {
+      const int r8 = 4 * i + (elane >> 4), erow = wrow0 + r8;
+      const int etok = erow / a.group, ehead = kvh_now * a.group + (erow - etok * a.group);
+      const int64_t o = whole_rb ? (int64_t)(it.tok0 + etok) * a.num_heads + ehead : wave * kRowsPerWave + r8;
+      off[i] = erow < rows_total ? (uint32_t)o : ~0u;
+    }
+    floatx4* T = reinterpret_cast<floatx4*>(S.q[wave]);
+    static_assert(sizeof(S.q[0]) >= 32 * 64 * sizeof(float), "64 features of 32 rows");
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj)
-          *reinterpret_cast<floatx4*>(op + 32 * t + 8 * jj) =
-              floatx4{(acc[t][4 * jj] + z_tot) * inv, (acc[t][4 * jj + 1] + z_tot) * inv,
-                      (acc[t][4 * jj + 2] + z_tot) * inv, (acc[t][4 * jj + 3] + z_tot) * inv};
+    for (int p = 0; p < 4; ++p) {
+      wave_sync_lds();
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const floatx16& c = acc[2 * p + tt];
+          T[16 * er + ((8 * tt + 2 * jj + eg) ^ (er & 15))] =
+              floatx4{(c[4 * jj] + z_tot) * inv, (c[4 * jj + 1] + z_tot) * inv, (c[4 * jj + 2] + z_tot) * inv,
+                      (c[4 * jj + 3] + z_tot) * inv};
+        }
+      wave_sync_lds();
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r8 = 4 * i + (elane >> 4);
+        const floatx4 x = T[16 * r8 + ((elane & 15) ^ (r8 & 15))];
+        if (off[i] != ~0u)
+          *reinterpret_cast<floatx4*>(base + (uint64_t)off[i] * kHeadDim + 64 * p + 4 * (elane & 15)) = x;
+      }
     }
   }
 }
@@ -1246,7 +1312,9 @@ int64_t host_head_units(int64_t n_new, int64_t cached, int64_t group) {
 }
 
 // Units per workgroup: one round of kShares workgroups, of at least kMinShare
-// units each (a partial of 256 rows is 264 KB, written and read again).
+// units each (a partial of 256 rows is 264 KB, written and read again: 77
+// tokens over 20K take 41 us + merge 10.7 in shares of 8, 36 + 12.9 of 6, 34 +
+// 14 of 5, 34 + 14.4 of 4).
 int64_t plan_share(int64_t units) {
   const int64_t s = (units + kShares - 1) / kShares;
   return s < kMinShare ? kMinShare : s;
