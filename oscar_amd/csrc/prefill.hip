@@ -50,6 +50,7 @@
 #include <utility>
 
 #include "prefill_operands.h"
+#include "step_launch.h"
 #include "../../include/oscar_amd.h"
 
 namespace oscar {
@@ -1577,7 +1578,9 @@ extern "C" size_t oscar_prefill_rotated_workspace_bytes(int32_t num_requests, co
   return most;
 }
 
-extern "C" int oscar_prefill_rotated(
+namespace oscar {
+
+int prefill_rotated(
     const void* query_bf16, int64_t query_token_stride, const void* key_bf16, const void* value_bf16,
     int64_t kv_token_stride, int32_t num_requests, const int32_t* first_tokens, const int32_t* new_tokens,
     const int64_t* cached_lens, const int32_t* table_rows, int32_t num_heads, int32_t num_kv_heads,
@@ -1586,7 +1589,7 @@ extern "C" int oscar_prefill_rotated(
     int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token,
     int64_t v_stride_head, const int32_t* block_table, int64_t block_table_stride, int32_t block_table_cols,
     const float* stage_k, const float* stage_v, const int64_t* stage_owner, int32_t stage_rows, float scale,
-    void* out_bf16, void* workspace, size_t workspace_size, hipStream_t stream) {
+    void* out_bf16, void* workspace, size_t workspace_size, const FusedWriteArgs* write, hipStream_t stream) {
   PrefillArgs base{};
   int st = fill_common(base, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages,
                        k_stride_page, k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
@@ -1628,11 +1631,33 @@ extern "C" int oscar_prefill_rotated(
     st = launch_rotate_operands(static_cast<const uint16_t*>(query_bf16), query_token_stride,
                                 static_cast<const uint16_t*>(key_bf16), static_cast<const uint16_t*>(value_bf16),
                                 kv_token_stride, num_heads, num_kv_heads, static_cast<const uint8_t*>(rot_k_operand),
-                                static_cast<const uint8_t*>(rot_v_operand), ops, o, stream);
+                                static_cast<const uint8_t*>(rot_v_operand), ops, o, write, stream);
+    write = nullptr;
     if (st != kOk) return st;
     int64_t wgs = 0;
     if ((st = launch_shares(a, wgs, stream)) != kOk) return st;
     if ((st = launch_output(a, wgs, rot_v_t_operand, out_bf16, stream)) != kOk) return st;
   }
   return kOk;
+}
+
+}  // namespace oscar
+
+extern "C" int oscar_prefill_rotated(
+    const void* query_bf16, int64_t query_token_stride, const void* key_bf16, const void* value_bf16,
+    int64_t kv_token_stride, int32_t num_requests, const int32_t* first_tokens, const int32_t* new_tokens,
+    const int64_t* cached_lens, const int32_t* table_rows, int32_t num_heads, int32_t num_kv_heads,
+    int32_t head_size, const void* rot_k_operand, const void* rot_v_operand, const void* rot_v_t_operand,
+    const void* k_cache, const void* v_cache, int32_t block_size, int64_t num_pages, int64_t k_stride_page,
+    int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token,
+    int64_t v_stride_head, const int32_t* block_table, int64_t block_table_stride, int32_t block_table_cols,
+    const float* stage_k, const float* stage_v, const int64_t* stage_owner, int32_t stage_rows, float scale,
+    void* out_bf16, void* workspace, size_t workspace_size, hipStream_t stream) {
+  return prefill_rotated(query_bf16, query_token_stride, key_bf16, value_bf16, kv_token_stride, num_requests, first_tokens,
+                         new_tokens, cached_lens, table_rows, num_heads, num_kv_heads, head_size,
+                         rot_k_operand, rot_v_operand, rot_v_t_operand, k_cache, v_cache,
+                         block_size, num_pages, k_stride_page, k_stride_token, k_stride_head,
+                         v_stride_page, v_stride_token, v_stride_head, block_table,
+                         block_table_stride, block_table_cols, stage_k, stage_v, stage_owner,
+                         stage_rows, scale, out_bf16, workspace, workspace_size, nullptr, stream);
 }

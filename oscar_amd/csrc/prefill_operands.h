@@ -21,6 +21,7 @@
 //      operand, conflict-free along features.
 #pragma once
 
+#include "bulk_write.h"
 #include "oscar_common.h"
 
 namespace oscar {
@@ -58,10 +59,11 @@ struct PrefillOperands {
   _Float16* vimg;
 };
 
-// quant_write.hip: operands from bf16 query / key / value, rotated on MFMA.
+// quant_write.hip: operands from bf16 query / key / value, rotated on MFMA,
+// and in the same launch the bulk write in `write`, if there is one.
 int launch_rotate_operands(const uint16_t* q, int64_t q_stride, const uint16_t* k, const uint16_t* v,
                            int64_t kv_stride, int32_t num_heads, int32_t num_kv_heads, const uint8_t* rot_k,
                            const uint8_t* rot_v, const OperandItems& items, const PrefillOperands& o,
-                           hipStream_t stream);
+                           const FusedWriteArgs* write, hipStream_t stream);
 
 }  // namespace oscar

@@ -26,6 +26,7 @@
 // after a seat-winner pass over the step's slots.
 #include <type_traits>
 
+#include "bulk_write.h"
 #include "int2_quant.h"
 #include "prefill_operands.h"
 #include "step_launch.h"
@@ -38,15 +39,6 @@ namespace {
 constexpr int kPerLane = kHeadDim / 2;      // 128 values of one vector per lane
 constexpr int kTokPerWave = 32;
 
-struct CacheArgs {
-  uint8_t* k_cache;
-  uint8_t* v_cache;
-  int64_t k_page, k_tok, k_head;     // byte strides
-  int64_t v_page, v_tok, v_head;
-  int32_t block_size;
-  int64_t num_slots;                 // pages * block_size (< 2^31); larger slots are skipped
-  FastDiv bs_div;                    // block_size
-};
 
 // Exact value of ascending-sorted |x| at index `idx` over the 256 values held
 // by this lane and its partner (l ^ 32).  Bitwise radix select on the IEEE
@@ -239,22 +231,6 @@ __device__ void quantize_store(const float (&v)[kPerLane], const QParams& p, int
   d4[1] = u32x4{words[4], words[5], words[6], words[7]};
   if (half == 0) *reinterpret_cast<uint32_t*>(kslot + 4 * side) = p.meta;
 }
-
-// The window arena of a bulk write (rows = 0: none).
-struct WindowArgs {
-  const int32_t* query_start;   // [num_requests + 1] on the device
-  const int32_t* seq_lens;      // [num_requests]
-  int32_t num_requests;
-  int32_t rows;
-  int32_t sink_eff, recent;
-  int32_t num_kv_heads;
-  float* stage_k;               // [rows][bs][Hk][D] fp32
-  float* stage_v;
-  int64_t* owner;               // [rows][bs]
-  int64_t* winner;              // seat winners (read after this call's pass)
-  _Float16* kimg;               // operand images, or null
-  _Float16* vimg;
-};
 
 __device__ __forceinline__ int64_t read_lane64(int64_t x, int lane) {
   return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), lane) << 32) |
@@ -586,25 +562,39 @@ __device__ __forceinline__ void store_v_images(const Value& value, int64_t seat_
 // tokens took 29 us with the window (their selection 10, its image 7), 1052
 // of a mixed step 36, 9256 29 and 65536 without one 71; this takes 11, 15, 20
 // and 67.  64 tokens to a workgroup (half the reading of R): 17, -, 25, 68.
-__global__ __launch_bounds__(kFwThreads, 4) void quant_write_fused_kernel(
-    const uint16_t* __restrict__ key, const uint16_t* __restrict__ value, int64_t n_tokens,
-    int64_t token_stride, const uint8_t* __restrict__ rot_k, const uint8_t* __restrict__ rot_v,
-    const int64_t* __restrict__ slots, CacheArgs c, int clip_k, int clip_v, WindowArgs w) {
-  // [k-step][row ^ k-step, half]; the selection's LDS once the products are done
-  __shared__ __attribute__((aligned(16))) uint16_t xs[kSteps][64][8];
-  static_assert(sizeof(RowSelLds) * (kFwThreads / 64) <= sizeof(xs), "the selection reuses the operands' LDS");
-  RowSelLds* sel = reinterpret_cast<RowSelLds*>(xs);
-  __shared__ floatx4 ys[kFwTokens * kHeadDim / 4];
-  __shared__ int64_t seat_tile[kFwTokens];
-  __shared__ int32_t seat_slot[kFwTokens];
-  __shared__ uint8_t inv[kFwThreads / 64][32];
+// 33 KB, so that four workgroups share a CU: the operands' rows [k-step][row ^
+// k-step, half] until the products are done, then the rotated values, in a
+// wave's share of which its selection works once the wave has read them.
+struct FusedWriteLds {
+  union {
+    uint16_t xs[kSteps][64][8];
+    floatx4 ys[kFwTokens * kHeadDim / 4];
+  };
+  int64_t seat_tile[kFwTokens];
+  int32_t seat_slot[kFwTokens];
+  uint8_t inv[kFwThreads / 64][32];
+  __device__ FusedWriteLds() {}
+};
+static_assert(sizeof(RowSelLds) <= kFwTokPerWave * kHeadDim * sizeof(float), "the selection fits its wave's values");
+
+__device__ __forceinline__ void fused_write(const FusedWriteArgs& a, FusedWriteLds& S, int block) {
+  auto& xs = S.xs;
+  auto& ys = S.ys;
+  auto& seat_tile = S.seat_tile;
+  auto& seat_slot = S.seat_slot;
+  auto& inv = S.inv;
+  const CacheArgs& c = a.c;
+  const WindowArgs& w = a.w;
+  const int64_t n_tokens = a.n_tokens;
+  const int64_t* slots = a.slots;
+  const int by = block / a.token_blocks, bx = block - by * a.token_blocks;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int head = blockIdx.y >> 1;
-  const int side = blockIdx.y & 1;
+  const int head = by >> 1;
+  const int side = by & 1;
   const int half = lane >> 5;
-  const int64_t tok0 = (int64_t)blockIdx.x * kFwTokens;
-  const u32x4* frag = reinterpret_cast<const u32x4*>(side == 0 ? rot_k : rot_v) + wave * 64 + lane;
+  const int64_t tok0 = (int64_t)bx * kFwTokens;
+  const u32x4* frag = reinterpret_cast<const u32x4*>(side == 0 ? a.rot_k : a.rot_v) + wave * 64 + lane;
   auto load_r = [&](int m, int p) { return __builtin_bit_cast(bf16x8, frag[(m * 16 + p * 8) * 64]); };
 
   // ---- rows to LDS: piece u & 31 (eight features) of token u >> 5; tokens
@@ -614,7 +604,7 @@ __global__ __launch_bounds__(kFwThreads, 4) void quant_write_fused_kernel(
   for (int i = 0; i < 2; ++i) {
     const int u = (int)threadIdx.x + kFwThreads * i;
     const int64_t tok = min(tok0 + (u >> 5), n_tokens - 1);
-    piece[i] = reinterpret_cast<const u32x4*>((side == 0 ? key : value) + tok * token_stride +
+    piece[i] = reinterpret_cast<const u32x4*>((side == 0 ? a.key : a.value) + tok * a.token_stride +
                                               (int64_t)head * kHeadDim)[u & 31];
   }
   // this lane's token from the exchange on
@@ -653,6 +643,7 @@ __global__ __launch_bounds__(kFwThreads, 4) void quant_write_fused_kernel(
   auto place = [](int rr, int jj, int q) {
     return rr * 64 + ((jj ^ (rr & 15)) * 4) + (q ^ ((rr >> 2) & 3) ^ ((jj >> 2) & 3));
   };
+  __syncthreads();
 #pragma unroll
   for (int q = 0; q < 4; ++q)
     ys[place(lane & 31, 8 * half + wave, q)] = floatx4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
@@ -678,11 +669,12 @@ __global__ __launch_bounds__(kFwThreads, 4) void quant_write_fused_kernel(
   mn = __uint_as_float(row_reduce(__float_as_uint(mn), [](uint32_t a, uint32_t b) {
     return __float_as_uint(fminf(__uint_as_float(a), __uint_as_float(b)));
   }));
-  const int clip = side == 0 ? clip_k : clip_v;
+  const int clip = side == 0 ? a.clip_k : a.clip_v;
   float thr = __builtin_inff();
   if (clip >= 0) {
     const uint32_t amax_bits = max(__float_as_uint(mx) & 0x7FFFFFFFu, __float_as_uint(mn) & 0x7FFFFFFFu);
-    thr = __uint_as_float(row_select(v, clip, amax_bits, sel[wave], lane));
+    thr = __uint_as_float(row_select(
+        v, clip, amax_bits, *reinterpret_cast<RowSelLds*>(&ys[wave * kFwTokPerWave * (kHeadDim / 4)]), lane));
   }
   const QParams p = make_qparams(mn, mx, thr, clip >= 0);
   uint32_t word = 0;
@@ -750,6 +742,8 @@ __global__ __launch_bounds__(kFwThreads, 4) void quant_write_fused_kernel(
     }
   }
   if (!v_images) return;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) ys[place(r, j, q)] = floatx4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
   if (j == 0) {
     seat_tile[r] = tile;
     seat_slot[r] = tt;
@@ -760,7 +754,11 @@ __global__ __launch_bounds__(kFwThreads, 4) void quant_write_fused_kernel(
                  seat_tile[lane & 31], seat_slot[lane & 31], inv[wave], w.vimg, wave, lane);
 }
 
-// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(kFwThreads, 8) void quant_write_fused_kernel(FusedWriteArgs a) {
+  __shared__ FusedWriteLds S;
+  fused_write(a, S, blockIdx.x);
+}
+
 // Rows rotated on MFMA: out = in @ R for rows of D = 256 features (the
 // prefill route's q / k / v rotations and its output's R_v^T,
 // oscar_ascend/backend.py:392-413).  in: bf16 (an exact operand) or fp32
@@ -932,6 +930,7 @@ __global__ __launch_bounds__(256, 2) void rotate_rows_kernel(const void* __restr
 // ring took 18.4 us for 3001 tokens, 12.6 for 1024, 11.0 for 77 and 41 for
 // 9256 (six query heads); this takes 14.9, 7.6, 5.8 and 38.  64 rows, which
 // read R half as often, took 15.2, 9.5, 7.9 and 34: only the last is better.
+// (Fragments four steps ahead spill a few registers: 7.4 us for 77 tokens.)
 struct RotateOperandArgs {
   const uint16_t* q;
   const uint16_t* k;
@@ -944,17 +943,21 @@ struct RotateOperandArgs {
   int32_t q_blocks, kv_blocks;
   OperandItems items;
 };
-constexpr int kOpAhead = 4;
+constexpr int kOpAhead = 2;
 
-__global__ __launch_bounds__(512, 4) void rotate_operands_kernel(RotateOperandArgs a) {
+struct OperandLds {
   // [k-step][row ^ k-step, half][8]: swizzled so that the 16 k-steps of one
   // row fall on different banks
-  __shared__ __attribute__((aligned(16))) uint16_t xs[kSteps][64][8];
-  __shared__ float qs[8][32];
+  __attribute__((aligned(16))) uint16_t xs[kSteps][64][8];
+  float qs[8][32];
+};
+
+__device__ __forceinline__ void rotate_operands(const RotateOperandArgs& a, OperandLds& S, int blk) {
+  auto& xs = S.xs;
+  auto& qs = S.qs;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int half = lane >> 5;
-  int blk = blockIdx.x;
   const int kind = blk < a.q_blocks ? 0 : (blk < a.q_blocks + a.kv_blocks ? 1 : 2);    // query, key, value
   blk -= kind == 0 ? 0 : (kind == 1 ? a.q_blocks : a.q_blocks + a.kv_blocks);
   const u32x4* frag = reinterpret_cast<const u32x4*>(kind == 2 ? a.rot_v : a.rot_k) + wave * 64 + lane;
@@ -1056,6 +1059,28 @@ __global__ __launch_bounds__(512, 4) void rotate_operands_kernel(RotateOperandAr
   }
 }
 
+__global__ __launch_bounds__(512, 4) void rotate_operands_kernel(RotateOperandArgs a) {
+  __shared__ OperandLds S;
+  rotate_operands(a, S, blockIdx.x);
+}
+
+// A step's bulk write and its prefill operands in one launch: neither reads
+// what the other writes, and neither fills the GPU up to some thousands of
+// tokens (3001: 11 + 15 us one after the other, 18.5 together; 1052 of a mixed
+// step 15 + 8 and 16.4; 9256 20 + 38 and 50).
+__global__ __launch_bounds__(512, 4) void write_operands_kernel(FusedWriteArgs w, RotateOperandArgs a) {
+  __shared__ union Lds {
+    FusedWriteLds w;
+    OperandLds o;
+    __device__ Lds() {}
+  } S;
+  const int writes = w.token_blocks * 2 * w.num_kv_heads;
+  if ((int)blockIdx.x < writes)
+    fused_write(w, S.w, blockIdx.x);
+  else
+    rotate_operands(a, S.o, (int)blockIdx.x - writes);
+}
+
 // One thread per operand element (2 x 16 x 8 x 64 x 8 = 131072 entries), then
 // one per element of the fp32 copy of R that follows them (65536 entries).
 __global__ void rotation_operand_kernel(const float* __restrict__ R, __bf16* __restrict__ out) {
@@ -1099,12 +1124,17 @@ std::atomic<uint64_t> g_rot_lds_set[4] = {{0}, {0}, {0}, {0}};   // the same for
 int launch_rotate_operands(const uint16_t* q, int64_t q_stride, const uint16_t* k, const uint16_t* v,
                            int64_t kv_stride, int32_t num_heads, int32_t num_kv_heads, const uint8_t* rot_k,
                            const uint8_t* rot_v, const OperandItems& items, const PrefillOperands& o,
-                           hipStream_t stream) {
+                           const FusedWriteArgs* write, hipStream_t stream) {
   RotateOperandArgs a{q, k, v, q_stride, kv_stride, num_heads, num_kv_heads, rot_k, rot_v, o, 0, 0, items};
   const int64_t rows = (int64_t)items.tokens * num_heads, units = (int64_t)items.tiles * num_kv_heads;
   a.q_blocks = (int32_t)((rows + 31) / 32);
   a.kv_blocks = (int32_t)units;
-  hipLaunchKernelGGL(rotate_operands_kernel, dim3((unsigned)(a.q_blocks + 2 * a.kv_blocks)), dim3(512), 0, stream, a);
+  const unsigned blocks = (unsigned)(a.q_blocks + 2 * a.kv_blocks);
+  if (write != nullptr)
+    hipLaunchKernelGGL(write_operands_kernel, dim3(blocks + (unsigned)(write->token_blocks * 2 * write->num_kv_heads)),
+                       dim3(512), 0, stream, *write, a);
+  else
+    hipLaunchKernelGGL(rotate_operands_kernel, dim3(blocks), dim3(512), 0, stream, a);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
@@ -1205,13 +1235,16 @@ struct StepLayout {
 };
 
 // oscar_quant_write with an optional window arena (w.rows > 0), whose request
-// layout is in w's device arrays, or to be stored there from host's.
+// layout is in w's device arrays, or to be stored there from host's.  With
+// `later`, a write that takes the tile kernel is left there for the caller to
+// launch (waits: it was), its winner pass done.
 int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_tokens, int32_t num_kv_heads,
                      int32_t head_size, int64_t token_stride, const void* rot_k_operand, const void* rot_v_operand,
                      const int64_t* slot_mapping, void* k_cache, void* v_cache, int32_t block_size,
                      int64_t num_pages, int64_t k_stride_page, int64_t k_stride_token, int64_t k_stride_head,
                      int64_t v_stride_page, int64_t v_stride_token, int64_t v_stride_head, int32_t clip_index_k,
-                     int32_t clip_index_v, const WindowArgs& w, const StepLayout* host, hipStream_t stream) {
+                     int32_t clip_index_v, const WindowArgs& w, const StepLayout* host, FusedWriteArgs* later,
+                     bool* waits, hipStream_t stream) {
   if (head_size != kHeadDim) return kErrUnsupportedHeadDim;
   if (num_tokens < 0 || num_kv_heads <= 0 || clip_index_k >= kHeadDim || clip_index_v >= kHeadDim)
     return kErrInvalidArgument;
@@ -1248,7 +1281,6 @@ int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_t
                       clip_index_k, clip_index_v, w.stage_k, w.stage_v, w.owner, w.kimg, w.vimg, w.rows,
                       w.sink_eff, w.recent, nullptr, nullptr, nullptr, stream);
   }
-  dim3 grid((unsigned)((num_tokens + kFwTokens - 1) / kFwTokens), (unsigned)(num_kv_heads * 2));
   if (w.rows > 0) {
     HostLayout h{};
     if (host != nullptr) {
@@ -1270,11 +1302,18 @@ int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_t
                        slot_mapping, (int32_t)num_tokens, w.winner, block_size, w.rows, h);
     if (hipGetLastError() != hipSuccess) return kErrLaunch;
   }
-  hipLaunchKernelGGL(quant_write_fused_kernel, grid, dim3(kFwThreads), 0, stream,
-                     static_cast<const uint16_t*>(key_bf16), static_cast<const uint16_t*>(value_bf16),
-                     num_tokens, token_stride, static_cast<const uint8_t*>(rot_k_operand),
-                     static_cast<const uint8_t*>(rot_v_operand), slot_mapping, c,
-                     (int)clip_index_k, (int)clip_index_v, w);
+  const FusedWriteArgs fw{static_cast<const uint16_t*>(key_bf16), static_cast<const uint16_t*>(value_bf16), num_tokens,
+                          token_stride, static_cast<const uint8_t*>(rot_k_operand),
+                          static_cast<const uint8_t*>(rot_v_operand), slot_mapping, c, clip_index_k, clip_index_v, w,
+                          (int32_t)((num_tokens + kFwTokens - 1) / kFwTokens), num_kv_heads};
+  if (later != nullptr) {
+    *later = fw;
+    *waits = true;
+    return kOk;
+  }
+  const int64_t blocks = (int64_t)fw.token_blocks * 2 * num_kv_heads;
+  if (blocks > INT32_MAX) return kErrInvalidArgument;
+  hipLaunchKernelGGL(quant_write_fused_kernel, dim3((unsigned)blocks), dim3(kFwThreads), 0, stream, fw);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
@@ -1293,7 +1332,7 @@ int oscar_quant_write(const void* key_bf16, const void* value_bf16, int64_t num_
   return quant_write_impl(key_bf16, value_bf16, num_tokens, num_kv_heads, head_size, token_stride, rot_k_operand,
                           rot_v_operand, slot_mapping, k_cache, v_cache, block_size, num_pages, k_stride_page,
                           k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
-                          clip_index_k, clip_index_v, WindowArgs{}, nullptr, stream);
+                          clip_index_k, clip_index_v, WindowArgs{}, nullptr, nullptr, nullptr, stream);
 }
 
 int oscar_quant_write_window(const void* key_bf16, const void* value_bf16, int64_t num_tokens,
@@ -1323,7 +1362,7 @@ int oscar_quant_write_window(const void* key_bf16, const void* value_bf16, int64
   return quant_write_impl(key_bf16, value_bf16, num_tokens, num_kv_heads, head_size, token_stride, rot_k_operand,
                           rot_v_operand, slot_mapping, k_cache, v_cache, block_size, num_pages, k_stride_page,
                           k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
-                          clip_index_k, clip_index_v, w, nullptr, stream);
+                          clip_index_k, clip_index_v, w, nullptr, nullptr, nullptr, stream);
 }
 
 }  // extern "C"
@@ -1333,7 +1372,8 @@ namespace oscar {
 int quant_write_step(const oscar_mtp_layer& L, const void* rot_k_operand, const void* rot_v_operand,
                      int64_t* seat_winner, const void* key_bf16, const void* value_bf16, int64_t kv_token_stride,
                      int32_t num_tokens, const int64_t* slot_mapping, const int32_t* query_start_loc,
-                     const int32_t* seq_lens, int32_t num_requests, int32_t* layout, hipStream_t stream) {
+                     const int32_t* seq_lens, int32_t num_requests, int32_t* layout, FusedWriteArgs* later, bool* waits,
+                     hipStream_t stream) {
   WindowArgs w{};
   const StepLayout host{query_start_loc, seq_lens};
   if (L.stage_rows > 0)
@@ -1343,7 +1383,7 @@ int quant_write_step(const oscar_mtp_layer& L, const void* rot_k_operand, const 
   return quant_write_impl(key_bf16, value_bf16, num_tokens, L.num_kv_heads, L.head_size, kv_token_stride,
                           rot_k_operand, rot_v_operand, slot_mapping, L.k_cache, L.v_cache, L.block_size, L.num_pages,
                           L.k_stride_page, L.k_stride_token, L.k_stride_head, L.v_stride_page, L.v_stride_token,
-                          L.v_stride_head, L.clip_index_k, L.clip_index_v, w, &host, stream);
+                          L.v_stride_head, L.clip_index_k, L.clip_index_v, w, &host, later, waits, stream);
 }
 
 }  // namespace oscar

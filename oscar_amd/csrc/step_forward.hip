@@ -3,7 +3,8 @@
 // (oscar_ascend/backend.py:239-319, 361-415):
 //   1. the INT2 write of every token and, with an arena, the window write
 //      (quant_write_step: a seat-winner pass that also carries the request
-//      layout to the device, then the fused write);
+//      layout to the device, then the fused write, which shares a launch with
+//      step 3's operand rotation);
 //   2. the short requests' q / k / v rotated in fp32, packed (one launch);
 //   3. the long requests: operand rotation, prefill read, merge, R_v^T;
 //   4. the short requests' paged read, whose merge writes their output rows.
@@ -142,9 +143,14 @@ extern "C" int oscar_step_forward(const oscar_mtp_layer* layer, const void* rot_
   const uint16_t* k = static_cast<const uint16_t*>(key_bf16);
   const uint16_t* v = static_cast<const uint16_t*>(value_bf16);
 
+  LongBatch b;
+  int32_t next = 0;
+  const bool any_long = next_batch(b, next, num_requests, query_start_loc, seq_lens, max_short);
+  FusedWriteArgs write;
+  bool waits = false;
   rc = quant_write_step(L, rot_k_operand, rot_v_operand, seat_winner, key_bf16, value_bf16, kv_token_stride,
                         num_tokens, slot_mapping, query_start_loc, seq_lens, num_requests,
-                        reinterpret_cast<int32_t*>(ws + p.layout), stream);
+                        reinterpret_cast<int32_t*>(ws + p.layout), any_long ? &write : nullptr, &waits, stream);
   if (rc != kOk) return rc;
 
   float* q_rot = reinterpret_cast<float*>(ws + p.q_rot);
@@ -176,17 +182,18 @@ extern "C" int oscar_step_forward(const oscar_mtp_layer* layer, const void* rot_
     if (runs.n > 0 && (rc = flush()) != kOk) return rc;
   }
 
-  LongBatch b;
-  for (int32_t i = 0; next_batch(b, i, num_requests, query_start_loc, seq_lens, max_short);) {
-    rc = oscar_prefill_rotated(query_bf16, query_token_stride, key_bf16, value_bf16, kv_token_stride, b.n, b.first,
-                               b.fresh, b.cached, b.row, L.num_heads, L.num_kv_heads, L.head_size, rot_k_operand,
-                               rot_v_operand, rot_v_t_operand, L.k_cache, L.v_cache, L.block_size, L.num_pages,
-                               L.k_stride_page, L.k_stride_token, L.k_stride_head, L.v_stride_page, L.v_stride_token,
-                               L.v_stride_head, block_table, block_table_stride, block_table_cols,
-                               L.stage_rows > 0 ? L.stage_k : nullptr, L.stage_rows > 0 ? L.stage_v : nullptr,
-                               L.stage_rows > 0 ? L.stage_owner : nullptr, L.stage_rows, L.scale, out_bf16,
-                               ws + p.rest, p.rest_bytes, stream);
+  for (bool more = any_long; more;
+       more = next_batch(b, next, num_requests, query_start_loc, seq_lens, max_short)) {
+    rc = prefill_rotated(query_bf16, query_token_stride, key_bf16, value_bf16, kv_token_stride, b.n, b.first, b.fresh,
+                         b.cached, b.row, L.num_heads, L.num_kv_heads, L.head_size, rot_k_operand, rot_v_operand,
+                         rot_v_t_operand, L.k_cache, L.v_cache, L.block_size, L.num_pages, L.k_stride_page,
+                         L.k_stride_token, L.k_stride_head, L.v_stride_page, L.v_stride_token, L.v_stride_head,
+                         block_table, block_table_stride, block_table_cols,
+                         L.stage_rows > 0 ? L.stage_k : nullptr, L.stage_rows > 0 ? L.stage_v : nullptr,
+                         L.stage_rows > 0 ? L.stage_owner : nullptr, L.stage_rows, L.scale, out_bf16, ws + p.rest,
+                         p.rest_bytes, waits ? &write : nullptr, stream);
     if (rc != kOk) return rc;
+    waits = false;
   }
 
   if (p.shorts == 0) return kOk;

@@ -1,6 +1,7 @@
 // What the sources launch of one another in a step's forward.
 #pragma once
 
+#include "bulk_write.h"
 #include "oscar_common.h"
 #include "../../include/oscar_amd.h"
 
@@ -49,11 +50,28 @@ int launch_decode_spans(const oscar_mtp_layer& layer, const DecodeSpans& d, void
 
 // oscar_quant_write_window (stage_rows > 0) or oscar_quant_write of a step
 // whose request layout is in host arrays; layout: 2 num_requests + 1 ints of
-// device scratch (quant_write.hip).
+// device scratch (quant_write.hip).  With `later`, a write of the bulk kernel is
+// not launched: its arguments are left there, *waits is set, and the caller
+// hands it to prefill_rotated.
 int quant_write_step(const oscar_mtp_layer& layer, const void* rot_k_operand, const void* rot_v_operand,
                      int64_t* seat_winner, const void* key_bf16, const void* value_bf16, int64_t kv_token_stride,
                      int32_t num_tokens, const int64_t* slot_mapping, const int32_t* query_start_loc,
-                     const int32_t* seq_lens, int32_t num_requests, int32_t* layout, hipStream_t stream);
+                     const int32_t* seq_lens, int32_t num_requests, int32_t* layout, FusedWriteArgs* later, bool* waits,
+                     hipStream_t stream);
+
+// oscar_prefill_rotated, whose first launch also carries out the write in
+// `write`, if there is one (prefill.hip).
+int prefill_rotated(
+    const void* query_bf16, int64_t query_token_stride, const void* key_bf16, const void* value_bf16,
+    int64_t kv_token_stride, int32_t num_requests, const int32_t* first_tokens, const int32_t* new_tokens,
+    const int64_t* cached_lens, const int32_t* table_rows, int32_t num_heads, int32_t num_kv_heads,
+    int32_t head_size, const void* rot_k_operand, const void* rot_v_operand, const void* rot_v_t_operand,
+    const void* k_cache, const void* v_cache, int32_t block_size, int64_t num_pages, int64_t k_stride_page,
+    int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token,
+    int64_t v_stride_head, const int32_t* block_table, int64_t block_table_stride, int32_t block_table_cols,
+    const float* stage_k, const float* stage_v, const int64_t* stage_owner, int32_t stage_rows, float scale,
+    void* out_bf16, void* workspace, size_t workspace_size, const FusedWriteArgs* write,
+    hipStream_t stream);
 
 // oscar_step_write, with the request layout in host arrays, or
 // (layout_on_device) in device arrays that are read on the stream.
