@@ -2376,7 +2376,10 @@ int launch_merge(const DecodeArgs& a, int64_t max_rows, unsigned nitems, const O
     // Rows per block: the fewest that keep the launch's blocks within one
     // round of the CUs, as far as the partials per row allow (one row of few
     // is quickest by itself: 24 rows of 193 partials take 7.0 us, 6 of 9
-    // partials 4.9).
+    // partials 4.9), in quarters of the features, in halves from two rows on
+    // where quarters would take a second round (168 rows of up to 127
+    // partials: 9.5 us as 2 rows x half, 12.9 as 4; 96 rows of 33: 6.9 as 2 x
+    // half, 6.2 as 2 x quarter).
     const int P = a.max_splits + a.fresh;
     const FastDiv heads_div = make_fast_div((uint32_t)a.num_heads), group_div = make_fast_div((uint32_t)a.group);
     auto blocks = [&](int kR, int kQ) { return 8u * kQ * (unsigned)((rows + 8 * kR - 1) / (8 * kR)); };
@@ -2386,8 +2389,10 @@ int launch_merge(const DecodeArgs& a, int64_t max_rows, unsigned nitems, const O
     };
     if (blocks(1, 4) <= 256)
       go(paged_decode_merge_rotate_kernel<1, 4>, 1, 4);
-    else if (blocks(2, 4) <= 256 || P > rot_max_partials(4))
+    else if (blocks(2, 4) <= 256)
       go(paged_decode_merge_rotate_kernel<2, 4>, 2, 4);
+    else if (blocks(2, 2) <= 256 || P > rot_max_partials(4))
+      go(paged_decode_merge_rotate_kernel<2, 2>, 2, 2);
     else if (blocks(4, 2) <= 256 || P > rot_max_partials(8))
       go(paged_decode_merge_rotate_kernel<4, 2>, 4, 2);
     else

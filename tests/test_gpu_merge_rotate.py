@@ -18,14 +18,15 @@ pytestmark = pytest.mark.gpu
 D = 256
 
 
-# Rows (tokens x query heads) of one row per block (64 is the most), two (128),
-# four (512) and eight, each at its last count and one more; groups that do
+# Rows (tokens x query heads) of one row per block (64 is the most), two (128 in
+# quarters, 256 in halves), four (512) and eight, at their last counts and more; groups that do
 # not divide the rows per block; several row tiles per request (16 tokens x 6
 # heads); requests without tokens; more items than one launch carries; 257
 # partials, which eight rows per block do not take.
 @pytest.mark.parametrize("hist,new,hq,hk,tiles,gap", [
     ([700], [16], 4, 1, 0, False), ([700], [13], 5, 1, 0, True), ([300, 5], [16, 16], 4, 2, 0, False),
-    ([40, 3000, 0], [16, 11, 16], 3, 3, 0, True), ([130] * 8, [16] * 8, 4, 1, 0, False),
+    ([40, 3000, 0], [16, 11, 16], 3, 3, 0, True), ([2000, 9, 77, 0], [16] * 4, 4, 1, 0, False),
+    ([20] * 6, [16] * 5 + [6], 3, 1, 0, True), ([0, 5000] * 3, [16, 12] * 3, 3, 1, 0, False), ([130] * 8, [16] * 8, 4, 1, 0, False),
     ([515, 0, 33] * 3, [16, 1, 16] * 3, 6, 1, 0, True), ([64] * 33, [16] * 33, 6, 2, 0, False),
     ([90] * 70, [2] * 70, 12, 2, 0, False), ([32768] + [10] * 40, [4] * 41, 6, 1, 4, False)])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
