@@ -17,8 +17,11 @@ Read path, per request (backend.py:273-313 routing):
   0 < q_len <= 16    -> paged MTP decode kernel over INT2 history + window
   q_len > 16         -> prefill-continuation kernel (f16 MFMA over dequantized
                         history tiles + the new tokens, right-aligned causal)
-Both read kernels work in the rotated domain; q/k/v are rotated with one
-fp32 matmul each and the output is mapped back with R_v^T.
+Both read kernels work in the rotated domain: a bf16 step rotates q/k/v in
+the library (fp32 for short requests, MFMA for long ones) and the reads' last
+pass applies R_v^T; the whole forward of a layer is one library call
+(oscar_mtp_forward, oscar_step_forward or oscar_decode_only_forward).  Other
+dtypes rotate with one fp32 matmul each.
 
 There is no fallback path: a missing library or a kernel error raises.
 """

@@ -557,11 +557,11 @@ __device__ __forceinline__ void store_v_images(const Value& value, int64_t seat_
 // Writes up to 8K tokens are bound by one workgroup's latency, larger ones by
 // the products (two bf16 passes, 28 us for 65536 tokens at the rate of a
 // large library product) beside the selection's vector instructions, which a
-// CU's three workgroups overlap.  With 128 tokens to a workgroup of four
+// CU's four workgroups overlap.  With 128 tokens to a workgroup of four
 // wavefronts, each with 32 tokens of its own and R through an LDS ring, 3001
 // tokens took 29 us with the window (their selection 10, its image 7), 1052
 // of a mixed step 36, 9256 29 and 65536 without one 71; this takes 11, 15, 20
-// and 67.  64 tokens to a workgroup (half the reading of R): 17, -, 25, 68.
+// and 64.  64 tokens to a workgroup (half the reading of R): 17, -, 25, 68.
 // 33 KB, so that four workgroups share a CU: the operands' rows [k-step][row ^
 // k-step, half] until the products are done, then the rotated values, in a
 // wave's share of which its selection works once the wave has read them.
