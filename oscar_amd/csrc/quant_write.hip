@@ -317,6 +317,9 @@ constexpr int kSteps = 16;
 constexpr int kMfmaEntries = kSteps * kChunkBytes / 2;
 constexpr size_t kMfmaOperandBytes = (size_t)kSteps * kChunkBytes;
 constexpr size_t kOperandBytes = kMfmaOperandBytes + sizeof(float) * kHeadDim * kHeadDim;
+constexpr size_t kRingLds = kFusedWaves * sizeof(SelLds) > kRing * kChunkBytes ? kFusedWaves * sizeof(SelLds)
+                                                                               : (size_t)kRing * kChunkBytes;
+constexpr int64_t kRingRound = 512;             // workgroups of the ring kernel resident at once: two per CU
 constexpr int64_t kShortWriteVectors = 2048;   // at most 1024 tokens (the step write's limit)
 constexpr int kDmaPerChunk = kChunkBytes / (kFusedWaves * 64 * 16);   // 2 per thread
 
@@ -877,6 +880,37 @@ __device__ __forceinline__ void rotate_tile(const uint8_t* __restrict__ xsrc, co
   }
 }
 
+// Large writes without a window whose workgroups fill the GPU's rounds: 128
+// tokens to a workgroup of four waves, each with 32 tokens of its own (lane l:
+// features 128 (l >> 5) .. +127 of token l & 31), R through the LDS ring.  It
+// reads R a quarter as often as quant_write_fused_kernel and needs no
+// exchange, but a round of it takes 33 us however few of its workgroups are
+// left: 32768 tokens (one whole round) 35.1 us against 36.3, 65536 (two) 62.4
+// against 65.2, but 24576 31.8 against 27.2 and 49152 67 against 51.  Same
+// products in the same order, same bytes.
+__global__ __launch_bounds__(256, 2) void quant_write_ring_kernel(FusedWriteArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t ring[];     // ring, then the selection buffers
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int by = (int)blockIdx.x / a.token_blocks, bx = (int)blockIdx.x - by * a.token_blocks;
+  const int head = by >> 1, side = by & 1, half = lane >> 5;
+  const int64_t tok = (int64_t)bx * (kFusedWaves * kTokPerWave) + wave * kTokPerWave + (lane & 31);
+  const bool live = tok < a.n_tokens;       // (else token 0 is computed and nothing stored)
+  floatx16 acc[8];
+  rotate_tile<false>(reinterpret_cast<const uint8_t*>((side == 0 ? a.key : a.value) + (live ? tok : 0) * a.token_stride +
+                                                      (int64_t)head * kHeadDim + half * kPerLane),
+                     side == 0 ? a.rot_k : a.rot_v, ring, wave, lane, acc);
+  __syncthreads();      // the ring becomes the waves' selection buffers
+  float v[kPerLane];
+#pragma unroll
+  for (int t = 0; t < 8; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[16 * t + i] = acc[t][i];
+  const QParams p =
+      vector_params(v, side == 0 ? a.clip_k : a.clip_v, reinterpret_cast<SelLds*>(ring)[wave], lane);
+  quantize_store(v, p, live ? a.slots[tok] : -1, head, side, half, a.c);
+}
+
 template <bool kF32In, bool kBf16Out>
 __global__ __launch_bounds__(256, 2) void rotate_rows_kernel(const void* __restrict__ in, int64_t in_stride,
                                                             int64_t rows, const uint8_t* __restrict__ rop,
@@ -1117,6 +1151,7 @@ int check_cache_args(CacheArgs& c) {
   return kOk;
 }
 
+std::atomic<uint64_t> g_ring_lds_set{0};   // dynamic-LDS attribute set, one bit per device
 std::atomic<uint64_t> g_rot_lds_set[4] = {{0}, {0}, {0}, {0}};   // the same for the rotate_rows instances
 
 }  // namespace
@@ -1180,19 +1215,19 @@ int oscar_rotate_rows(const void* in, int32_t in_f32, int64_t in_row_stride, int
                       reinterpret_cast<const void*>(rotate_rows_kernel<true, false>),
                       reinterpret_cast<const void*>(rotate_rows_kernel<true, true>)};
   const int which = 2 * in_f32 + out_bf16;
-  constexpr int kRingLds = kRing * kChunkBytes;
-  if (set_dynamic_lds(k[which], kRingLds, g_rot_lds_set[which]) != kOk) return kErrLaunch;
+  constexpr int kRotLds = kRing * kChunkBytes;
+  if (set_dynamic_lds(k[which], kRotLds, g_rot_lds_set[which]) != kOk) return kErrLaunch;
   if (in_f32 && out_bf16)
-    hipLaunchKernelGGL((rotate_rows_kernel<true, true>), grid, dim3(256), kRingLds, stream, in, in_row_stride, rows,
+    hipLaunchKernelGGL((rotate_rows_kernel<true, true>), grid, dim3(256), kRotLds, stream, in, in_row_stride, rows,
                        rop, out, out_row_stride);
   else if (in_f32)
-    hipLaunchKernelGGL((rotate_rows_kernel<true, false>), grid, dim3(256), kRingLds, stream, in, in_row_stride, rows,
+    hipLaunchKernelGGL((rotate_rows_kernel<true, false>), grid, dim3(256), kRotLds, stream, in, in_row_stride, rows,
                        rop, out, out_row_stride);
   else if (out_bf16)
-    hipLaunchKernelGGL((rotate_rows_kernel<false, true>), grid, dim3(256), kRingLds, stream, in, in_row_stride, rows,
+    hipLaunchKernelGGL((rotate_rows_kernel<false, true>), grid, dim3(256), kRotLds, stream, in, in_row_stride, rows,
                        rop, out, out_row_stride);
   else
-    hipLaunchKernelGGL((rotate_rows_kernel<false, false>), grid, dim3(256), kRingLds, stream, in, in_row_stride, rows,
+    hipLaunchKernelGGL((rotate_rows_kernel<false, false>), grid, dim3(256), kRotLds, stream, in, in_row_stride, rows,
                        rop, out, out_row_stride);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
@@ -1306,6 +1341,18 @@ int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_t
                           token_stride, static_cast<const uint8_t*>(rot_k_operand),
                           static_cast<const uint8_t*>(rot_v_operand), slot_mapping, c, clip_index_k, clip_index_v, w,
                           (int32_t)((num_tokens + kFwTokens - 1) / kFwTokens), num_kv_heads};
+  const int64_t ring_blocks = (num_tokens + kFusedWaves * kTokPerWave - 1) / (kFusedWaves * kTokPerWave);
+  const int64_t ring_wgs = ring_blocks * 2 * num_kv_heads, last_round = ring_wgs % kRingRound;
+  if (w.rows == 0 && ring_wgs >= kRingRound && (last_round == 0 || last_round > kRingRound - kRingRound / 16)) {
+    FusedWriteArgs rw = fw;
+    rw.token_blocks = (int32_t)ring_blocks;
+    if (ring_wgs > INT32_MAX) return kErrInvalidArgument;
+    if (set_dynamic_lds(reinterpret_cast<const void*>(quant_write_ring_kernel), (int)kRingLds, g_ring_lds_set) != kOk)
+      return kErrLaunch;
+    hipLaunchKernelGGL(quant_write_ring_kernel, dim3((unsigned)ring_wgs), dim3(kFusedWaves * 64), kRingLds, stream,
+                       rw);
+    return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+  }
   if (later != nullptr) {
     *later = fw;
     *waits = true;

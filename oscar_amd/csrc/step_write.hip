@@ -26,6 +26,8 @@
 // keys and values finds the clip threshold by a bitwise radix select over the
 // 256 |x| (ballots), quantizes with the exact thresholds of int2_quant.h,
 // writes the slot and, when it is its seat's winner, the window.
+#include <type_traits>
+
 #include "int2_quant.h"
 #include "step_launch.h"
 #include "window_images.h"
@@ -72,7 +74,6 @@ struct StepArgs {
   const int32_t* query_start;   // the request layout on the device, or null: keep holds the rule
   const int32_t* seq_lens;
   int32_t num_requests, sink_eff, recent;
-  TokenRuns runs;               // n > 0: the inputs' tokens of the packed order
 };
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t x) { return __uint_as_float((uint32_t)x << 16); }
@@ -314,7 +315,14 @@ __device__ __forceinline__ int run_token(const TokenRuns& r, int p, int lane) {
   return __builtin_amdgcn_readlane(tok, i) + p - __builtin_amdgcn_readlane(pos, i);
 }
 
-__global__ __launch_bounds__(kThreads) void step_write_kernel(StepArgs a) {
+// (runs: the inputs' tokens in the packed order of a rotation without a write.
+// A kernel of its own: half a kilobyte more of arguments cost every short
+// write 0.3 us.)
+struct NoRuns {};
+
+template <class Runs>
+__global__ __launch_bounds__(kThreads) void step_write_kernel(StepArgs a, Runs runs) {
+  constexpr bool kRuns = std::is_same<Runs, TokenRuns>::value;
   __shared__ __attribute__((aligned(16))) float xs[kGroupVecs][kHeadDim];
   __shared__ __attribute__((aligned(16))) float part[kWaves][kGroupVecs][kHeadDim];
   const Scalars c = load_scalars(a);
@@ -360,7 +368,8 @@ __global__ __launch_bounds__(kThreads) void step_write_kernel(StepArgs a) {
   for (int idx = tid; idx < nv * kHeadDim; idx += kThreads) {
     const int vv = __builtin_amdgcn_readfirstlane(idx >> 8), f = idx & 255;
     const int e = e0 + vv, h = e % heads;
-    const int t = a.runs.n > 0 ? run_token(a.runs, e / heads, lane) : e / heads;
+    int t = e / heads;
+    if constexpr (kRuns) t = run_token(runs, t, lane);
     xs[vv][f] = bf16_to_f32(src[(int64_t)t * stride + (int64_t)h * kHeadDim + f]);
   }
   __syncthreads();
@@ -397,14 +406,16 @@ __global__ __launch_bounds__(kThreads) void step_write_kernel(StepArgs a) {
 // Vectors per workgroup: one while the step has few vectors (every workgroup
 // streams R once; fewer vectors each finish sooner), up to four for larger
 // steps.
-int launch(StepArgs& a, hipStream_t stream) {
+template <class Runs = NoRuns>
+int launch(StepArgs& a, hipStream_t stream, const Runs& runs = Runs{}) {
   const int64_t n = a.n_tokens;
   const int64_t vectors = n * (a.num_heads + 2 * a.num_kv_heads);
   const int64_t per = vectors <= 512 ? 1 : (vectors <= 2048 ? 2 : 4);
   a.vecs_per_group = (int32_t)per;
   a.kv_groups = (int32_t)((n * a.num_kv_heads + per - 1) / per);
   const int64_t q_groups = (n * a.num_heads + per - 1) / per;
-  hipLaunchKernelGGL(step_write_kernel, dim3((unsigned)(2 * a.kv_groups + q_groups)), dim3(kThreads), 0, stream, a);
+  hipLaunchKernelGGL(step_write_kernel<Runs>, dim3((unsigned)(2 * a.kv_groups + q_groups)), dim3(kThreads), 0, stream, a,
+                     runs);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
@@ -446,8 +457,7 @@ int launch_rotate_runs(const uint16_t* q, int64_t q_stride, const uint16_t* k, c
   a.q_rot = q_rot;
   a.k_rot = k_rot;
   a.v_rot = v_rot;
-  a.runs = runs;
-  return launch(a, stream);
+  return launch(a, stream, runs);
 }
 
 int step_write(bool layout_on_device, const void* query_bf16, int64_t query_token_stride,

@@ -34,9 +34,21 @@ def _vectors(kind, n, hk, g):
 @pytest.mark.parametrize("ratios", [(0.96, 0.92), (0.0, 0.5), (1.0, 0.004), (0.84, 0.85)])
 @pytest.mark.parametrize("n,hk", [(1027, 1), (544, 2)])
 def test_bytes_with_an_exact_rotation(device, kind, ratios, n, hk):
+    _check(device, kind, ratios, n, hk)
+
+
+# The kernel of whole rounds of 128-token workgroups: exactly one round with a
+# remainder in the last workgroup, the fewest workgroups of a round that take
+# it, and one less (the kernel above).
+@pytest.mark.parametrize("n,hk", [(32765, 1), (30721, 1), (30720, 1), (16300, 2)])
+def test_bytes_of_whole_rounds(device, n, hk):
+    _check(device, "ties" if n % 2 else "range", (0.96, 0.5), n, hk)
+
+
+def _check(device, kind, ratios, n, hk):
     g = torch.Generator().manual_seed(n)
     k, v = _vectors(kind, n, hk, g), _vectors(kind, n, hk, g)
-    bs, pages = 32, 40
+    bs, pages = 32, n // 32 + 7
     caches = make_caches(pages, bs, hk, torch.int8, seed=4)
     slots = torch.randperm(pages * bs, generator=g)[:n]
     slots[::17] = -1
