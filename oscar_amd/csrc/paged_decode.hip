@@ -99,19 +99,30 @@ typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 
 // Work items of one launch travel inside the kernel arguments (no device
 // round trip for the metadata); larger batches are launched in chunks.
-constexpr int kMaxInlineItems = 128;    // (and kv heads, so that kvh fits its byte)
+constexpr int kMaxInlineItems = 128;
 
+// Five words: every split and merge launch carries 128 of them, and each
+// further 512 bytes of arguments cost it about 0.3 us (six words: plain merge
+// of 96 rows 5.42 -> 5.78 us, of 1024 tokens 4.80 -> 5.06).
 struct ItemInfo {
   int32_t qa;        // first query row (token) of the request
   int32_t prefix;    // history length
   int32_t pbase;     // first partial slot of the item: history splits 0 .. nsplit - 1, then the fresh one
-  int32_t out0;      // first output token of the request (rotated merge)
-  int32_t req;       // block-table row, from the launch chunk's first
-  int8_t nq;         // query tokens of the request
-  int8_t kvh;        // kv head
+  int16_t nq;        // query tokens of the request
+  int16_t req;       // block-table row, from the launch chunk's first
+  int16_t kvh;       // kv head
   int16_t nsplit;    // history splits of the item: split s takes steps s, s + nsplit, s + 2 nsplit, ...
 };
 constexpr int kItemWords = sizeof(ItemInfo) / sizeof(int);
+static_assert(sizeof(ItemInfo) == 5 * sizeof(int), "ItemInfo is five words");
+
+// First output tokens of a launch chunk's requests, where the queries are
+// packed and the output is not (the short requests of a step with long ones);
+// other launches write a token's output at its query row and carry NoSpans.
+struct SpanTokens {
+  int32_t tok[kMaxInlineItems];
+};
+struct NoSpans {};
 
 struct DecodeArgs {
   const float* q;          // [n, Hq, D]
@@ -1861,11 +1872,19 @@ __global__ __launch_bounds__(256) void paged_decode_merge_small_kernel(DecodeArg
 // last request that starts at or before the token (a request without tokens
 // starts where the next one does).  As in find_item, every lane reads two
 // requests' items and a ballot counts the starts.  Called by every lane of
-// the wavefront with wave-uniform arguments.
-__device__ __forceinline__ ItemInfo find_token_item(const DecodeArgs& a, int tok, int kvh) {
+// the wavefront with wave-uniform arguments.  out_tok: the token's row of the
+// output.
+template <class Spans>
+__device__ __forceinline__ ItemInfo find_token_item(const DecodeArgs& a, const Spans& spans, int tok, int kvh,
+                                                    int& out_tok) {
+  constexpr bool kSpans = std::is_same<Spans, SpanTokens>::value;
   const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
   const int hk = a.num_kv_heads, n = a.nitems;     // items are [request][kv head]
-  if (n == hk) return a.items[kvh];
+  out_tok = tok;
+  if (n == hk) {
+    if constexpr (kSpans) out_tok += spans.tok[0] - a.items[kvh].qa;
+    return a.items[kvh];
+  }
   const int i0 = lane * hk + kvh, i1 = (lane + 64) * hk + kvh;
   const int* f0 = reinterpret_cast<const int*>(&a.items[i0 < n ? i0 : kvh]);
   const int* f1 = reinterpret_cast<const int*>(&a.items[i1 < n ? i1 : kvh]);
@@ -1874,6 +1893,11 @@ __device__ __forceinline__ ItemInfo find_token_item(const DecodeArgs& a, int tok
   for (int k = 0; k < kItemWords; ++k) {
     w0[k] = f0[k];
     w1[k] = f1[k];
+  }
+  int t0 = 0, t1 = 0;
+  if constexpr (kSpans) {
+    t0 = spans.tok[lane];
+    t1 = spans.tok[lane + 64];
   }
   static_assert(offsetof(ItemInfo, qa) == 0, "qa is the first word");
   const int c = __popcll(__ballot(i0 < n && w0[0] <= tok)) + __popcll(__ballot(i1 < n && w1[0] <= tok));
@@ -1886,6 +1910,10 @@ __device__ __forceinline__ ItemInfo find_token_item(const DecodeArgs& a, int tok
   }
   ItemInfo it;
   __builtin_memcpy(&it, fld, sizeof(it));
+  if constexpr (kSpans) {
+    const int v0 = __builtin_amdgcn_readlane(t0, req & 63), v1 = __builtin_amdgcn_readlane(t1, req & 63);
+    out_tok += (req < 64 ? v0 : v1) - it.qa;
+  }
   return it;
 }
 
@@ -1920,10 +1948,10 @@ constexpr int kRotMl = 2;                        // (m, l) pairs per thread, at 
 constexpr int rot_max_partials(int kR) { return kRotMl * kRotThreads / kR; }
 static_assert(rot_max_partials(2) >= kMaxPartials, "one or two rows per block take any launch");
 
-template <int kR, int kQ>
+template <int kR, int kQ, class Spans>
 __global__ __launch_bounds__(kRotThreads) void paged_decode_merge_rotate_kernel(
-    DecodeArgs a, int tok0, int rows, FastDiv heads_div, FastDiv group_div, const float* __restrict__ rot_t, void* __restrict__ out, int64_t out_stride,
-    int out_bf16) {
+    DecodeArgs a, Spans spans, int tok0, int rows, FastDiv heads_div, FastDiv group_div,
+    const float* __restrict__ rot_t, void* __restrict__ out, int64_t out_stride, int out_bf16) {
   constexpr int W = kRotWaves / kR;              // waves per row
   constexpr int kMl = kR == 1 ? 1 : kRotMl;
   constexpr int CW = 4 / kQ;                     // waves side by side over the block's output features
@@ -1964,7 +1992,8 @@ __global__ __launch_bounds__(kRotThreads) void paged_decode_merge_rotate_kernel(
   const int tok = tok0 + to;
   const int h = trow - to * a.num_heads;
   const int kvh = (int)fast_div((uint32_t)h, group_div);
-  const ItemInfo it = find_token_item(a, tok, kvh);
+  int out_tok;
+  const ItemInfo it = find_token_item(a, spans, tok, kvh, out_tok);
   const int row = (tok - it.qa) * a.group + (h - kvh * a.group);
   const int rt = row / kRows, r = row % kRows;
   const int steps = (it.prefix + kStepTok - 1) / kStepTok;
@@ -1998,7 +2027,7 @@ __global__ __launch_bounds__(kRotThreads) void paged_decode_merge_rotate_kernel(
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) mloc = fmaxf(mloc, __shfl_xor(mloc, o, 64));
   if (lane == 0) red[0][w] = mloc;
-  if (lane == 0 && wr == 0) otok[w / W] = it.out0 + (tok - it.qa);
+  if (lane == 0 && wr == 0) otok[w / W] = out_tok;
   __syncthreads();
   float mx = red[0][w - wr];
 #pragma unroll
@@ -2365,8 +2394,9 @@ struct OutRotation {
   int32_t out_bf16;
 };
 
+// (spans: the requests' output tokens, only with a rotation; or null)
 int launch_merge(const DecodeArgs& a, int64_t max_rows, unsigned nitems, const OutRotation& orot,
-                 hipStream_t stream) {
+                 const SpanTokens* spans, hipStream_t stream) {
   const int mr = merge_rows(max_rows);
   if (orot.rot_t != nullptr) {
     const int tok0 = a.items[0].qa;
@@ -2383,20 +2413,33 @@ int launch_merge(const DecodeArgs& a, int64_t max_rows, unsigned nitems, const O
     const int P = a.max_splits + a.fresh;
     const FastDiv heads_div = make_fast_div((uint32_t)a.num_heads), group_div = make_fast_div((uint32_t)a.group);
     auto blocks = [&](int kR, int kQ) { return 8u * kQ * (unsigned)((rows + 8 * kR - 1) / (8 * kR)); };
-    auto go = [&](auto kernel, int kR, int kQ) {
-      hipLaunchKernelGGL(kernel, dim3(blocks(kR, kQ)), dim3(kRotThreads), 0, stream, a, tok0, rows, heads_div, group_div, orot.rot_t,
-                         orot.out, orot.out_stride, (int)orot.out_bf16);
+    auto go = [&](auto rows_tag, auto parts_tag) {
+      constexpr int kR = decltype(rows_tag)::value, kQ = decltype(parts_tag)::value;
+      const dim3 grid(blocks(kR, kQ));
+      if (spans != nullptr)
+        hipLaunchKernelGGL((paged_decode_merge_rotate_kernel<kR, kQ, SpanTokens>), grid, dim3(kRotThreads), 0, stream, a,
+                           *spans, tok0, rows, heads_div, group_div, orot.rot_t, orot.out, orot.out_stride,
+                           (int)orot.out_bf16);
+      else
+        hipLaunchKernelGGL((paged_decode_merge_rotate_kernel<kR, kQ, NoSpans>), grid, dim3(kRotThreads), 0, stream, a,
+                           NoSpans{}, tok0, rows, heads_div, group_div, orot.rot_t, orot.out, orot.out_stride,
+                           (int)orot.out_bf16);
     };
+    using std::integral_constant;
+    constexpr integral_constant<int, 1> one{};
+    constexpr integral_constant<int, 2> two{};
+    constexpr integral_constant<int, 4> four{};
+    constexpr integral_constant<int, 8> eight{};
     if (blocks(1, 4) <= 256)
-      go(paged_decode_merge_rotate_kernel<1, 4>, 1, 4);
+      go(one, four);
     else if (blocks(2, 4) <= 256)
-      go(paged_decode_merge_rotate_kernel<2, 4>, 2, 4);
+      go(two, four);
     else if (blocks(2, 2) <= 256 || P > rot_max_partials(4))
-      go(paged_decode_merge_rotate_kernel<2, 2>, 2, 2);
+      go(two, two);
     else if (blocks(4, 2) <= 256 || P > rot_max_partials(8))
-      go(paged_decode_merge_rotate_kernel<4, 2>, 4, 2);
+      go(four, two);
     else
-      go(paged_decode_merge_rotate_kernel<8, 2>, 8, 2);
+      go(eight, two);
   } else if (a.max_splits + a.fresh <= kSmallP) {
     dim3 grid((unsigned)((mr * 4 + 15) / 16), nitems, (unsigned)a.row_tiles);
     hipLaunchKernelGGL(paged_decode_merge_small_kernel, grid, dim3(256), 0, stream, a);
@@ -2529,9 +2572,11 @@ int launch_decode(DecodeLaunch& L, hipStream_t stream) {
   // next split in stream order).
   const int32_t per = requests_per_launch(L.num_kv_heads);
   int32_t packed = 0;                   // query tokens of the requests so far
+  SpanTokens spans;
   for (int32_t c0 = 0; c0 < L.num_requests;) {
     int32_t nreq = 0, first = c0;
-    for (; c0 < L.num_requests && nreq < per; ++c0) {
+    // (a chunk's requests span at most as many table rows as `req` can tell)
+    for (; c0 < L.num_requests && nreq < per && (nreq == 0 || c0 - first <= INT16_MAX); ++c0) {
       const int32_t tok = L.qsl[c0];
       const int32_t nq = L.qsl[c0 + 1] - tok;
       if (L.spans > 0 && (nq <= 0 || nq > L.spans)) continue;
@@ -2539,7 +2584,8 @@ int launch_decode(DecodeLaunch& L, hipStream_t stream) {
       const int32_t qa = L.spans > 0 ? packed : tok;
       for (int32_t h = 0; h < L.num_kv_heads; ++h)
         a.items[nreq * L.num_kv_heads + h] =
-            ItemInfo{qa, L.seqs[c0] - nq, 0, tok, c0 - first, (int8_t)nq, (int8_t)h, 0};
+            ItemInfo{qa, L.seqs[c0] - nq, 0, (int16_t)nq, (int16_t)(c0 - first), (int16_t)h, 0};
+      spans.tok[nreq] = tok;
       packed += nq;
       ++nreq;
     }
@@ -2553,7 +2599,8 @@ int launch_decode(DecodeLaunch& L, hipStream_t stream) {
     const unsigned gx = split_workgroups(a);
     if (gx > 0) launch_split(a, nitems, dim3(gx, 1, (unsigned)a.row_tiles), stream);
     if (hipGetLastError() != hipSuccess) return kErrLaunch;
-    const int rc = launch_merge(a, (int64_t)L.max_query_len * a.group, nitems, L.orot, stream);
+    const int rc = launch_merge(a, (int64_t)L.max_query_len * a.group, nitems, L.orot,
+                                L.spans > 0 ? &spans : nullptr, stream);
     if (rc != kOk) return rc;
   }
   return kOk;
@@ -2669,7 +2716,7 @@ int decode_only(const float* q_rot, int32_t num_heads, int32_t num_kv_heads, int
     const int32_t nreq = num_requests - c0 < per ? num_requests - c0 : per;
     for (int32_t i = 0; i < nreq; ++i)
       for (int32_t h = 0; h < num_kv_heads; ++h)
-        a.items[i * num_kv_heads + h] = ItemInfo{c0 + i, seq_lens[c0 + i], 0, c0 + i, i, 1, (int8_t)h, 0};
+        a.items[i * num_kv_heads + h] = ItemInfo{c0 + i, seq_lens[c0 + i], 0, 1, (int16_t)i, (int16_t)h, 0};
     a.block_table = block_table ? block_table + (int64_t)c0 * block_table_stride : nullptr;
     const unsigned nitems = (unsigned)(nreq * num_kv_heads);
     if (!plan_splits(a, nitems, max_history, tiles_per_split, 0)) return kErrInvalidArgument;
@@ -2683,7 +2730,7 @@ int decode_only(const float* q_rot, int32_t num_heads, int32_t num_kv_heads, int
       launch_split(a, nitems, dim3(gx, 1, (unsigned)a.row_tiles), stream);
       if (hipGetLastError() != hipSuccess) return kErrLaunch;
     }
-    if ((rc = launch_merge(a, a.group, nitems, orot, stream)) != kOk) return rc;
+    if ((rc = launch_merge(a, a.group, nitems, orot, nullptr, stream)) != kOk) return rc;
   }
   return kOk;
 }
