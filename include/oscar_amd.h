@@ -488,6 +488,8 @@ int oscar_quant_write_window(const void* key_bf16, const void* value_bf16, int64
  *     [tokens], block_table [num_requests][block_table_stride];
  *   out_bf16 [tokens][num_heads][D], 16-byte aligned;
  *   workspace: 16-byte aligned, >= oscar_step_forward_workspace_bytes(...).
+ * Every argument is checked before anything is enqueued: a step that is
+ * refused has neither written the caches or the arena nor read them.
  */
 size_t oscar_step_forward_workspace_bytes(int32_t num_requests, const int32_t* query_start_loc,
                                           const int32_t* seq_lens, int32_t num_heads, int32_t num_kv_heads,

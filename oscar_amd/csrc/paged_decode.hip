@@ -2922,7 +2922,7 @@ int oscar_mtp_forward(const oscar_mtp_layer* layer, const oscar_mtp_step* step, 
 namespace oscar {
 
 int launch_decode_spans(const oscar_mtp_layer& L, const DecodeSpans& d, void* out_bf16, int64_t out_token_stride,
-                        void* workspace, size_t workspace_size, hipStream_t stream) {
+                        void* workspace, size_t workspace_size, bool check_only, hipStream_t stream) {
   const int32_t rows = L.stage_rows;
   DecodeLaunch D;
   const int rc = prepare_decode(D, d.q_rot, d.k_rot, d.v_rot, d.query_start_loc[d.num_requests], L.num_heads,
@@ -2935,7 +2935,7 @@ int launch_decode_spans(const oscar_mtp_layer& L, const DecodeSpans& d, void* ou
                                 reinterpret_cast<float*>(out_bf16),
                                 OutRotation{L.rot_v_t, out_bf16, out_token_stride, 1}, workspace, workspace_size,
                                 d.spans);
-  return rc != kOk ? rc : launch_decode(D, stream);
+  return rc != kOk || check_only ? rc : launch_decode(D, stream);
 }
 
 }  // namespace oscar

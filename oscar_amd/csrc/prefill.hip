@@ -1589,7 +1589,8 @@ int prefill_rotated(
     int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token,
     int64_t v_stride_head, const int32_t* block_table, int64_t block_table_stride, int32_t block_table_cols,
     const float* stage_k, const float* stage_v, const int64_t* stage_owner, int32_t stage_rows, float scale,
-    void* out_bf16, void* workspace, size_t workspace_size, const FusedWriteArgs* write, hipStream_t stream) {
+    void* out_bf16, void* workspace, size_t workspace_size, const FusedWriteArgs* write, bool check_only,
+    hipStream_t stream) {
   PrefillArgs base{};
   int st = fill_common(base, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages,
                        k_stride_page, k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
@@ -1617,6 +1618,7 @@ int prefill_rotated(
   if (workspace_size < oscar_prefill_rotated_workspace_bytes(num_requests, new_tokens, cached_lens, num_heads,
                                                              num_kv_heads))
     return kErrWorkspaceTooSmall;
+  if (check_only) return kOk;
   for (int32_t r0 = 0; r0 < num_requests; r0 += kMaxPrefillItems) {
     PrefillArgs a = base;
     OperandItems ops{};
@@ -1659,5 +1661,5 @@ extern "C" int oscar_prefill_rotated(
                          block_size, num_pages, k_stride_page, k_stride_token, k_stride_head,
                          v_stride_page, v_stride_token, v_stride_head, block_table,
                          block_table_stride, block_table_cols, stage_k, stage_v, stage_owner,
-                         stage_rows, scale, out_bf16, workspace, workspace_size, nullptr, stream);
+                         stage_rows, scale, out_bf16, workspace, workspace_size, nullptr, false, stream);
 }

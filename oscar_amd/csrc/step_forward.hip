@@ -143,8 +143,35 @@ extern "C" int oscar_step_forward(const oscar_mtp_layer* layer, const void* rot_
   const uint16_t* k = static_cast<const uint16_t*>(key_bf16);
   const uint16_t* v = static_cast<const uint16_t*>(value_bf16);
 
+  float* q_rot = reinterpret_cast<float*>(ws + p.q_rot);
+  float* k_rot = reinterpret_cast<float*>(ws + p.k_rot);
+  float* v_rot = reinterpret_cast<float*>(ws + p.v_rot);
+  auto read_long = [&](const LongBatch& b, const FusedWriteArgs* write, bool check_only) {
+    return prefill_rotated(query_bf16, query_token_stride, key_bf16, value_bf16, kv_token_stride, b.n, b.first, b.fresh,
+                           b.cached, b.row, L.num_heads, L.num_kv_heads, L.head_size, rot_k_operand, rot_v_operand,
+                           rot_v_t_operand, L.k_cache, L.v_cache, L.block_size, L.num_pages, L.k_stride_page,
+                           L.k_stride_token, L.k_stride_head, L.v_stride_page, L.v_stride_token, L.v_stride_head,
+                           block_table, block_table_stride, block_table_cols,
+                           L.stage_rows > 0 ? L.stage_k : nullptr, L.stage_rows > 0 ? L.stage_v : nullptr,
+                           L.stage_rows > 0 ? L.stage_owner : nullptr, L.stage_rows, L.scale, out_bf16, ws + p.rest,
+                           p.rest_bytes, write, check_only, stream);
+  };
+  auto read_short = [&](bool check_only) {
+    return launch_decode_spans(L, DecodeSpans{q_rot, k_rot, v_rot, query_start_loc, seq_lens, num_requests, max_short,
+                                              p.max_query_len, p.max_history, block_table, block_table_stride,
+                                              block_table_cols},
+                               out_bf16, width, ws + p.rest, p.rest_bytes, check_only, stream);
+  };
+
+  // Whatever a part of the step refuses is refused before the first launch
+  // (the write's own checks precede its launches, which come first).
   LongBatch b;
   int32_t next = 0;
+  while (next_batch(b, next, num_requests, query_start_loc, seq_lens, max_short))
+    if ((rc = read_long(b, nullptr, true)) != kOk) return rc;
+  if (p.shorts > 0 && (rc = read_short(true)) != kOk) return rc;
+
+  next = 0;
   const bool any_long = next_batch(b, next, num_requests, query_start_loc, seq_lens, max_short);
   FusedWriteArgs write;
   bool waits = false;
@@ -153,9 +180,6 @@ extern "C" int oscar_step_forward(const oscar_mtp_layer* layer, const void* rot_
                         reinterpret_cast<int32_t*>(ws + p.layout), any_long ? &write : nullptr, &waits, stream);
   if (rc != kOk) return rc;
 
-  float* q_rot = reinterpret_cast<float*>(ws + p.q_rot);
-  float* k_rot = reinterpret_cast<float*>(ws + p.k_rot);
-  float* v_rot = reinterpret_cast<float*>(ws + p.v_rot);
   if (p.shorts > 0) {
     TokenRuns runs{};
     int64_t done = 0;                                // packed tokens of earlier launches
@@ -184,21 +208,9 @@ extern "C" int oscar_step_forward(const oscar_mtp_layer* layer, const void* rot_
 
   for (bool more = any_long; more;
        more = next_batch(b, next, num_requests, query_start_loc, seq_lens, max_short)) {
-    rc = prefill_rotated(query_bf16, query_token_stride, key_bf16, value_bf16, kv_token_stride, b.n, b.first, b.fresh,
-                         b.cached, b.row, L.num_heads, L.num_kv_heads, L.head_size, rot_k_operand, rot_v_operand,
-                         rot_v_t_operand, L.k_cache, L.v_cache, L.block_size, L.num_pages, L.k_stride_page,
-                         L.k_stride_token, L.k_stride_head, L.v_stride_page, L.v_stride_token, L.v_stride_head,
-                         block_table, block_table_stride, block_table_cols,
-                         L.stage_rows > 0 ? L.stage_k : nullptr, L.stage_rows > 0 ? L.stage_v : nullptr,
-                         L.stage_rows > 0 ? L.stage_owner : nullptr, L.stage_rows, L.scale, out_bf16, ws + p.rest,
-                         p.rest_bytes, waits ? &write : nullptr, stream);
-    if (rc != kOk) return rc;
+    if ((rc = read_long(b, waits ? &write : nullptr, false)) != kOk) return rc;
     waits = false;
   }
 
-  if (p.shorts == 0) return kOk;
-  return launch_decode_spans(L, DecodeSpans{q_rot, k_rot, v_rot, query_start_loc, seq_lens, num_requests, max_short,
-                                            p.max_query_len, p.max_history, block_table, block_table_stride,
-                                            block_table_cols},
-                             out_bf16, width, ws + p.rest, p.rest_bytes, stream);
+  return p.shorts > 0 ? read_short(false) : (int)kOk;
 }

@@ -45,8 +45,9 @@ struct DecodeSpans {
   int64_t block_table_stride;
   int32_t block_table_cols;
 };
+// (check_only: the arguments' checks alone, nothing enqueued)
 int launch_decode_spans(const oscar_mtp_layer& layer, const DecodeSpans& d, void* out_bf16, int64_t out_token_stride,
-                        void* workspace, size_t workspace_size, hipStream_t stream);
+                        void* workspace, size_t workspace_size, bool check_only, hipStream_t stream);
 
 // oscar_quant_write_window (stage_rows > 0) or oscar_quant_write of a step
 // whose request layout is in host arrays; layout: 2 num_requests + 1 ints of
@@ -60,7 +61,8 @@ int quant_write_step(const oscar_mtp_layer& layer, const void* rot_k_operand, co
                      hipStream_t stream);
 
 // oscar_prefill_rotated, whose first launch also carries out the write in
-// `write`, if there is one (prefill.hip).
+// `write`, if there is one (prefill.hip).  check_only: the arguments' checks
+// alone, nothing enqueued.
 int prefill_rotated(
     const void* query_bf16, int64_t query_token_stride, const void* key_bf16, const void* value_bf16,
     int64_t kv_token_stride, int32_t num_requests, const int32_t* first_tokens, const int32_t* new_tokens,
@@ -70,7 +72,7 @@ int prefill_rotated(
     int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token,
     int64_t v_stride_head, const int32_t* block_table, int64_t block_table_stride, int32_t block_table_cols,
     const float* stage_k, const float* stage_v, const int64_t* stage_owner, int32_t stage_rows, float scale,
-    void* out_bf16, void* workspace, size_t workspace_size, const FusedWriteArgs* write,
+    void* out_bf16, void* workspace, size_t workspace_size, const FusedWriteArgs* write, bool check_only,
     hipStream_t stream);
 
 // oscar_step_write, with the request layout in host arrays, or
