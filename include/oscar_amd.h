@@ -249,10 +249,10 @@ int oscar_prefill_continuation(const float* q_rot, const float* k_new, const flo
                                const int64_t* stage_owner, int32_t stage_rows, float scale,
                                float* out, oscar_stream_t stream);
 
-/* The same read with its work spread over the whole GPU: the row blocks (128
+/* The same read with its work spread over the whole GPU: the row blocks (256
  * (token, head) rows) and their key blocks are cut into equal shares, and row
  * blocks that a cut runs through are merged from fp32 partials.  workspace:
- * device memory of at least oscar_prefill_workspace_bytes(num_new, Hq, Hk,
+ * device memory, 16-byte aligned, of at least oscar_prefill_workspace_bytes(num_new, Hq, Hk,
  * cached_len) bytes (the new tokens' MFMA operands and the partials); its
  * contents need no initialisation and mean nothing after the call.
  */
@@ -280,7 +280,7 @@ int oscar_prefill_continuation_split(const float* q_rot, const float* k_new, con
  *     R_k, R_v and R_v^T;
  *   block_table [rows][block_table_stride];
  *   out_bf16 [tokens][Hq][D]: rows of the requests' tokens are written;
- *   workspace: at least oscar_prefill_rotated_workspace_bytes bytes.
+ *   workspace: 16-byte aligned, at least oscar_prefill_rotated_workspace_bytes bytes.
  */
 size_t oscar_prefill_rotated_workspace_bytes(int32_t num_requests, const int32_t* new_tokens,
                                              const int64_t* cached_lens, int32_t num_heads, int32_t num_kv_heads);

@@ -219,6 +219,12 @@ __device__ __forceinline__ void locate_unit(const PrefillItem& it, int group, in
   }
 }
 
+// A V slot's code word and four fp32 values where the caller's strides and
+// addresses promise less than their size (any V stride; an output or an arena
+// aligned to its elements): the same one instruction each.
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef floatx4 floatx4_any __attribute__((aligned(4)));
+
 // Raw bytes of one history block for one thread of wave w: K role (token 4w +
 // lane / 16, code word lane % 16: features 16 (lane % 16) .. +15) and owner
 // tag of token lane % 32; V role (token 4w + lane % 4, code word lane / 4);
@@ -320,7 +326,7 @@ __device__ __forceinline__ u32x2 load_meta(const Hot& h, int k0, int32_t page, c
 __device__ __forceinline__ uint32_t load_v(const Hot& h, int k0, int32_t page, const Roles& r) {
   const int64_t pg = page >= 0 ? page : 0;
   const uint8_t* vp = h.vbase + pg * h.v_page + (uint64_t)fast_mod((uint32_t)k0, h.bs_div) * h.vtok;
-  return *reinterpret_cast<const uint32_t*>(vp + r.vo);
+  return *reinterpret_cast<const u32_any*>(vp + r.vo);
 }
 
 // fp16 pair (1 + c/4) of the codes at bits [sh, sh + 2) and [sh + 16, sh + 18)
@@ -419,7 +425,7 @@ __device__ __forceinline__ void window_tiles(uint32_t kmask, int32_t kpage, int 
   const uint32_t nib = (vmask >> (4 * w)) & 15u;
   floatx4 xk[4] = {}, y[4];
   if (mine) {
-    const floatx4* src = reinterpret_cast<const floatx4*>(stage_row(false, kpage, k0, t, kvh) + 16 * (lane & 15));
+    const floatx4_any* src = reinterpret_cast<const floatx4_any*>(stage_row(false, kpage, k0, t, kvh) + 16 * (lane & 15));
 #pragma unroll
     for (int e = 0; e < 4; ++e) xk[e] = src[e];
   }
@@ -428,7 +434,7 @@ __device__ __forceinline__ void window_tiles(uint32_t kmask, int32_t kpage, int 
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       if ((nib >> k) & 1u)
-        y[k] = *reinterpret_cast<const floatx4*>(stage_row(true, vpage, v0, 4 * w + k, kvh) + 4 * lane);
+        y[k] = *reinterpret_cast<const floatx4_any*>(stage_row(true, vpage, v0, 4 * w + k, kvh) + 4 * lane);
       else
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[k][e] = 1.f + 0.25f * (float)((codes >> (8 * k + 2 * e)) & 3u);
@@ -972,7 +978,7 @@ __global__ __launch_bounds__(512, 2) void prefill_kernel(PrefillArgs a) {
         const int r8 = 4 * i + (elane >> 4);
         const floatx4 x = T[16 * r8 + ((elane & 15) ^ (r8 & 15))];
         if (off[i] != ~0u)
-          *reinterpret_cast<floatx4*>(base + (uint64_t)off[i] * kHeadDim + 64 * p + 4 * (elane & 15)) = x;
+          *reinterpret_cast<floatx4_any*>(base + (uint64_t)off[i] * kHeadDim + 64 * p + 4 * (elane & 15)) = x;
       }
     }
   }
@@ -1065,7 +1071,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   const floatx4 o = merge_row<kWavesPerRow>(slot, n, pr, wave % kWavesPerRow, lane);
   if (wave % kWavesPerRow != 0) return;
   const int tok = row / a.group, head = kvh * a.group + (row - tok * a.group);
-  *reinterpret_cast<floatx4*>(a.out + ((int64_t)(it.tok0 + tok) * a.num_heads + head) * kHeadDim + 4 * lane) = o;
+  *reinterpret_cast<floatx4_any*>(a.out + ((int64_t)(it.tok0 + tok) * a.num_heads + head) * kHeadDim + 4 * lane) = o;
 }
 
 // The read's bf16 output: rows merged where the shares cut their row block
@@ -1347,8 +1353,9 @@ Layout workspace_layout(int64_t tokens, int64_t tiles, int64_t units, int32_t hq
   return w;
 }
 
-// The cache, block table, arena and geometry half of the arguments, checked.
-int fill_common(PrefillArgs& a, int32_t num_heads, int32_t num_kv_heads, int32_t head_size, const void* k_cache,
+// The cache, block table, arena and geometry half of the arguments, checked
+// (of a call without new tokens, `empty`, only the counts).
+int fill_common(PrefillArgs& a, bool empty, int32_t num_heads, int32_t num_kv_heads, int32_t head_size, const void* k_cache,
                 const void* v_cache, int32_t block_size, int64_t num_pages, int64_t k_stride_page,
                 int64_t k_stride_token, int64_t k_stride_head, int64_t v_stride_page, int64_t v_stride_token,
                 int64_t v_stride_head, const int32_t* block_table, int64_t block_table_stride,
@@ -1356,12 +1363,13 @@ int fill_common(PrefillArgs& a, int32_t num_heads, int32_t num_kv_heads, int32_t
                 int32_t stage_rows, float scale) {
   if (head_size != kHeadDim) return kErrUnsupportedHeadDim;
   if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || block_size <= 0 || num_pages <= 0 ||
-      stage_rows < 0 || block_table_cols < 0 || !k_cache || !v_cache)
+      stage_rows < 0 || block_table_cols < 0)
     return kErrInvalidArgument;
+  if (empty) return kOk;
+  if (!k_cache || !v_cache) return kErrInvalidArgument;
   if (stage_rows > 0 && (!stage_k || !stage_v || !stage_owner)) return kErrInvalidArgument;
   if (k_stride_head < kKCodeOff + kCodeBytes || v_stride_head < kCodeBytes || (k_stride_head & 7) ||
-      (k_stride_token & 7) || (k_stride_page & 7) || (v_stride_head & 1) || (v_stride_token & 1) ||
-      (v_stride_page & 1) || block_size % kBlk != 0)
+      (k_stride_token & 7) || (k_stride_page & 7) || block_size % kBlk != 0)
     return kErrUnsupportedGeometry;
   a.num_heads = num_heads;
   a.num_kv_heads = num_kv_heads;
@@ -1501,14 +1509,15 @@ extern "C" int oscar_prefill_continuation_split(
     const float* stage_k, const float* stage_v, const int64_t* stage_owner, int32_t stage_rows,
     float scale, float* out, void* workspace, size_t workspace_size, hipStream_t stream) {
   PrefillArgs a{};
-  int st = fill_common(a, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages, k_stride_page,
-                       k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head, block_table_row,
-                       0, block_table_cols, stage_k, stage_v, stage_owner, stage_rows, scale);
-  if (st != kOk) return st;
+  if (num_new < 0 || cached_len < 0) return kErrInvalidArgument;
+  int st = fill_common(a, num_new == 0, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages,
+                       k_stride_page, k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
+                       block_table_row, 0, block_table_cols, stage_k, stage_v, stage_owner, stage_rows, scale);
+  if (st != kOk || num_new == 0) return st;
   if ((st = check_request(num_new, cached_len, num_heads, block_size, block_table_row, block_table_cols)) != kOk)
     return st;
-  if (num_new == 0) return kOk;
-  if (!q_rot || !k_new || !v_new || !out || !workspace) return kErrInvalidArgument;
+  if (!q_rot || !k_new || !v_new || !out || !workspace || (reinterpret_cast<uintptr_t>(workspace) & 15))
+    return kErrInvalidArgument;
   OperandItems ops{};
   add_item(a, ops, num_new, cached_len, 0, 0);
   const Layout w = workspace_layout(ops.tokens, ops.tiles, a.units, num_heads, num_kv_heads, false);
@@ -1535,13 +1544,13 @@ extern "C" int oscar_prefill_continuation(
     const float* stage_k, const float* stage_v, const int64_t* stage_owner, int32_t stage_rows,
     float scale, float* out, hipStream_t stream) {
   PrefillArgs a{};
-  int st = fill_common(a, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages, k_stride_page,
-                       k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head, block_table_row,
-                       0, block_table_cols, stage_k, stage_v, stage_owner, stage_rows, scale);
-  if (st != kOk) return st;
+  if (num_new < 0 || cached_len < 0) return kErrInvalidArgument;
+  int st = fill_common(a, num_new == 0, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages,
+                       k_stride_page, k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
+                       block_table_row, 0, block_table_cols, stage_k, stage_v, stage_owner, stage_rows, scale);
+  if (st != kOk || num_new == 0) return st;
   if ((st = check_request(num_new, cached_len, num_heads, block_size, block_table_row, block_table_cols)) != kOk)
     return st;
-  if (num_new == 0) return kOk;
   if (!q_rot || !k_new || !v_new || !out) return kErrInvalidArgument;
   a.q = q_rot;
   a.k_new = k_new;
@@ -1592,7 +1601,7 @@ int prefill_rotated(
     void* out_bf16, void* workspace, size_t workspace_size, const FusedWriteArgs* write, bool check_only,
     hipStream_t stream) {
   PrefillArgs base{};
-  int st = fill_common(base, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages,
+  int st = fill_common(base, false, num_heads, num_kv_heads, head_size, k_cache, v_cache, block_size, num_pages,
                        k_stride_page, k_stride_token, k_stride_head, v_stride_page, v_stride_token, v_stride_head,
                        block_table, block_table_stride, block_table_cols, stage_k, stage_v, stage_owner, stage_rows,
                        scale);
@@ -1607,7 +1616,8 @@ int prefill_rotated(
       (query_token_stride & 7) || (kv_token_stride & 7) || (reinterpret_cast<uintptr_t>(query_bf16) & 15) ||
       (reinterpret_cast<uintptr_t>(key_bf16) & 15) || (reinterpret_cast<uintptr_t>(value_bf16) & 15) ||
       (reinterpret_cast<uintptr_t>(out_bf16) & 15) || (reinterpret_cast<uintptr_t>(rot_k_operand) & 15) ||
-      (reinterpret_cast<uintptr_t>(rot_v_operand) & 15) || (reinterpret_cast<uintptr_t>(rot_v_t_operand) & 15))
+      (reinterpret_cast<uintptr_t>(rot_v_operand) & 15) || (reinterpret_cast<uintptr_t>(rot_v_t_operand) & 15) ||
+      (reinterpret_cast<uintptr_t>(workspace) & 15))
     return kErrInvalidArgument;
   for (int32_t i = 0; i < num_requests; ++i) {
     if (first_tokens[i] < 0 || table_rows[i] < 0) return kErrInvalidArgument;

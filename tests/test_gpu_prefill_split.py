@@ -112,3 +112,42 @@ def test_workspace_is_checked(device):
             *vst, bt.data_ptr(), 16, 1000, None, None, None, 0, ctypes.c_float(0.1), z.data_ptr(), ws.data_ptr(),
             size, _lib.stream_handle(z.device))
     assert run(need - 1) == -3
+
+
+@pytest.mark.parametrize("split", [False, True])
+def test_rows_of_less_alignment_than_a_load(device, split):
+    # V slots 67 bytes apart from an odd address, an output and an arena that
+    # start 4 bytes past a 16-byte line: the same results as aligned ones.
+    hq, hk, hist, new, bs = 6, 1, 300, 45, 32
+    case = decode_case([hist], [new], hq=hq, hk=hk, bs=bs, seed=8, window=True, sink=bs, recent=40)
+    L = case.layer
+    q, k, v = (t.to(device) for t in case.rotated())
+    kc, vc, bt = L.k_cache.to(device), L.v_cache.to(device), case.bt[0].to(device)
+    sk, sv, owner = (t.to(device).contiguous() for t in L.stage())
+    pages = kc.shape[0]
+    packed = torch.zeros(1 + pages * bs * 67, dtype=torch.int8, device=device)
+    packed[1:].view(pages, bs, 67)[:, :, :64] = vc[:, :, 0, :64]
+    shifted = [torch.zeros(t.numel() + 1, dtype=torch.float32, device=device) for t in (sk, sv)]
+    for s, t in zip(shifted, (sk, sv)):
+        s[1:] = t.reshape(-1)
+    gbs, _, kst, vst = cache_geometry(kc, vc)
+    lib = _lib.load()
+    ws = torch.empty(lib.oscar_prefill_workspace_bytes(new, hq, hk, hist), dtype=torch.uint8, device=device)
+
+    def run(vptr, vst, skp, svp, out):
+        args = (*map(_lib.ptr, (q, k, v)), new, hq, hk, D, _lib.ptr(kc), vptr, gbs, pages, *kst, *vst, _lib.ptr(bt),
+                bt.numel(), hist, skp, svp, _lib.ptr(owner), owner.shape[0], L.scale, out.data_ptr())
+        stream = _lib.stream_handle(out.device)
+        if split:
+            _lib.call("oscar_prefill_continuation_split", *args, _lib.ptr(ws), ws.numel(), stream)
+        else:
+            _lib.call("oscar_prefill_continuation", *args, stream)
+        torch.cuda.synchronize()
+        return out.cpu()
+
+    n = new * hq * D
+    want = run(vc.data_ptr(), vst, sk.data_ptr(), sv.data_ptr(), torch.zeros(n, device=device))
+    got = run(packed.data_ptr() + 1, (bs * 67, 67, 64), shifted[0].data_ptr() + 4, shifted[1].data_ptr() + 4,
+              torch.zeros(n + 1, device=device)[1:])
+    assert torch.equal(got, want)
+    _close(want.view(new, hq, D), _want(case, 0, *case.rotated(), hk))
