@@ -392,8 +392,9 @@ class OscarAttentionBackendImpl:
         return True
 
     def _mtp_layer(self, layer, kv_cache, dev) -> step.MtpLayer:
-        """The layer half of the short-step forward, kept on the layer and
-        rebuilt only when its rotations, caches or window arena are replaced."""
+        """The layer half of the one-call forwards, kept on the layer and
+        rebuilt when its rotations, caches or window arena are replaced or
+        when a setting it was packed from has another value."""
         cfg = self._oscar
         if cfg.window_enabled:
             self._ensure_staging(layer, kv_cache)
@@ -402,9 +403,10 @@ class OscarAttentionBackendImpl:
             rots = self._layer_rots(layer, dev)
         arena = (layer._oscar_stage_k, layer._oscar_stage_v, layer._oscar_slot_owner, layer._oscar_stage_kimg,
                  layer._oscar_stage_vimg) if cfg.window_enabled else (None,) * 5
-        ml = getattr(layer, "_oscar_mtp", None)
+        ml, was = getattr(layer, "_oscar_mtp", None), getattr(layer, "_oscar_mtp_settings", None)
+        settings = (cfg, self.scale, self.num_heads, self.num_kv_heads)
         rvT = getattr(layer, "_oscar_rvT", None)
-        if ml is not None and ml.bound_to(rots[0], rots[1], rvT, self.key_cache, self.value_cache, *arena):
+        if ml is not None and was == settings and ml.bound_to(rots[0], rots[1], rvT, self.key_cache, self.value_cache, *arena):
             return ml
         rk, rv = self._layer_rots(layer, dev)
         D = self.head_size
@@ -413,7 +415,7 @@ class OscarAttentionBackendImpl:
                            self.num_kv_heads, quant.clip_index(cfg.k_clip_ratio, D),
                            quant.clip_index(cfg.v_clip_ratio, D), self.scale,
                            arena if cfg.window_enabled else None, (cfg.sink_tokens // bs) * bs, cfg.recent_tokens)
-        layer._oscar_mtp = ml
+        layer._oscar_mtp, layer._oscar_mtp_settings = ml, settings
         return ml
 
     def _decode_only_step(self, layer, query, kv_cache, attn_metadata, output) -> bool:
