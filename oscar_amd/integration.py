@@ -10,9 +10,11 @@ whole cache blocks.  Per OSCAR layer the fixed buffers here are
   * its fp16 MFMA operand images (high and    rows * bs * 4 * Hk * D * 2
     low parts of K and of V)
   * the arena's seat-winner buffer             rows * bs * 8 + 16
-and, once per device, the split-decode workspace of the largest batch and
-the library's no-allocation decode array (32 MiB, a static device array every
-GPU that loads the library holds whether or not that entry is called).
+and, once per device, the split-decode workspace of the largest batch, the
+scratch of the largest step with long requests (oscar_step_forward's, 135 MB of
+it for the pieces of cut row blocks) and the library's no-allocation decode
+array (32 MiB, a static device array every GPU that loads the library holds
+whether or not that entry is called).
 
 The engine seams (``install_runner_hooks``) apply that budget before vLLM
 allocates its caches and print one READY manifest per rank after it did;
@@ -128,6 +130,30 @@ def decode_workspace_bytes(max_requests: int, num_kv_heads: int, num_heads: int,
         DECODE_PARTIAL_FLOATS * 4
 
 
+PREFILL_SHARES = 256                   # workgroups of a prefill read: one per CU, two partial slots each
+PREFILL_PARTIAL_BYTES = 256 * (256 + 2) * 4       # 256 rows x 256 + max + sum, fp32
+PREFILL_LAUNCH_REQUESTS = 48
+PREFILL_TILE = 32                      # tokens of a key tile (16 KB each of K and V operands per kv head)
+
+
+def step_workspace_bytes(max_tokens: int, max_requests: int, num_kv_heads: int, num_heads: int, max_history: int,
+                         max_short: int = 16) -> int:
+    """At least oscar_step_forward_workspace_bytes of every step of up to
+    max_tokens new tokens in up to max_requests requests of up to max_history
+    tokens, of which those of 1 .. max_short new tokens take the paged read (no
+    library needed)."""
+    # a short token's fp32 q / k / v; a long one's fp16 operands with their sum
+    # and fp32 output row (its key tiles are rounded up once per request)
+    short = (num_heads + 2 * num_kv_heads) * 256 * 4
+    tile = 2 * num_kv_heads * PREFILL_TILE * 256 * 2
+    long = num_heads * (256 * 2 + 4 + 256 * 4) + tile // PREFILL_TILE
+    read = decode_workspace_bytes(min(max_requests, max_tokens), num_kv_heads, num_heads, max_short, max_history) \
+        if max_short else 0
+    pieces = 2 * PREFILL_SHARES * PREFILL_PARTIAL_BYTES
+    tiles = min(max_requests, PREFILL_LAUNCH_REQUESTS) * tile
+    return 4 * (2 * max_requests + 1) + max_tokens * max(short, long) + max(pieces + tiles, read) + 16 * 256
+
+
 def kv_block_bytes(block_size: int, num_kv_heads: int, slot_width: int, layers: int) -> int:
     """Native bytes of one cache block across the OSCAR layers (K and V caches)."""
     return 2 * block_size * num_kv_heads * slot_width * layers
@@ -136,11 +162,15 @@ def kv_block_bytes(block_size: int, num_kv_heads: int, slot_width: int, layers: 
 def plan_capacity(available: int, layers: int, head_dim: int = 256, num_kv_heads: int = 1,
                   num_heads: int = 6, block_size: int = 128, slot_width: int = 256, sink: int = 128,
                   recent: int = 256, staging: int = 8192, window: bool = True, max_requests: int = 256,
-                  max_query_len: int = 4, max_history: int = 262144) -> dict:
-    """Budget one GPU: how many cache blocks (and INT2 tokens) fit."""
+                  max_query_len: int = 4, max_history: int = 262144, max_step_tokens: int = 0) -> dict:
+    """Budget one GPU: how many cache blocks (and INT2 tokens) fit.
+    max_step_tokens: the largest step's new tokens, whose scratch is set aside
+    (0: none, for a server whose prompts are computed elsewhere)."""
     fixed = layers * fixed_bytes_per_layer(head_dim, num_kv_heads, block_size, sink, recent, staging, window)
     fixed += decode_workspace_bytes(max_requests, num_kv_heads, num_heads, max_query_len, max_history)
     fixed += NOALLOC_SCRATCH_BYTES
+    if max_step_tokens > 0:
+        fixed += step_workspace_bytes(max_step_tokens, max_requests, num_kv_heads, num_heads, max_history)
     native = kv_block_bytes(block_size, num_kv_heads, slot_width, layers)
     budget = memory_budget(available, native, 0, fixed)
     blocks = budget // native
@@ -186,10 +216,12 @@ def _oscar_modules(ctx: dict) -> dict:
 def oscar_fixed_bytes(runner, specs: dict, targets: dict) -> int:
     """Persistent bytes the OSCAR layers allocate after profiling (rotations,
     MFMA operands, window arena and its images, at the engine page size),
-    plus, once per device, the split-decode workspace of the largest batch
+    plus, once per device, the split-decode workspace of the largest batch,
+    the scratch of the largest step the scheduler makes (max_num_batched_tokens)
     and the library's 32 MiB no-allocation decode array."""
     fixed = 0
     hk = heads = 1
+    short = 0
     for name, module in targets.items():
         impl = module.impl
         c = impl._oscar
@@ -197,6 +229,7 @@ def oscar_fixed_bytes(runner, specs: dict, targets: dict) -> int:
         fixed += fixed_bytes_per_layer(impl.head_size, impl.num_kv_heads, bs, c.sink_tokens, c.recent_tokens,
                                        c.staging_tokens, c.window_enabled)
         hk, heads = impl.num_kv_heads, impl.num_heads
+        short = c.paged_max_q_len if c.use_paged else 0
     cfg = runner.vllm_config
     max_reqs = int(getattr(cfg.scheduler_config, "max_num_seqs", 256) or 256)
     max_len = int(getattr(cfg.model_config, "max_model_len", 0) or 0)
@@ -204,6 +237,9 @@ def oscar_fixed_bytes(runner, specs: dict, targets: dict) -> int:
     max_q = 1 + int(getattr(spec_cfg, "num_speculative_tokens", 0) or 0) if spec_cfg is not None else 1
     if targets and max_len > 0:
         fixed += decode_workspace_bytes(max_reqs, hk, heads, max_q, max_len)
+        max_tokens = int(getattr(cfg.scheduler_config, "max_num_batched_tokens", 0) or 0)
+        if max_tokens > 0:
+            fixed += step_workspace_bytes(max_tokens, max_reqs, hk, heads, max_len, short)
     if targets:
         fixed += NOALLOC_SCRATCH_BYTES
     return fixed
