@@ -880,14 +880,12 @@ __device__ __forceinline__ void rotate_tile(const uint8_t* __restrict__ xsrc, co
   }
 }
 
-// Large writes without a window whose workgroups fill the GPU's rounds: 128
-// tokens to a workgroup of four waves, each with 32 tokens of its own (lane l:
-// features 128 (l >> 5) .. +127 of token l & 31), R through the LDS ring.  It
-// reads R a quarter as often as quant_write_fused_kernel and needs no
-// exchange, but a round of it takes 33 us however few of its workgroups are
-// left: 32768 tokens (one whole round) 35.1 us against 36.3, 65536 (two) 62.4
-// against 65.2, but 24576 31.8 against 27.2 and 49152 67 against 51.  Same
-// products in the same order, same bytes.
+// Large writes without a window: 128 tokens to a workgroup of four waves, each
+// with 32 tokens of its own (lane l: features 128 (l >> 5) .. +127 of token l &
+// 31), R through the LDS ring.  It reads R a quarter as often as
+// quant_write_fused_kernel and needs no exchange, but a round of it takes about
+// 30 us however few of its workgroups are left.  Same products in the same
+// order, same bytes.  prefers_ring says when it is taken.
 __global__ __launch_bounds__(256, 2) void quant_write_ring_kernel(FusedWriteArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t ring[];     // ring, then the selection buffers
   const int lane = threadIdx.x & 63;
@@ -1151,6 +1149,20 @@ int check_cache_args(CacheArgs& c) {
   return kOk;
 }
 
+// Whether a write of that many 128-token workgroups takes the ring kernel: its
+// last round is full to a sixteenth, or there are more than 3 1/8 rounds, which
+// a partial last one no longer decides.  us, ring against tile kernel, by rounds
+// (one kv head): 0.875 31.9 / 31.0, 0.94 32.6 / 33.9, 1 33.4 / 34.7, 1.01 46 / 37,
+// 1.5 66 / 51, 1.75 68 / 58, 2 61-72 (by process) / 65.5, 2.25 86 / 76, 2.75 95 /
+// 93, 3 100.7 / 100.3, 3.06 105 / 103, 3.19 106.7 / 107.3, 3.5 112.6 / 117.3, 5.5
+// 169 / 180, 8 236 / 260; two heads 1 33.2 / 34.5, 3.25 112 / 110, 3.5 115 / 117;
+// four 3.25 111 / 109, 4 131.6 / 132.5.
+bool prefers_ring(int64_t workgroups) {
+  const int64_t last = workgroups % kRingRound;
+  return workgroups > 3 * kRingRound + kRingRound / 8 ||
+         (workgroups >= kRingRound && (last == 0 || last > kRingRound - kRingRound / 16));
+}
+
 std::atomic<uint64_t> g_ring_lds_set{0};   // dynamic-LDS attribute set, one bit per device
 std::atomic<uint64_t> g_rot_lds_set[4] = {{0}, {0}, {0}, {0}};   // the same for the rotate_rows instances
 
@@ -1342,8 +1354,8 @@ int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_t
                           static_cast<const uint8_t*>(rot_v_operand), slot_mapping, c, clip_index_k, clip_index_v, w,
                           (int32_t)((num_tokens + kFwTokens - 1) / kFwTokens), num_kv_heads};
   const int64_t ring_blocks = (num_tokens + kFusedWaves * kTokPerWave - 1) / (kFusedWaves * kTokPerWave);
-  const int64_t ring_wgs = ring_blocks * 2 * num_kv_heads, last_round = ring_wgs % kRingRound;
-  if (w.rows == 0 && ring_wgs >= kRingRound && (last_round == 0 || last_round > kRingRound - kRingRound / 16)) {
+  const int64_t ring_wgs = ring_blocks * 2 * num_kv_heads;
+  if (w.rows == 0 && prefers_ring(ring_wgs)) {
     FusedWriteArgs rw = fw;
     rw.token_blocks = (int32_t)ring_blocks;
     if (ring_wgs > INT32_MAX) return kErrInvalidArgument;
