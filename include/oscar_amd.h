@@ -50,7 +50,8 @@ int oscar_rotation_operand(const float* rotation, void* operand, int32_t head_si
 /* Rows rotated on MFMA: out[r] = in[r] @ R for rows of head_size features.
  * Replaces the prefill route's fp32 rotations (oscar_ascend/backend.py:392-413:
  * q / k / v `x.float() @ rk` / `@ rv` before the attention, `out.float() @
- * rv.t()` after it).
+ * rv.t()` after it) for callers of oscar_prefill_continuation; oscar_prefill_rotated
+ * and oscar_step_forward rotate by themselves.
  *   in:          [rows][in_row_stride] bf16 (in_f32 = 0) or fp32 (in_f32 = 1);
  *   rot_operand: oscar_rotation_operand of R (of R_v^T for the output);
  *   out:         [rows][out_row_stride] fp32 (out_bf16 = 0) or bf16 (out_bf16 = 1,
@@ -236,7 +237,11 @@ int oscar_decode_only(const float* q_rot, int32_t num_heads, int32_t num_kv_head
  * kernels/prefill.py:69-72) for one request.
  *   q_rot [num_new][Hq][D], k_new / v_new [num_new][Hk][D]: fp32 rotated;
  *   block_table_row [block_table_cols] int32: the request's pages;
+ *   k_cache is 8-byte aligned with strides that are multiples of 8, V slots
+ *   and strides may have any alignment;
  *   staging as in oscar_paged_decode; out [num_new][Hq][D] fp32 rotated-V.
+ * Without a workspace: a workgroup walks all keys of a whole row block.  For
+ * callers that have none; the Python layer uses the entry below.
  */
 int oscar_prefill_continuation(const float* q_rot, const float* k_new, const float* v_new,
                                int32_t num_new, int32_t num_heads, int32_t num_kv_heads,

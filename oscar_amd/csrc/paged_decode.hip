@@ -101,9 +101,10 @@ typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 // round trip for the metadata); larger batches are launched in chunks.
 constexpr int kMaxInlineItems = 128;
 
-// Five words: every split and merge launch carries 128 of them, and each
-// further 512 bytes of arguments cost it about 0.3 us (six words: plain merge
-// of 96 rows 5.42 -> 5.78 us, of 1024 tokens 4.80 -> 5.06).
+// Five words: every split and merge launch carries 128 of them, and with six
+// (512 bytes more) the plain merge of 24 rows of 194 partials took 5.78 us for
+// 5.56, of 48 rows of 65 5.06 for 4.85, and the one-row rotated merge 7.33 for
+// 6.93.
 struct ItemInfo {
   int32_t qa;        // first query row (token) of the request
   int32_t prefix;    // history length
@@ -1697,9 +1698,11 @@ __global__ __launch_bounds__(256, 2) void paged_decode_split_small_kernel(Decode
 }
 
 // One 256-thread block per (output row, quarter of the features) of an item.
-// Every load the block needs goes out in one round: the partials' (m, l)
+// The loads the block needs are written as one round: the partials' (m, l)
 // (thread per partial) and the block's 64-feature slice of every partial row
 // (thread: partial group t / 16, features 4 * (t % 16) .. +3 of the quarter).
+// Each row's load is behind a branch of its own, and the compiled code waits
+// for all before it after the second: two memory round trips.
 constexpr int kMergeGroups = 16;                 // partial groups per block
 constexpr int kMergeBatch = 16;                  // partial loads per thread per round
 constexpr int kMaxPartials = kMaxSplits + 1;
@@ -1728,7 +1731,7 @@ __global__ __launch_bounds__(256) void paged_decode_merge_kernel(DecodeArgs a) {
   const int64_t pstride = (int64_t)a.row_tiles * kPartialFloats;
   const int f0 = 64 * qd + 4 * fl;
 
-  // ---- issue every load ----
+  // ---- the loads ----
   float mreg[kMaxPartials / 256], lreg[kMaxPartials / 256];
 #pragma unroll
   for (int k = 0; k < kMaxPartials / 256; ++k) {
@@ -1923,11 +1926,14 @@ __device__ __forceinline__ ItemInfo find_token_item(const DecodeArgs& a, const S
 // features).  Output rows are the launch's (token, head) pairs in memory
 // order, so a block's rows may belong to several requests and no block is
 // launched for a row that a request does not have.  The sixteen waves are
-// dealt to the rows, W = 16 / kR each.  Every load of the first round goes out
-// before any wait: the rows' partials' (m, l) (thread per partial), the
-// partial rows (wave wr of a row: partials wr, wr + W, ..., lane: four rotated
-// features) and, where a thread needs only 16 of them, the block's columns of
-// R_v^T (else they are fetched under the exchange of the row sums).  The block
+// dealt to the rows, W = 16 / kR each.  The first round's loads: where a thread
+// needs only 16 of them, the block's columns of R_v^T (else they are fetched
+// under the exchange of the row sums); the rows' items, if there are several;
+// then the rows' partials' (m, l) (thread per partial) and the partial rows
+// (wave wr of a row: partials wr, wr + W, ..., lane: four rotated features).
+// The items are waited for with what went out before them, and the compiled
+// code, which has a branch around each partial row, waits once more after the
+// first of those: three memory round trips (two for one request).  The block
 // LSE-combines each row over all 256 rotated features, normalises it,
 // multiplies it by its columns of R_v^T in fp32 (chunks of rotated features
 // per wave, added in chunk order) and writes fp32 or bf16 (RNE).
@@ -1975,7 +1981,7 @@ __global__ __launch_bounds__(kRotThreads) void paged_decode_merge_rotate_kernel(
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = w % W;
 
-  // ---- every load of the first round ----
+  // ---- the first round's loads ----
   float rv[FK];
   const int col = CW == 1 ? lane : 64 * (w % CW) + lane;
   const float* rcol = rot_t + (int64_t)(FK * (w / CW)) * kHeadDim + 64 * CW * qd + col;

@@ -6,8 +6,9 @@
 // the 256x256 rotation's output features for all of them on MFMA (bf16 hi + lo
 // split of R, two passes); the values change hands through LDS, after which a
 // row of 16 lanes holds a vector and everything that concerns it stays in the
-// row.  The pre-rotated entry has one wavefront to 32 tokens, lane l holding
-// features 128 (l >> 5) .. +127 of token l & 31.
+// row.  The pre-rotated entry, and the kernel of large writes without a window
+// (prefers_ring), have one wavefront to 32 tokens, lane l holding features 128
+// (l >> 5) .. +127 of token l & 31.
 //
 // Clip threshold (the idx-th smallest |x| of a vector, i.e. its kk-th largest
 // with kk = 256 - idx) without sorting: a 64-bucket histogram of |x| keyed on
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(256) void quant_write_prerotated_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Fused entry: bf16 input, rotation on MFMA.
+// Rotation on MFMA of bf16 rows.
 //
 // Rotation operand (prepared once per layer by oscar_rotation_operand):
 //   op[m][p][T][lane][u] (bf16), m = 16-row K step, p = 0 hi / 1 lo split,
@@ -301,12 +302,15 @@ __global__ __launch_bounds__(256) void quant_write_prerotated_kernel(
 //     f = 128*((r >> 2) & 1) + 16*T + 4*(r >> 3) + (r & 3), r = lane & 31
 //   so that accumulator register i of tile T in lane l is feature
 //   128*(l >> 5) + 16*T + i of token (l & 31) -- the per-lane layout above.
-// grid = (ceil(N / 128), Hk * 2), block = 256 (4 waves x 32 tokens; two
-// blocks per CU).  The 16 K-step chunks (16 KB each) stream through a 4-slot
-// LDS ring filled with buffer_load_dwordx4 ... lds: chunk m + 3 is requested
-// while chunk m is multiplied, into the slot chunk m - 1 left.  Each K step
-// issues the 8 tiles' hi passes, then their lo passes, so no MFMA waits on the
-// previous.
+// Two ways to multiply by it: eight waves of a workgroup take a tile T each for
+// the same 32 rows and read their fragments straight from L2 (fused_write and
+// rotate_operands below); or four waves take all tiles for 32 rows each
+// (rotate_tile: quant_write_ring_kernel and rotate_rows_kernel, block = 256,
+// two blocks per CU), the 16 K-step chunks (16 KB each) streaming through a
+// 4-slot LDS ring filled with buffer_load_dwordx4 ... lds: chunk m + 3 is
+// requested while chunk m is multiplied, into the slot chunk m - 1 left, and
+// each K step issues the 8 tiles' hi passes, then their lo passes, so that no
+// MFMA waits on the previous.
 // ---------------------------------------------------------------------------
 constexpr int kFusedWaves = 4;
 constexpr int kChunkBytes = 2 * 8 * 64 * 16;   // one K step: 2 passes x 8 tiles x 64 lanes x 16 B
@@ -560,12 +564,14 @@ __device__ __forceinline__ void store_v_images(const Value& value, int64_t seat_
 // Writes up to 8K tokens are bound by one workgroup's latency, larger ones by
 // the products (two bf16 passes, 28 us for 65536 tokens at the rate of a
 // large library product) beside the selection's vector instructions, which a
-// CU's four workgroups overlap.  With 128 tokens to a workgroup of four
+// CU's workgroups overlap: four of them (64 registers), two where the write
+// shares a launch with the prefill operands (106).  With 128 tokens to a workgroup of four
 // wavefronts, each with 32 tokens of its own and R through an LDS ring, 3001
 // tokens took 29 us with the window (their selection 10, its image 7), 1052
 // of a mixed step 36, 9256 29 and 65536 without one 71; this takes 11, 15, 20
-// and 64.  64 tokens to a workgroup (half the reading of R): 17, -, 25, 68.
-// 33 KB, so that four workgroups share a CU: the operands' rows [k-step][row ^
+// and 64 (a write of that size takes the ring kernel, see prefers_ring).  64
+// tokens to a workgroup (half the reading of R): 17, -, 25, 68.
+// 33 KB, so that four workgroups fit a CU: the operands' rows [k-step][row ^
 // k-step, half] until the products are done, then the rotated values, in a
 // wave's share of which its selection works once the wave has read them.
 struct FusedWriteLds {
@@ -763,14 +769,16 @@ __global__ __launch_bounds__(kFwThreads, 8) void quant_write_fused_kernel(FusedW
 }
 
 // Rows rotated on MFMA: out = in @ R for rows of D = 256 features (the
-// prefill route's q / k / v rotations and its output's R_v^T,
-// oscar_ascend/backend.py:392-413).  in: bf16 (an exact operand) or fp32
+// reference's q / k / v rotations and R_v^T around its dense read,
+// oscar_ascend/backend.py:392-413).  An entry for callers who rotate rows of
+// their own: the prefill read here rotates in rotate_operands and
+// prefill_output_kernel.  in: bf16 (an exact operand) or fp32
 // (its bf16 high and low parts); R: the operand's bf16 high and low parts;
 // fp32 accumulation (about 2^-16 of each product); out: fp32, or bf16
 // rounded to nearest even.
 // grid = ceil(rows / 128), block = 256 (4 waves x 32 rows): lane l takes row
 // (l & 31) of its wave, input and output features 128 (l >> 5) .. +127, and
-// the operand streams through the fused kernel's 4-slot LDS ring.  A bf16
+// the operand streams through the 4-slot LDS ring.  A bf16
 // input's first half (K steps 0-7) is requested before the ring and its
 // second half during step 4; an fp32 input (twice the registers) comes in
 // quarters, the first before the ring and quarter q (steps 4q .. 4q + 3)
@@ -1099,7 +1107,8 @@ __global__ __launch_bounds__(512, 4) void rotate_operands_kernel(RotateOperandAr
 // A step's bulk write and its prefill operands in one launch: neither reads
 // what the other writes, and neither fills the GPU up to some thousands of
 // tokens (3001: 11 + 15 us one after the other, 18.5 together; 1052 of a mixed
-// step 15 + 8 and 16.4; 9256 20 + 38 and 50).
+// step 15 + 8 and 16.4; 9256 20 + 38 and 50).  Both halves run with the
+// operands' 106 registers, two workgroups a CU.
 __global__ __launch_bounds__(512, 4) void write_operands_kernel(FusedWriteArgs w, RotateOperandArgs a) {
   __shared__ union Lds {
     FusedWriteLds w;
