@@ -1158,18 +1158,26 @@ int check_cache_args(CacheArgs& c) {
   return kOk;
 }
 
-// Whether a write of that many 128-token workgroups takes the ring kernel: its
-// last round is full to a sixteenth, or there are more than 3 1/8 rounds, which
-// a partial last one no longer decides.  us, ring against tile kernel, by rounds
-// (one kv head): 0.875 31.9 / 31.0, 0.94 32.6 / 33.9, 1 33.4 / 34.7, 1.01 46 / 37,
-// 1.5 66 / 51, 1.75 68 / 58, 2 61-72 (by process) / 65.5, 2.25 86 / 76, 2.75 95 /
-// 93, 3 100.7 / 100.3, 3.06 105 / 103, 3.19 106.7 / 107.3, 3.5 112.6 / 117.3, 5.5
-// 169 / 180, 8 236 / 260; two heads 1 33.2 / 34.5, 3.25 112 / 110, 3.5 115 / 117;
-// four 3.25 111 / 109, 4 131.6 / 132.5.
-bool prefers_ring(int64_t workgroups) {
-  const int64_t last = workgroups % kRingRound;
-  return workgroups > 3 * kRingRound + kRingRound / 8 ||
-         (workgroups >= kRingRound && (last == 0 || last > kRingRound - kRingRound / 16));
+// Whether a write of that many 128-token workgroups takes the ring kernel, whose
+// rounds of kRingRound cost the same however full the last one is: where that
+// one is 13/16 (the first round) or 15/16 full (the second), and from 2 11/16
+// rounds on, where a partial last one no longer decides.  us, ring against tile
+// kernel, by rounds (one kv head): 0.5 23.9 / 23.0, 0.75 32.7 / 31.2, 0.81 32.0 /
+// 33.1, 0.875 32.5 / 34.4, 0.94 33.3 / 38.2, 0.98 34.0 / 38.4, 1.02 53.6 / 40.9,
+// 1.5 65.9 / 55.5, 1.75 67.4 / 60.7, 1.875 68.0 / 65.2, 1.92 68.7 / 68.0, 2.03 74.5
+// / 72.5, 2.5 84.9 / 83.3, 2.75 87.8 / 91.5, 2.94 88.0 / 96.8, 3.06 95.1 / 102.3,
+// 3.5 112.6 / 117.3, 5.5 169 / 180, 8 236 / 260; two heads 0.94 33.7 / 37.8, 1.875
+// 64.4 / 65.4, 2.75 88.4 / 90.8; four 0.94 33.5 / 38.5, 1.875 67.3 / 64.6, 2.75 90.4
+// / 90.4.  A write that can share its launch with a step's prefill operands
+// (shares) does so up to those 2 11/16 rounds: a whole step of four kv heads
+// without a window 240 us with the ring kernel and 227 with the shared launch at
+// 0.82 rounds, 297 / 287 at 1, 815 / 810 at 2, 1427 / 1443 at 2.8; of one kv head
+// 610 / 599 at 0.92.
+bool prefers_ring(int64_t workgroups, bool shares) {
+  const int64_t sixteenth = kRingRound / 16;
+  if (workgroups >= 43 * sixteenth) return true;
+  return !shares && ((workgroups >= 13 * sixteenth && workgroups <= kRingRound) ||
+                     (workgroups > 31 * sixteenth && workgroups <= 2 * kRingRound));
 }
 
 std::atomic<uint64_t> g_ring_lds_set{0};   // dynamic-LDS attribute set, one bit per device
@@ -1364,7 +1372,7 @@ int quant_write_impl(const void* key_bf16, const void* value_bf16, int64_t num_t
                           (int32_t)((num_tokens + kFwTokens - 1) / kFwTokens), num_kv_heads};
   const int64_t ring_blocks = (num_tokens + kFusedWaves * kTokPerWave - 1) / (kFusedWaves * kTokPerWave);
   const int64_t ring_wgs = ring_blocks * 2 * num_kv_heads;
-  if (w.rows == 0 && prefers_ring(ring_wgs)) {
+  if (w.rows == 0 && prefers_ring(ring_wgs, later != nullptr)) {
     FusedWriteArgs rw = fw;
     rw.token_blocks = (int32_t)ring_blocks;
     if (ring_wgs > INT32_MAX) return kErrInvalidArgument;

@@ -2,8 +2,8 @@
 kernel writes, from the same products in the same order): every byte equal.
 
 Sizes around the 128-token workgroups' rounds of 512, where the kernel changes:
-the last round a sixteenth short of full, whole, one workgroup over, and more
-than 3 1/8 rounds, with whole and partial last workgroups."""
+13/16 of a round, a whole round, one workgroup over, two rounds but a sixteenth,
+and 2 11/16 rounds, with whole and partial last workgroups."""
 import pytest
 import torch
 
@@ -14,8 +14,8 @@ pytestmark = pytest.mark.gpu
 D = 256
 
 
-@pytest.mark.parametrize("N,hk", [(30720, 1), (30721, 1), (32768, 1), (32769, 1), (16384, 2), (16400, 2), (102400, 1),
-                                  (102401, 1), (26000, 4)])
+@pytest.mark.parametrize("N,hk", [(26496, 1), (26497, 1), (6656, 4), (30720, 1), (32768, 1), (32769, 1), (16384, 2),
+                                  (16400, 2), (63488, 1), (63489, 1), (87936, 1), (87937, 1), (102401, 1), (26000, 4)])
 @pytest.mark.parametrize("clip", [(245, 235), (-1, -1)])
 def test_bytes_equal_the_parts(device, N, hk, clip):
     bs = 128
