@@ -160,7 +160,8 @@ class OscarAttentionBackendImpl:
             rv = get_layer_rotation(cfg.v_rotation_path, layer.layer_name, self.head_size, device, mode="v", strict=True)
             layer._oscar_rots = (rk, rv)
         rk, rv = layer._oscar_rots
-        if rk.device != torch.device(device) or rk.dtype != torch.float32:
+        if rk.device != torch.device(device) or rk.dtype != torch.float32 \
+                or not rk.is_contiguous() or not rv.is_contiguous():
             rk = rk.to(device=device, dtype=torch.float32).contiguous()
             rv = rv.to(device=device, dtype=torch.float32).contiguous()
             layer._oscar_rots = (rk, rv)

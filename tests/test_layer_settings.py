@@ -37,3 +37,18 @@ def test_layer_half_is_rebuilt_when_a_setting_changes(change):
     assert (a.clip_index_k, a.clip_index_v, a.sink_eff, a.recent, a.scale) == (
         quant.clip_index(cfg.k_clip_ratio, D), quant.clip_index(cfg.v_clip_ratio, D), cfg.sink_tokens // 32 * 32,
         cfg.recent_tokens, impl.scale)          # (powers of two: exact in the struct's float)
+
+
+def test_rotations_of_any_stride(monkeypatch):
+    # a transposed view, as the fp32 products of the general route take it
+    impl = make_impl(2, 1, sink=0, recent=0)
+    caches = [torch.zeros(4, 32, 1, D, dtype=torch.int8) for _ in range(2)]
+    impl._set_caches(caches)
+    monkeypatch.setattr(quant, "rotation_operand", lambda R: R.contiguous())
+    rk, rv = synthetic.rotations(D, 1)
+    layer = NS(layer_name="model.layers.0.self_attn.attn", _oscar_rots=(rk.t(), rv.t()))
+    dev = torch.device("cpu")
+    half = impl._mtp_layer(layer, caches, dev)
+    for got, want in zip(half.tensors, (rk.t(), rv.t(), rv)):
+        assert got.is_contiguous() and torch.equal(got, want)
+    assert impl._mtp_layer(layer, caches, dev) is half
