@@ -256,7 +256,8 @@ int oscar_prefill_continuation(const float* q_rot, const float* k_new, const flo
 
 /* The same read with its work spread over the whole GPU: the row blocks (256
  * (token, head) rows) and their key blocks are cut into equal shares, and row
- * blocks that a cut runs through are merged from fp32 partials.  workspace:
+ * blocks that a cut runs through are merged from fp32 partials (few rows or
+ * keys are read by whole row blocks all the same).  workspace:
  * device memory, 16-byte aligned, of at least oscar_prefill_workspace_bytes(num_new, Hq, Hk,
  * cached_len) bytes (the new tokens' MFMA operands and the partials); its
  * contents need no initialisation and mean nothing after the call.

@@ -20,7 +20,9 @@
 // long as its key blocks, form one line of units; every workgroup (one per CU)
 // takes an equal share of it, whatever row blocks that cuts.  A row block that
 // lies in one share is finished there; of a cut one each share writes fp32
-// partials (m, l, unnormalised O), which prefill_merge_kernel combines.
+// partials (m, l, unnormalised O), which prefill_merge_kernel combines.  Reads of
+// fp32 rows without a workspace, or of few key blocks, take whole row blocks
+// instead (prefers_rows, prefers_rows_shares).
 //
 // A block is two phases of a wavefront:
 //   M (matrix): O^T += V^T P^T of block i - 1 and S^T = K Q^T of block i (16
@@ -46,6 +48,7 @@
 // takes about 5 and 2.5 us: unit, pages and Q^T, first words, first tile; and
 // the partial.  One request, 6 heads, D = 256, this kernel: 9256 tokens over
 // 15360 1988 -> 1200 us, 77 over 20011 1016 -> 34 us, 3001 alone 170 -> 50 us.
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -1308,14 +1311,21 @@ __global__ __launch_bounds__(256) void convert_operands_kernel(ConvertArgs a) {
 std::atomic<uint64_t> g_lds_set[2] = {{0}, {0}};   // dynamic-LDS attribute set, one bit per device
 
 // ---- host side ----
-int64_t host_head_units(int64_t n_new, int64_t cached, int64_t group) {
-  const int64_t rows = n_new * group, nrb = (rows + kTileRows - 1) / kTileRows, nh = (cached + kBlk - 1) / kBlk;
-  int64_t n = nrb * (nh + kPieceCost);
+
+// Row blocks of `tile` rows of one kv head, and all their key blocks.
+int64_t host_row_blocks(int64_t n_new, int64_t group, int tile) { return (n_new * group + tile - 1) / tile; }
+int64_t host_key_blocks(int64_t n_new, int64_t cached, int64_t group, int tile) {
+  const int64_t rows = n_new * group, nrb = host_row_blocks(n_new, group, tile);
+  int64_t n = nrb * ((cached + kBlk - 1) / kBlk);
   for (int64_t rb = 0; rb < nrb; ++rb) {
-    const int64_t last = ((rb + 1) * kTileRows < rows ? (rb + 1) * kTileRows : rows) - 1;
+    const int64_t last = ((rb + 1) * tile < rows ? (rb + 1) * tile : rows) - 1;
     n += last / group / kBlk + 1;
   }
   return n;
+}
+
+int64_t host_head_units(int64_t n_new, int64_t cached, int64_t group) {
+  return host_row_blocks(n_new, group, kTileRows) * kPieceCost + host_key_blocks(n_new, cached, group, kTileRows);
 }
 
 // Units per workgroup: one round of kShares workgroups, of at least kMinShare
@@ -1445,6 +1455,59 @@ int launch_shares(PrefillArgs& a, int64_t& wgs, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
+// A read of one request by whole row blocks of `tile` rows, in key blocks walked
+// one after the other: the last row block's, and a CU's mean of all of them.
+struct WholeLength {
+  double last, mean;
+  int64_t workgroups;
+};
+WholeLength whole_length(const PrefillArgs& a, int tile) {
+  const PrefillItem& it = a.items[0];
+  const int64_t last = ((int64_t)it.cached + kBlk - 1) / kBlk + (it.n_new - 1) / kBlk + 1;
+  const int64_t all = host_key_blocks(it.n_new, it.cached, a.group, tile) * a.num_kv_heads;
+  return WholeLength{(double)last, (double)all / kShares, host_row_blocks(it.n_new, a.group, tile) * a.num_kv_heads};
+}
+
+// Whether that read takes row blocks of 128 rows (prefill_rows.hip), not of 256
+// (prefill_kernel<false>): of history, a key block of the latter takes a third
+// longer for twice the rows; new tokens' fp32 rows are fetched ahead by the
+// former only.  us, 128 against 256 rows: 6 heads, 17 tokens over 100 19.4 / 20.2,
+// 100 over 800 56 / 69, 1500 alone 88 / 128, 6000 alone 305 / 462; 16 heads of two
+// kv heads, 3000 over 2400 379 / 367; 64 of eight, 600 over 400 106 / 88, 1000
+// alone 129 / 97; 32 heads, 3000 over 2400 636 / 500.
+bool prefers_rows(const PrefillArgs& a) {
+  const WholeLength w1 = whole_length(a, kPrefillSmallTile), w2 = whole_length(a, kTileRows);
+  return 0.85 * std::max(w1.last, 1.3 * w1.mean) < std::max(w2.last, 1.3 * w2.mean);
+}
+
+// Whether a read of one request with a workspace takes row blocks of 128 rows
+// whole all the same: one launch instead of three, without operands and
+// partials.  In us beside what both take: 1.6 a key block (of every round of the
+// CUs where several kv heads are one after the other) against 1.6 a unit of a
+// share, 0.25 a row block (operands, partials) and 10 for the launches.  Of 423
+// shapes it picks the slower one by 13 % at most, by 0.1 on average.  us, whole
+// against shares: 6 heads, 17 tokens alone 14.1 / 22, over 100 19.4 / 24.7, over 400
+// 35 / 26.6, 200 alone 23 / 29.5, over 300 39 / 32; 32 heads, 1500 alone 91 / 108;
+// 64 of eight kv heads, 400 over 100 44 / 61, 600 over 400 106 / 92.
+bool prefers_rows_shares(const PrefillArgs& a) {
+  const WholeLength w = whole_length(a, kPrefillSmallTile);
+  const int64_t rounds = a.num_kv_heads > 1 ? (w.workgroups + kShares - 1) / kShares : 1;
+  const int64_t rbs = host_row_blocks(a.items[0].n_new, a.group, kTileRows) * a.num_kv_heads;
+  return 1.6 * std::max(w.last * (double)rounds, 1.15 * w.mean) <
+         10. + 1.6 * (double)plan_share(a.units) + 0.25 * (double)rbs;
+}
+
+// That read (prefill_rows.hip).
+int launch_rows(const PrefillArgs& a, const float* q_rot, const float* k_new, const float* v_new, float* out,
+                hipStream_t stream) {
+  const PrefillItem& it = a.items[0];
+  return launch_prefill_rows(PrefillRows{q_rot, k_new, v_new, it.n_new, a.num_heads, a.num_kv_heads, a.group,
+                                         a.k_cache, a.v_cache, a.k_page, a.k_tok, a.k_head, a.v_page, a.v_tok,
+                                         a.v_head, a.block_size, a.bs_div, a.rows_div, a.num_pages, a.bt, a.bt_cols,
+                                         it.cached, a.stage_k, a.stage_v, a.owner, a.stage_rows, a.scale_log2, out},
+                             stream);
+}
+
 // Few row blocks in many shares: a workgroup per row merges them.
 bool many_pieces(const PrefillArgs& a, int64_t wgs) { return launch_row_blocks(a) * kMergeManyPieces <= wgs; }
 
@@ -1522,6 +1585,7 @@ extern "C" int oscar_prefill_continuation_split(
   add_item(a, ops, num_new, cached_len, 0, 0);
   const Layout w = workspace_layout(ops.tokens, ops.tiles, a.units, num_heads, num_kv_heads, false);
   if (workspace_size < w.total) return kErrWorkspaceTooSmall;
+  if (prefers_rows_shares(a)) return launch_rows(a, q_rot, k_new, v_new, out, stream);
   ConvertArgs c{q_rot, k_new, v_new, num_heads, num_kv_heads, PrefillOperands{}, 0, 0, ops};
   bind_workspace(a, c.o, w, static_cast<uint8_t*>(workspace));
   a.out = out;
@@ -1558,6 +1622,7 @@ extern "C" int oscar_prefill_continuation(
   a.out = out;
   OperandItems ops{};
   add_item(a, ops, num_new, cached_len, 0, 0);
+  if (prefers_rows(a)) return launch_rows(a, q_rot, k_new, v_new, out, stream);
   const int64_t rows = (int64_t)num_new * a.group;
   const dim3 grid((unsigned)((rows + kTileRows - 1) / kTileRows), (unsigned)num_kv_heads);
   if (set_dynamic_lds(reinterpret_cast<const void*>(prefill_kernel<false>), (int)kPrefillLds, g_lds_set[0]) != kOk)

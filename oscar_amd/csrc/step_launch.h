@@ -75,6 +75,34 @@ int prefill_rotated(
     void* out_bf16, void* workspace, size_t workspace_size, const FusedWriteArgs* write, bool check_only,
     hipStream_t stream);
 
+// The read of one request over its fp32 rows by whole row blocks of
+// kPrefillSmallTile rows (prefill_rows.hip); the arguments have been checked.
+constexpr int kPrefillSmallTile = 128;
+struct PrefillRows {
+  const float* q;        // [N][Hq][D]
+  const float* k_new;    // [N][Hk][D]
+  const float* v_new;
+  int32_t n_new;
+  int32_t num_heads, num_kv_heads, group;
+  const uint8_t* k_cache;
+  const uint8_t* v_cache;
+  int64_t k_page, k_tok, k_head, v_page, v_tok, v_head;
+  int32_t block_size;
+  FastDiv bs_div;        // block_size
+  FastDiv rows_div;      // stage_rows (1 without an arena)
+  int64_t num_pages;
+  const int32_t* bt;     // the request's block-table row
+  int32_t bt_cols;
+  int64_t cached;        // C
+  const float* stage_k;
+  const float* stage_v;
+  const int64_t* owner;
+  int32_t stage_rows;
+  float scale_log2;
+  float* out;
+};
+int launch_prefill_rows(const PrefillRows& a, hipStream_t stream);
+
 // oscar_step_write, with the request layout in host arrays, or
 // (layout_on_device) in device arrays that are read on the stream.
 int step_write(bool layout_on_device, const void* query_bf16, int64_t query_token_stride, const void* key_bf16,
