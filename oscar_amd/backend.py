@@ -37,6 +37,18 @@ from .format import HEAD_DIM, K_IDX_OFF, VALUES_PER_BYTE, check_d
 from .kernels import _lib, decode, prefill, quant, staging, step
 from .rotation import get_layer_rotation
 
+# (token, head) rows of a step that the one-call forwards rotate in fp32 by
+# themselves, each workgroup reading R for a few of them: of more rows torch's
+# matrix products are quicker, whatever the copies around them.  us, one call
+# against the general route: DecodeOnly over 1500 tokens, 16 heads x 250 109 /
+# 140, 64 x 60 141 / 139, 12 x 500 287 / 265, 32 x 250 155 / 143, 128 x 250 531 /
+# 338; over 100 tokens, 16 x 500 156 / 184, 128 x 60 108 / 95, 32 x 500 247 / 187.
+# Short requests beside a long one: 25600 rows of 32 heads 453 / 987, of 16 500 /
+# 612, 30720 of 32 527 / 518, 51200 813 / 654, 61440 of 64 1130 / 806.
+DECODE_ONLY_ROWS = 4096
+DECODE_ONLY_SHORT_HISTORY = 512        # up to which twice as many rows are quicker in one call
+STEP_SHORT_ROWS = 32768
+
 
 def metadata_batch_lists(attn_metadata) -> tuple[list, list]:
     """(query_start_loc, seq_lens) as host lists (backend.py:25-55).
@@ -359,7 +371,8 @@ class OscarAttentionBackendImpl:
         """The whole forward of a bf16 step with long requests in one library
         call (write, window, paged read of the short requests, prefill read
         of the long ones).  Returns False (nothing done) when the step's
-        types, shapes or layout need the general route."""
+        types, shapes or layout need the general route, or its short requests'
+        rows are quicker there."""
         cfg = self._oscar
         N = attn_metadata.num_actual_tokens
         num_tokens = query.shape[0]
@@ -375,6 +388,9 @@ class OscarAttentionBackendImpl:
         slots, bt = attn_metadata.slot_mapping, attn_metadata.block_tables
         qsl, seqs = metadata_batch_lists(attn_metadata)
         B = len(qsl) - 1
+        shorts = sum(n for n in (b - a for a, b in itertools.pairwise(qsl)) if n <= limit)
+        if shorts * self.num_heads > STEP_SHORT_ROWS:
+            return False
         if B < 1 or len(seqs) < B or qsl[0] != 0 or qsl[-1] != N or not 0 <= limit <= decode.MAX_QUERY_LEN \
                 or any(not 0 <= b - a <= s for (a, b), s in zip(itertools.pairwise(qsl), seqs)) \
                 or slots.ndim != 1 or slots.shape[0] < N or bt.ndim != 2 or bt.shape[0] < B or bt.shape[1] == 0:
@@ -424,7 +440,7 @@ class OscarAttentionBackendImpl:
         query rotation, read, and R_v^T with the cast in its merge.  Returns
         False (nothing done) for what takes the general route: other dtypes,
         small pages, an arena that no step has written yet, a query count that
-        route refuses."""
+        route refuses, more rows than the library rotates quickly."""
         cfg = self._oscar
         N = query.shape[0]
         if query.dtype != torch.bfloat16 or output.dtype != torch.bfloat16 or output.device != query.device \
@@ -433,8 +449,12 @@ class OscarAttentionBackendImpl:
             return False
         if cfg.window_enabled and not getattr(layer, "_oscar_stage_ready", False):
             return False
+        rows = N * self.num_heads
+        if rows > 2 * DECODE_ONLY_ROWS:
+            return False
         qsl, seqs = metadata_batch_lists(attn_metadata)
-        if N != len(seqs) or any(b - a != 1 for a, b in itertools.pairwise(qsl[:N + 1])):
+        if N != len(seqs) or rows > DECODE_ONLY_ROWS and max(seqs) > DECODE_ONLY_SHORT_HISTORY \
+                or any(b - a != 1 for a, b in itertools.pairwise(qsl[:N + 1])):
             return False
         dev = query.device
         return step.decode_only_forward(self._mtp_layer(layer, kv_cache, dev), query, attn_metadata.block_tables,
