@@ -420,10 +420,11 @@ class OscarAttentionBackendImpl:
             rots = self._layer_rots(layer, dev)
         arena = (layer._oscar_stage_k, layer._oscar_stage_v, layer._oscar_slot_owner, layer._oscar_stage_kimg,
                  layer._oscar_stage_vimg) if cfg.window_enabled else (None,) * 5
-        ml, was = getattr(layer, "_oscar_mtp", None), getattr(layer, "_oscar_mtp_settings", None)
+        ml = getattr(layer, "_oscar_mtp", None)
         settings = (cfg, self.scale, self.num_heads, self.num_kv_heads)
         rvT = getattr(layer, "_oscar_rvT", None)
-        if ml is not None and was == settings and ml.bound_to(rots[0], rots[1], rvT, self.key_cache, self.value_cache, *arena):
+        if ml is not None and ml.settings == settings and ml.bound_to(rots[0], rots[1], rvT, self.key_cache,
+                                                                      self.value_cache, *arena):
             return ml
         rk, rv = self._layer_rots(layer, dev)
         D = self.head_size
@@ -432,7 +433,8 @@ class OscarAttentionBackendImpl:
                            self.num_kv_heads, quant.clip_index(cfg.k_clip_ratio, D),
                            quant.clip_index(cfg.v_clip_ratio, D), self.scale,
                            arena if cfg.window_enabled else None, (cfg.sink_tokens // bs) * bs, cfg.recent_tokens)
-        layer._oscar_mtp, layer._oscar_mtp_settings = ml, settings
+        ml.settings = settings              # (with its half: another thread sees both or neither)
+        layer._oscar_mtp = ml
         return ml
 
     def _decode_only_step(self, layer, query, kv_cache, attn_metadata, output) -> bool:

@@ -120,9 +120,10 @@ class MtpLayer:
     R_v^T (fp32 [D, D]), the paged caches and the window arena (stage =
     (stage_k, stage_v, owner, k_image, v_image) or None).  Holds the tensors
     it points at; ``bound_to`` says whether the same tensors are still the
-    layer's (identity, so a rebound cache or replaced rotation rebuilds)."""
+    layer's (identity, so a rebound cache or replaced rotation rebuilds);
+    ``settings``: what its keeper compares beside them."""
 
-    __slots__ = ("tensors", "ids", "args", "ref", "num_heads", "num_kv_heads", "head_size")
+    __slots__ = ("tensors", "ids", "args", "ref", "num_heads", "num_kv_heads", "head_size", "settings")
 
     def __init__(self, R_k, R_v, R_v_t, k_cache, v_cache, num_heads: int, num_kv_heads: int, clip_k: int,
                  clip_v: int, scale: float, stage=None, sink_eff: int = 0, recent: int = 0):
@@ -150,6 +151,7 @@ class MtpLayer:
         self.tensors = (R_k, R_v, R_v_t, k_cache, v_cache) + arena
         self.ids = tuple(map(id, self.tensors))     # stable: the tensors are held here
         self.num_heads, self.num_kv_heads, self.head_size = num_heads, num_kv_heads, D
+        self.settings = None
         ptrs = [_lib.ptr(t) for t in self.tensors]
         self.args = MtpLayerArgs(*ptrs[:5], pages, *kst, *vst, bs, num_heads, num_kv_heads, D, clip_k, clip_v,
                                  float(scale), rows, *ptrs[5:], int(sink_eff), int(recent))
