@@ -1497,6 +1497,8 @@ bool prefers_rows_shares(const PrefillArgs& a) {
          10. + 1.6 * (double)plan_share(a.units) + 0.25 * (double)rbs;
 }
 
+constexpr size_t kRowsWorkspace = 16;   // that such a read asks for (it uses none; zero means a refused shape)
+
 // That read (prefill_rows.hip).
 int launch_rows(const PrefillArgs& a, const float* q_rot, const float* k_new, const float* v_new, float* out,
                 hipStream_t stream) {
@@ -1559,8 +1561,14 @@ using namespace oscar;
 extern "C" size_t oscar_prefill_workspace_bytes(int32_t num_new, int32_t num_heads, int32_t num_kv_heads,
                                                 int64_t cached_len) {
   if (num_new <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || cached_len < 0) return 0;
-  const int64_t units = host_head_units(num_new, cached_len, num_heads / num_kv_heads) * num_kv_heads;
-  return workspace_layout(num_new, (num_new + kBlk - 1) / kBlk, units, num_heads, num_kv_heads, false).total;
+  if (cached_len + num_new >= ((int64_t)1 << 31)) return 0;
+  PrefillArgs a{};
+  a.num_kv_heads = num_kv_heads;
+  a.group = num_heads / num_kv_heads;
+  OperandItems ops{};
+  add_item(a, ops, num_new, cached_len, 0, 0);
+  if (prefers_rows_shares(a)) return kRowsWorkspace;
+  return workspace_layout(ops.tokens, ops.tiles, a.units, num_heads, num_kv_heads, false).total;
 }
 
 extern "C" int oscar_prefill_continuation_split(
@@ -1583,9 +1591,11 @@ extern "C" int oscar_prefill_continuation_split(
     return kErrInvalidArgument;
   OperandItems ops{};
   add_item(a, ops, num_new, cached_len, 0, 0);
+  if (prefers_rows_shares(a))
+    return workspace_size < kRowsWorkspace ? (int)kErrWorkspaceTooSmall
+                                           : launch_rows(a, q_rot, k_new, v_new, out, stream);
   const Layout w = workspace_layout(ops.tokens, ops.tiles, a.units, num_heads, num_kv_heads, false);
   if (workspace_size < w.total) return kErrWorkspaceTooSmall;
-  if (prefers_rows_shares(a)) return launch_rows(a, q_rot, k_new, v_new, out, stream);
   ConvertArgs c{q_rot, k_new, v_new, num_heads, num_kv_heads, PrefillOperands{}, 0, 0, ops};
   bind_workspace(a, c.o, w, static_cast<uint8_t*>(workspace));
   a.out = out;

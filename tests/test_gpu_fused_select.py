@@ -37,10 +37,10 @@ def test_bytes_with_an_exact_rotation(device, kind, ratios, n, hk):
     _check(device, kind, ratios, n, hk)
 
 
-# The kernel of whole rounds of 128-token workgroups: exactly one round with a
-# remainder in the last workgroup, the fewest workgroups of a round that take
-# it, and one less (the kernel above).
-@pytest.mark.parametrize("n,hk", [(32765, 1), (30721, 1), (30720, 1), (16300, 2)])
+# The kernel of 128-token workgroups: exactly one round of them with a remainder
+# in the last, most of a round, the fewest that take it, and one less (the kernel
+# above).
+@pytest.mark.parametrize("n,hk", [(32765, 1), (30721, 1), (30720, 1), (16300, 2), (26497, 1), (26496, 1)])
 def test_bytes_of_whole_rounds(device, n, hk):
     _check(device, "ties" if n % 2 else "range", (0.96, 0.5), n, hk)
 

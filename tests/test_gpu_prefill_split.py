@@ -4,7 +4,9 @@ against the oracle's dense read in fp32 (bar of the prefill kernel:
 the bf16 outputs of whole requests after R_v^T likewise).
 
 A workgroup takes 256 (token, head) rows and walks 32-key blocks; equal shares
-of all row blocks' key blocks may cut a row block anywhere.
+of all row blocks' key blocks may cut a row block anywhere.  (Reads of fp32 rows
+with few rows or keys take whole blocks of 128 rows: tests/test_gpu_prefill_whole.py
+has both at their edges.)
 """
 import ctypes
 

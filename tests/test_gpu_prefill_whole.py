@@ -16,12 +16,14 @@ D = 256
 
 
 # 128-row blocks that are short of, exactly and over full (21 / 22 tokens of group
-# 6, 128 / 129 of group 1, 8 of group 16); several kv heads; 128-row blocks of
-# more than a round of the CUs, where 256 rows are taken without a workspace (128
-# heads of one kv head); histories of as many key blocks as whole row blocks are
-# read with a workspace, and of more, which shares are.
-@pytest.mark.parametrize("hq,hk,new", [(6, 1, 21), (6, 1, 22), (1, 1, 128), (1, 1, 129), (16, 1, 8), (16, 2, 33),
-                                       (4, 4, 200), (64, 8, 40), (128, 1, 500)])
+# 6, 128 / 129 of group 1, 8 of group 16), and 256-row blocks (42 / 43, 256 / 257);
+# several kv heads; 128-row blocks of more than a round of the CUs, where 256 rows
+# are taken without a workspace (128 heads of one kv head, half a block at the
+# end); histories of as many key blocks as whole row blocks are read with a
+# workspace (none, two), and of more, which shares are.
+@pytest.mark.parametrize("hq,hk,new", [(6, 1, 21), (6, 1, 22), (6, 1, 42), (6, 1, 43), (1, 1, 128), (1, 1, 129),
+                                       (1, 1, 256), (1, 1, 257), (16, 1, 8), (16, 2, 33), (4, 4, 200), (64, 8, 40),
+                                       (128, 1, 501)])
 @pytest.mark.parametrize("hist", [0, 33, 900])
 @pytest.mark.parametrize("window", [False, True])
 def test_both_entries(device, hq, hk, new, hist, window):

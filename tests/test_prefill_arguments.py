@@ -10,7 +10,7 @@ from oscar_amd.kernels import _lib
 
 pytestmark = pytest.mark.skipif(torch.cuda.is_available(), reason="the addresses are host memory")
 D = 256
-OK, INVALID, LAUNCH, GEOMETRY = 0, -1, -4, -5
+OK, INVALID, SMALL, LAUNCH, GEOMETRY = 0, -1, -3, -4, -5
 
 
 @pytest.mark.parametrize("split", [False, True])
@@ -19,11 +19,12 @@ def test_accepted_and_refused(split):
     buf = torch.zeros(256, dtype=torch.uint8)
     at = (buf.data_ptr() + 15) & ~15
 
-    def call(new, cached=64, hq=2, hk=1, bs=32, cache=at, kst=(8192, 256, 256), vst=(8192, 256, 256), cols=4, ws=at):
+    def call(new, cached=64, hq=2, hk=1, bs=32, cache=at, kst=(8192, 256, 256), vst=(8192, 256, 256), cols=4, ws=at,
+             size=1 << 40):
         args = (at, at, at, new, hq, hk, D, cache, cache, bs, 64, *kst, *vst, at, cols, cached, None, None, None, 0,
                 ctypes.c_float(0.1), at)
         if split:
-            return lib.oscar_prefill_continuation_split(*args, ws, 1 << 40, None)
+            return lib.oscar_prefill_continuation_split(*args, ws, size, None)
         return lib.oscar_prefill_continuation(*args, None)
 
     assert call(20) == LAUNCH
@@ -38,3 +39,9 @@ def test_accepted_and_refused(split):
     assert call(0, cached=-1) == INVALID and call(0, hq=3, hk=2) == INVALID and call(-1) == INVALID
     if split:
         assert call(20, ws=at + 8) == INVALID
+        # as much scratch as is asked for: next to none where whole row blocks
+        # are read, partials and operands where shares are
+        for new, cached, most in ((20, 64, 256), (2000, 64, 1 << 28)):
+            need = lib.oscar_prefill_workspace_bytes(new, 2, 1, cached)
+            assert 0 < need <= most and call(new, cached, size=need) == LAUNCH and call(new, cached, size=need - 1) == SMALL
+        assert need > 1 << 20
