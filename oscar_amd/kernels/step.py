@@ -239,20 +239,15 @@ def mtp_step(qsl, seqs, num_tokens: int, slot_mapping, block_table, num_heads: i
 
 def _row_stride(x: torch.Tensor, N: int, features: int) -> int:
     """Elements between consecutive tokens of x read as [tokens][features]
-    rows with contiguous features (of one token, whose stride may be anything,
-    the features); -1 when x is not such a view."""
+    rows with contiguous features; -1 when x is not such a view."""
     shape, st = x.shape, x.stride()
     if shape[0] < N:
         return -1
     if len(shape) == 2:
-        rows = shape[1] == features and st[1] == 1
-    elif len(shape) == 3:
-        rows = shape[1] * shape[2] == features and st[2] == 1 and st[1] == shape[2]
-    else:
-        rows = False
-    if not rows:
-        return -1
-    return st[0] if N > 1 else features
+        return st[0] if shape[1] == features and st[1] == 1 else -1
+    if len(shape) == 3:
+        return st[0] if shape[1] * shape[2] == features and st[2] == 1 and st[1] == shape[2] else -1
+    return -1
 
 
 def mtp_forward(layer: MtpLayer, st: MtpStep, query, key, value, out, stream: int) -> torch.Tensor:
@@ -294,14 +289,19 @@ def decode_only_forward(layer: MtpLayer, query, block_table, seqs, out, stream: 
     rows do not hold Hq * D contiguous features each of their own."""
     B = len(seqs)
     hq, hk, D = layer.num_heads, layer.num_kv_heads, layer.head_size
+    # (of a single row the stride may be anything)
     os_ = _row_stride(out, B, hq * D)
+    if B == 1 and os_ >= 0:
+        os_ = hq * D
     if os_ < hq * D:
         return False
     if any(s < 0 for s in seqs) or block_table.ndim != 2 or block_table.shape[0] < B:
         raise ValueError("DecodeOnly needs a non-negative length and a block-table row per request")
     qs = _row_stride(query, B, hq * D)
     if qs < hq * D:
-        query, qs = _rows(query, B, hq * D)[0].contiguous(), hq * D
+        if B > 1 or qs < 0:
+            query = _rows(query, B, hq * D)[0].contiguous()
+        qs = hq * D
     if block_table.dtype != torch.int32 or block_table.device != query.device or block_table.stride(1) != 1:
         block_table = block_table.to(device=query.device, dtype=torch.int32).contiguous()
     seq_t = (_i32 * B)(*seqs)
